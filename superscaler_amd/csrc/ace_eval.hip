@@ -20,6 +20,7 @@
 
 #include "ace_edit_kernels.h"
 #include "ace_score_loop.h"
+#include "ace_spread.h"
 
 // Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans (the
 // layout ace_score_body's DEFER variant uses: [workgroup][stage][lane][ACE_WS_REC]).  Every GPU the library runs on holds
@@ -67,6 +68,26 @@ __global__ __launch_bounds__(BLOCK) void ace_score_kernel(const AceKernelArgs a)
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_score_body<BD, RANGED, WIN, DEFER, BLOCK, COLL>(a, lds_raw, 0u, (int)threadIdx.x, (long long)blockIdx.x, gridDim.x);
 }
+
+// Small batches: a plan (or single-stage query) per workgroup, see ace_spread.h.
+template <bool BD, bool RANGED, bool COLL>
+__global__ __launch_bounds__(kSpreadLanes) void ace_spread_kernel(const AceKernelArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    ace_spread_body<BD, RANGED, COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+}
+// Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has four workgroups
+// (1,024 plans), that of the kernels with a plan per lane not before 16,384; they cross between 4,096 and 16,384 plans,
+// earlier without stage records (the lane-per-plan kernel defers the stage tails there).  Measured, us per launch,
+// lane per plan -> plan per workgroup (launches back to back: 13 to 20 us is what the host needs for one):
+//   plain    315 ops:    1 plan  49 -> 13, 1,024  65 -> 16, 4,096  66 -> 45;  1,251 ops: 1  169 -> 26, 4,096  254 -> 118
+//   records  523 ops:    1 plan 117 -> 19, 1,024 312 -> 24, 4,096 321 -> 80, 16,384 322 -> 274 (315 ops: 147 -> 194)
+//   queries  523 ops:   64      163 -> 20, 1,024 189 -> 21, 4,096 194 -> 38, 16,384 169 -> 112 (315 ops: 106 -> 122)
+#ifndef ACE_SPREAD_MAX_PLAIN
+#define ACE_SPREAD_MAX_PLAIN 4096
+#endif
+#ifndef ACE_SPREAD_MAX_RECORDS
+#define ACE_SPREAD_MAX_RECORDS 8192
+#endif
 
 // ------------------------------------------------------------------------------------------
 // top-k: radix select on the order-preserving 64-bit image of the iteration time, then a
@@ -921,6 +942,7 @@ struct ace_handle {
     // device copies
     double *d_rows;
     uint32_t *d_pos_info;
+    ace_u2 *d_pos_spread;      // per position, for the kernel of small batches (null: more ops than it takes)
     uint32_t *d_pos_types;     // d_pos_info with row indices in place of LDS slots (windowed rows, at most 256 of them; else null)
     ace_u4 *d_pos4;            // per position, for the assembly op loop (null when its pair-kind table has no room in LDS)
     ace_u4 *d_win_dma;         // windowed rows: what the assembly op loop fetches its windows by (setup_windowed_asm), or null
@@ -1034,6 +1056,14 @@ static int upload_pos4(ace_handle *h, const ace_tables_t *t, size_t pos_entries,
     const int rc = upload((void **)&h->d_pos4, p4, pos_entries * sizeof(ace_u4));
     delete[] p4;
     return rc;
+}
+
+static int upload_pos_spread(ace_handle *h, const ace_tables_t *t, size_t pos_entries) {
+    h->d_pos_spread = nullptr;
+    if (t->num_ops > kSpreadMaxOps || (uint64_t)t->num_types * (uint64_t)t->row_doubles * 8u > 0xffffffffull) return ACE_OK;
+    std::vector<ace_u2> ps(pos_entries);
+    ace_pos_spread(t, ps.data(), pos_entries);
+    return upload((void **)&h->d_pos_spread, ps.data(), pos_entries * sizeof(ace_u2));
 }
 
 // Windowed rows: the position descriptors with each row's index in `rows` where its LDS slot is.
@@ -1288,10 +1318,11 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
     double *scratch_here = nullptr;
     if ((rc = hipGetDevice(&h->device) == hipSuccess ? ACE_OK : ACE_EHIP) ||
         (rc = static_scratch_ptr(&scratch_here)) ||
-        (rc = upload((void **)&h->d_rows, t->rows, (size_t)t->num_types * row_bytes)) ||
+        // (zeros behind the last row: a code byte that names no profiled entry may point a few entries past its row)
+        (rc = upload((void **)&h->d_rows, t->rows, (size_t)t->num_types * row_bytes, (size_t)t->num_types * row_bytes + 4096u)) ||
         (rc = upload((void **)&h->d_pos_info, t->pos_info, (size_t)(t->num_ops + 1) * 4, pos_entries * 4)) ||
         (rc = upload_pos4(h, t, pos_entries, pk32_off)) ||
-        (rc = upload_pos_types(h, t, pos_entries)) ||
+        (rc = upload_pos_types(h, t, pos_entries)) || (rc = upload_pos_spread(h, t, pos_entries)) ||
         (rc = upload((void **)&h->d_pair_kinds, t->pair_kinds, (size_t)rk_bytes)) ||
         (rc = upload((void **)&h->d_stage_lut, t->stage_lut, (size_t)stg_words * 4)) ||
         (rc = upload((void **)&h->d_nbm1, t->nb_minus_1, (size_t)t->n_mbs * 8)) ||
@@ -1314,7 +1345,8 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
 
 void ace_destroy(ace_handle_t *h) {
     if (!h) return;
-    (void)hipFree(h->d_rows); (void)hipFree(h->d_pos_info); (void)hipFree(h->d_pos_types); (void)hipFree(h->d_pair_kinds);
+    (void)hipFree(h->d_rows); (void)hipFree(h->d_pos_info); (void)hipFree(h->d_pos_types); (void)hipFree(h->d_pos_spread);
+    (void)hipFree(h->d_pair_kinds);
     if (h->d_pos4) (void)hipFree(h->d_pos4);
     if (h->d_win_dma) (void)hipFree(h->d_win_dma);
     (void)hipFree(h->d_stage_lut); (void)hipFree(h->d_nbm1); (void)hipFree(h->d_win_pos);
@@ -1338,7 +1370,7 @@ static int fill_args(ace_handle_t *h, const ace_batch_t *b, double memory_limit,
     a->hdr = reinterpret_cast<const ace_u4 *>(b->d_hdr);
     a->range = reinterpret_cast<const ace_u2 *>(b->d_range);
     a->order = b->d_order;
-    a->rows = h->d_rows; a->pos_info = h->d_pos_info; a->pos_types = h->d_pos_types; a->pos4 = h->d_pos4; a->win_dma = h->d_win_dma; a->pair_kinds = h->d_pair_kinds; a->stage_lut = h->d_stage_lut;
+    a->rows = h->d_rows; a->pos_info = h->d_pos_info; a->pos_types = h->d_pos_types; a->pos4 = h->d_pos4; a->win_dma = h->d_win_dma; a->pos_spread = h->d_pos_spread; a->pair_kinds = h->d_pair_kinds; a->stage_lut = h->d_stage_lut;
     a->nbm1 = h->d_nbm1; a->win_pos = h->d_win_pos; a->win_row_begin = h->d_win_row_begin; a->win_rows = h->d_win_rows;
     a->n_windows = h->n_windows; a->row_doubles = h->row_doubles; a->rk_bytes = h->rk_bytes; a->stg_words = h->stg_words;
     a->flat_rows16 = h->flat_rows16;
@@ -1378,7 +1410,25 @@ static void launch_score_w(const ace_handle_t *h, const AceKernelArgs &a, hipStr
     else launch_score_b<BD, RANGED, false, false>(h, a, s);
 }
 
+template <bool BD, bool RANGED, bool COLL>
+static void launch_spread_c(const AceKernelArgs &a, hipStream_t s) {
+    SpreadShared sh;
+    const uint32_t lds = ace_spread_layout(SpreadCols<BD, COLL>::kCols, a.g.G, (uint32_t)a.rk_bytes, nullptr, &sh);
+    hipLaunchKernelGGL((ace_spread_kernel<BD, RANGED, COLL>), dim3((unsigned)a.g.P), dim3(kSpreadLanes), lds, s, a);
+}
+template <bool BD, bool RANGED>
+static void launch_spread(const AceKernelArgs &a, hipStream_t s) {
+    if (a.g.flags & ACE_F_COLLECTIVE_MEM) launch_spread_c<BD, RANGED, true>(a, s);
+    else launch_spread_c<BD, RANGED, false>(a, s);
+}
+
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    if (a.pos_spread && a.g.P <= (a.stage_out ? ACE_SPREAD_MAX_RECORDS : ACE_SPREAD_MAX_PLAIN)) {
+        if (a.range) launch_spread<true, true>(a, s);
+        else if (a.stage_out) launch_spread<true, false>(a, s);
+        else launch_spread<false, false>(a, s);
+        return;
+    }
     if (a.range) launch_score_w<true, true>(h, a, s);
     else if (a.stage_out) launch_score_w<true, false>(h, a, s);
     else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);

@@ -194,8 +194,8 @@ uint32_t ace_lds_pk32(uint32_t lds_end, uint32_t rk_bytes, uint32_t *pk32_off) {
 // BD: per-stage records for the caller.  RANGED: one stage over an op sub-range.  DEFER: stage
 // tails are not evaluated where the stage ends (where only the few lanes that cut at this op are
 // active) but stashed to a per-plan workspace and replayed after the op loop with every lane busy.
-// GROWS (with DEFER): the rows are windowed, so the evaluation of the stashed stages looks the stage boundaries up in
-// the rows' global copy (its caller passes the geometry with row offsets as they are there).
+// GROWS: the stage boundaries are looked up in the rows' global copy (the caller passes the geometry with row offsets as
+// they are there): with DEFER, where the rows are windowed; in the kernel for small batches (ace_spread.h) always.
 template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROWS = false> struct PlanState {
     template <class T> ACE_HD static T row_ld(const AceLds &lds, uint32_t a) {
         if (GROWS) return lds.template gld<T>(a);
@@ -340,7 +340,7 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
         in_comm = row_ld<double>(lds, a + (in_cross ? 16u : 8u));        // size / inter- or intra-node bandwidth
         if (BD) {
             uint32_t ai = row + g.start_off + ideal_start_v + (c & (uint32_t)(g.n_algo - 1)) * ACE_START_STRIDE;
-            id_in = lds.ld<double>(ai + (in_cross ? 16u : 8u));
+            id_in = row_ld<double>(lds, ai + (in_cross ? 16u : 8u));
             id_fwd = 0.0; id_bwd = 0.0;
         }
     }
@@ -514,7 +514,7 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
             r[ACE_R_SAVED] = saved; r[ACE_R_PEAK] = peak; r[ACE_R_RESERVED] = reserved;
             // ideal pass: output_size[ops[-1]][mbs index of micro_bs][tp index 0][algo[-1]]
             uint32_t iidx = ((bidx * (uint32_t)g.n_tp + 0u) << g.A_shift) + a_last;
-            ace_d2 ie = lds.ld<ace_d2>(lastrow + g.out_off + iidx * 16u);
+            ace_d2 ie = row_ld<ace_d2>(lds, lastrow + g.out_off + iidx * 16u);
             r[ACE_R_IDEAL_FWD] = id_fwd; r[ACE_R_IDEAL_BWD] = id_bwd; r[ACE_R_IDEAL_IN] = id_in;
             r[ACE_R_IDEAL_OUT] = out_cross ? ie.y : ie.x;
             r[ACE_R_STAGE_MS] = t; r[ACE_R_STAGE_MB] = mem;

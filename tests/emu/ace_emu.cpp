@@ -6,6 +6,7 @@
 #define ACE_HOST_EMU 1
 #include "ace_edit_kernels.h"
 #include "ace_score_loop.h"
+#include "ace_spread.h"
 
 #include <sys/mman.h>
 
@@ -138,12 +139,45 @@ void run_lanes(const AceKernelArgs &a, unsigned char *lds, uint32_t lds_bytes) {
     }
 }
 
+// The kernel of small batches: its workgroup's lanes one after the other within each phase, LDS behind guard pages.
+template <bool BD, bool RANGED, bool COLL>
+void run_spread(const AceKernelArgs &a, GuardedPool &pool) {
+    SpreadShared sh;
+    const uint32_t bytes = ace_spread_layout(SpreadCols<BD, COLL>::kCols, a.g.G, (uint32_t)a.rk_bytes, nullptr, &sh);
+    unsigned char *lds = (unsigned char *)pool.place(nullptr, bytes);
+    for (long long p = 0; p < a.g.P; ++p) {
+        memset(lds, 0xff, bytes);
+        ace_spread_body<BD, RANGED, COLL>(a, lds, 0, p);
+    }
+}
+template <bool BD, bool RANGED> void run_spread_c(const AceKernelArgs &a, GuardedPool &pool) {
+    if (a.g.flags & ACE_F_COLLECTIVE_MEM) run_spread<BD, RANGED, true>(a, pool);
+    else run_spread<BD, RANGED, false>(a, pool);
+}
+
+int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, const uint32_t *order, long long P,
+               double memory_limit, int strict, double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, double *stage_out,
+               bool spread);
+
 }  // namespace
 
 // codes: uint8 [G][P][16] (the kernel's layout).  Chooses the kernel variant as the library's launcher does.
 extern "C" int ace_emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range,
                               const uint32_t *order /* nullable [P] */, long long P, double memory_limit, int strict,
                               double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, double *stage_out) {
+    return emu_kernel(t, codes, hdr, range, order, P, memory_limit, strict, iter_ms, peak_mb, feasible, status, stage_out, false);
+}
+// ... and the kernel of small batches.
+extern "C" int ace_emu_spread(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range,
+                              const uint32_t *order /* nullable [P] */, long long P, double memory_limit, int strict,
+                              double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, double *stage_out) {
+    return emu_kernel(t, codes, hdr, range, order, P, memory_limit, strict, iter_ms, peak_mb, feasible, status, stage_out, true);
+}
+
+namespace {
+int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, const uint32_t *order, long long P,
+               double memory_limit, int strict, double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, double *stage_out,
+               bool spread) {
     if (range && !stage_out) return -1;
     AceKernelArgs a;
     memset(&a, 0, sizeof(a));
@@ -202,6 +236,25 @@ extern "C" int ace_emu_kernel(const ace_tables_t *t, const uint8_t *codes, const
     const size_t rec_bytes = (size_t)P * (range ? 1 : ACE_MAX_STAGES) * ACE_STAGE_REC * 8;
     a.stage_out = stage_out ? (double *)pool.place(stage_out, rec_bytes, 8) : nullptr;   // (records of unused stages stay as the caller left them)
     unsigned char *lds = (unsigned char *)pool.place(nullptr, lds_bytes);
+    if (spread) {
+        // (as the library uploads them: positions padded, zeros behind the last row)
+        ace_u2 *ps = (ace_u2 *)pool.place(nullptr, (G * 16 + 16) * 8, 8);
+        ace_pos_spread(t, ps, G * 16 + 16);
+        a.pos_spread = ps;
+        const size_t rows = (size_t)t->num_types * t->row_doubles * 8;
+        double *padded = (double *)pool.place(nullptr, rows + 4096);
+        memcpy(padded, t->rows, rows);
+        a.rows = padded;
+        if (range) run_spread_c<true, true>(a, pool);
+        else if (stage_out) run_spread_c<true, false>(a, pool);
+        else run_spread_c<false, false>(a, pool);
+        memcpy(iter_ms, a.iter_ms, (size_t)P * 8);
+        memcpy(peak_mb, a.peak_mb, (size_t)P * 8);
+        memcpy(feasible, a.feasible, (size_t)P);
+        if (status) memcpy(status, a.status, (size_t)P);
+        if (stage_out) memcpy(stage_out, a.stage_out, rec_bytes);
+        return 0;
+    }
     const bool win = t->n_windows > 1;
     const bool coll = (t->flags & ACE_F_COLLECTIVE_MEM) != 0;
     const bool defer = !range && !stage_out && (!win || a.pos_types) && g.N < 32768 && !coll;
@@ -227,7 +280,7 @@ extern "C" int ace_emu_kernel(const ace_tables_t *t, const uint8_t *codes, const
     if (stage_out) memcpy(stage_out, a.stage_out, rec_bytes);
     return 0;
 }
-
+}  // namespace
 
 // ------------------------------------------------------------------------------------------
 // The plan-editing kernels (ace_edit_kernels.h) on the CPU, one call per work item, arrays behind

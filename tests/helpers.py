@@ -55,7 +55,7 @@ def emu_lib():
     if _emu is None:
         so = os.path.join(ROOT, "tests", "emu", "libace_emu.so")
         src = os.path.join(ROOT, "tests", "emu", "ace_emu.cpp")
-        hdrs = [os.path.join(ROOT, "superscaler_amd", "csrc", h) for h in ("ace_plan_state.h", "ace_score_loop.h")]
+        hdrs = [os.path.join(ROOT, "superscaler_amd", "csrc", h) for h in ("ace_plan_state.h", "ace_score_loop.h", "ace_spread.h")]
         if (not os.path.exists(so)) or os.path.getmtime(so) < max(os.path.getmtime(f) for f in [src] + hdrs):
             subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC",
                             "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "superscaler_amd", "csrc"),
@@ -63,6 +63,7 @@ def emu_lib():
         _emu = ctypes.CDLL(so)
         _emu.ace_emu_score.restype = ctypes.c_int
         _emu.ace_emu_kernel.restype = ctypes.c_int
+        _emu.ace_emu_spread.restype = ctypes.c_int
     return _emu
 
 
@@ -97,10 +98,11 @@ def kernel_layout(codes):
     return np.ascontiguousarray(out.reshape(P, G, 16).transpose(1, 0, 2))
 
 
-def emu_kernel_score(tables, batch, memory_limit=None, strict=False, breakdown=False, ranges=None, raw_codes=None, order=None):
+def emu_kernel_score(tables, batch, memory_limit=None, strict=False, breakdown=False, ranges=None, raw_codes=None, order=None, spread=False):
     """The scoring kernel's own loop (csrc/ace_score_loop.h) on the CPU with guard pages behind every array:
     an out-of-range index ends the process with SIGSEGV, so call this from a child process.
-    `raw_codes`: a [G][P][16] array to use as is (e.g. with junk in the padding bytes)."""
+    `raw_codes`: a [G][P][16] array to use as is (e.g. with junk in the padding bytes).
+    `spread`: the kernel of small batches (csrc/ace_spread.h)."""
     lib = emu_lib()
     ts = tables.as_struct()
     P = batch.n_plans
@@ -116,7 +118,8 @@ def emu_kernel_score(tables, batch, memory_limit=None, strict=False, breakdown=F
     vp = ctypes.c_void_p
     if order is not None:
         order = np.ascontiguousarray(order, dtype=np.uint32)
-    rc = lib.ace_emu_kernel(ctypes.byref(ts), codes.ctypes.data_as(vp), hdr.ctypes.data_as(vp),
+    entry = lib.ace_emu_spread if spread else lib.ace_emu_kernel
+    rc = entry(ctypes.byref(ts), codes.ctypes.data_as(vp), hdr.ctypes.data_as(vp),
                             ranges.ctypes.data_as(vp) if ranges is not None else None,
                             order.ctypes.data_as(vp) if order is not None else None, ctypes.c_longlong(P),
                             ctypes.c_double(limit), ctypes.c_int(int(strict)), it.ctypes.data_as(vp), pk.ctypes.data_as(vp),
