@@ -213,6 +213,37 @@ int ace_apply_moves(const uint8_t *d_template_codes, const uint32_t *d_template_
                     const uint32_t *d_moves, size_t n_moves, int num_ops, int n_algo, uint8_t *d_codes_out,
                     uint32_t *d_hdr_out, uint64_t *d_keys_out, void *stream);
 
+/* The visited set of a search over such keys, on the host (aceso_search.py:47,105 over aceso_utils.py:831-850).  A key is a
+ * pair of 64-bit words, keys are uint64[n][2] in HOST memory.  Not safe for concurrent changes of one set.
+ * ace_keyset_unseen sets mask[i] (uint8[n]) for keys that are in none of the n_sets sets and not earlier in `keys`;
+ * ace_keyset_claim does that and adds those keys to sets[0]; ace_keyset_add adds keys (repeats are ignored);
+ * ace_keyset_move adds everything in `from` to `to` and empties `from`. */
+typedef struct ace_keyset ace_keyset_t;
+int ace_keyset_create(ace_keyset_t **out);
+void ace_keyset_destroy(ace_keyset_t *s);
+size_t ace_keyset_size(const ace_keyset_t *s);
+int ace_keyset_add(ace_keyset_t *s, const uint64_t *keys, size_t n);
+int ace_keyset_unseen(const ace_keyset_t *const *sets, int n_sets, const uint64_t *keys, size_t n, uint8_t *mask);
+int ace_keyset_claim(ace_keyset_t *const *sets, int n_sets, const uint64_t *keys, size_t n, uint8_t *mask);
+int ace_keyset_move(ace_keyset_t *to, ace_keyset_t *from);
+int ace_keyset_keys(const ace_keyset_t *s, uint64_t *keys_out /* [size][2], in no order */);
+
+/* Single-move neighbours of one plan as move descriptors and templates (HOST memory throughout), from choices that the
+ * caller has drawn: per kind k of neighbour, `count[k]` rows of the result and their choices.
+ *   0 op migration: x = stage whose first boundary moves, y = by how many ops (signed); 1 tp <-> dp: x = stage, y = 1 or
+ *   -1; 2 micro-batch size: x = 1 or -1; 3 recompute: x = first op, y = how many; 4 algorithm: x = op; 5 devices:
+ *   from stage x to stage y.
+ * A move that leaves the profiled grid (stage_lut, as in ace_tables_t) becomes a copy of the plan.  codes: the plan's num_ops code bytes, hdr: its header.
+ * moves_out: uint32[n][4] as ace_apply_moves reads them; templates go to t_codes_out (uint8[max_templates][num_ops]) and
+ * t_hdr_out (uint32[max_templates][4]); at most 3 + S * (S - 1) for a plan of S stages, the plan itself first. */
+typedef struct ace_move_draws {
+    size_t n, count[6];
+    const int64_t *rows[6], *x[6], *y[6];
+} ace_move_draws_t;
+int ace_build_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
+                    int gpus_per_node, const ace_move_draws_t *draws, uint32_t *moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out,
+                    int max_templates, int *n_templates_out);
+
 /* Sort keys for grouped storage (ace_batch_t.d_order) of a batch that is already on the device: d_keys[i]
  * (uint64[n_plans]) orders the plans by pipeline depth, deepest first, then by the positions of their first two
  * stage boundaries.  The caller sorts the keys (stably), deals the sorted wavefronts of 64 to the workgroups and

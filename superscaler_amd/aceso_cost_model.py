@@ -121,9 +121,7 @@ class CostModel:
         ev = self.evaluator
         d = ev.upload(batch)
         it, pk, fe, st = ev.score(d, memory_limit, strict)
-        idx, val, cnt = ev.topk(it, fe, k)
-        n = int(cnt.item())
-        return idx[:n].cpu().numpy(), val[:n].cpu().numpy()
+        return ev.read_topk(ev.topk_packed(it, fe, k), k)
 
     @staticmethod
     def _raise_for_status(status):

@@ -19,6 +19,8 @@
 #include <vector>
 
 #include "ace_edit_kernels.h"
+#include "ace_keyset.h"
+#include "ace_moves_host.h"
 #include "ace_score_loop.h"
 #include "ace_spread.h"
 
@@ -1665,6 +1667,111 @@ int ace_recompute_select(const ace_rc_tables_t *t, uint8_t *d_codes_rw, int n_st
                        memory_limit, d_alive);
     ACE_HIP(hipGetLastError());
     return ACE_OK;
+}
+
+int ace_keyset_create(ace_keyset_t **out) {
+    if (!out) return ACE_EINVAL;
+    try {
+        *out = reinterpret_cast<ace_keyset_t *>(new AceKeySet);
+    } catch (const std::bad_alloc &) {
+        *out = nullptr;
+        return ACE_ENOMEM;
+    }
+    return ACE_OK;
+}
+
+static AceKeySet *key_set(ace_keyset_t *s) { return reinterpret_cast<AceKeySet *>(s); }
+static const AceKeySet *key_set(const ace_keyset_t *s) { return reinterpret_cast<const AceKeySet *>(s); }
+
+void ace_keyset_destroy(ace_keyset_t *s) { delete key_set(s); }
+
+size_t ace_keyset_size(const ace_keyset_t *s) { return s ? key_set(s)->size() : 0; }
+
+int ace_keyset_add(ace_keyset_t *s, const uint64_t *keys, size_t n) {
+    if (!s || (n && !keys)) return ACE_EINVAL;
+    try {
+        AceKeySet *set = key_set(s);
+        ace_each_key(keys, n, &set, 1, [&](size_t, const AceKey &k) { set->add(k); });
+    } catch (const std::bad_alloc &) {
+        return ACE_ENOMEM;
+    }
+    return ACE_OK;
+}
+
+// the sets behind the handles (at most four), or 0
+static int key_sets(const ace_keyset_t *const *sets, int n_sets, const AceKeySet **out) {
+    if (n_sets < 0 || n_sets > 4 || (n_sets && !sets)) return 0;
+    for (int i = 0; i < n_sets; ++i) {
+        if (!sets[i]) return 0;
+        out[i] = key_set(sets[i]);
+    }
+    return 1;
+}
+
+int ace_keyset_unseen(const ace_keyset_t *const *sets, int n_sets, const uint64_t *keys, size_t n, uint8_t *mask) {
+    const AceKeySet *in[5];
+    if (!key_sets(sets, n_sets, in) || (n && (!keys || !mask))) return ACE_EINVAL;
+    try {
+        AceKeySet here;
+        here.reserve(n);
+        in[n_sets] = &here;
+        ace_each_key(keys, n, in, n_sets + 1, [&](size_t i, const AceKey &k) {
+            bool fresh = true;
+            for (int j = 0; j < n_sets && fresh; ++j) fresh = !in[j]->has(k);
+            mask[i] = (uint8_t)(fresh && here.add(k));
+        });
+    } catch (const std::bad_alloc &) {
+        return ACE_ENOMEM;
+    }
+    return ACE_OK;
+}
+
+int ace_keyset_claim(ace_keyset_t *const *sets, int n_sets, const uint64_t *keys, size_t n, uint8_t *mask) {
+    const AceKeySet *in[4];
+    if (n_sets < 1 || !key_sets(sets, n_sets, in) || (n && (!keys || !mask))) return ACE_EINVAL;
+    try {
+        AceKeySet *set = key_set(sets[0]);
+        ace_each_key(keys, n, in, n_sets, [&](size_t i, const AceKey &k) {
+            bool fresh = true;
+            for (int j = 1; j < n_sets && fresh; ++j) fresh = !in[j]->has(k);
+            mask[i] = (uint8_t)(fresh && set->add(k));
+        });
+    } catch (const std::bad_alloc &) {
+        return ACE_ENOMEM;
+    }
+    return ACE_OK;
+}
+
+int ace_keyset_move(ace_keyset_t *to, ace_keyset_t *from) {
+    if (!to || !from || to == from) return ACE_EINVAL;
+    try {
+        AceKeySet *t = key_set(to);
+        std::vector<uint64_t> keys;
+        keys.reserve(2 * key_set(from)->size());
+        key_set(from)->each([&](const AceKey &k) { keys.push_back(k.a); keys.push_back(k.b); });
+        t->reserve(t->size() + keys.size() / 2);
+        ace_each_key(keys.data(), keys.size() / 2, &t, 1, [&](size_t, const AceKey &k) { t->add(k); });
+        key_set(from)->clear();
+    } catch (const std::bad_alloc &) {
+        return ACE_ENOMEM;
+    }
+    return ACE_OK;
+}
+
+int ace_keyset_keys(const ace_keyset_t *s, uint64_t *keys_out) {
+    if (!s || !keys_out) return ACE_EINVAL;
+    key_set(s)->each([&](const AceKey &k) { *keys_out++ = k.a; *keys_out++ = k.b; });
+    return ACE_OK;
+}
+
+int ace_build_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
+                    int gpus_per_node, const ace_move_draws_t *draws, uint32_t *moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out,
+                    int max_templates, int *n_templates_out) {
+    if (!codes || !hdr || !stage_lut || !draws || !moves_out || !t_codes_out || !t_hdr_out || !n_templates_out || num_ops <= 0 ||
+        num_ops >= 65536 || (n_algo != 1 && n_algo != 2) || n_tp <= 0 || n_tp > 4 || n_mbs <= 0 || gpus_per_node <= 0)
+        return ACE_EINVAL;
+    return ace_build_moves_body(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, *draws, moves_out, t_codes_out, t_hdr_out,
+                                max_templates, n_templates_out);
 }
 
 }  // extern "C"

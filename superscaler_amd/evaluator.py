@@ -17,7 +17,9 @@ _lib = None
 
 EXPORTS = ["ace_abi_version", "ace_strerror", "ace_last_hip_error", "ace_create", "ace_destroy",
            "ace_score_batch", "ace_score_batch_static", "ace_reserve", "ace_topk_workspace_bytes", "ace_topk", "ace_time_score_kernel", "ace_apply_moves",
-           "ace_recompute_groups", "ace_recompute_select", "ace_group_keys", "ace_gather_plans"]
+           "ace_recompute_groups", "ace_recompute_select", "ace_group_keys", "ace_gather_plans",
+           "ace_keyset_create", "ace_keyset_destroy", "ace_keyset_size", "ace_keyset_add", "ace_keyset_unseen", "ace_keyset_claim",
+           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves"]
 
 
 class AceBatchStruct(ctypes.Structure):
@@ -29,6 +31,11 @@ class AceRcTablesStruct(ctypes.Structure):
     _fields_ = [("d_codes", ctypes.c_void_p), ("n_plans", ctypes.c_size_t), ("d_type_of_pos", ctypes.c_void_p),
                 ("d_activations", ctypes.c_void_p), ("d_no_recompute", ctypes.c_void_p), ("num_ops", ctypes.c_int32),
                 ("num_types", ctypes.c_int32), ("n_mbs", ctypes.c_int32), ("n_tp", ctypes.c_int32), ("n_algo", ctypes.c_int32)]
+
+
+class AceMoveDrawsStruct(ctypes.Structure):
+    _fields_ = [("n", ctypes.c_size_t), ("count", ctypes.c_size_t * 6), ("rows", ctypes.c_void_p * 6),
+                ("x", ctypes.c_void_p * 6), ("y", ctypes.c_void_p * 6)]
 
 
 class AceError(RuntimeError):
@@ -83,6 +90,19 @@ def load_library():
     lib.ace_recompute_select.restype = ctypes.c_int
     lib.ace_recompute_select.argtypes = ([ctypes.POINTER(AceRcTablesStruct), ctypes.c_void_p, ctypes.c_int] +
                                          [ctypes.c_void_p] * 9 + [ctypes.c_double, ctypes.c_void_p, ctypes.c_void_p])
+    vp, sz = ctypes.c_void_p, ctypes.c_size_t
+    lib.ace_keyset_create.argtypes = [ctypes.POINTER(vp)]
+    lib.ace_keyset_destroy.restype = None
+    lib.ace_keyset_destroy.argtypes = [vp]
+    lib.ace_keyset_size.restype = sz
+    lib.ace_keyset_size.argtypes = [vp]
+    lib.ace_keyset_add.argtypes = [vp, vp, sz]
+    lib.ace_keyset_unseen.argtypes = [ctypes.POINTER(vp), ctypes.c_int, vp, sz, vp]
+    lib.ace_keyset_claim.argtypes = [ctypes.POINTER(vp), ctypes.c_int, vp, sz, vp]
+    lib.ace_keyset_move.argtypes = [vp, vp]
+    lib.ace_keyset_keys.argtypes = [vp, vp]
+    ci = ctypes.c_int
+    lib.ace_build_moves.argtypes = [vp, vp, ci, ci, ci, ci, vp, ci, ctypes.POINTER(AceMoveDrawsStruct), vp, vp, vp, ci, ctypes.POINTER(ci)]
     if lib.ace_abi_version() != ABI_VERSION:
         raise AceError("libace_eval.so has a different ABI version")
     _lib = lib
@@ -326,20 +346,31 @@ class PlanEvaluator:
     def topk(self, iter_ms, feasible, k: int):
         """Device-wide top-k: (indices int64[k], times f64[k], count)."""
         torch = self._torch
+        buf = self.topk_packed(iter_ms, feasible, k)
+        return buf[:8 * k].view(torch.int64), buf[8 * k:16 * k].view(torch.float64), buf[16 * k:16 * k + 4].view(torch.int32)
+
+    def topk_packed(self, iter_ms, feasible, k: int):
+        """topk() in one device buffer (indices, times, count: one copy brings all of them to the host)."""
+        torch = self._torch
         n = iter_ms.numel()
         need = self.lib.ace_topk_workspace_bytes(n, k)
         if self._topk_ws is None or self._topk_ws.numel() < need:
             # (a captured step keeps its own reference to the workspace it recorded, so the old one stays alive for it)
             self._topk_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
-        idx = torch.empty(k, dtype=torch.int64, device=self.device)
-        val = torch.empty(k, dtype=torch.float64, device=self.device)
-        cnt = torch.empty(1, dtype=torch.int32, device=self.device)
+        buf = torch.empty(16 * k + 8, dtype=torch.uint8, device=self.device)
+        at = buf.data_ptr()
         with torch.cuda.device(self.device):
-            rc = self.lib.ace_topk(self.handle, iter_ms.data_ptr(), feasible.data_ptr(), n, k, idx.data_ptr(),
-                                   val.data_ptr(), cnt.data_ptr(), self._topk_ws.data_ptr(), self._topk_ws.numel(),
-                                   self._stream())
+            rc = self.lib.ace_topk(self.handle, iter_ms.data_ptr(), feasible.data_ptr(), n, k, at, at + 8 * k, at + 16 * k,
+                                   self._topk_ws.data_ptr(), self._topk_ws.numel(), self._stream())
         _check(self.lib, rc, "ace_topk")
-        return idx, val, cnt
+        return buf
+
+    @staticmethod
+    def read_topk(buf, k: int):
+        """topk_packed's result on the host: (indices, times) of the feasible ones."""
+        host = buf.cpu().numpy()
+        n = int(host[16 * k:16 * k + 4].view(np.int32)[0])
+        return host[:8 * k].view(np.int64)[:n], host[8 * k:16 * k].view(np.float64)[:n]
 
     def capture_step(self, dbatch: DeviceBatch, k: int, memory_limit: Optional[float] = None, strict: bool = False):
         """Score + top-k of a resident batch recorded once in a HIP graph (the library's launches record into a
@@ -403,10 +434,9 @@ class PlanEvaluator:
             pending = upload(nxt) if nxt is not None else None     # overlaps with the scoring below
             main.wait_event(ready)
             t, pk, fe, st = self.score(d, memory_limit, strict)
-            idx, val, cnt = self.topk(t, fe, k)
-            n = int(cnt.item())                                      # synchronises this batch
-            best_idx = np.concatenate([best_idx, idx[:n].cpu().numpy() + offset])
-            best_val = np.concatenate([best_val, val[:n].cpu().numpy()])
+            idx, val = self.read_topk(self.topk_packed(t, fe, k), k)   # synchronises this batch
+            best_idx = np.concatenate([best_idx, idx + offset])
+            best_val = np.concatenate([best_val, val])
             order = np.lexsort((best_idx, best_val))[:k]
             best_idx, best_val = best_idx[order], best_val[order]
             offset += d.n_plans
@@ -422,16 +452,19 @@ class PlanEvaluator:
         T, N = templates.codes.shape
         G = (N + 15) // 16
         n = int(moves.shape[0])
-        tc = np.zeros((T, G * 16), dtype=np.uint8)
-        tc[:, :N] = templates.codes
-        d_tc = torch.from_numpy(tc).to(self.device)
-        d_th = torch.from_numpy(np.ascontiguousarray(templates.hdr).view(np.int32)).to(self.device)
-        d_mv = torch.from_numpy(np.ascontiguousarray(moves, dtype=np.uint32).view(np.int32)).to(self.device)
+        # one upload: descriptors, template headers, template code rows
+        off_hdr, off_codes = 16 * n, 16 * (n + T)
+        up = np.zeros(off_codes + T * G * 16, dtype=np.uint8)
+        up[:off_hdr].view(np.uint32).reshape(n, 4)[...] = moves
+        up[off_hdr:off_codes].view(np.uint32).reshape(T, 4)[...] = templates.hdr
+        up[off_codes:].reshape(T, G * 16)[:, :N] = templates.codes
+        d_up = torch.from_numpy(up).to(self.device)
+        at = d_up.data_ptr()
         codes = torch.empty((G, n, 16), dtype=torch.uint8, device=self.device)
         hdr = torch.empty((n, 4), dtype=torch.int32, device=self.device)
         keys = torch.zeros((n, 2), dtype=torch.int64, device=self.device) if with_keys else None
         with torch.cuda.device(self.device):
-            rc = self.lib.ace_apply_moves(d_tc.data_ptr(), d_th.data_ptr(), T, d_mv.data_ptr(), n, N,
+            rc = self.lib.ace_apply_moves(at + off_codes, at + off_hdr, T, at, n, N,
                                           self.tables.db.n_algo, codes.data_ptr(), hdr.data_ptr(),
                                           keys.data_ptr() if with_keys else None, self._stream())
         _check(self.lib, rc, "ace_apply_moves")

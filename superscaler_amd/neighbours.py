@@ -7,6 +7,7 @@ row / header, so thousands of neighbours of one plan are produced with a few num
 scored by one kernel launch.  The search policy of the reference (aceso_policy.py) is not
 reproduced: `hill_climb` is a plain best-neighbour descent used to exercise the batched path.
 """
+import ctypes
 from typing import Tuple
 
 import numpy as np
@@ -40,6 +41,88 @@ def _set_header(hdr_row, S, bidx, glogs, gpn):
 OP_NONE, OP_MIGRATE, OP_TP_STEP, OP_RC_TOGGLE, OP_ALGO_TOGGLE = 0, 1, 2, 3, 4
 
 
+def _draw_moves(n: int, S: int, tables: CompiledTables, rng: np.random.Generator, max_move: int = 8):
+    """Everything random about n single-move neighbours of a plan of S stages (their kinds, the stages, counts and
+    directions), none of which depends on the plan itself: hill_climb draws for its next step while the GPU scores the
+    current one.  Returns int64 arrays: per kind the neighbours of that kind, and their choices."""
+    N = tables.graph.num_ops
+    kinds = rng.integers(0, 6, size=n)
+    order = np.argsort(kinds.astype(np.uint8), kind="stable")
+    ends = np.cumsum(np.bincount(kinds, minlength=6))
+    rows = [order[lo:hi] for lo, hi in zip([0, *ends[:-1]], ends)]
+    none = np.zeros(0, dtype=np.int64)
+    out = {"n": n, "rows": list(rows), "x": [none] * 6, "y": [none] * 6}
+
+    def sign(m):
+        return np.where(rng.random(m) < 0.5, 1, -1)
+
+    # kind 0, op migration: which boundary, by how many ops, which way
+    m = len(rows[0])
+    if S > 1 and m:
+        out["x"][0] = rng.integers(1, S, size=m)
+        out["y"][0] = rng.integers(1, max_move + 1, size=m) * sign(m)
+    else:
+        out["rows"][0] = none
+    # kind 1, tp <-> dp inside one stage
+    m = len(rows[1])
+    if m:
+        out["x"][1] = rng.integers(0, S, size=m)
+        out["y"][1] = sign(m)
+    # kind 2, micro-batch size one step up or down
+    m = len(rows[2])
+    if m:
+        out["x"][2] = sign(m)
+    # kind 3, recompute: a short run of ops
+    m = len(rows[3])
+    if m:
+        out["x"][3] = rng.integers(0, N, size=m)
+        out["y"][3] = rng.integers(1, 14, size=m)
+    # kind 4, partition algorithm of one tunable op
+    m = len(rows[4])
+    if tables.db.n_algo == 2 and m:
+        cand = np.flatnonzero((tables.graph.flags[tables.graph.type_of_pos] & og.F_TUNABLE) != 0)
+        out["x"][4] = cand[rng.integers(0, len(cand), size=m)]
+    else:
+        out["rows"][4] = none
+    # kind 5, devices from one stage to another
+    m = len(rows[5])
+    if S > 1 and m:
+        out["x"][5] = rng.integers(0, S, size=m)
+        out["y"][5] = (out["x"][5] + rng.integers(1, S, size=m)) % S
+    else:
+        out["rows"][5] = none
+    return out
+
+
+def _build_moves(base: PlanBatch, tables: CompiledTables, draws) -> Tuple[PlanBatch, np.ndarray]:
+    """The drawn moves on base plan 0 as (templates, moves): the library's ace_build_moves."""
+    from .evaluator import AceMoveDrawsStruct, _check, load_library
+    lib = load_library()
+    N, M, n = tables.graph.num_ops, len(tables.db.mbs_list), draws["n"]
+    if N >= 65536:
+        raise ValueError("move descriptors hold 16-bit op positions")
+    S = int(base.hdr[0, 0] & 0xff)
+    cap = 3 + S * (S - 1)
+    t_codes, t_hdr = np.empty((cap, N), dtype=np.uint8), np.empty((cap, 4), dtype=np.uint32)
+    moves = np.empty((n, 4), dtype=np.uint32)
+    row, hdr = np.ascontiguousarray(base.codes[0]), np.ascontiguousarray(base.hdr[0])
+    d = AceMoveDrawsStruct()
+    d.n = n
+    keep = []
+    for name in ("rows", "x", "y"):
+        for k, a in enumerate(draws[name]):
+            a = np.ascontiguousarray(a, dtype=np.int64)
+            keep.append(a)
+            getattr(d, name)[k] = a.ctypes.data
+            if name == "rows":
+                d.count[k] = len(a)
+    n_templates = ctypes.c_int(0)
+    _check(lib, lib.ace_build_moves(row.ctypes.data, hdr.ctypes.data, N, tables.db.n_algo, len(tables.db.tp_list), M,
+                                    tables.stage_lut.ctypes.data, tables.settings.num_gpus_per_node, ctypes.byref(d), moves.ctypes.data, t_codes.ctypes.data,
+                                    t_hdr.ctypes.data, cap, ctypes.byref(n_templates)), "ace_build_moves")
+    return PlanBatch(t_codes[:n_templates.value], t_hdr[:n_templates.value]), moves
+
+
 def sample_moves(base: PlanBatch, tables: CompiledTables, n: int, rng: np.random.Generator,
                  max_move: int = 8) -> Tuple[PlanBatch, np.ndarray]:
     """n single-move neighbours of base plan 0 as (templates, moves).  A neighbour is one template row
@@ -52,126 +135,7 @@ def sample_moves(base: PlanBatch, tables: CompiledTables, n: int, rng: np.random
         OP_ALGO_TOGGLE  p0 = op position
     Moves that would leave the profiled grid become (template 0, OP_NONE): a copy of the base plan.
     `apply_moves_host` (numpy) and the library's ace_apply_moves (on the device) expand them."""
-    A = tables.db.n_algo
-    N = tables.graph.num_ops
-    if N >= 65536:
-        raise ValueError("move descriptors hold 16-bit op positions")
-    gpn = tables.settings.num_gpus_per_node
-    row0, hdr0 = base.codes[0], base.hdr[0]
-    S = int(hdr0[0] & 0xff)
-    bidx = int(hdr0[0] >> 8) & 0xff
-    gword = int(hdr0[1]) | (int(hdr0[2]) << 32)
-    glogs = np.array([(gword >> (4 * s)) & 15 for s in range(S)], dtype=np.int64)
-    starts, ends = _stage_bounds(row0)
-    tunable = (tables.graph.flags[tables.graph.type_of_pos] & og.F_TUNABLE) != 0
-    M = len(tables.db.mbs_list)
-    tp0 = ((row0 & 7) // A).astype(np.int64)
-    stage_of_pos = np.cumsum((row0 >> 4) & 1) - 1
-    kinds = rng.integers(0, 6, size=n)
-    moves = np.zeros((n, 4), dtype=np.uint32)
-    t_codes, t_hdr = [row0.copy()], [hdr0.copy()]
-
-    def allowed(b, gl):
-        return tables.allowed_tp_logs(b, gl)
-
-    def ok_bits(b, gl):
-        return sum(1 << t for t in allowed(b, gl))
-
-    # kind 0, op migration: move a stage boundary by up to max_move ops; the ops that change stage
-    # take the tp of the op they now follow / precede in the receiving stage
-    rows = np.flatnonzero(kinds == 0)
-    if S > 1 and len(rows):
-        j = rng.integers(1, S, size=len(rows))
-        d = rng.integers(1, max_move + 1, size=len(rows)) * np.where(rng.random(len(rows)) < 0.5, 1, -1)
-        cut = starts[j]
-        new_cut = cut + d
-        good = (new_cut > starts[j - 1]) & (new_cut < ends[j])
-        rows, cut, new_cut, d = rows[good], cut[good], new_cut[good], d[good]
-        ref = np.where(d > 0, tp0[cut - 1], tp0[cut])        # stage j-1 grows to the right / stage j to the left
-        moves[rows, 0] = OP_MIGRATE << 16
-        moves[rows, 1] = cut | (new_cut << 16)
-        moves[rows, 2] = ref
-
-    # kind 1, tp <-> dp inside one stage: all ops one step up or down, if the stage allows it
-    rows = np.flatnonzero(kinds == 1)
-    if len(rows):
-        s = rng.integers(0, S, size=len(rows))
-        step = np.where(rng.random(len(rows)) < 0.5, 1, -1)
-        # a stage's ops may sit on different tp: the move is legal iff every tp value present has a legal target
-        bits = np.array([ok_bits(bidx, int(g)) for g in glogs], dtype=np.int64)
-        present = np.array([sum(1 << int(v) for v in np.unique(tp0[starts[k]:ends[k]])) for k in range(S)], dtype=np.int64)
-        want = np.where(step > 0, present[s] << 1, present[s] >> 1)
-        lost = (step < 0) & ((present[s] & 1) == 1)                      # tp = 1 cannot go down
-        good = ((want & ~bits[s]) == 0) & ~lost
-        rows, s, step = rows[good], s[good], step[good]
-        moves[rows, 0] = OP_TP_STEP << 16
-        moves[rows, 1] = starts[s] | (ends[s] << 16)
-        moves[rows, 2] = (step > 0).astype(np.uint32)
-
-    # kind 2, micro-batch size one step up or down, if every op stays on the profiled grid: a header-only template
-    rows = np.flatnonzero(kinds == 2)
-    if len(rows):
-        up = rng.random(len(rows)) < 0.5
-        for sign, sel in ((1, up), (-1, ~up)):
-            b2 = bidx + sign
-            if not 0 <= b2 < M or not sel.any():
-                continue
-            bits = np.array([ok_bits(b2, int(g)) for g in glogs], dtype=np.int64)[stage_of_pos]
-            if (((bits >> tp0) & 1) == 1).all():
-                h = hdr0.copy()
-                h[0] = S | (b2 << 8)
-                t_codes.append(row0.copy())
-                t_hdr.append(h)
-                moves[rows[sel], 0] = len(t_codes) - 1
-
-    # kind 3, recompute: toggle a short run of ops
-    rows = np.flatnonzero(kinds == 3)
-    if len(rows):
-        lo = rng.integers(0, N, size=len(rows))
-        hi = np.minimum(N, lo + rng.integers(1, 14, size=len(rows)))
-        moves[rows, 0] = OP_RC_TOGGLE << 16
-        moves[rows, 1] = lo | (hi << 16)
-
-    # kind 4, partition algorithm of one tunable op
-    rows = np.flatnonzero(kinds == 4)
-    if A == 2 and len(rows):
-        cand = np.flatnonzero(tunable)
-        moves[rows, 0] = OP_ALGO_TOGGLE << 16
-        moves[rows, 1] = cand[rng.integers(0, len(cand), size=len(rows))]
-
-    # kind 5, move half of stage a's devices to a stage b that has exactly that many (sizes stay powers
-    # of two and the total is unchanged); few distinct (a, b) pairs, each a template of its own
-    rows = np.flatnonzero(kinds == 5)
-    if S > 1 and len(rows):
-        a = rng.integers(0, S, size=len(rows))
-        b = (a + rng.integers(1, S, size=len(rows))) % S
-        for pa, pb in sorted({(int(x), int(y)) for x, y in zip(a, b)}):
-            if glogs[pa] - 1 != glogs[pb]:
-                continue
-            g2 = glogs.copy()
-            g2[pa] -= 1
-            g2[pb] += 1
-            row = row0.copy()
-            good = True
-            for st in (pa, pb):
-                ok = allowed(bidx, int(g2[st]))
-                if not ok:
-                    good = False
-                    break
-                lo, hi = int(starts[st]), int(ends[st])
-                t = np.clip(tp0[lo:hi], min(ok), max(ok))
-                if not np.all(np.isin(t, ok)):
-                    good = False
-                    break
-                row[lo:hi] = (row[lo:hi] & 0xF8) | (t * A + (row[lo:hi] & (A - 1))).astype(np.uint8)
-            if not good:
-                continue
-            h = hdr0.copy()
-            _set_header(h, S, bidx, g2, gpn)
-            t_codes.append(row)
-            t_hdr.append(h)
-            moves[rows[(a == pa) & (b == pb)], 0] = len(t_codes) - 1
-    return PlanBatch(np.stack(t_codes), np.stack(t_hdr)), moves
+    return _build_moves(base, tables, _draw_moves(n, int(base.hdr[0, 0] & 0xff), tables, rng, max_move))
 
 
 # ---- the reference's own primitives as descriptors --------------------------------------------------------------
@@ -411,47 +375,83 @@ def as_key128(keys) -> np.ndarray:
     return k.view(KEY128).ravel()
 
 
+class _KeySet:
+    """A native set of 128-bit keys (ace_keyset_*)."""
+
+    def __init__(self):
+        from .evaluator import _check, load_library
+        self._lib, self._check = load_library(), _check
+        self.handle = ctypes.c_void_p()
+        _check(self._lib, self._lib.ace_keyset_create(ctypes.byref(self.handle)), "ace_keyset_create")
+
+    def __del__(self):
+        if getattr(self, "handle", None):
+            self._lib.ace_keyset_destroy(self.handle)
+
+    def __len__(self):
+        return self._lib.ace_keyset_size(self.handle)
+
+    def keys(self) -> np.ndarray:
+        out = np.empty((len(self), 2), dtype=np.uint64)
+        self._check(self._lib, self._lib.ace_keyset_keys(self.handle, out.ctypes.data), "ace_keyset_keys")
+        return out
+
+    def add(self, keys: np.ndarray) -> None:
+        self._check(self._lib, self._lib.ace_keyset_add(self.handle, keys.ctypes.data, len(keys)), "ace_keyset_add")
+
+    def take(self, other: "_KeySet") -> None:
+        self._check(self._lib, self._lib.ace_keyset_move(self.handle, other.handle), "ace_keyset_move")
+
+    def __getstate__(self):
+        return self.keys()
+
+    def __setstate__(self, keys):
+        self.__init__()
+        self.add(np.ascontiguousarray(keys))
+
+
+def _first_of_each(keys: np.ndarray, sets=(), claim: bool = False) -> np.ndarray:
+    """Mask of the keys (anything viewable as pairs of 64-bit words, one pair per row) that are in none of the sets and do
+    not repeat an earlier one; `claim`: they are added to sets[0]."""
+    from .evaluator import _check, load_library
+    lib = load_library()
+    keys = np.ascontiguousarray(keys)
+    mask = np.empty(len(keys), dtype=np.uint8)
+    handles = (ctypes.c_void_p * max(1, len(sets)))(*[s.handle for s in sets])
+    fn = lib.ace_keyset_claim if claim else lib.ace_keyset_unseen
+    _check(lib, fn(handles, len(sets), keys.ctypes.data, len(keys), mask.ctypes.data), "ace_keyset")
+    return mask.view(bool)
+
+
 class VisitedKeys:
-    """A visited set over 128-bit plan keys (for neighbours that only exist on the device): two sorted
-    arrays, a large one and a small one that takes the new keys and is folded into the large one
-    when it has grown (so marking costs a merge of the small array only).  Two plans are taken for the
-    same plan when both 64-bit halves of their keys agree; the reference's sets compare the plans' full
-    strings (aceso_utils.py:831-850)."""
+    """A visited set over 128-bit plan keys (for neighbours that only exist on the device): two native hash sets, a
+    large one and a small one that takes the new keys -- it stays in the core's cache -- and is folded into the large
+    one when it has grown.  Two plans are taken for the same plan when both 64-bit halves of their keys agree; the
+    reference's sets compare the plans' full strings (aceso_utils.py:831-850)."""
 
     SMALL_LIMIT = 65536
 
     def __init__(self):
-        self._sorted = np.empty(0, dtype=KEY128)
-        self._small = np.empty(0, dtype=KEY128)
+        self._large = _KeySet()
+        self._small = _KeySet()
 
     def __len__(self):
-        return len(self._sorted) + len(self._small)
-
-    @staticmethod
-    def _absent(sorted_keys: np.ndarray, keys: np.ndarray) -> np.ndarray:
-        if len(sorted_keys) == 0:
-            return np.ones(len(keys), dtype=bool)
-        pos = np.searchsorted(sorted_keys, keys)
-        return sorted_keys[np.minimum(pos, len(sorted_keys) - 1)] != keys
+        return len(self._large) + len(self._small)
 
     def unseen(self, keys: np.ndarray) -> np.ndarray:
         """Mask of the keys not marked before that do not repeat an earlier entry of `keys`."""
-        keys = as_key128(keys)
-        _, first = np.unique(keys, return_index=True)
-        mask = np.zeros(len(keys), dtype=bool)
-        mask[first] = True
-        cand = np.flatnonzero(mask)
-        ok = self._absent(self._sorted, keys[cand]) & self._absent(self._small, keys[cand])
-        mask[cand[~ok]] = False
+        return _first_of_each(as_key128(keys), (self._small, self._large))
+
+    def claim(self, keys: np.ndarray) -> np.ndarray:
+        """unseen(), and those keys marked."""
+        # (only what the large set lacks goes to the small one: the two stay disjoint, __len__ is their sum)
+        mask = _first_of_each(as_key128(keys), (self._small, self._large), claim=True)
+        if len(self._small) > self.SMALL_LIMIT:
+            self._large.take(self._small)
         return mask
 
     def mark(self, keys: np.ndarray) -> None:
-        k = np.unique(as_key128(keys))
-        k = k[self._absent(self._sorted, k)]              # (the two arrays stay disjoint: __len__ is their sum)
-        self._small = np.union1d(self._small, k)
-        if len(self._small) > self.SMALL_LIMIT:
-            self._sorted = np.union1d(self._sorted, self._small)
-            self._small = np.empty(0, dtype=KEY128)
+        self.claim(keys)
 
 
 def hill_climb(cm, start: PlanBatch, steps: int, n_neighbours: int, seed: int = 0, max_move: int = 8,
@@ -479,36 +479,39 @@ def hill_climb(cm, start: PlanBatch, steps: int, n_neighbours: int, seed: int = 
     cur_m = float(pk[0])
     if visited is not None:
         visited.mark(plan_keys_host(cur) if device_moves else cur)
+    draws = None
     for step in range(steps):
         if device_moves:
-            templates, moves = sample_moves(cur, tables, n_neighbours, rng, max_move)
+            if draws is None:
+                draws = _draw_moves(n_neighbours, int(cur.hdr[0, 0] & 0xff), tables, rng, max_move)
+            templates, moves = _build_moves(cur, tables, draws)
+            draws = None
             if visited is None:
-                # equal descriptors are equal plans: keep one of each (template < 2^16, op < 2^8, p1 < 2^8)
-                packed = (moves[:, 0] | (moves[:, 2] << 24)).astype(np.uint64) | (moves[:, 1].astype(np.uint64) << np.uint64(32))
-                # (first occurrences, in the order they were drawn: among neighbours of equal time the earliest wins,
-                # as it does when the duplicates are scored too)
-                moves = moves[np.sort(np.unique(packed, return_index=True)[1])]
+                # equal descriptors are equal plans: keep one of each (first occurrences, in the order they were drawn:
+                # among neighbours of equal time the earliest wins, as it does when the duplicates are scored too)
+                moves = moves[_first_of_each(moves)]
                 d = ev.apply_moves(templates, moves)
             else:
                 d, keys = ev.apply_moves(templates, moves, with_keys=True)
-                keys = as_key128(keys.cpu().numpy().view(np.uint64))
-                keep = np.flatnonzero(visited.unseen(keys))
+                keep = np.flatnonzero(visited.claim(keys.cpu().numpy().view(np.uint64)))
                 if len(keep) == 0:
                     if on_step is not None:
                         on_step(step, cur_t, cur_m)
                     continue
-                visited.mark(keys[keep])
                 moves = moves[keep]
                 d = ev.select(d, ev._torch.from_numpy(keep).to(d.hdr.device))
             if greedy_recompute:
                 d = cm.update_recompute_device(d)
             it, pk, fe, st = ev.score(d)
-            idx, val, cnt = ev.topk(it, fe, 1)
-            if int(cnt.item()) == 1 and float(val[0].item()) < cur_t:
-                best_i = int(idx[0].item())
-                cur = ev.download(d, idx[:1]) if greedy_recompute else \
+            top = ev.topk_packed(it, fe, 1)
+            if step + 1 < steps:
+                draws = _draw_moves(n_neighbours, int(cur.hdr[0, 0] & 0xff), tables, rng, max_move)
+            idx, val = ev.read_topk(top, 1)
+            if len(idx) and float(val[0]) < cur_t:
+                best_i, cur_t = int(idx[0]), float(val[0])
+                cur_m = float(pk[best_i].item())
+                cur = ev.download(d, ev._torch.tensor([best_i], device=d.hdr.device)) if greedy_recompute else \
                     apply_moves_host(templates, moves[best_i:best_i + 1], tables.db.n_algo)
-                cur_t, cur_m = float(val[0].item()), float(pk[best_i].item())
             if on_step is not None:
                 on_step(step, cur_t, cur_m)
             continue
