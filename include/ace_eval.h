@@ -291,6 +291,20 @@ int ace_recompute_select(const ace_rc_tables_t *t, uint8_t *d_codes_rw, int n_st
                          const double *d_sum_size, const int32_t *d_first_pos, uint8_t *d_recomputed, const double *d_mem,
                          double memory_limit, uint8_t *d_alive, void *stream);
 
+/* check_recompute (aceso_cost_model.py:822-872) for every stage of every plan of a batch in one launch: the loop above
+ * from the first evaluation to the last round on the device.
+ * ace_recompute_prepare uploads what it needs beside the handle's tables, once (HOST pointers): type_of_pos
+ * int32[num_ops]; activations double[num_types][n_mbs][n_tp][n_algo] and no_recompute uint8[num_types] as in
+ * ace_rc_tables_t.  ACE_ETOOBIG: more ops than a workgroup's LDS holds (4,000; ace_recompute_groups / _select then).
+ * ace_recompute_batch writes the batch's code bytes with check_recompute's recompute bits to d_codes_out (same layout as
+ * d_codes, not overlapping it).  peak_backward: args.peak_mem_in_backward.  d_status: what ace_score_batch said of these plans.
+ * d_flags: int32[4] ZEROED by the caller: [0] stage-start bits minus stage counts over the batch (the plans that do not
+ * match, if any, come back with their recompute bits cleared), [1] some plan's first op opens no stage, [2] an op of a
+ * stage above the limit sits outside the profiled grid, [3] some d_status is not 0. */
+int ace_recompute_prepare(ace_handle_t *h, const int32_t *type_of_pos, const double *activations, const uint8_t *no_recompute);
+int ace_recompute_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_limit, double peak_backward, const uint8_t *d_status,
+                        uint8_t *d_codes_out, int32_t *d_flags, void *stream);
+
 /* Average duration in milliseconds of the `reps` scoring-kernel launches of one
  * ace_score_batch-equivalent call sequence, measured with hipEvents on `stream`
  * (for bench.py's roofline figure; not part of the reference). */

@@ -9,6 +9,7 @@ LIB = os.path.join(HERE, "libace_eval.so")
 SOURCES = [os.path.join(HERE, "csrc", "ace_eval.hip")]
 HEADERS = [os.path.join(HERE, "csrc", "ace_plan_state.h"), os.path.join(HERE, "csrc", "ace_score_loop.h"),
            os.path.join(HERE, "csrc", "ace_score_loop_asm.inc"), os.path.join(HERE, "csrc", "ace_spread.h"),
+           os.path.join(HERE, "csrc", "ace_recompute.h"),
            os.path.join(HERE, "csrc", "ace_edit_kernels.h"), os.path.join(HERE, "csrc", "ace_keyset.h"),
            os.path.join(HERE, "csrc", "ace_moves_host.h"),
            os.path.join(ROOT, "include", "ace_eval.h")]

@@ -23,6 +23,7 @@
 #include "ace_moves_host.h"
 #include "ace_score_loop.h"
 #include "ace_spread.h"
+#include "ace_recompute.h"
 
 // Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans (the
 // layout ace_score_body's DEFER variant uses: [workgroup][stage][lane][ACE_WS_REC]).  Every GPU the library runs on holds
@@ -77,6 +78,11 @@ __global__ __launch_bounds__(kSpreadLanes) void ace_spread_kernel(const AceKerne
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_spread_body<BD, RANGED, COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
+template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+}
+
 // Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has four workgroups
 // (1,024 plans), that of the kernels with a plan per lane not before 16,384; they cross between 4,096 and 16,384 plans,
 // earlier without stage records (the lane-per-plan kernel defers the stage tails there).  Measured, us per launch,
@@ -956,6 +962,8 @@ struct ace_handle {
     int32_t *d_win_pos, *d_win_row_begin;
     uint32_t *d_win_rows;
     int32_t flat_rows16;       // see AceKernelArgs
+    ace_u2 *d_rc_pos;          // check_recompute's tables (ace_recompute_prepare), or null
+    double *d_rc_act;
     double *d_stage_ws;        // grow-only workspace for deferred stage tails
     size_t stage_ws_plans;     // capacity in plans
     int stage_ws_fixed;        // ace_reserve(..., fixed): a larger batch is an error instead of a reallocation
@@ -1353,6 +1361,8 @@ void ace_destroy(ace_handle_t *h) {
     if (h->d_win_dma) (void)hipFree(h->d_win_dma);
     (void)hipFree(h->d_stage_lut); (void)hipFree(h->d_nbm1); (void)hipFree(h->d_win_pos);
     (void)hipFree(h->d_win_row_begin); (void)hipFree(h->d_win_rows);
+    if (h->d_rc_pos) (void)hipFree(h->d_rc_pos);
+    if (h->d_rc_act) (void)hipFree(h->d_rc_act);
     if (h->d_stage_ws) (void)hipFree(h->d_stage_ws);
     delete h;
 }
@@ -1665,6 +1675,56 @@ int ace_recompute_select(const ace_rc_tables_t *t, uint8_t *d_codes_rw, int n_st
     hipLaunchKernelGGL(rc_select_kernel, dim3((n_stages + 127) / 128), dim3(128), 0, (hipStream_t)stream, k, d_codes_rw,
                        n_stages, d_plan, d_lo, d_hi, d_nsb, d_mrow, d_sum_size, d_first_pos, d_recomputed, d_mem,
                        memory_limit, d_alive);
+    ACE_HIP(hipGetLastError());
+    return ACE_OK;
+}
+
+int ace_recompute_prepare(ace_handle_t *h, const int32_t *type_of_pos, const double *activations, const uint8_t *no_recompute) {
+    if (!h || !type_of_pos || !activations || !no_recompute) return ACE_EINVAL;
+    const int N = h->geom.N;
+    if (N > kRcMaxOps || !h->d_pos_spread || h->num_types > 0xffff) return ACE_ETOOBIG;
+    for (int i = 0; i < N; ++i)
+        if (type_of_pos[i] < 0 || type_of_pos[i] >= h->num_types) return ACE_EINVAL;
+    RcShared s;
+    const uint32_t lds = ace_rc_layout(N, h->geom.G, nullptr, &s);
+    if (lds > kMaxLds) return ACE_ETOOBIG;
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_rc_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_rc_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    std::vector<ace_u2> pos((size_t)N);
+    ace_rc_positions(type_of_pos, no_recompute, N, h->num_types, pos.data());
+    if (h->d_rc_pos) (void)hipFree(h->d_rc_pos);
+    if (h->d_rc_act) (void)hipFree(h->d_rc_act);
+    h->d_rc_pos = nullptr;
+    h->d_rc_act = nullptr;
+    const size_t n_act = (size_t)h->num_types * h->geom.n_mbs * h->geom.n_tp * h->geom.n_algo;
+    int rc = upload((void **)&h->d_rc_pos, pos.data(), pos.size() * sizeof(ace_u2));
+    if (rc == ACE_OK) rc = upload((void **)&h->d_rc_act, activations, n_act * sizeof(double));
+    return rc;
+}
+
+int ace_recompute_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_limit, double peak_backward, const uint8_t *d_status,
+                        uint8_t *d_codes_out, int32_t *d_flags, void *stream) {
+    if (!h || !batch || batch->d_range || batch->d_order || !d_status || !d_codes_out || !d_flags || ((uintptr_t)d_codes_out & 15u))
+        return ACE_EINVAL;
+    if (!h->d_rc_pos || !h->d_rc_act) return ACE_EINVAL;
+    RcArgs a;
+    // (the scoring outputs are not written: any pointer will do)
+    double *unused = h->d_rc_act;
+    int rc = fill_args(h, batch, memory_limit, 0, unused, unused, d_codes_out, nullptr, nullptr, &a.k);
+    if (rc) return rc;
+    a.pos = h->d_rc_pos;
+    a.act = h->d_rc_act;
+    a.status = d_status;
+    a.codes_out = reinterpret_cast<ace_u4 *>(d_codes_out);
+    a.flags = d_flags;
+    a.limit = memory_limit;
+    a.peak_backward = peak_backward;
+    RcShared s;
+    const uint32_t lds = ace_rc_layout(a.k.g.N, a.k.g.G, nullptr, &s);
+    if (a.k.g.flags & ACE_F_COLLECTIVE_MEM)
+        hipLaunchKernelGGL((ace_rc_kernel<true>), dim3((unsigned)a.k.g.P), dim3(kSpreadLanes), lds, (hipStream_t)stream, a);
+    else
+        hipLaunchKernelGGL((ace_rc_kernel<false>), dim3((unsigned)a.k.g.P), dim3(kSpreadLanes), lds, (hipStream_t)stream, a);
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }

@@ -19,7 +19,7 @@ EXPORTS = ["ace_abi_version", "ace_strerror", "ace_last_hip_error", "ace_create"
            "ace_score_batch", "ace_score_batch_static", "ace_reserve", "ace_topk_workspace_bytes", "ace_topk", "ace_time_score_kernel", "ace_apply_moves",
            "ace_recompute_groups", "ace_recompute_select", "ace_group_keys", "ace_gather_plans",
            "ace_keyset_create", "ace_keyset_destroy", "ace_keyset_size", "ace_keyset_add", "ace_keyset_unseen", "ace_keyset_claim",
-           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves"]
+           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves", "ace_recompute_prepare", "ace_recompute_batch"]
 
 
 class AceBatchStruct(ctypes.Structure):
@@ -36,6 +36,9 @@ class AceRcTablesStruct(ctypes.Structure):
 class AceMoveDrawsStruct(ctypes.Structure):
     _fields_ = [("n", ctypes.c_size_t), ("count", ctypes.c_size_t * 6), ("rows", ctypes.c_void_p * 6),
                 ("x", ctypes.c_void_p * 6), ("y", ctypes.c_void_p * 6)]
+
+
+ACE_ETOOBIG = -2
 
 
 class AceError(RuntimeError):
@@ -101,6 +104,8 @@ def load_library():
     lib.ace_keyset_claim.argtypes = [ctypes.POINTER(vp), ctypes.c_int, vp, sz, vp]
     lib.ace_keyset_move.argtypes = [vp, vp]
     lib.ace_keyset_keys.argtypes = [vp, vp]
+    lib.ace_recompute_prepare.argtypes = [vp] * 4
+    lib.ace_recompute_batch.argtypes = [vp, ctypes.POINTER(AceBatchStruct), ctypes.c_double, ctypes.c_double] + [vp] * 4
     ci = ctypes.c_int
     lib.ace_build_moves.argtypes = [vp, vp, ci, ci, ci, ci, vp, ci, ctypes.POINTER(AceMoveDrawsStruct), vp, vp, vp, ci, ctypes.POINTER(ci)]
     if lib.ace_abi_version() != ABI_VERSION:
@@ -267,6 +272,7 @@ class PlanEvaluator:
         self._deal_cache = {}
         self._topk_ws = None
         self._small = None
+        self._rc_ready = None
         self._graphs_alive = 0
 
     def close(self):
@@ -470,6 +476,33 @@ class PlanEvaluator:
         _check(self.lib, rc, "ace_apply_moves")
         d = DeviceBatch.from_device(codes, hdr, N)
         return (d, keys) if with_keys else d
+
+    def prepare_recompute(self, no_recompute: np.ndarray) -> bool:
+        """Upload what check_recompute needs beside the tables (once); False if the op graph is too long for the kernel."""
+        if self._rc_ready is None:
+            t = self.tables
+            types = np.ascontiguousarray(t.graph.type_of_pos, dtype=np.int32)
+            act = np.ascontiguousarray(t.db.tables["activations"], dtype=np.float64)
+            norec = np.ascontiguousarray(no_recompute, dtype=np.uint8)
+            with self.device_context():
+                rc = self.lib.ace_recompute_prepare(self.handle, types.ctypes.data, act.ctypes.data, norec.ctypes.data)
+            if rc != ACE_ETOOBIG:
+                _check(self.lib, rc, "ace_recompute_prepare")
+            self._rc_ready = rc == 0
+        return self._rc_ready
+
+    def recompute(self, d: DeviceBatch, memory_limit: float, peak_backward: float):
+        """check_recompute's choice for every stage of every plan, after prepare_recompute: (the new batch, status of the
+        plans, int32[4] flags of ace_recompute_batch), on the device."""
+        torch = self._torch
+        status = self.score(d, memory_limit)[3]
+        codes = torch.empty_like(d.codes)
+        flags = torch.zeros(4, dtype=torch.int32, device=self.device)
+        with self.device_context():
+            _check(self.lib, self.lib.ace_recompute_batch(self.handle, ctypes.byref(d.struct), float(memory_limit), float(peak_backward),
+                                                          status.data_ptr(), codes.data_ptr(), flags.data_ptr(), self._stream()),
+                   "ace_recompute_batch")
+        return DeviceBatch.from_device(codes, d.hdr, d.num_ops), status, flags
 
     def select(self, d: DeviceBatch, index) -> DeviceBatch:
         """The plans `index` (device int64 tensor) of a device-resident batch, as a new batch."""

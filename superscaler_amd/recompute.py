@@ -180,10 +180,12 @@ def update_recompute_arrays(cm, batch: PlanBatch) -> PlanBatch:
 
 def update_recompute_device(cm, dbatch):
     """update_recompute for every stage of every plan of a device-resident batch (evaluator.DeviceBatch),
-    without the plans ever visiting the host: the same greedy loop as `update_recompute_arrays`, with
-    the selection done by the library's ace_recompute_groups / ace_recompute_select kernels and the
-    memory bookkeeping by element-wise fp64 tensor operations (the reference's order of operations,
-    one rounding each).  Returns a new DeviceBatch; bit-identical to the host form."""
+    without the plans ever visiting the host: the same greedy loop as `update_recompute_arrays`, run from
+    start to end by one launch (ace_recompute_batch).  Returns a new DeviceBatch; bit-identical to the host form.
+
+    Op graphs too long for that kernel's LDS (4,000 ops) take the loop round by round: selection by
+    ace_recompute_groups / ace_recompute_select, the memory bookkeeping by element-wise fp64 tensor operations (the
+    reference's order of operations, one rounding each)."""
     import ctypes
     import torch
     from .evaluator import AceRcTablesStruct, DeviceBatch, _check
@@ -193,13 +195,24 @@ def update_recompute_device(cm, dbatch):
     dev = dbatch.hdr.device
     N, P = dbatch.num_ops, dbatch.n_plans
     G = (N + 15) // 16
-    codes = dbatch.codes.clone()
     if not args.flex_recompute:
-        codes |= 8
+        codes = dbatch.codes | 8
         if G * 16 != N:
             codes.view(G, P, 16)[G - 1, :, N - (G - 1) * 16:] = 0
         return DeviceBatch.from_device(codes, dbatch.hdr, N)
-    codes &= 0xF7
+    n_types = len(tables.db.op_names)
+    norec = ((np.asarray(tables.graph.flags)[:n_types] & og.F_NO_RECOMPUTE) != 0).astype(np.uint8)
+    if hasattr(ev, "recompute") and ev.prepare_recompute(norec):
+        out, status, flags = ev.recompute(dbatch, args.memory_limit, args.peak_mem_in_backward)
+        count, first, grid, bad = flags.tolist()
+        if count or first:
+            raise ValueError("malformed encoding: stage bits do not match the stage counts")
+        if bad:
+            cm._raise_for_status(status.cpu().numpy())
+        if grid:
+            raise KeyError("a stage's micro-batch size per replica is not in the profile database")
+        return out
+    codes = dbatch.codes & 0xF7
     hdr = dbatch.hdr.to(torch.int64) & 0xFFFFFFFF
     # ---- every stage of every plan: (plan, first op, one past the last op, stage index) ----------
     rows = codes.permute(1, 0, 2).reshape(P, G * 16)[:, :N]
@@ -238,11 +251,9 @@ def update_recompute_device(cm, dbatch):
         return DeviceBatch.from_device(codes, dbatch.hdr, N)
 
     # ---- device tables of the selection kernels ----------------------------------------------------
-    n_types = len(tables.db.op_names)
     act_tab = np.ascontiguousarray(tables.db.tables["activations"], dtype=np.float64)
     d_act = torch.from_numpy(act_tab).to(dev)
     d_types = torch.from_numpy(np.ascontiguousarray(tables.graph.type_of_pos, dtype=np.int32)).to(dev)
-    norec = ((np.asarray(tables.graph.flags)[:n_types] & og.F_NO_RECOMPUTE) != 0).astype(np.uint8)
     d_norec = torch.from_numpy(norec).to(dev)
     lut = torch.from_numpy(np.ascontiguousarray(tables.stage_lut).astype(np.int64)).to(dev)
     t = AceRcTablesStruct(codes.data_ptr(), P, d_types.data_ptr(), d_act.data_ptr(), d_norec.data_ptr(), N, n_types,

@@ -7,6 +7,7 @@
 #include "ace_edit_kernels.h"
 #include "ace_score_loop.h"
 #include "ace_spread.h"
+#include "ace_recompute.h"
 
 #include <sys/mman.h>
 
@@ -155,9 +156,17 @@ template <bool BD, bool RANGED> void run_spread_c(const AceKernelArgs &a, Guarde
     else run_spread<BD, RANGED, false>(a, pool);
 }
 
+struct RcJob {
+    const int32_t *type_of_pos;
+    const double *activations;
+    const uint8_t *no_recompute, *status;
+    double peak_backward;
+    uint8_t *codes_out;
+    int32_t *flags;
+};
 int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, const uint32_t *order, long long P,
                double memory_limit, int strict, double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, double *stage_out,
-               bool spread);
+               bool spread, const RcJob *rc = nullptr);
 
 }  // namespace
 
@@ -174,10 +183,20 @@ extern "C" int ace_emu_spread(const ace_tables_t *t, const uint8_t *codes, const
     return emu_kernel(t, codes, hdr, range, order, P, memory_limit, strict, iter_ms, peak_mb, feasible, status, stage_out, true);
 }
 
+// ace_recompute_batch: codes and codes_out uint8 [G][P][16], flags int32 [4] zeroed by the caller.
+extern "C" int ace_emu_recompute(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, long long P, double memory_limit,
+                                 double peak_backward, const int32_t *type_of_pos, const double *activations, const uint8_t *no_recompute,
+                                 const uint8_t *status, uint8_t *codes_out, int32_t *flags) {
+    const RcJob rc{type_of_pos, activations, no_recompute, status, peak_backward, codes_out, flags};
+    std::vector<double> d((size_t)P);
+    std::vector<uint8_t> b((size_t)P);
+    return emu_kernel(t, codes, hdr, nullptr, nullptr, P, memory_limit, 0, d.data(), d.data(), b.data(), nullptr, nullptr, true, &rc);
+}
+
 namespace {
 int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, const uint32_t *order, long long P,
                double memory_limit, int strict, double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, double *stage_out,
-               bool spread) {
+               bool spread, const RcJob *rc) {
     if (range && !stage_out) return -1;
     AceKernelArgs a;
     memset(&a, 0, sizeof(a));
@@ -245,6 +264,30 @@ int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr,
         double *padded = (double *)pool.place(nullptr, rows + 4096);
         memcpy(padded, t->rows, rows);
         a.rows = padded;
+        if (rc) {
+            const size_t N = (size_t)g.N, n_act = (size_t)t->num_types * t->n_mbs * t->n_tp * t->n_algo;
+            RcArgs r;
+            r.k = a;
+            ace_u2 *pos = (ace_u2 *)pool.place(nullptr, N * 8, 8);
+            ace_rc_positions(rc->type_of_pos, rc->no_recompute, g.N, t->num_types, pos);
+            r.pos = pos;
+            r.act = (const double *)pool.place(rc->activations, n_act * 8, 8);
+            r.status = (const uint8_t *)pool.place(rc->status, (size_t)P, 1);
+            r.codes_out = (ace_u4 *)pool.place(nullptr, G * (size_t)P * 16);
+            r.flags = rc->flags;
+            r.limit = memory_limit;
+            r.peak_backward = rc->peak_backward;
+            RcShared sh;
+            const uint32_t bytes = ace_rc_layout(g.N, g.G, nullptr, &sh);
+            unsigned char *rlds = (unsigned char *)pool.place(nullptr, bytes);
+            for (long long p = 0; p < P; ++p) {
+                memset(rlds, 0xff, bytes);
+                if (g.flags & ACE_F_COLLECTIVE_MEM) ace_rc_body<true>(r, rlds, 0, p);
+                else ace_rc_body<false>(r, rlds, 0, p);
+            }
+            memcpy(rc->codes_out, r.codes_out, G * (size_t)P * 16);
+            return 0;
+        }
         if (range) run_spread_c<true, true>(a, pool);
         else if (stage_out) run_spread_c<true, false>(a, pool);
         else run_spread_c<false, false>(a, pool);
