@@ -258,6 +258,17 @@ int ace_group_keys(const uint8_t *d_codes, const uint32_t *d_hdr, size_t n_plans
 int ace_gather_plans(const uint8_t *d_codes_in, const uint32_t *d_hdr_in, const uint32_t *d_perm, size_t n_plans, int num_ops,
                      uint8_t *d_codes_out, uint32_t *d_hdr_out, void *stream);
 
+/* Plans from the host's layout -- d_rows: uint8[n_plans][num_ops], a row of code bytes per plan, as it was copied to the
+ * device -- to the layout of ace_batch_t (d_codes_out: uint8[ceil(num_ops / 16)][n_plans][16], zero padded), and back.
+ * With d_hdr (uint32[n_plans][4]) the packing also checks the batch and ORs what it finds into *d_flags (int32, zeroed by the
+ * caller): 1 a number of stages outside 1..ACE_MAX_STAGES, 2 stage-start bits that disagree with it, 4 a first op that opens no
+ * stage, 8 a micro-batch index >= n_mbs, 16 a code (bits 0-2) >= n_codes.  ace_check_plans: the same check in host memory,
+ * returns those bits.  Device pointers are 16-byte aligned. */
+int ace_pack_plans(const uint8_t *d_rows, size_t n_plans, int num_ops, const uint32_t *d_hdr, int n_mbs, int n_codes,
+                   uint8_t *d_codes_out, int32_t *d_flags, void *stream);
+int ace_unpack_plans(const uint8_t *d_codes, size_t n_plans, int num_ops, uint8_t *d_rows_out, void *stream);
+int ace_check_plans(const uint8_t *codes, const uint32_t *hdr, size_t n_plans, int num_ops, int n_mbs, int n_codes);
+
 /* The two steps of check_recompute's greedy loop (aceso_cost_model.py:822-872) that are not a stage
  * evaluation, for many encoded stages at once (one stage = the ops [lo, hi) of one plan of the batch).
  * The caller runs the loop: evaluate the stages (ace_score_batch with d_range), update their memory

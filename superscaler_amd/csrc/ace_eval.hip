@@ -20,6 +20,7 @@
 
 #include "ace_edit_kernels.h"
 #include "ace_keyset.h"
+#include "ace_pack.h"
 #include "ace_moves_host.h"
 #include "ace_score_loop.h"
 #include "ace_spread.h"
@@ -987,6 +988,16 @@ __global__ __launch_bounds__(256) void gather_plans_kernel(const ace_u4 *codes_i
     gather_plans_body((unsigned long long)blockIdx.x * 256 + threadIdx.x, codes_in, hdr_in, perm, n, G, codes_out, hdr_out);
 }
 
+__global__ __launch_bounds__(kPackLanes) void pack_plans_kernel(const PackArgs a) {
+    __shared__ PackShared s;
+    ace_pack_body(a, s, (int)threadIdx.x, (long long)blockIdx.x);
+}
+
+__global__ __launch_bounds__(kPackLanes) void unpack_plans_kernel(const PackArgs a) {
+    __shared__ PackShared s;
+    ace_unpack_body(a, s, (int)threadIdx.x, (long long)blockIdx.x);
+}
+
 __global__ void rc_groups_kernel(RcTables t, int n, const int32_t *q_plan, const int32_t *q_lo, const int32_t *q_hi,
                                  const int32_t *q_nsb, const uint32_t *q_mrow, double *sum_size, int32_t *first_pos,
                                  int32_t *bad) {
@@ -1644,6 +1655,34 @@ int ace_gather_plans(const uint8_t *d_codes_in, const uint32_t *d_hdr_in, const 
                        (unsigned long long)n_plans, G, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<ace_u4 *>(d_hdr_out));
     ACE_HIP(hipGetLastError());
     return ACE_OK;
+}
+
+int ace_pack_plans(const uint8_t *d_rows, size_t n_plans, int num_ops, const uint32_t *d_hdr, int n_mbs, int n_codes,
+                   uint8_t *d_codes_out, int32_t *d_flags, void *stream) {
+    if (!d_rows || !d_codes_out || n_plans == 0 || n_plans > 0x7fffffffull || num_ops <= 0 || num_ops >= (1 << 20) || (d_hdr && !d_flags) ||
+        n_codes < 1 || n_codes > 8 || ((uintptr_t)d_rows & 15u) || ((uintptr_t)d_codes_out & 15u) || ((uintptr_t)d_hdr & 15u))
+        return ACE_EINVAL;
+    PackArgs a{d_rows, nullptr, nullptr, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<const ace_u4 *>(d_hdr), d_flags,
+               (long long)n_plans, num_ops, (num_ops + 15) / 16, n_mbs, n_codes};
+    hipLaunchKernelGGL(pack_plans_kernel, dim3((unsigned)((n_plans + kPackPlans - 1) / kPackPlans)), dim3(kPackLanes), 0, (hipStream_t)stream, a);
+    ACE_HIP(hipGetLastError());
+    return ACE_OK;
+}
+
+int ace_unpack_plans(const uint8_t *d_codes, size_t n_plans, int num_ops, uint8_t *d_rows_out, void *stream) {
+    if (!d_codes || !d_rows_out || n_plans == 0 || n_plans > 0x7fffffffull || num_ops <= 0 || num_ops >= (1 << 20) ||
+        ((uintptr_t)d_codes & 15u) || ((uintptr_t)d_rows_out & 15u))
+        return ACE_EINVAL;
+    PackArgs a{nullptr, d_rows_out, reinterpret_cast<const ace_u4 *>(d_codes), nullptr, nullptr, nullptr, (long long)n_plans, num_ops,
+               (num_ops + 15) / 16, 0, 8};
+    hipLaunchKernelGGL(unpack_plans_kernel, dim3((unsigned)((n_plans + kPackPlans - 1) / kPackPlans)), dim3(kPackLanes), 0, (hipStream_t)stream, a);
+    ACE_HIP(hipGetLastError());
+    return ACE_OK;
+}
+
+int ace_check_plans(const uint8_t *codes, const uint32_t *hdr, size_t n_plans, int num_ops, int n_mbs, int n_codes) {
+    if (!codes || !hdr || num_ops <= 0 || n_codes < 1 || n_codes > 8) return ACE_EINVAL;
+    return ace_check_plans_host(codes, hdr, n_plans, num_ops, n_mbs, n_codes);
 }
 
 int ace_recompute_groups(const ace_rc_tables_t *t, int n_stages, const int32_t *d_plan, const int32_t *d_lo,

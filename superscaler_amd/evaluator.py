@@ -9,7 +9,7 @@ from typing import Optional
 
 import numpy as np
 
-from .plan import PlanBatch, validate_batch
+from .plan import PlanBatch, check_shape, finding, validate_batch
 from .tables import ABI_VERSION, MAX_STAGES, STAGE_REC, AceTablesStruct, CompiledTables
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libace_eval.so")
@@ -19,7 +19,8 @@ EXPORTS = ["ace_abi_version", "ace_strerror", "ace_last_hip_error", "ace_create"
            "ace_score_batch", "ace_score_batch_static", "ace_reserve", "ace_topk_workspace_bytes", "ace_topk", "ace_time_score_kernel", "ace_apply_moves",
            "ace_recompute_groups", "ace_recompute_select", "ace_group_keys", "ace_gather_plans",
            "ace_keyset_create", "ace_keyset_destroy", "ace_keyset_size", "ace_keyset_add", "ace_keyset_unseen", "ace_keyset_claim",
-           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves", "ace_recompute_prepare", "ace_recompute_batch"]
+           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves", "ace_recompute_prepare", "ace_recompute_batch",
+           "ace_pack_plans", "ace_unpack_plans", "ace_check_plans"]
 
 
 class AceBatchStruct(ctypes.Structure):
@@ -104,6 +105,9 @@ def load_library():
     lib.ace_keyset_claim.argtypes = [ctypes.POINTER(vp), ctypes.c_int, vp, sz, vp]
     lib.ace_keyset_move.argtypes = [vp, vp]
     lib.ace_keyset_keys.argtypes = [vp, vp]
+    lib.ace_pack_plans.argtypes = [vp, sz, ctypes.c_int, vp, ctypes.c_int, ctypes.c_int, vp, vp, vp]
+    lib.ace_unpack_plans.argtypes = [vp, sz, ctypes.c_int, vp, vp]
+    lib.ace_check_plans.argtypes = [vp, vp, sz, ctypes.c_int, ctypes.c_int, ctypes.c_int]
     lib.ace_recompute_prepare.argtypes = [vp] * 4
     lib.ace_recompute_batch.argtypes = [vp, ctypes.POINTER(AceBatchStruct), ctypes.c_double, ctypes.c_double] + [vp] * 4
     ci = ctypes.c_int
@@ -186,57 +190,92 @@ def pack_small_inputs(buf: np.ndarray, batch: PlanBatch, ranges) -> int:
     return n_in
 
 
+STAGING_PIECE = 8 << 20      # bytes of plans staged at a time: the copy to the device of one runs beside the staging of the next
+
+
+def rows_to_device(batch: PlanBatch, device, staging=None):
+    """The code rows (uint8 [P, N]) and headers (int32 [P, 4]) of a host batch on the device, in the host's layout.  Plans in
+    page-locked memory (PlanEvaluator.pinned_plan_batch) are read where they are; others go through `staging` (see
+    DeviceBatch), if there is one, piece by piece."""
+    import torch
+    pinned = getattr(batch, "pinned_tensors", None)
+    if pinned is not None:
+        return pinned[0].to(device, non_blocking=True), pinned[1].to(device, non_blocking=True)
+    host_rows = torch.from_numpy(np.ascontiguousarray(batch.codes))
+    host_hdr = torch.from_numpy(np.ascontiguousarray(batch.hdr).view(np.int32))
+    if staging is None:
+        return host_rows.to(device), host_hdr.to(device)
+    P, N = host_rows.shape
+    stage = staging[:P * N].view(P, N)
+    stage_hdr = staging[P * N:P * N + 16 * P].view(P, 16)
+    rows = torch.empty((P, N), dtype=torch.uint8, device=device)
+    per = max(1, STAGING_PIECE // N)
+    for lo in range(0, P, per):
+        stage[lo:lo + per].copy_(host_rows[lo:lo + per])
+        rows[lo:lo + per].copy_(stage[lo:lo + per], non_blocking=True)
+    stage_hdr.copy_(host_hdr.view(torch.uint8).view(P, 16))
+    hdr = torch.empty((P, 4), dtype=torch.int32, device=device)
+    hdr.view(torch.uint8).view(P, 16).copy_(stage_hdr, non_blocking=True)
+    return rows, hdr
+
+
+def pack_rows(rows, hdr, check=None):
+    """Code rows [P, N] on the device -> [ceil(N / 16), P, 16] (plan-minor, sixteen ops per 16-byte word, zero padded);
+    `check` as in DeviceBatch."""
+    import torch
+    P, N = rows.shape
+    G = (N + 15) // 16
+    if rows.device.type != "cuda":
+        return torch.nn.functional.pad(rows, (0, G * 16 - N)).view(P, G, 16).permute(1, 0, 2).contiguous()
+    lib = load_library()
+    codes = torch.empty((G, P, 16), dtype=torch.uint8, device=rows.device)
+    n_mbs, n_codes = check or (0, 8)
+    flags = torch.zeros(1, dtype=torch.int32, device=rows.device) if check else None
+    with torch.cuda.device(rows.device):
+        _check(lib, lib.ace_pack_plans(rows.data_ptr(), P, N, hdr.data_ptr() if check else None, n_mbs, n_codes, codes.data_ptr(),
+                                       flags.data_ptr() if check else None,
+                                       torch.cuda.current_stream(rows.device).cuda_stream), "ace_pack_plans")
+    if check:
+        msg = finding(int(flags.item()))
+        if msg:
+            raise ValueError(msg)
+    return codes
+
+
 class DeviceBatch:
     """A PlanBatch resident in HBM in the layout the kernel streams."""
 
     def __init__(self, batch: PlanBatch, device="cuda:0", ranges: Optional[np.ndarray] = None, staging=None,
-                 group_by_depth: bool = False):
-        """`staging`: a pinned uint8 host tensor of at least P * N bytes; the plan bytes then go through
+                 group_by_depth: bool = False, check=None):
+        """`staging`: a pinned uint8 host tensor of at least P * N + 16 * P bytes; the plans then go through
         it and the copy to the device does not block the host (the caller must not reuse the tensor
         before that copy has completed).
         `group_by_depth`: store the plans sorted by pipeline depth (deepest first) and position of the
         first two stage boundaries, with the permutation alongside (`order`), so that the lanes of a
-        wavefront close their stages together; results still come back in the caller's order."""
+        wavefront close their stages together; results still come back in the caller's order.
+        `check`: (micro-batch sizes, codes) of the tables; the plans' structure is then checked on the way
+        (ValueError)."""
         import torch
-        self.n_plans = batch.n_plans
-        self.num_ops = batch.num_ops
         P, N = batch.codes.shape
-        G = (N + 15) // 16
-        host_codes, host_hdr = batch.codes, batch.hdr
-        self.order = None
+        order = None
         if group_by_depth and P > 1:
             perm = depth_order(batch)
-            host_codes, host_hdr = host_codes[perm], host_hdr[perm]
+            batch = PlanBatch(batch.codes[perm], batch.hdr[perm])
             if ranges is not None:
                 ranges = np.asarray(ranges)[perm]
-            self.order = torch.from_numpy(perm.astype(np.int32)).to(device)
-        pinned = getattr(batch, "pinned_tensors", None) if host_codes is batch.codes else None
-        if pinned is not None:
-            # the plans were produced in page-locked memory (PlanEvaluator.pinned_plan_batch): the copy to the device reads
-            # them where they are, no staging copy on the host
-            codes = pinned[0].to(device, non_blocking=True)
-        elif staging is not None:
-            stage = staging[:P * N].view(P, N)
-            stage.copy_(torch.from_numpy(np.ascontiguousarray(host_codes)))
-            codes = stage.to(device, non_blocking=True)
-        else:
-            codes = torch.from_numpy(np.ascontiguousarray(host_codes)).to(device)
-        if G * 16 != N:
-            codes = torch.nn.functional.pad(codes, (0, G * 16 - N))
-        # [P, G, 16] -> [G, P, 16]: plan-minor, sixteen ops per 16-byte word
-        self.codes = codes.view(P, G, 16).permute(1, 0, 2).contiguous()
-        if pinned is not None:
-            self.hdr = pinned[1].to(device, non_blocking=True)
-        else:
-            self.hdr = torch.from_numpy(np.ascontiguousarray(host_hdr).view(np.int32)).to(device)
-        self.ranges = None
+            order = torch.from_numpy(perm.astype(np.int32)).to(device)
+        rows, hdr = rows_to_device(batch, device, staging)
         if ranges is not None:
             r = np.ascontiguousarray(ranges, dtype=np.uint32)
             assert r.shape == (P, 2)
-            self.ranges = torch.from_numpy(r.view(np.int32)).to(device)
-        self.struct = AceBatchStruct(self.codes.data_ptr(), self.hdr.data_ptr(),
-                                     self.ranges.data_ptr() if self.ranges is not None else None, P,
-                                     self.order.data_ptr() if self.order is not None else None)
+            ranges = torch.from_numpy(r.view(np.int32)).to(device)
+        self._set(pack_rows(rows, hdr, check), hdr, N, ranges, order)
+
+    def _set(self, codes, hdr, num_ops, ranges, order):
+        self.n_plans, self.num_ops = int(hdr.shape[0]), int(num_ops)
+        self.codes, self.hdr, self.ranges, self.order = codes, hdr, ranges, order
+        self.struct = AceBatchStruct(codes.data_ptr(), hdr.data_ptr(), ranges.data_ptr() if ranges is not None else None,
+                                     self.n_plans, order.data_ptr() if order is not None else None)
 
     @classmethod
     def from_device(cls, codes, hdr, num_ops: int, ranges=None, order=None):
@@ -244,10 +283,7 @@ class DeviceBatch:
         [P, 4], ranges (single-stage queries) int32 [P, 2] or None, order int32 [P] (result index of the plan in
         each slot) or None."""
         self = cls.__new__(cls)
-        self.n_plans, self.num_ops = int(hdr.shape[0]), int(num_ops)
-        self.codes, self.hdr, self.ranges, self.order = codes, hdr, ranges, order
-        self.struct = AceBatchStruct(codes.data_ptr(), hdr.data_ptr(), ranges.data_ptr() if ranges is not None else None,
-                                     self.n_plans, order.data_ptr() if order is not None else None)
+        self._set(codes, hdr, num_ops, ranges, order)
         return self
 
     @property
@@ -290,11 +326,16 @@ class PlanEvaluator:
                staging=None, group_by_depth: bool = False) -> DeviceBatch:
         """`validate` checks the encoding on the host first (a clear message instead of per-plan status
         bytes; the kernel itself is safe for any byte content).  `group_by_depth`: see DeviceBatch."""
+        check = None
         if validate and ranges is None:
-            msg = validate_batch(batch, self.tables)
+            # (small batches are checked before they go anywhere; for others the check rides on the device's packing of the
+            # plans and costs the read-back of its findings)
+            small = batch.codes.size <= self.HOST_CHECK_BYTES
+            msg = validate_batch(batch, self.tables) if small else check_shape(batch, self.tables)
             if msg:
                 raise ValueError(msg)
-        return DeviceBatch(batch, self.device, ranges, staging, group_by_depth)
+            check = None if small else (len(self.tables.db.mbs_list), self.tables.C)
+        return DeviceBatch(batch, self.device, ranges, staging, group_by_depth, check)
 
     def pinned_plan_batch(self, n_plans: int) -> PlanBatch:
         """An empty PlanBatch (codes uint8 [n_plans, N], hdr uint32 [n_plans, 4]) whose arrays live in page-locked host
@@ -422,23 +463,25 @@ class PlanEvaluator:
         def upload(b):
             # buffer `turn` was last used two batches ago, and that batch has been scored and synchronised
             # (plans that already sit in page-locked memory need no staging buffer)
-            need = b.n_plans * b.num_ops
+            need = b.n_plans * (b.num_ops + 16)
             if getattr(b, "pinned_tensors", None) is None and (staging[turn[0]] is None or staging[turn[0]].numel() < need):
                 staging[turn[0]] = torch.empty(need, dtype=torch.uint8, pin_memory=True)
+            # (only copies on the second stream, so that the bus never waits for a kernel)
             with torch.cuda.stream(copy_stream):
-                d = self.upload(b, validate=False, staging=staging[turn[0]])
+                rows, hdr = rows_to_device(b, self.device, staging[turn[0]])
                 ev = torch.cuda.Event()
                 ev.record(copy_stream)
             turn[0] ^= 1
-            return d, ev
+            return rows, hdr, ev
 
         nxt = next(it, None)
         pending = upload(nxt) if nxt is not None else None
         while pending is not None:
-            d, ready = pending
+            rows, hdr, ready = pending
             nxt = next(it, None)
             pending = upload(nxt) if nxt is not None else None     # overlaps with the scoring below
             main.wait_event(ready)
+            d = DeviceBatch.from_device(pack_rows(rows, hdr), hdr, rows.shape[1])
             t, pk, fe, st = self.score(d, memory_limit, strict)
             idx, val = self.read_topk(self.topk_packed(t, fe, k), k)   # synchronises this batch
             best_idx = np.concatenate([best_idx, idx + offset])
@@ -446,7 +489,7 @@ class PlanEvaluator:
             order = np.lexsort((best_idx, best_val))[:k]
             best_idx, best_val = best_idx[order], best_val[order]
             offset += d.n_plans
-            del d
+            del d, rows, hdr
         return best_idx, best_val, offset
 
     def apply_moves(self, templates: PlanBatch, moves: np.ndarray, with_keys: bool = False):
@@ -517,9 +560,21 @@ class PlanEvaluator:
             d = self.select(d, index)
         if d.order is not None:
             raise ValueError("download: the batch is stored in grouped order (group_by_depth)")
-        G, P, _ = d.codes.shape
-        codes = d.codes.permute(1, 0, 2).reshape(P, G * 16)[:, :d.num_ops].contiguous().cpu().numpy()
-        return PlanBatch(codes, d.hdr.cpu().numpy().view(np.uint32).copy())
+        torch = self._torch
+        P, N = d.n_plans, d.num_ops
+        both = torch.empty(16 * P + P * N, dtype=torch.uint8, device=self.device)
+        both[:16 * P].copy_(d.hdr.view(torch.uint8).view(-1))
+        with self.device_context():
+            _check(self.lib, self.lib.ace_unpack_plans(d.codes.data_ptr(), P, N, both.data_ptr() + 16 * P, self._stream()), "ace_unpack_plans")
+        # (up to PINNED_RESULT_BYTES the arrays handed out are page-locked: one copy at the bus's rate, no second one)
+        if both.numel() <= self.PINNED_RESULT_BYTES:
+            host = torch.empty(both.numel(), dtype=torch.uint8, pin_memory=True)
+            host.copy_(both, non_blocking=True)
+            torch.cuda.current_stream(self.device).synchronize()
+        else:
+            host = both.cpu()
+        host = host.numpy()
+        return PlanBatch(host[16 * P:].reshape(P, N), host[:16 * P].view(np.uint32).reshape(P, 4))
 
     def group(self, d: DeviceBatch) -> DeviceBatch:
         """A copy of a device-resident batch in grouped storage order (see DeviceBatch), made on the
@@ -559,6 +614,9 @@ class PlanEvaluator:
         pick = out[4][torch.from_numpy(np.ascontiguousarray(plan_idx)).to(self.device),
                       torch.from_numpy(np.ascontiguousarray(stage_idx)).to(self.device)]
         return out[3].cpu().numpy(), pick.cpu().numpy()
+
+    PINNED_RESULT_BYTES = 64 << 20
+    HOST_CHECK_BYTES = 128 << 10     # (the host checks 4 to 8 GB/s, the read-back is 20 us)
 
     # ---- small host-in / host-out calls ------------------------------------------------------------
     # The reference's search calls the cost model for one plan or one stage at a time, so the time of such
@@ -614,16 +672,16 @@ class PlanEvaluator:
     # convenience: host in, host out
     def score_host(self, batch: PlanBatch, memory_limit=None, strict=False, breakdown=False, ranges=None,
                    group_by_depth: bool = False):
-        if ranges is None:
-            msg = validate_batch(batch, self.tables)
-            if msg:
-                raise ValueError(msg)
-        if not group_by_depth and batch.n_plans <= 4096:
+        if not group_by_depth and batch.n_plans <= 4096 and batch.codes.size < self.SMALL_IO_BYTES:
+            if ranges is None:
+                msg = validate_batch(batch, self.tables)
+                if msg:
+                    raise ValueError(msg)
             limit = float(self.tables.settings.memory_limit if memory_limit is None else memory_limit)
             out = self._score_small(batch, limit, strict, breakdown, ranges)
             if out is not None:
                 return out
-        d = self.upload(batch, validate=False, ranges=ranges, group_by_depth=group_by_depth)
+        d = self.upload(batch, ranges=ranges, group_by_depth=group_by_depth)
         out = self.score(d, memory_limit, strict, breakdown)
         self._torch.cuda.synchronize(self.device)
         return tuple(None if t is None else t.cpu().numpy() for t in out)

@@ -255,25 +255,34 @@ class PlanBatch:
         return np.ascontiguousarray(padded.reshape(P, G, 16).transpose(1, 0, 2))
 
 
-def validate_batch(batch: PlanBatch, tables: CompiledTables) -> Optional[str]:
-    """Cheap structural check of an array-form batch; returns a message or None."""
+# what the structural check of a batch finds wrong (ace_check_plans / ace_pack_plans), in this order
+FINDINGS = ("num_stages outside 1..16", "stage-start bits disagree with num_stages", "op 0 must start a stage",
+            "micro-batch index outside the profile database", "tp/algo code outside the profile database")
+
+
+def finding(bits: int) -> Optional[str]:
+    """The message for the first of the findings."""
+    return next((m for k, m in enumerate(FINDINGS) if bits >> k & 1), None)
+
+
+def check_shape(batch: PlanBatch, tables: CompiledTables) -> Optional[str]:
     P, N = batch.codes.shape
     if N != tables.graph.num_ops:
         return f"batch has {N} ops per plan, op graph {tables.graph.num_ops}"
     if P == 0:
         return "empty batch"
-    S = batch.hdr[:, 0] & 0xff
-    if np.any(S < 1) or np.any(S > MAX_STAGES):
-        return "num_stages outside 1..16"
-    if np.any(((batch.codes >> 4) & 1).sum(axis=1) != S):
-        return "stage-start bits disagree with num_stages"
-    if np.any((batch.codes[:, 0] & 16) == 0):
-        return "op 0 must start a stage"
-    if np.any((batch.hdr[:, 0] >> 8) & 0xff >= len(tables.db.mbs_list)):
-        return "micro-batch index outside the profile database"
-    if np.any((batch.codes & 7) >= tables.C):
-        return "tp/algo code outside the profile database"
     return None
+
+
+def validate_batch(batch: PlanBatch, tables: CompiledTables) -> Optional[str]:
+    """Cheap structural check of an array-form batch; returns a message or None."""
+    msg = check_shape(batch, tables)
+    if msg:
+        return msg
+    from .evaluator import load_library
+    codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr)
+    return finding(load_library().ace_check_plans(codes.ctypes.data, hdr.ctypes.data, codes.shape[0], codes.shape[1],
+                                                  len(tables.db.mbs_list), tables.C))
 
 
 # model_size -> (num_layers, seq_len, hidden, ffn_hidden, heads, kv_channels, vocab)  (aceso_utils.py:27-34)

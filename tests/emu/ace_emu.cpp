@@ -8,6 +8,7 @@
 #include "ace_score_loop.h"
 #include "ace_spread.h"
 #include "ace_recompute.h"
+#include "ace_pack.h"
 
 #include <sys/mman.h>
 
@@ -445,3 +446,31 @@ extern "C" int ace_emu_gather_plans(const uint8_t *codes_in, const uint32_t *hdr
     return 0;
 }
 
+// ace_pack_plans (with the check) / ace_unpack_plans; returns the findings.
+extern "C" int ace_emu_pack(const uint8_t *rows, const uint32_t *hdr, long long P, int N, int n_mbs, int C, uint8_t *codes_out) {
+    GuardedPool pool;
+    const int G = (N + 15) / 16;
+    int32_t flags = 0;
+    PackShared *s = (PackShared *)pool.place(nullptr, sizeof(PackShared));
+    PackArgs a{(const uint8_t *)pool.place(rows, (size_t)P * N), nullptr, nullptr, (ace_u4 *)pool.place(nullptr, (size_t)G * P * 16),
+               (const ace_u4 *)pool.place(hdr, (size_t)P * 16), &flags, P, N, G, n_mbs, C};
+    for (long long b = 0; b < (P + kPackPlans - 1) / kPackPlans; ++b) {
+        memset((void *)s, 0xff, sizeof(*s));
+        ace_pack_body(a, *s, 0, b);
+    }
+    memcpy(codes_out, a.codes_out, (size_t)G * P * 16);
+    return flags;
+}
+extern "C" int ace_emu_unpack(const uint8_t *codes, long long P, int N, uint8_t *rows_out) {
+    GuardedPool pool;
+    const int G = (N + 15) / 16;
+    PackShared *s = (PackShared *)pool.place(nullptr, sizeof(PackShared));
+    PackArgs a{nullptr, (uint8_t *)pool.place(nullptr, (size_t)P * N), (const ace_u4 *)pool.place(codes, (size_t)G * P * 16), nullptr, nullptr, nullptr,
+               P, N, G, 0, 8};
+    for (long long b = 0; b < (P + kPackPlans - 1) / kPackPlans; ++b) {
+        memset((void *)s, 0xff, sizeof(*s));
+        ace_unpack_body(a, *s, 0, b);
+    }
+    memcpy(rows_out, a.rows_out, (size_t)P * N);
+    return 0;
+}
