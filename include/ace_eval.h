@@ -159,6 +159,19 @@ int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_lim
                     double *d_iter_ms, double *d_peak_mb, uint8_t *d_feasible, uint8_t *d_status,
                     double *d_stage_out, void *stream);
 
+/* A small batch in HOST memory, scored and waited for in one call: what a search that asks about one plan or stage at a time
+ * waits for.  codes: uint8[n_plans][num_ops] (a row of code bytes per plan), hdr: uint32[n_plans][4], range: NULL or
+ * uint32[n_plans][2] (single-stage queries).  times: double[2][n_plans] (iteration times, then peak memory), flags:
+ * uint8[2][n_plans] (feasible, then status), stage_out: NULL (only without range) or the stage records as in
+ * ace_score_batch, zero where a plan has no stage.  The kernel reads and writes page-locked buffers of the handle (1 MiB each
+ * way, allocated on first use) where they are.  ACE_ETOOBIG: the batch does not fit them, nothing was done. */
+int ace_score_host(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, size_t n_plans,
+                   double memory_limit, int strict, double *times, uint8_t *flags, double *stage_out, void *stream);
+
+/* What ace_score_host hands to the kernel, laid out in `out` (HOST memory; NULL: only the size): codes [G][P][16], zero padded,
+ * then the headers, then the ranges if there are any.  Returns the number of bytes. */
+size_t ace_pack_host(const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, size_t n_plans, int num_ops, uint8_t *out);
+
 /* ace_score_batch for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): plain scoring (no d_stage_out, no batch->d_range) of at most
  * ACE_STATIC_MAX_PLANS plans, with the deferred-stage-tail records in a static device array of the library

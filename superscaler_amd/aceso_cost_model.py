@@ -27,6 +27,7 @@ from typing import List, Optional, Sequence
 import numpy as np
 
 from . import opgraph as og
+from .evaluator import load_objects
 from .plan import AcesoConfig, AcesoStageInfo, PlanBatch, get_config  # noqa: F401 (re-exported)
 from .profile_db import CostModelSettings, ProfileDB
 from .tables import (MAX_STAGES, R_ACT, R_BWD, R_FWD, R_IDEAL_BWD, R_IDEAL_FWD, R_IDEAL_IN, R_IDEAL_OUT, R_IN_COMM,
@@ -146,6 +147,10 @@ class CostModel:
     def _fill_breakdown(self, config, rec, print_time=False, print_memory=False):
         """aceso_cost_model.py:541-672 from the kernel's per-stage records."""
         args = self.settings
+        if not print_time and not print_memory and load_objects().fill(config, rec, args.memory_limit, args.memory_main_params,
+                                                                       args.memory_optimizer, args.consider_reserved_space):
+            return
+        # (what follows is the same in Python: for the printed breakdown, and for plan objects of other shapes than a search's)
         num_batches = config.global_bs // config.micro_bs
         _time_list, memory_list, compute_time_list, efficiency_list, gpu_time_list = [], [], [], [], []
         ideal_per_gpu, eff_loss_list, recomp_list = [], [], []

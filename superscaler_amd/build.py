@@ -20,6 +20,21 @@ FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-shared", "-fPIC", "-ffp
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(HERE, "csrc")]
 
+# walks plan objects for the one-call-at-a-time API: a CPython extension module, host code only (no contraction: see above)
+OBJECTS_SOURCE = os.path.join(HERE, "csrc", "ace_objects.cpp")
+OBJECTS_LIB = os.path.join(HERE, "_ace_objects.so")
+
+
+def build_objects(verbose: bool = True) -> str:
+    import sysconfig
+    cmd = ["g++", "-O2", "-std=c++17", "-shared", "-fPIC", "-ffp-contract=off", "-I" + sysconfig.get_paths()["include"], OBJECTS_SOURCE, "-o", OBJECTS_LIB]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + proc.stdout)
+    return OBJECTS_LIB
+
 
 def source_hash() -> str:
     """sha256 over the library's sources (the files `build` compiles, in a fixed order): names what a set of
@@ -44,14 +59,15 @@ def build(verbose: bool = True) -> str:
         raise RuntimeError("hipcc failed:\n" + out)
     if verbose and out.strip():
         print(out)
+    build_objects(verbose)
     return LIB
 
 
 def is_stale() -> bool:
-    if not os.path.exists(LIB):
+    if not os.path.exists(LIB) or not os.path.exists(OBJECTS_LIB):
         return True
-    t = os.path.getmtime(LIB)
-    return any(os.path.getmtime(p) > t for p in SOURCES + HEADERS)
+    t = min(os.path.getmtime(LIB), os.path.getmtime(OBJECTS_LIB))
+    return any(os.path.getmtime(p) > t for p in SOURCES + HEADERS + [OBJECTS_SOURCE])
 
 
 if __name__ == "__main__":

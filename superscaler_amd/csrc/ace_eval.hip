@@ -44,6 +44,7 @@ constexpr int kSmallBlock = 256;         // ... for small batches: 4 wavefronts,
 #endif
 constexpr int kSmallBatchBlocks = ACE_SMALL_BATCH_BLOCKS;   // batches of fewer than this many kBlock workgroups use kSmallBlock
 constexpr uint32_t kMaxLds = 160 * 1024;  // CDNA4 LDS per workgroup
+constexpr size_t kHostIoBytes = 1 << 20;  // page-locked buffers of ace_score_host, each way
 static_assert(ACE_STATIC_MAX_PLANS % ACE_BLOCK == 0, "the static scratch holds whole workgroups");
 
 thread_local char g_hip_err[256] = "";
@@ -965,6 +966,7 @@ struct ace_handle {
     int32_t flat_rows16;       // see AceKernelArgs
     ace_u2 *d_rc_pos;          // check_recompute's tables (ace_recompute_prepare), or null
     double *d_rc_act;
+    unsigned char *host_in, *host_out;   // page-locked buffers of ace_score_host (null until the first call)
     double *d_stage_ws;        // grow-only workspace for deferred stage tails
     size_t stage_ws_plans;     // capacity in plans
     int stage_ws_fixed;        // ace_reserve(..., fixed): a larger batch is an error instead of a reallocation
@@ -1374,6 +1376,8 @@ void ace_destroy(ace_handle_t *h) {
     (void)hipFree(h->d_win_row_begin); (void)hipFree(h->d_win_rows);
     if (h->d_rc_pos) (void)hipFree(h->d_rc_pos);
     if (h->d_rc_act) (void)hipFree(h->d_rc_act);
+    if (h->host_in) (void)hipHostFree(h->host_in);
+    if (h->host_out) (void)hipHostFree(h->host_out);
     if (h->d_stage_ws) (void)hipFree(h->d_stage_ws);
     delete h;
 }
@@ -1505,6 +1509,65 @@ int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_lim
     launch_score(h, a, (hipStream_t)stream);
     ACE_HIP(hipGetLastError());
     return ACE_OK;
+}
+
+size_t ace_pack_host(const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, size_t n_plans, int num_ops, uint8_t *out) {
+    const size_t P = n_plans, N = (size_t)num_ops, G = (N + 15) / 16, off_hdr = G * P * 16, off_rng = off_hdr + P * 16;
+    if (out) {
+        for (size_t p = 0; p < P; ++p) {
+            const uint8_t *row = codes + p * N;
+            for (size_t g = 0; g + 1 < G; ++g) memcpy(out + (g * P + p) * 16, row + g * 16, 16);
+            unsigned char last[16] = {0};
+            memcpy(last, row + (G - 1) * 16, N - (G - 1) * 16);
+            memcpy(out + ((G - 1) * P + p) * 16, last, 16);
+        }
+        memcpy(out + off_hdr, hdr, P * 16);
+        if (range) memcpy(out + off_rng, range, P * 8);
+    }
+    return off_rng + (range ? P * 8 : 0);
+}
+
+int ace_score_host(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, size_t n_plans,
+                   double memory_limit, int strict, double *times, uint8_t *flags, double *stage_out, void *stream) {
+    if (!h || !codes || !hdr || !times || !flags || n_plans == 0 || (range && !stage_out)) return ACE_EINVAL;
+    const size_t P = n_plans, N = (size_t)h->geom.N, G = (size_t)h->geom.G;
+    const size_t rec_bytes = stage_out ? P * (range ? 1 : ACE_MAX_STAGES) * ACE_STAGE_REC * sizeof(double) : 0;
+    // in: codes [G][P][16] | headers | ranges; out: times | records | flags
+    const size_t off_hdr = G * P * 16, off_rng = off_hdr + P * 16, n_in = ace_pack_host(nullptr, nullptr, range, P, (int)N, nullptr);
+    const size_t off_rec = 16 * P, off_flags = off_rec + rec_bytes, n_out = off_flags + 2 * P;
+    if (P > kHostIoBytes || n_in > kHostIoBytes || n_out > kHostIoBytes) return ACE_ETOOBIG;
+    int dev = -1;
+    ACE_HIP(hipGetDevice(&dev));
+    if (dev != h->device) ACE_HIP(hipSetDevice(h->device));
+    int rc = ACE_OK;
+    if (!h->host_in && (hipHostMalloc((void **)&h->host_in, kHostIoBytes, hipHostMallocDefault) != hipSuccess ||
+                        hipHostMalloc((void **)&h->host_out, kHostIoBytes, hipHostMallocDefault) != hipSuccess)) {
+        if (h->host_in) (void)hipHostFree(h->host_in);
+        h->host_in = nullptr;
+        h->host_out = nullptr;
+        rc = ACE_ENOMEM;
+    }
+    if (rc == ACE_OK) {
+        unsigned char *in = h->host_in, *out = h->host_out;
+        ace_pack_host(codes, hdr, range, P, (int)N, in);
+        if (rec_bytes) memset(out + off_rec, 0, rec_bytes);      // (a plan has records for its stages only)
+        const ace_batch_t b{in, reinterpret_cast<const uint32_t *>(in + off_hdr), range ? reinterpret_cast<const uint32_t *>(in + off_rng) : nullptr,
+                            P, nullptr};
+        double *t = reinterpret_cast<double *>(out);
+        rc = ace_score_batch(h, &b, memory_limit, strict, t, t + P, out + off_flags, out + off_flags + P,
+                             rec_bytes ? reinterpret_cast<double *>(out + off_rec) : nullptr, stream);
+        if (rc == ACE_OK && hipStreamSynchronize((hipStream_t)stream) != hipSuccess) {
+            snprintf(g_hip_err, sizeof(g_hip_err), "hipStreamSynchronize failed");
+            rc = ACE_EHIP;
+        }
+        if (rc == ACE_OK) {
+            memcpy(times, t, 16 * P);
+            memcpy(flags, out + off_flags, 2 * P);
+            if (rec_bytes) memcpy(stage_out, out + off_rec, rec_bytes);
+        }
+    }
+    if (dev != h->device) ACE_HIP(hipSetDevice(dev));
+    return rc;
 }
 
 int ace_score_batch_static(ace_handle_t *h, const ace_batch_t *batch, double memory_limit, int strict, double *d_iter_ms,

@@ -20,7 +20,7 @@ EXPORTS = ["ace_abi_version", "ace_strerror", "ace_last_hip_error", "ace_create"
            "ace_recompute_groups", "ace_recompute_select", "ace_group_keys", "ace_gather_plans",
            "ace_keyset_create", "ace_keyset_destroy", "ace_keyset_size", "ace_keyset_add", "ace_keyset_unseen", "ace_keyset_claim",
            "ace_keyset_move", "ace_keyset_keys", "ace_build_moves", "ace_recompute_prepare", "ace_recompute_batch",
-           "ace_pack_plans", "ace_unpack_plans", "ace_check_plans"]
+           "ace_pack_plans", "ace_unpack_plans", "ace_check_plans", "ace_score_host", "ace_pack_host"]
 
 
 class AceBatchStruct(ctypes.Structure):
@@ -108,6 +108,9 @@ def load_library():
     lib.ace_pack_plans.argtypes = [vp, sz, ctypes.c_int, vp, ctypes.c_int, ctypes.c_int, vp, vp, vp]
     lib.ace_unpack_plans.argtypes = [vp, sz, ctypes.c_int, vp, vp]
     lib.ace_check_plans.argtypes = [vp, vp, sz, ctypes.c_int, ctypes.c_int, ctypes.c_int]
+    lib.ace_score_host.argtypes = [vp, vp, vp, vp, sz, ctypes.c_double, ctypes.c_int, vp, vp, vp, vp]
+    lib.ace_pack_host.restype = sz
+    lib.ace_pack_host.argtypes = [vp, vp, vp, sz, ctypes.c_int, vp]
     lib.ace_recompute_prepare.argtypes = [vp] * 4
     lib.ace_recompute_batch.argtypes = [vp, ctypes.POINTER(AceBatchStruct), ctypes.c_double, ctypes.c_double] + [vp] * 4
     ci = ctypes.c_int
@@ -116,6 +119,21 @@ def load_library():
         raise AceError("libace_eval.so has a different ABI version")
     _lib = lib
     return lib
+
+
+_objects = None
+
+
+def load_objects():
+    """The native module that walks plan objects (csrc/ace_objects.cpp)."""
+    global _objects
+    if _objects is None:
+        try:
+            from . import _ace_objects
+        except ImportError as e:
+            raise AceError(f"superscaler_amd/_ace_objects.so cannot be loaded ({e}): build it with `python -m superscaler_amd.build`") from e
+        _objects = _ace_objects
+    return _objects
 
 
 def _check(lib, rc, what):
@@ -170,24 +188,16 @@ def depth_order(batch: PlanBatch) -> np.ndarray:
 
 
 def pack_small_inputs(buf: np.ndarray, batch: PlanBatch, ranges) -> int:
-    """Lay a small batch out for the kernel in `buf` (uint8): codes [ceil(N/16)][P][16] (zero padded), then the
-    headers uint32 [P][4], then the ranges uint32 [P][2] if given.  Returns the number of bytes used."""
-    P, N = batch.codes.shape
-    G = (N + 15) // 16
-    off_hdr = G * P * 16
-    off_rng = off_hdr + P * 16
-    n_in = off_rng + (P * 8 if ranges is not None else 0)
-    lay = buf[:off_hdr].reshape(G, P, 16)
-    full = N // 16
-    if full:
-        lay[:full] = batch.codes[:, :full * 16].reshape(P, full, 16).transpose(1, 0, 2)
-    if full < G:
-        lay[full, :, :N - full * 16] = batch.codes[:, full * 16:]
-        lay[full, :, N - full * 16:] = 0
-    buf[off_hdr:off_rng].view(np.uint32).reshape(P, 4)[...] = batch.hdr
-    if ranges is not None:
-        buf[off_rng:n_in].view(np.uint32).reshape(P, 2)[...] = ranges
-    return n_in
+    """Lay a small batch out for the kernel in `buf` (uint8) as ace_score_host does: codes [ceil(N/16)][P][16] (zero padded),
+    then the headers uint32 [P][4], then the ranges uint32 [P][2] if given.  Returns the number of bytes used."""
+    codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr, dtype=np.uint32)
+    rg = None if ranges is None else np.ascontiguousarray(ranges, dtype=np.uint32)
+    P, N = codes.shape
+    args = (codes.ctypes.data, hdr.ctypes.data, None if rg is None else rg.ctypes.data, P, N)
+    lib = load_library()
+    if lib.ace_pack_host(*args, None) > buf.nbytes:
+        raise ValueError("the buffer is too small")
+    return lib.ace_pack_host(*args, buf.ctypes.data)
 
 
 STAGING_PIECE = 8 << 20      # bytes of plans staged at a time: the copy to the device of one runs beside the staging of the next
@@ -307,7 +317,6 @@ class PlanEvaluator:
         self.handle = h
         self._deal_cache = {}
         self._topk_ws = None
-        self._small = None
         self._rc_ready = None
         self._graphs_alive = 0
 
@@ -620,54 +629,29 @@ class PlanEvaluator:
 
     # ---- small host-in / host-out calls ------------------------------------------------------------
     # The reference's search calls the cost model for one plan or one stage at a time, so the time of such
-    # a call is what a host-side search sees.  Small batches therefore go through one pinned buffer each
-    # way: the plans are laid out for the kernel on the host in page-locked memory, which the kernel reads
-    # and writes where it is.
+    # a call is what a host-side search sees.  Small batches therefore take one library call (ace_score_host): laid out in
+    # page-locked memory, which the kernel reads and writes where it is.
     SMALL_IO_BYTES = 1 << 20
 
-    def _small_io(self):
-        if self._small is None:
-            torch = self._torch
-            n = self.SMALL_IO_BYTES
-            h_in = torch.empty(n, dtype=torch.uint8, pin_memory=True)
-            h_out = torch.empty(n, dtype=torch.uint8, pin_memory=True)
-            self._small = (h_in, h_in.numpy(), h_out, h_out.numpy())
-        return self._small
-
     def _score_small(self, batch: PlanBatch, limit: float, strict: bool, breakdown: bool, ranges):
-        """score_host for a batch whose inputs and outputs fit SMALL_IO_BYTES; None if they do not."""
+        """score_host for a batch whose inputs and outputs fit the library's page-locked buffers; None if they do not."""
         P, N = batch.codes.shape
-        G = (N + 15) // 16
         breakdown = breakdown or ranges is not None
-        off_hdr = G * P * 16
-        off_rng = off_hdr + P * 16
-        n_in = off_rng + (P * 8 if ranges is not None else 0)
         n_rec = 1 if ranges is not None else MAX_STAGES          # a single-stage query has one record
-        rec_bytes = P * n_rec * STAGE_REC * 8 if breakdown else 0
-        off_fe = 16 * P + rec_bytes
-        n_out = off_fe + 2 * P
-        if n_in > self.SMALL_IO_BYTES or n_out > self.SMALL_IO_BYTES:
+        codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr)
+        if ranges is not None:
+            ranges = np.ascontiguousarray(ranges, dtype=np.uint32)
+        times = np.empty((2, P))
+        flags = np.empty((2, P), dtype=np.uint8)
+        rec = np.empty((P, n_rec, STAGE_REC)) if breakdown else None
+        rc = self.lib.ace_score_host(self.handle, codes.ctypes.data, hdr.ctypes.data, ranges.ctypes.data if ranges is not None else None, P,
+                                     limit, int(strict), times.ctypes.data, flags.ctypes.data, rec.ctypes.data if breakdown else None,
+                                     self._torch._C._cuda_getCurrentRawStream(self.device.index or 0))
+        if rc == ACE_ETOOBIG:
             return None
-        # the kernel reads the plans from, and writes its results to, page-locked host memory directly (the device sees it
-        # at the same address): a kilobyte each way over the bus costs less than two copies and their bookkeeping
-        # (measured: 5 to 12 us of a 70 to 140 us call)
-        h_in, np_in, h_out, np_out = self._small_io()
-        pack_small_inputs(np_in, batch, ranges)
-        if breakdown:
-            np_out[16 * P:off_fe] = 0
-        base_in, base_out = h_in.data_ptr(), h_out.data_ptr()
-        struct = AceBatchStruct(base_in, base_in + off_hdr, base_in + off_rng if ranges is not None else None, P, None)
-        with self._torch.cuda.device(self.device):
-            rc = self.lib.ace_score_batch(self.handle, ctypes.byref(struct), limit, int(strict), base_out, base_out + 8 * P,
-                                          base_out + off_fe, base_out + off_fe + P,
-                                          base_out + 16 * P if breakdown else None, self._stream())
-        _check(self.lib, rc, "ace_score_batch")
-        self._torch.cuda.current_stream(self.device).synchronize()
-        f64 = np_out[:off_fe].view(np.float64)
-        out = (f64[:P].copy(), f64[P:2 * P].copy(), np_out[off_fe:off_fe + P].copy(), np_out[off_fe + P:n_out].copy())
-        if breakdown:
-            out += (f64[2 * P:].reshape(P, n_rec, STAGE_REC).copy(),)
-        return out
+        _check(self.lib, rc, "ace_score_host")
+        out = (times[0], times[1], flags[0], flags[1])
+        return out + (rec,) if breakdown else out
 
     # convenience: host in, host out
     def score_host(self, batch: PlanBatch, memory_limit=None, strict=False, breakdown=False, ranges=None,

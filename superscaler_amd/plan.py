@@ -11,7 +11,6 @@ plus four 32-bit words per plan --
     [1..2] log2(stage gpus), 4 bits per stage
     [3] in-cross-node bit per stage | out-cross-node bits << 16   (aceso_cost_model.py:572-574)
 """
-import itertools
 import json
 from dataclasses import dataclass, field
 from typing import List, Optional, Sequence
@@ -166,62 +165,69 @@ class PlanBatch:
         profiled (as aceso_cost_model.py:22-25 does) and ValueError for plans the encoding cannot
         hold.  `single_stage_intra_node` forces both cross-node flags off, which is what the
         single-stage queries do (aceso_cost_model.py:494-495)."""
-        db = tables.db
-        N = tables.graph.num_ops
-        A = db.n_algo
-        mbs_index = {m: k for k, m in enumerate(db.mbs_list)}
-        # tp size -> index in the profile database (0xff: not profiled), as a lookup table
-        tp_lut = np.full(max(db.tp_list) + 2, 0xff, dtype=np.uint8)
-        tp_lut[np.asarray(db.tp_list)] = np.arange(len(db.tp_list), dtype=np.uint8)
-        P = len(configs)
-        codes = np.zeros((P, N), dtype=np.uint8)
-        hdr = np.zeros((P, 4), dtype=np.uint32)
-        gpn = tables.settings.num_gpus_per_node
-        chain = itertools.chain.from_iterable
-        for p, cfg in enumerate(configs):
-            S = cfg.num_stages
-            if S < 1 or S > MAX_STAGES:
-                raise ValueError(f"plan {p}: {S} stages (1..{MAX_STAGES} supported)")
-            bidx = mbs_index[cfg.micro_bs]
-            stages = cfg.stages
-            lens = [len(st.ops) for st in stages]
-            glogs = 0
-            gl = []
-            for s, st in enumerate(stages):
-                if lens[s] == 0:
-                    raise ValueError(f"plan {p}: stage {s} is empty")
-                g = st.tp_size[0] * st.dp_size[0]
-                if g & (g - 1) or g.bit_length() - 1 > 15:
-                    raise ValueError(f"plan {p}: stage {s} has {g} devices (power of two expected)")
-                gl.append(g)
-                glogs |= (g.bit_length() - 1) << (4 * s)
-                for d in set(st.dp_size):
-                    if cfg.micro_bs // d not in mbs_index:
-                        raise KeyError(cfg.micro_bs // d)
-            total = sum(lens)
-            if total != N:
-                raise ValueError(f"plan {p} has {total} ops, the op graph {N}")
-            # the per-op lists of all stages, flattened once each
-            tp, dp, al, rc = (_flat_ints(stages, key, N) for key in ("tp_size", "dp_size", "algo", "recompute_ops"))
-            g_of_op = np.repeat(np.asarray(gl, dtype=np.int64), lens)
-            bad = np.flatnonzero(tp * dp != g_of_op)
-            if len(bad):
-                s = int(np.searchsorted(np.cumsum(lens), bad[0], side="right"))
-                raise ValueError(f"plan {p}: stage {s} mixes tp*dp products")
-            t = tp_lut[np.clip(tp, 0, len(tp_lut) - 1)]
-            if (t == 0xff).any():
-                raise ValueError(f"plan {p}: tp size {int(tp[np.flatnonzero(t == 0xff)[0]])} is not in the profile database")
-            if ((al < 0) | (al >= A)).any():
-                raise ValueError(f"plan {p}: algo index outside the profile database")
-            row = (t * A + al.astype(np.uint8)) | ((rc == 1).astype(np.uint8) << 3)
-            starts = np.cumsum([0] + lens[:-1])
-            row[starts] |= 1 << 4
-            codes[p] = row
-            hdr[p, 0] = S | (bidx << 8)
-            hdr[p, 1] = glogs & 0xFFFFFFFF
-            hdr[p, 2] = glogs >> 32
-            hdr[p, 3] = 0 if single_stage_intra_node else cross_node_bits(gl, gpn)
+        from .evaluator import load_objects
+        db, N, P = tables.db, tables.graph.num_ops, len(configs)
+        mbs, tp_lut = tables.encode_luts
+        codes = np.empty((P, N), dtype=np.uint8)
+        hdr = np.empty((P, 4), dtype=np.uint32)
+        done = 0
+        while done < P:
+            # (native code for plans that are lists of small ints and fit the encoding; it stops at the first other one)
+            done = load_objects().encode(configs, done, N, db.n_algo, tables.settings.num_gpus_per_node, single_stage_intra_node, mbs,
+                                         tp_lut, codes, hdr)
+            if done < P:
+                cls._encode_config(done, configs[done], tables, single_stage_intra_node, codes[done], hdr[done])
+                done += 1
         return cls(codes, hdr)
+
+    @staticmethod
+    def _encode_config(p, cfg, tables: CompiledTables, single_stage_intra_node: bool, row_out: np.ndarray, hdr_out: np.ndarray):
+        """Plan p of from_configs: any sequences of integers, and the errors."""
+        db, N, A = tables.db, tables.graph.num_ops, tables.db.n_algo
+        mbs_index = {m: k for k, m in enumerate(db.mbs_list)}
+        tp_lut = tables.encode_luts[1]
+        S = cfg.num_stages
+        if S < 1 or S > MAX_STAGES:
+            raise ValueError(f"plan {p}: {S} stages (1..{MAX_STAGES} supported)")
+        bidx = mbs_index[cfg.micro_bs]
+        stages = cfg.stages
+        lens = [len(st.ops) for st in stages]
+        glogs = 0
+        gl = []
+        for s, st in enumerate(stages):
+            if lens[s] == 0:
+                raise ValueError(f"plan {p}: stage {s} is empty")
+            g = st.tp_size[0] * st.dp_size[0]
+            if g & (g - 1) or g.bit_length() - 1 > 15:
+                raise ValueError(f"plan {p}: stage {s} has {g} devices (power of two expected)")
+            gl.append(g)
+            glogs |= (g.bit_length() - 1) << (4 * s)
+            for d in set(st.dp_size):
+                if cfg.micro_bs // d not in mbs_index:
+                    raise KeyError(cfg.micro_bs // d)
+        total = sum(lens)
+        if total != N:
+            raise ValueError(f"plan {p} has {total} ops, the op graph {N}")
+        # the per-op lists of all stages, flattened once each
+        tp, dp, al, rc = (_flat_ints(stages, key, N) for key in ("tp_size", "dp_size", "algo", "recompute_ops"))
+        g_of_op = np.repeat(np.asarray(gl, dtype=np.int64), lens)
+        bad = np.flatnonzero(tp * dp != g_of_op)
+        if len(bad):
+            s = int(np.searchsorted(np.cumsum(lens), bad[0], side="right"))
+            raise ValueError(f"plan {p}: stage {s} mixes tp*dp products")
+        t = tp_lut[np.clip(tp, 0, len(tp_lut) - 1)]
+        if (t == 0xff).any():
+            raise ValueError(f"plan {p}: tp size {int(tp[np.flatnonzero(t == 0xff)[0]])} is not in the profile database")
+        if ((al < 0) | (al >= A)).any():
+            raise ValueError(f"plan {p}: algo index outside the profile database")
+        row = (t * A + al.astype(np.uint8)) | ((rc == 1).astype(np.uint8) << 3)
+        starts = np.cumsum([0] + lens[:-1])
+        row[starts] |= 1 << 4
+        row_out[...] = row
+        hdr_out[0] = S | (bidx << 8)
+        hdr_out[1] = glogs & 0xFFFFFFFF
+        hdr_out[2] = glogs >> 32
+        hdr_out[3] = 0 if single_stage_intra_node else cross_node_bits(gl, tables.settings.num_gpus_per_node)
 
     # ---- array form -> object form -------------------------------------------------------------
     def to_config(self, p: int, tables: CompiledTables, cls_config=AcesoConfig, cls_stage=AcesoStageInfo):

@@ -29,6 +29,7 @@ maxima of table entries:
   pos_info[i]  LDS slot of op i's row | slot of op i+1's row << 8 | kind of the (i, i+1) pair << 16 | flags << 24
 """
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 from typing import Dict, List, Optional, Tuple
@@ -100,6 +101,15 @@ class CompiledTables:
     @property
     def C(self):
         return len(self.db.tp_list) * self.db.n_algo
+
+    @functools.cached_property
+    def encode_luts(self):
+        """For encoding plan objects: micro-batch sizes (int32), and tp size -> index in the profile database (uint8, 0xff:
+        not profiled)."""
+        db = self.db
+        tp_lut = np.full(max(db.tp_list) + 2, 0xff, dtype=np.uint8)
+        tp_lut[np.asarray(db.tp_list)] = np.arange(len(db.tp_list), dtype=np.uint8)
+        return np.asarray(db.mbs_list, dtype=np.int32), tp_lut
 
     def as_struct(self) -> AceTablesStruct:
         db = self.db

@@ -1,0 +1,71 @@
+"""The native walk over plan objects (superscaler_amd/csrc/ace_objects.cpp) against the Python code it stands in for: the same
+arrays and lists for a search's plans, the same arrays and errors for everything it leaves to that code."""
+import copy
+
+import numpy as np
+import pytest
+
+from superscaler_amd import synth
+from superscaler_amd.evaluator import load_objects
+from superscaler_amd.plan import PlanBatch
+from tests.helpers import emu_score, odd_workloads
+from tests.test_recompute_kernel import cost_model
+from tests.test_small_batches import WORKLOADS
+
+
+def by_python(configs, tables, intra=False):
+    P, N = len(configs), tables.graph.num_ops
+    codes, hdr = np.empty((P, N), dtype=np.uint8), np.empty((P, 4), dtype=np.uint32)
+    for p, c in enumerate(configs):
+        PlanBatch._encode_config(p, c, tables, intra, codes[p], hdr[p])
+    return codes, hdr
+
+
+@pytest.mark.parametrize("name", ["gpt3_13b", "t5_770m", "wresnet_1b", "gpt3_175b", "gpt_1tp_1mbs", "gpt_wide_stages", "resnet_16gpus"])
+def test_encode_and_fill_equal_the_python_code(name):
+    w = WORKLOADS[name]
+    cm = cost_model(w)
+    batch = synth.make_plans(w, cm.tables, n_plans=12, seed_offset=2)
+    configs = [batch.to_config(p, cm.tables) for p in range(12)]
+    for intra in (False, True):
+        native, (codes, hdr) = PlanBatch.from_configs(configs, cm.tables, intra), by_python(configs, cm.tables, intra)
+        assert np.array_equal(native.codes, codes) and np.array_equal(native.hdr, hdr) and np.array_equal(codes, batch.codes)
+    rec = emu_score(cm.tables, batch, breakdown=True)[4]
+    s = cm.settings
+    for p, c in enumerate(configs):
+        other = copy.deepcopy(c)
+        assert load_objects().fill(c, rec[p], s.memory_limit, s.memory_main_params, s.memory_optimizer, s.consider_reserved_space) is True
+        other.stages = tuple(other.stages)              # (left to the Python code)
+        assert load_objects().fill(other, rec[p], s.memory_limit, s.memory_main_params, s.memory_optimizer, s.consider_reserved_space) is False
+        cm._fill_breakdown(other, rec[p])
+        other.stages = list(other.stages)
+        assert c == other and c.time_list and all(type(x) is float for x in c.time_list + c.memory_list + c.efficient_time_list)
+
+
+def test_other_plan_objects_and_errors_take_the_python_code():
+    w = odd_workloads()[2]
+    tables = synth.make_tables(w)
+    batch = synth.make_plans(w, tables, n_plans=6, seed_offset=1)
+    good = [batch.to_config(p, tables) for p in range(6)]
+    odd = copy.deepcopy(good)
+    odd[1].stages[0].tp_size = tuple(odd[1].stages[0].tp_size)                 # not a list
+    odd[3].stages[-1].algo = [np.int64(a) for a in odd[3].stages[-1].algo]      # not ints
+    odd[4].stages[0].recompute_ops = [2 * r for r in odd[4].stages[0].recompute_ops]   # only 1 means recomputed
+    got = PlanBatch.from_configs(odd, tables)
+    want = PlanBatch.from_configs(good, tables)
+    n = len(good[4].stages[0].ops)
+    want.codes[4, :n] &= 0xF7
+    assert np.array_equal(got.codes, want.codes) and np.array_equal(got.hdr, want.hdr)
+
+    def change(**kw):
+        c = copy.deepcopy(good[2])
+        for k, v in kw.items():
+            setattr(c if hasattr(c, k) else c.stages[0], k, v(getattr(c if hasattr(c, k) else c.stages[0], k)))
+        return c
+    bad = [(KeyError, change(micro_bs=lambda m: 3)), (ValueError, change(num_stages=lambda n: 17)), (ValueError, change(ops=lambda o: [])),
+           (ValueError, change(tp_size=lambda t: [3] * len(t))), (ValueError, change(algo=lambda a: [9] * len(a))),
+           (ValueError, change(ops=lambda o: o[:-1], tp_size=lambda t: t[:-1])), (ValueError, change(dp_size=lambda d: d[:1] + [2 * x for x in d[1:]])),
+           (AttributeError, object())]
+    for error, c in bad:
+        with pytest.raises(error):
+            PlanBatch.from_configs([good[0], c], tables)
