@@ -64,7 +64,7 @@ def test_other_plan_objects_and_errors_take_the_python_code():
         return c
     bad = [(KeyError, change(micro_bs=lambda m: 3)), (ValueError, change(num_stages=lambda n: 17)), (ValueError, change(ops=lambda o: [])),
            (ValueError, change(tp_size=lambda t: [3] * len(t))), (ValueError, change(algo=lambda a: [9] * len(a))),
-           (ValueError, change(ops=lambda o: o[:-1], tp_size=lambda t: t[:-1])), (ValueError, change(dp_size=lambda d: d[:1] + [2 * x for x in d[1:]])),
+           (ValueError, change(ops=lambda o: o[:-1], tp_size=lambda t: t[:-1])), ((KeyError, ValueError), change(dp_size=lambda d: d[:1] + [2 * x for x in d[1:]])),
            (AttributeError, object())]
     for error, c in bad:
         with pytest.raises(error):
