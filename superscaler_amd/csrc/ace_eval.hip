@@ -332,29 +332,18 @@ __global__ __launch_bounds__(1024) void topk_finish(TopkState *st, Cand *less, C
 }
 
 // ------------------------------------------------------------------------------------------
-// top-k, short form (small k): three launches instead of seventeen.  The k-th smallest key of an evenly spaced SAMPLE
-// bounds the k-th smallest key of the whole input from above, so one pass keeps everything at or below it (about
-// n * k / kSample entries), and one workgroup then selects among those (held in registers, or in LDS): radix select on the 96-bit order
-// (key, index), which makes ties fall to the lower index, a gather of the k winners and a small sort.
+// top-k, short form (k <= 256): workgroups of 1,024 lanes select the k best of a stretch of the input each, one workgroup the
+// k best of what they found (up to 16,384 entries: that workgroup alone).  A selection keeps its entries in registers: radix
+// select on the 96-bit order (key, index) -- so ties fall to the lower index --, starting below the bits that all keys
+// share, cut short as soon as the bucket that holds the k-th entry is small enough to be ranked as it is.  Exact for any
+// input, whatever its order and however many keys are equal: no bound is guessed and no list can overflow.
+// Bound by the latency of the two selections (about three dozen workgroup barriers each), not by reading the input.
+// Launches back to back (10 us is what the host needs for a call), us, against a sampled bound, a filter pass and one
+// selection: k = 64, 4,096 entries 23 -> 10, 262,144 entries 27 -> 17, 2^20 entries 34 -> 23; k = 256, 2^20 entries 80 -> 40.
 // ------------------------------------------------------------------------------------------
-constexpr int kSample = 8192;            // sampled keys, selected from by one workgroup (eight per lane)
-static_assert(kSample == 1 << 13, "topk_sample's index arithmetic");
-constexpr unsigned kCandCap = 12000;     // candidates the last kernel can hold in LDS (12 bytes each)
 constexpr int kShortMaxK = 256;
-constexpr size_t kShortMaxNK = 1ull << 26;   // n * k up to this: about kSample candidates expected, kCandCap is 4 sigma above
-// Equal keys: the threshold is the sample's exact k-th key; entries below it and entries equal to it are kept apart,
-// and of the equal ones only the lowest indices are ever needed (k minus the number of entries below).  Few of them go
-// into a list of their own; masses of them (a search neighbourhood whose plans share the bottleneck stage all have the
-// same time) are only COUNTED per filter workgroup, and the last kernel reads the first few of them from the input in
-// index order.  Cost: 0.03-0.05 ms at n = 2^20, k = 64 whatever the keys; only when more than kCandCap entries lie
-// strictly below the sample's k-th key (feasible plans crowded between the sampled positions) does the last kernel
-// select from the whole input in global memory instead (ShortSource below): one workgroup, about nine passes over
-// n entries, 3.8 ms at n = 2^20.
-constexpr unsigned kTieCap = 2048;       // equal-to-threshold entries listed one by one; beyond that: per-workgroup counts
-constexpr unsigned kMaxFilterGroups = 8192;   // n <= kShortMaxNK entries in workgroups of 8,192
-static_assert(kShortMaxNK / (1024 * 8) <= kMaxFilterGroups, "one count per filter workgroup");
-
-struct ShortTopk { unsigned long long thr; unsigned int count; unsigned int count_eq; };
+constexpr unsigned kShortMaxEntries = 16384;     // entries one workgroup selects from: sixteen per lane
+constexpr unsigned kShortBucket = 512;           // bucket entries that fit the histogram's LDS as (key, index) pairs
 
 // Which of the kRadix buckets of `hist` (LDS) holds the rem-th entry (1-based), counting buckets in order: returns the
 // bucket, the entries before it in `before` and the total in `total` to every lane of the 1024-lane workgroup (no bucket:
@@ -391,62 +380,41 @@ __device__ __forceinline__ unsigned int short_pick(const unsigned int *hist, uns
     return bucket;
 }
 
-// Smallest and largest finite key of a strided view of the lanes' own keys (kmin = kInfKey: none), to every lane.  The bits
-// above the highest bit in which the two differ are common to all keys: the radix passes start below them, where the
-// histogram spreads (a pass over common bits would send every LDS atomic to one bucket, one after the other).
-// `cnt`: the lane's number of finite keys; `total` their number in all.
-__device__ __forceinline__ void short_minmax(unsigned long long mn, unsigned long long mx, unsigned long long cnt,
-                                             unsigned long long *wmm /* [48] */, unsigned long long &kmin, unsigned long long &kmax,
-                                             unsigned long long &total) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    for (int off = 32; off > 0; off >>= 1) {
-        const unsigned long long a = __shfl_xor(mn, off, 64), b = __shfl_xor(mx, off, 64);
-        cnt += __shfl_xor(cnt, off, 64);
-        mn = a < mn ? a : mn;
-        mx = b > mx ? b : mx;
+// Rank in (key, index) order of entry tid / parts of `list` (LDS, cnt <= 1,024 / parts entries) for every entry at once:
+// `parts` neighbouring lanes compare an entry with a part of the others each; every one of them gets the rank.
+template <int parts> __device__ __forceinline__ unsigned int short_rank(const Cand *list, unsigned int cnt, Cand &me) {
+    const unsigned int i = threadIdx.x / parts, part = threadIdx.x % parts;
+    me = list[i < cnt ? i : 0u];
+    unsigned int rank = 0;
+#pragma unroll 8
+    for (unsigned int j = part; j < cnt; j += parts) {
+        const Cand o = list[j];
+        rank += o.key < me.key || (o.key == me.key && o.idx < me.idx) ? 1u : 0u;
     }
-    if (lane == 0) { wmm[3 * wave] = mn; wmm[3 * wave + 1] = mx; wmm[3 * wave + 2] = cnt; }
-    __syncthreads();
-    kmin = kInfKey; kmax = 0; total = 0;
-    for (int w2 = 0; w2 < 16; ++w2) {
-        const unsigned long long a = wmm[3 * w2], b = wmm[3 * w2 + 1];
-        kmin = a < kmin ? a : kmin;
-        kmax = b > kmax ? b : kmax;
-        total += wmm[3 * w2 + 2];
-    }
-    __syncthreads();
+#pragma unroll
+    for (int off = 1; off < parts; off <<= 1) rank += __shfl_xor(rank, off, 64);
+    return i < cnt ? rank : ~0u;
 }
 
-// The sample's k-th smallest key: an upper bound of the input's k-th smallest key (with fewer than k feasible entries in
-// the sample: the largest finite key, so that every feasible entry is kept).
-__global__ __launch_bounds__(1024) void topk_sample(const double *t, const uint8_t *f, size_t n, int k, ShortTopk *st) {
-    constexpr int kPer = kSample / 1024;
-    __shared__ unsigned int hist[kRadix];
-    __shared__ unsigned int wsum[20];
-    __shared__ unsigned long long s_wref[16];
-    __shared__ unsigned long long small_keys[64];
-    __shared__ unsigned long long s_kth;
-    __shared__ unsigned int s_nsmall, s_nfin, s_cur;
+struct ShortShared {
+    union {
+        unsigned int hist[kRadix];
+        Cand bucket[kShortBucket];               // after the passes
+    };
+    Cand win[kShortMaxK];
+    unsigned int wsum[20];
+    unsigned long long wref[16];
+    unsigned int nfin, cur, nwin, nbucket;
+};
+
+// The k smallest of the workgroup's entries (kPer per lane; kInfKey: none) in (key, index) order, into s.win in no order;
+// returns how many there are (k, or all of them).
+template <int kPer>
+__device__ __forceinline__ unsigned int short_select(ShortShared &s, const unsigned long long (&rk)[kPer], const unsigned int (&ri)[kPer], int k) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    if (tid == 0) { s_nfin = 0; s_cur = 0; }
-    // the sample: evenly spaced runs of consecutive entries (consecutive entries share cache lines); all of a short input.
-    // 64 runs of 128 entries up to 2^18 entries, then more and shorter runs, so that the stretch between two runs stays at
-    // about 4,096 entries (8,192 single entries from 2^25 on): an input in which the best entries are neighbours -- times
-    // that fall or rise along the batch -- then leaves fewer of them between two runs than the last kernel can hold.
-    // The keys stay in registers, eight per lane: no pass of the selection reads anything.
-    const size_t m = n < (size_t)kSample ? n : (size_t)kSample;
-    int run_shift = 7;                                          // log2(entries per run)
-    while (run_shift > 0 && (n >> (13 - run_shift)) > 4096) --run_shift;
-    const size_t run_step = n >> (13 - run_shift);              // (kSample = 2^13 entries in 2^(13 - run_shift) runs)
-    unsigned long long rk[kPer];
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const int j = tid + q * 1024;
-        const size_t i = n <= (size_t)kSample ? (size_t)j : (size_t)(j >> run_shift) * run_step + (size_t)(j & ((1 << run_shift) - 1));
-        rk[q] = (size_t)j < m ? time_key(t[i], f[i]) : kInfKey;
-    }
-    // how many keys are finite, and which bits vary among them: the highest bit in which any key differs from one of
-    // them (the first finite key in lane order), one 32-bit maximum over the workgroup
+    if (tid == 0) { s.nfin = 0; s.cur = 0; s.nwin = 0; s.nbucket = 0; }
+    // how many keys there are, and which bits vary among them: the highest bit in which any key differs from one of
+    // them (the first one in lane order), one 32-bit maximum over the workgroup
     unsigned long long mine = kInfKey;
     unsigned int wave_cnt = 0;
 #pragma unroll
@@ -459,453 +427,146 @@ __global__ __launch_bounds__(1024) void topk_sample(const double *t, const uint8
     const unsigned long long wave_ref = __shfl(mine, has ? __ffsll((long long)has) - 1 : 0, 64);
     __syncthreads();                                           // (the counters are zero)
     if (lane == 0) {
-        s_wref[wave] = wave_ref;
-        if (wave_cnt) atomicAdd(&s_nfin, wave_cnt);
+        s.wref[wave] = wave_ref;
+        if (wave_cnt) atomicAdd(&s.nfin, wave_cnt);
     }
     __syncthreads();
-    unsigned long long ref = kInfKey;
-    for (int w2 = 15; w2 >= 0; --w2) {
-        const unsigned long long v = s_wref[w2];
-        if (v != kInfKey) ref = v;
-    }
-    const unsigned long long nfin = s_nfin;
-    int hb = 0;
+    const unsigned int nfin = s.nfin;
+    const bool all = nfin <= (unsigned)k;
+    int cur = 0, icur = 32, small_shift = 0;
+    unsigned long long prefix = 0;
+    unsigned int iprefix = 0, rem = (unsigned)k;
+    bool small = false;
+    if (!all) {
+        unsigned long long ref = kInfKey;
+        for (int w2 = 15; w2 >= 0; --w2) {
+            const unsigned long long v = s.wref[w2];
+            if (v != kInfKey) ref = v;
+        }
+        int hb = 0;
 #pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        if (rk[q] != kInfKey) {
-            const unsigned long long x = rk[q] ^ ref;
+        for (int q = 0; q < kPer; ++q) {
+            const unsigned long long x = rk[q] == kInfKey ? 0ull : rk[q] ^ ref;
             const int b = x ? 64 - __clzll((long long)x) : 0;
             hb = b > hb ? b : hb;
         }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(hb, off, 64);
-        hb = o > hb ? o : hb;
-    }
-    if (lane == 0 && hb) atomicMax(&s_cur, (unsigned int)hb);
-    __syncthreads();
-    int cur = nfin == 0 ? 0 : (int)s_cur;                      // the low `cur` bits vary
-    unsigned long long prefix = cur >= 64 ? 0ull : (ref >> cur) << cur;
-    unsigned int rem = (unsigned)k;
-    bool enough = nfin >= (unsigned long long)k;           // fewer than k feasible entries in the sample: keep every feasible entry
-    for (int pass = 0; pass < 8 && enough && cur > 0; ++pass) {
-        for (int j = tid; j < kRadix; j += 1024) hist[j] = 0;
-        __syncthreads();
-        const int bits = cur < kRadixBits ? cur : kRadixBits, shift = cur - bits;
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const unsigned long long x = rk[q];
-            if (x != kInfKey && (cur >= 64 || (x >> cur) == (prefix >> cur)))
-                atomicAdd(&hist[(unsigned)((x >> shift) & ((1ull << bits) - 1ull))], 1u);
+        for (int off = 32; off > 0; off >>= 1) {
+            const int o = __shfl_xor(hb, off, 64);
+            hb = o > hb ? o : hb;
         }
+        if (lane == 0 && hb) atomicMax(&s.cur, (unsigned int)hb);
         __syncthreads();
-        unsigned int before, total;
-        const unsigned int b = short_pick(hist, rem, wsum, before, total);
-        (void)total;
-        prefix |= (unsigned long long)b << shift;
-        rem -= before;
-        cur = shift;
-        const unsigned int in_bucket = hist[b];
-        __syncthreads();                                       // (hist[b] read by all before anything clears it)
-        if (cur > 0 && in_bucket <= 64u) {
-            // a handful of keys left in the bucket (distinct keys: after two passes): the rem-th smallest of them directly,
-            // each wavefront ranking some of them by ballot
-            if (tid == 0) s_nsmall = 0;
+        cur = (int)s.cur;                                      // the low `cur` key bits vary
+        prefix = cur >= 64 ? 0ull : (ref >> cur) << cur;
+        // key digits from the highest varying bit down, then index digits among the entries with the selected key
+        while (!small && (cur > 0 || icur > 0)) {
+            for (int j = tid; j < kRadix; j += 1024) s.hist[j] = 0;
             __syncthreads();
+            const bool on_key = cur > 0;
+            const int top = on_key ? cur : icur;
+            const int bits = top < kRadixBits ? top : kRadixBits, shift = top - bits;
 #pragma unroll
             for (int q = 0; q < kPer; ++q) {
-                const unsigned long long x = rk[q];
-                if (x != kInfKey && (x >> cur) == (prefix >> cur)) small_keys[atomicAdd(&s_nsmall, 1u) & 63u] = x;
-            }
-            __syncthreads();
-            for (unsigned int i = (unsigned int)wave; i < in_bucket; i += 16) {
-                const unsigned long long me = small_keys[i];
-                bool less = false;
-                if ((unsigned int)lane < in_bucket) {
-                    const unsigned long long o = small_keys[lane];
-                    less = o < me || (o == me && (unsigned int)lane < i);
+                const unsigned long long key = rk[q];
+                if (key == kInfKey) continue;
+                if (on_key) {
+                    if (cur >= 64 || (key >> cur) == (prefix >> cur))
+                        atomicAdd(&s.hist[(unsigned)((key >> shift) & ((1ull << bits) - 1ull))], 1u);
+                } else if (key == prefix) {
+                    if (icur >= 32 || (ri[q] >> icur) == (iprefix >> icur)) atomicAdd(&s.hist[(ri[q] >> shift) & ((1u << bits) - 1u)], 1u);
                 }
-                const unsigned int rank = (unsigned int)__popcll(__ballot(less));
-                if (lane == 0 && rank + 1u == rem) s_kth = me;
             }
             __syncthreads();
-            prefix = s_kth;
-            cur = 0;
-        }
-    }
-    if (tid == 0) {
-        // the sample's k-th smallest key itself (all digits found; all sampled keys equal: that key)
-        unsigned long long thr = enough ? prefix : kInfKey;
-        if (thr == kInfKey) thr = kInfKey - 1;
-        st->thr = thr; st->count = 0; st->count_eq = 0;
-    }
-}
-
-constexpr int kFilterPer = 8;             // entries per lane of topk_filter
-__global__ __launch_bounds__(1024) void topk_filter(const double *t, const uint8_t *f, size_t n, ShortTopk *st, Cand *cand,
-                                                    Cand *tiecand, unsigned int *group_ties) {
-    // One atomic on each shared counter per WORKGROUP (atomics on one address are served one after the other, about ten
-    // nanoseconds each): the lanes count their hits in LDS first.  Below the threshold: a candidate.  Equal to it: counted
-    // for this workgroup's stretch of the input (group_ties), and listed while the list has room.
-    __shared__ unsigned int s_hits, s_base, s_ties, s_tbase;
-    const unsigned long long thr = st->thr;
-    const size_t i0 = (size_t)blockIdx.x * 1024 * kFilterPer + threadIdx.x;
-    unsigned long long key[kFilterPer];
-    if (threadIdx.x == 0) { s_hits = 0; s_ties = 0; }
-#pragma unroll
-    for (int q = 0; q < kFilterPer; ++q) {
-        const size_t i = i0 + (size_t)q * 1024;
-        key[q] = i < n ? time_key(t[i], f[i]) : kInfKey;
-    }
-    __syncthreads();
-    unsigned int mine = 0, mine_eq = 0;
-#pragma unroll
-    for (int q = 0; q < kFilterPer; ++q) { mine += key[q] < thr ? 1u : 0u; mine_eq += key[q] == thr ? 1u : 0u; }
-    unsigned int first = 0, first_eq = 0;
-    if (mine) first = atomicAdd(&s_hits, mine);
-    if (mine_eq) first_eq = atomicAdd(&s_ties, mine_eq);
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        if (s_hits) s_base = atomicAdd(&st->count, s_hits);
-        if (s_ties) s_tbase = atomicAdd(&st->count_eq, s_ties);
-        group_ties[blockIdx.x] = s_ties;
-    }
-    __syncthreads();
-    if (mine) {
-        unsigned int p = s_base + first;
-#pragma unroll
-        for (int q = 0; q < kFilterPer; ++q) {
-            if (key[q] < thr) {
-                if (p < kCandCap) cand[p] = Cand{key[q], (long long)(i0 + (size_t)q * 1024)};
-                ++p;
-            }
-        }
-    }
-    if (mine_eq) {
-        unsigned int p = s_tbase + first_eq;
-#pragma unroll
-        for (int q = 0; q < kFilterPer; ++q) {
-            if (key[q] == thr) {
-                if (p < kTieCap) tiecand[p] = Cand{key[q], (long long)(i0 + (size_t)q * 1024)};
-                ++p;
-            }
-        }
-    }
-}
-
-// Entry j of the selection's input: the candidates in LDS, or -- when more entries passed the filter than LDS holds --
-// the whole input again, read from global memory (slow, exact, and rare: see kShortMaxNK).
-struct ShortSource {
-    const unsigned long long *lkey; const unsigned int *lidx;     // LDS
-    const double *t; const uint8_t *f;                             // global
-    bool global;
-    __device__ __forceinline__ void get(size_t j, unsigned long long &key, unsigned int &idx) const {
-        if (global) { key = time_key(t[j], f[j]); idx = (unsigned int)j; }
-        else { key = lkey[j]; idx = lidx[j]; }
-    }
-};
-
-// Rank of `me` among the first `cnt` entries of `list` (LDS) in (key, index) order, for a whole wavefront at once: every
-// lane compares one entry, the ballots are counted (a lane that walks the list alone waits for one LDS read per entry).
-__device__ __forceinline__ unsigned int short_rank(const Cand *list, unsigned int cnt, const Cand me) {
-    const unsigned int lane = threadIdx.x & 63u;
-    unsigned int rank = 0;
-    for (unsigned int c = 0; c < cnt; c += 64) {
-        const unsigned int j = c + lane;
-        bool less = false;
-        if (j < cnt) {
-            const Cand o = list[j];
-            less = o.key < me.key || (o.key == me.key && o.idx < me.idx);
-        }
-        rank += (unsigned int)__popcll(__ballot(less));
-    }
-    return rank;
-}
-
-// (the selection in general: candidates in LDS or the whole input in global memory, equal keys at the threshold)
-__device__ __forceinline__ void short_final_any(unsigned char *smem, const double *t, const uint8_t *f, size_t n, ShortTopk *st,
-                                                const Cand *cand, const Cand *tiecand, const unsigned int *group_ties, int k,
-                                                long long *out_idx, double *out_val, int *out_count) {
-    unsigned long long *lkey = reinterpret_cast<unsigned long long *>(smem);                       // [kCandCap]
-    unsigned int *lidx = reinterpret_cast<unsigned int *>(smem + (size_t)kCandCap * 8);            // [kCandCap]
-    unsigned int *hist = lidx + kCandCap;                                                          // [kRadix]
-    Cand *win = reinterpret_cast<Cand *>(hist + kRadix);                                           // [kShortMaxK]
-    __shared__ unsigned int wsum[20];
-    __shared__ unsigned int s_nwin;
-    const int tid = threadIdx.x;
-    const unsigned int count_lt = st->count, count_eq = st->count_eq;
-    ShortSource src{lkey, lidx, t, f, count_lt > kCandCap};
-    // Entries equal to the threshold matter only if fewer than k lie below it.  Then: all of them join the candidates if
-    // they were listed one by one and fit; otherwise every entry below wins, and the lowest-indexed equal ones are read
-    // from the input (tie_scan, after the selection).
-    const bool want_ties = !src.global && count_lt < (unsigned)k && count_eq > 0;
-    const bool ties_listed = want_ties && count_eq <= kTieCap && count_lt + count_eq <= kCandCap;
-    const bool tie_scan = want_ties && !ties_listed;
-    const unsigned int count = count_lt + (ties_listed ? count_eq : 0u);
-    const size_t m = src.global ? n : (size_t)count;
-    if (!src.global) {
-        for (unsigned j = tid; j < count_lt; j += 1024) { const Cand c = cand[j]; lkey[j] = c.key; lidx[j] = (unsigned int)c.idx; }
-        if (ties_listed)
-            for (unsigned j = tid; j < count_eq; j += 1024) { const Cand c = tiecand[j]; lkey[count_lt + j] = c.key; lidx[count_lt + j] = (unsigned int)c.idx; }
-    }
-    if (tid == 0) s_nwin = 0;
-    // radix select on the 96-bit order (key, index): 6 passes over the key bits, then 3 over the index bits of the entries
-    // whose key is the selected one -- cut short as soon as the bucket that holds the k-th entry is small enough to be sorted
-    // as it is (usually after two passes).  State is kept by every lane alike (short_pick returns the same values to all).
-    constexpr unsigned kSmall = 512;                           // bucket entries that fit the histogram's LDS as (key, index) pairs
-    Cand *bucket = reinterpret_cast<Cand *>(hist);
-    __shared__ unsigned int s_nbucket;
-    __shared__ unsigned long long wmm[48];
-    unsigned long long mn = kInfKey, mx = 0, nf = 0;
-    __syncthreads();
-    for (size_t j = tid; j < m; j += 1024) {
-        unsigned long long key; unsigned int idx;
-        src.get(j, key, idx);
-        if (key != kInfKey) { mn = key < mn ? key : mn; mx = key > mx ? key : mx; ++nf; }
-    }
-    unsigned long long kmin, kmax, nfin;
-    short_minmax(mn, mx, nf, wmm, kmin, kmax, nfin);
-    const bool all = nfin < (unsigned long long)k;             // fewer (feasible) candidates than asked for: all of them win
-    int cur = (nfin == 0 || kmin == kmax) ? 0 : 64 - __clzll((long long)(kmin ^ kmax));      // the low `cur` key bits vary
-    unsigned long long prefix = cur >= 64 ? 0ull : (kmin >> cur) << cur;
-    unsigned int iprefix = 0, rem = (unsigned)k;
-    bool small = false;
-    int small_shift = 0, icur = 32;
-    if (tid == 0) s_nbucket = 0;
-    // key digits from the highest varying bit down, then index digits among the entries with the selected key
-    while (!all && !small && (cur > 0 || icur > 0)) {
-        for (int j = tid; j < kRadix; j += 1024) hist[j] = 0;
-        __syncthreads();
-        const bool on_key = cur > 0;
-        const int top = on_key ? cur : icur;
-        const int bits = top < kRadixBits ? top : kRadixBits, shift = top - bits;
-        for (size_t j = tid; j < m; j += 1024) {
-            unsigned long long key; unsigned int idx;
-            src.get(j, key, idx);
-            if (key == kInfKey) continue;
+            unsigned int before, total;
+            const unsigned int b = short_pick(s.hist, rem, s.wsum, before, total);
+            (void)total;
+            rem -= before;
             if (on_key) {
-                if (cur >= 64 || (key >> cur) == (prefix >> cur))
-                    atomicAdd(&hist[(unsigned)((key >> shift) & ((1ull << bits) - 1ull))], 1u);
-            } else if (key == prefix) {
-                if (icur >= 32 || (idx >> icur) == (iprefix >> icur)) atomicAdd(&hist[(idx >> shift) & ((1u << bits) - 1u)], 1u);
+                prefix |= (unsigned long long)b << shift;
+                cur = shift;
+                if (s.hist[b] <= kShortBucket) { small = true; small_shift = shift; }
+            } else {
+                iprefix |= b << shift;
+                icur = shift;
             }
+            __syncthreads();                                   // (hist[b] read by all before the next pass clears it)
         }
-        __syncthreads();
-        unsigned int before, total;
-        const unsigned int b = short_pick(hist, rem, wsum, before, total);
-        (void)total;
-        rem -= before;
-        if (on_key) {
-            prefix |= (unsigned long long)b << shift;
-            cur = shift;
-            if (hist[b] <= kSmall) { small = true; small_shift = shift; }
-        } else {
-            iprefix |= b << shift;
-            icur = shift;
-        }
-        __syncthreads();                                       // (hist[b] read by all before the next pass clears it)
-    }
-    // gather the winners
-    for (size_t j = tid; j < m; j += 1024) {
-        unsigned long long key; unsigned int idx;
-        src.get(j, key, idx);
-        if (key == kInfKey) continue;
-        bool wins;
-        if (all) wins = true;
-        else if (small) {
-            // the key bits from small_shift up are fixed: below the bucket -> a winner; in it -> sorted below
-            const unsigned long long hk = key >> small_shift, hp = prefix >> small_shift;
-            wins = hk < hp;
-            if (hk == hp) {
-                const unsigned int p = atomicAdd(&s_nbucket, 1u);
-                if (p < kSmall) bucket[p] = Cand{key, (long long)idx};
-            }
-        } else wins = key < prefix || (key == prefix && idx <= iprefix);
-        if (wins) {
-            const unsigned int p = atomicAdd(&s_nwin, 1u);
-            if (p < (unsigned)kShortMaxK) win[p] = Cand{key, (long long)idx};
-        }
-    }
-    __syncthreads();
-    if (small) {
-        // the `rem` smallest (key, index) of the bucket join the winners: an entry's rank is the number of entries before
-        // it in that order (the pairs are distinct); a wavefront ranks one entry at a time by ballot
-        const unsigned int nb = s_nbucket < kSmall ? s_nbucket : kSmall;
-        const unsigned int base = s_nwin;
-        for (unsigned int i = (unsigned int)tid >> 6; i < nb; i += 16) {
-            const Cand me = bucket[i];
-            const unsigned int rank = short_rank(bucket, nb, me);
-            if ((tid & 63) == 0 && rank < rem && base + rank < (unsigned)kShortMaxK) win[base + rank] = me;
-        }
-        __syncthreads();
-        if (tid == 0) s_nwin = base + rem;
-    }
-    __syncthreads();
-    if (tie_scan) {
-        // every candidate below the threshold has won (there are fewer than k: `all`); the rest of the k are the entries
-        // EQUAL to the threshold with the lowest indices.  group_ties[g] says how many of them stretch g of the input
-        // (8,192 consecutive entries) holds: stretches without any are skipped, the others read 1,024 entries at a time
-        // in index order, each lane ranking its entry among the equal ones of the step (wavefront ballots, one
-        // exchange through LDS), until enough are found.
-        const unsigned long long thr = st->thr;
-        const unsigned int need = (unsigned)k - s_nwin, base = s_nwin;
-        const unsigned int n_groups = (unsigned int)((n + 1024 * (size_t)kFilterPer - 1) / (1024 * (size_t)kFilterPer));
-        __shared__ unsigned int s_wave_ties[16];
-        unsigned int found = 0;
-        for (unsigned int g = 0; g < n_groups && found < need; ++g) {
-            if (group_ties[g] == 0) continue;                  // (the same for every lane)
-            for (int c = 0; c < kFilterPer && found < need; ++c) {
-                const size_t i = (size_t)g * 1024 * kFilterPer + (size_t)c * 1024 + (size_t)tid;
-                const bool eq = i < n && time_key(t[i], f[i]) == thr;
-                const unsigned long long mask = __ballot(eq);
-                const int lane = tid & 63, wave = tid >> 6;
-                if (lane == 0) s_wave_ties[wave] = (unsigned int)__popcll(mask);
-                __syncthreads();
-                unsigned int before = 0, total = 0;
-                for (int w = 0; w < 16; ++w) { const unsigned int v = s_wave_ties[w]; before += w < wave ? v : 0u; total += v; }
-                const unsigned int rank = found + before + (unsigned int)__popcll(mask & ((1ull << lane) - 1ull));
-                if (eq && rank < need && base + rank < (unsigned)kShortMaxK) win[base + rank] = Cand{thr, (long long)i};
-                found += total;
-                __syncthreads();
-            }
-        }
-        if (tid == 0) s_nwin = base + (found < need ? found : need);
-        __syncthreads();
-    }
-    const unsigned int nwin = s_nwin < (unsigned)k ? s_nwin : (unsigned)k;
-    // the winners in ascending (key, index) order, by rank as above
-    for (unsigned j = tid; j < (unsigned)k; j += 1024) {
-        if (j >= nwin) {
-            out_idx[j] = -1;
-            out_val[j] = __longlong_as_double(0x7ff0000000000000ll);
-        }
-    }
-    for (unsigned int i = (unsigned int)tid >> 6; i < nwin; i += 16) {
-        const Cand me = win[i];
-        const unsigned int rank = short_rank(win, nwin, me);
-        if ((tid & 63) == 0) {
-            unsigned long long b = me.key;
-            b = (b >> 63) ? (b & 0x7fffffffffffffffull) : ~b;
-            out_idx[rank] = me.idx;
-            out_val[rank] = __longlong_as_double((long long)b);
-        }
-    }
-    if (tid == 0 && out_count) *out_count = (int)nwin;
-}
-
-// The selection's common case -- at least k candidates below the threshold and no more than LDS-sized lists were made
-// for -- with the candidates in REGISTERS (twelve per lane, read once from global memory): the same radix select on
-// (key, index), but no pass reads anything, the bits that vary are found from key XOR threshold (every candidate lies
-// below the threshold, so the bits above the highest differing one are the threshold's: one 32-bit maximum over the
-// workgroup instead of a 64-bit minimum and maximum), and the two small sorts rank by ballot.
-__device__ __forceinline__ void short_final_fast(unsigned char *smem, const ShortTopk *st, const Cand *cand, unsigned int m, int k,
-                                                 long long *out_idx, double *out_val, int *out_count) {
-    constexpr int kPer = (int)((kCandCap + 1023u) / 1024u);
-    constexpr unsigned kSmall = 512;                           // bucket entries that fit the histogram's LDS as (key, index) pairs
-    unsigned int *hist = reinterpret_cast<unsigned int *>(smem);                                   // [kRadix]
-    Cand *bucket = reinterpret_cast<Cand *>(hist);                                                 // [kSmall], after the passes
-    Cand *win = reinterpret_cast<Cand *>(hist + kRadix);                                           // [kShortMaxK]
-    __shared__ unsigned int wsum[20];
-    __shared__ unsigned int s_nwin, s_nbucket, s_cur;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    unsigned long long rk[kPer];
-    unsigned int ri[kPer];
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        const unsigned int j = (unsigned int)tid + (unsigned int)q * 1024u;
-        rk[q] = kInfKey;
-        ri[q] = 0;
-        if (j < m) { const Cand c = cand[j]; rk[q] = c.key; ri[q] = (unsigned int)c.idx; }
-    }
-    if (tid == 0) { s_nwin = 0; s_nbucket = 0; s_cur = 0; }
-    const unsigned long long thr = st->thr;
-    int hb = 0;
-#pragma unroll
-    for (int q = 0; q < kPer; ++q) {
-        if (rk[q] != kInfKey) {
-            const int b = 64 - __clzll((long long)(rk[q] ^ thr));
-            hb = b > hb ? b : hb;
-        }
-    }
-    for (int off = 32; off > 0; off >>= 1) {
-        const int o = __shfl_xor(hb, off, 64);
-        hb = o > hb ? o : hb;
-    }
-    __syncthreads();
-    if (lane == 0) atomicMax(&s_cur, (unsigned int)hb);
-    __syncthreads();
-    int cur = (int)s_cur;                                      // the low `cur` key bits vary (>= 1: every key differs from thr)
-    unsigned long long prefix = cur >= 64 ? 0ull : (thr >> cur) << cur;
-    unsigned int iprefix = 0, rem = (unsigned)k;
-    bool small = false;
-    int small_shift = 0, icur = 32;
-    // key digits from the highest varying bit down, then index digits among the entries with the selected key
-    while (!small && (cur > 0 || icur > 0)) {
-        for (int j = tid; j < kRadix; j += 1024) hist[j] = 0;
-        __syncthreads();
-        const bool on_key = cur > 0;
-        const int top = on_key ? cur : icur;
-        const int bits = top < kRadixBits ? top : kRadixBits, shift = top - bits;
-#pragma unroll
-        for (int q = 0; q < kPer; ++q) {
-            const unsigned long long key = rk[q];
-            if (key == kInfKey) continue;
-            if (on_key) {
-                if (cur >= 64 || (key >> cur) == (prefix >> cur))
-                    atomicAdd(&hist[(unsigned)((key >> shift) & ((1ull << bits) - 1ull))], 1u);
-            } else if (key == prefix) {
-                if (icur >= 32 || (ri[q] >> icur) == (iprefix >> icur)) atomicAdd(&hist[(ri[q] >> shift) & ((1u << bits) - 1u)], 1u);
-            }
-        }
-        __syncthreads();
-        unsigned int before, total;
-        const unsigned int b = short_pick(hist, rem, wsum, before, total);
-        (void)total;
-        rem -= before;
-        if (on_key) {
-            prefix |= (unsigned long long)b << shift;
-            cur = shift;
-            if (hist[b] <= kSmall) { small = true; small_shift = shift; }
-        } else {
-            iprefix |= b << shift;
-            icur = shift;
-        }
-        __syncthreads();                                       // (hist[b] read by all before the next pass clears it)
     }
     // gather the winners (the bucket's entries go where the histogram was)
 #pragma unroll
     for (int q = 0; q < kPer; ++q) {
         const unsigned long long key = rk[q];
         if (key == kInfKey) continue;
-        bool wins;
+        bool wins = true;
         if (small) {
+            // the key bits from small_shift up are fixed: below the bucket -> a winner; in it -> ranked below
             const unsigned long long hk = key >> small_shift, hp = prefix >> small_shift;
             wins = hk < hp;
             if (hk == hp) {
-                const unsigned int p = atomicAdd(&s_nbucket, 1u);
-                if (p < kSmall) bucket[p] = Cand{key, (long long)ri[q]};
+                const unsigned int p = atomicAdd(&s.nbucket, 1u);
+                if (p < kShortBucket) s.bucket[p] = Cand{key, (long long)ri[q]};
             }
-        } else wins = key < prefix || (key == prefix && ri[q] <= iprefix);
+        } else if (!all) wins = key < prefix || (key == prefix && ri[q] <= iprefix);
         if (wins) {
-            const unsigned int p = atomicAdd(&s_nwin, 1u);
-            if (p < (unsigned)kShortMaxK) win[p] = Cand{key, (long long)ri[q]};
+            const unsigned int p = atomicAdd(&s.nwin, 1u);
+            if (p < (unsigned)kShortMaxK) s.win[p] = Cand{key, (long long)ri[q]};
         }
     }
     __syncthreads();
+    unsigned int nwin = s.nwin;
     if (small) {
         // the `rem` smallest (key, index) of the bucket join the winners, each at its rank
-        const unsigned int nb = s_nbucket < kSmall ? s_nbucket : kSmall;
-        const unsigned int base = s_nwin;
-        for (unsigned int i = (unsigned int)wave; i < nb; i += 16) {
-            const Cand me = bucket[i];
-            const unsigned int rank = short_rank(bucket, nb, me);
-            if (lane == 0 && rank < rem && base + rank < (unsigned)kShortMaxK) win[base + rank] = me;
-        }
+        const unsigned int nb = s.nbucket < kShortBucket ? s.nbucket : kShortBucket;
+        static_assert(kShortBucket * 2 <= 1024, "two lanes per entry");
+        Cand me;
+        const unsigned int rank = short_rank<2>(s.bucket, nb, me);
+        if (!(tid & 1) && rank < rem && nwin + rank < (unsigned)kShortMaxK) s.win[nwin + rank] = me;
+        nwin += rem;
         __syncthreads();
-        if (tid == 0) s_nwin = base + rem;
     }
-    __syncthreads();
-    const unsigned int nwin = s_nwin < (unsigned)k ? s_nwin : (unsigned)k;
+    return nwin < (unsigned)k ? nwin : (unsigned)k;
+}
+
+// The k best of each stretch of 1,024 * kPer entries: cand[k * workgroup ...], kInfKey behind the last one.
+template <int kPer>
+__global__ __launch_bounds__(1024) void topk_local(const double *t, const uint8_t *f, size_t n, int k, Cand *cand) {
+    __shared__ ShortShared s;
+    unsigned long long rk[kPer];
+    unsigned int ri[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const size_t i = ((size_t)blockIdx.x * kPer + q) * 1024 + threadIdx.x;
+        rk[q] = i < n ? time_key(t[i], f[i]) : kInfKey;
+        ri[q] = (unsigned int)i;
+    }
+    const unsigned int nwin = short_select<kPer>(s, rk, ri, k);
+    for (unsigned int j = threadIdx.x; j < (unsigned)k; j += 1024)
+        cand[(size_t)blockIdx.x * k + j] = j < nwin ? s.win[j] : Cand{kInfKey, 0x7fffffffffffffffll};
+}
+
+// The k best of all: of the input itself (cand == nullptr) or of the m entries that topk_local left.
+template <int kPer>
+__global__ __launch_bounds__(1024) void topk_final(const double *t, const uint8_t *f, const Cand *cand, unsigned int m, int k,
+                                                   long long *out_idx, double *out_val, int *out_count) {
+    __shared__ ShortShared s;
+    const int tid = threadIdx.x;
+    unsigned long long rk[kPer];
+    unsigned int ri[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const unsigned int i = (unsigned int)q * 1024u + (unsigned int)tid;
+        rk[q] = kInfKey;
+        ri[q] = i;
+        if (i < m) {
+            if (cand) {
+                const Cand c = cand[i];
+                rk[q] = c.key;
+                ri[q] = (unsigned int)c.idx;
+            } else
+                rk[q] = time_key(t[i], f[i]);
+        }
+    }
+    const unsigned int nwin = short_select<kPer>(s, rk, ri, k);
     for (unsigned j = tid; j < (unsigned)k; j += 1024) {
         if (j >= nwin) {
             out_idx[j] = -1;
@@ -913,28 +574,29 @@ __device__ __forceinline__ void short_final_fast(unsigned char *smem, const Shor
         }
     }
     // the winners in ascending (key, index) order
-    for (unsigned int i = (unsigned int)wave; i < nwin; i += 16) {
-        const Cand me = win[i];
-        const unsigned int rank = short_rank(win, nwin, me);
-        if (lane == 0) {
-            unsigned long long b = me.key;
-            b = (b >> 63) ? (b & 0x7fffffffffffffffull) : ~b;
-            out_idx[rank] = me.idx;
-            out_val[rank] = __longlong_as_double((long long)b);
-        }
+    static_assert(kShortMaxK * 4 <= 1024, "four lanes per winner");
+    Cand me;
+    const unsigned int rank = short_rank<4>(s.win, nwin, me);
+    if (!(tid & 3) && rank < nwin) {
+        unsigned long long b = me.key;
+        b = (b >> 63) ? (b & 0x7fffffffffffffffull) : ~b;
+        out_idx[rank] = me.idx;
+        out_val[rank] = __longlong_as_double((long long)b);
     }
     if (tid == 0 && out_count) *out_count = (int)nwin;
 }
 
-__global__ __launch_bounds__(1024) void topk_short_final(const double *t, const uint8_t *f, size_t n, ShortTopk *st, const Cand *cand,
-                                                         const Cand *tiecand, const unsigned int *group_ties, int k,
-                                                         long long *out_idx, double *out_val, int *out_count) {
-    extern __shared__ __align__(16) unsigned char smem[];
-    const unsigned int count_lt = st->count;
-    if (count_lt >= (unsigned)k && count_lt <= kCandCap) short_final_fast(smem, st, cand, count_lt, k, out_idx, out_val, out_count);
-    else short_final_any(smem, t, f, n, st, cand, tiecand, group_ties, k, out_idx, out_val, out_count);
+// Entries per workgroup of topk_local for n entries (0: topk_final alone): short stretches while the selection from what they
+// leave stays short too (4,096 entries), longer ones while it fits one workgroup, or none at all (~0u).
+unsigned int short_stretch(size_t n, int k) {
+    if (k > kShortMaxK || n > 0xffffffffull) return ~0u;
+    if (n <= kShortMaxEntries) return 0;
+    const auto found = [&](size_t per) { return (n + per - 1) / per * (size_t)k; };
+    if (found(4096) <= 4096) return 4096;
+    if (found(8192) <= kShortMaxEntries) return 8192;
+    if (found(16384) <= kShortMaxEntries) return 16384;
+    return ~0u;
 }
-constexpr size_t kShortLds = (size_t)kCandCap * 12 + (size_t)kRadix * 4 + (size_t)kShortMaxK * sizeof(Cand);
 
 unsigned int next_pow2(unsigned int v) {
     unsigned int p = 1;
@@ -1353,8 +1015,6 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = upload((void **)&h->d_win_row_begin, t->win_row_begin, (size_t)(t->n_windows + 1) * 4)) ||
         (rc = upload((void **)&h->d_win_rows, t->win_rows, (size_t)n_win_rows * 8)) ||
         (rc = setup_windowed_asm(h, t, pos_entries, rk_bytes, stg_words)) ||
-        (rc = hipFuncSetAttribute(reinterpret_cast<const void *>(&topk_short_final), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                  (int)kShortLds) == hipSuccess ? ACE_OK : ACE_EHIP) ||
         (rc = allow_big_lds<false, false, false, false>()) || (rc = allow_big_lds<false, false, true, false>()) ||
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
@@ -1620,9 +1280,8 @@ size_t ace_topk_workspace_bytes(size_t n, int k) {
     if (k <= 0) return 0;
     const unsigned cap = topk_cap(k);
     const unsigned p2 = next_pow2(2 * cap);
-    // (the last part: state and candidates of the short form)
-    return 256 + sizeof(unsigned int) * kRadix + sizeof(Cand) * ((size_t)cap * 2 + p2) + 256 + sizeof(Cand) * (kCandCap + kTieCap) +
-           sizeof(unsigned int) * kMaxFilterGroups;
+    // (the last part: what the short form's first launch leaves)
+    return 256 + sizeof(unsigned int) * kRadix + sizeof(Cand) * ((size_t)cap * 2 + p2) + sizeof(Cand) * kShortMaxEntries;
 }
 
 int ace_topk(ace_handle_t *h, const double *d_iter_ms, const uint8_t *d_feasible, size_t n, int k, int64_t *d_idx,
@@ -1641,16 +1300,15 @@ int ace_topk(ace_handle_t *h, const double *d_iter_ms, const uint8_t *d_feasible
     unsigned blocks = (unsigned)((n + kTopBlock * 8 - 1) / (kTopBlock * 8));
     if (blocks < 1) blocks = 1;
     if (blocks > 2048) blocks = 2048;
-    if (k <= kShortMaxK && n * (size_t)k <= kShortMaxNK && n <= 0xffffffffull) {
-        ShortTopk *sst = (ShortTopk *)(buf + p2);
-        Cand *cand = (Cand *)((unsigned char *)sst + 256);
-        Cand *tiecand = cand + kCandCap;
-        unsigned int *group_ties = (unsigned int *)(tiecand + kTieCap);      // (at most kMaxFilterGroups filter workgroups: n <= kShortMaxNK)
-        hipLaunchKernelGGL(topk_sample, dim3(1), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, sst);
-        hipLaunchKernelGGL(topk_filter, dim3((unsigned)((n + 1024 * kFilterPer - 1) / (1024 * kFilterPer))), dim3(1024), 0, s, d_iter_ms,
-                           d_feasible, n, sst, cand, tiecand, group_ties);
-        hipLaunchKernelGGL(topk_short_final, dim3(1), dim3(1024), kShortLds, s, d_iter_ms, d_feasible, n, sst, cand, tiecand, group_ties, k,
-                           (long long *)d_idx, d_val, d_count);
+    const unsigned int per = short_stretch(n, k);
+    if (per != ~0u) {
+        Cand *cand = per ? buf + p2 : nullptr;
+        const unsigned int groups = per ? (unsigned int)((n + per - 1) / per) : 0u, m = per ? groups * (unsigned int)k : (unsigned int)n;
+        if (per == 4096) hipLaunchKernelGGL(topk_local<4>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, cand);
+        else if (per == 8192) hipLaunchKernelGGL(topk_local<8>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, cand);
+        else if (per) hipLaunchKernelGGL(topk_local<16>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, cand);
+        const auto last = m <= 4096 ? topk_final<4> : m <= 8192 ? topk_final<8> : topk_final<16>;
+        hipLaunchKernelGGL(last, dim3(1), dim3(1024), 0, s, d_iter_ms, d_feasible, cand, m, k, (long long *)d_idx, d_val, d_count);
         ACE_HIP(hipGetLastError());
         return ACE_OK;
     }
