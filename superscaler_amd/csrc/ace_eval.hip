@@ -24,6 +24,7 @@
 #include "ace_moves_host.h"
 #include "ace_score_loop.h"
 #include "ace_spread.h"
+#include "ace_duo.h"
 #include "ace_recompute.h"
 
 // Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans (the
@@ -80,6 +81,11 @@ __global__ __launch_bounds__(kSpreadLanes) void ace_spread_kernel(const AceKerne
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_spread_body<BD, RANGED, COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
+// Mid-sized batches: several lanes per plan, see ace_duo.h.
+template <int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(const AceKernelArgs a) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    ace_duo_body<L>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+}
 template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
@@ -94,6 +100,12 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
 //   queries  523 ops:   64      163 -> 20, 1,024 189 -> 21, 4,096 194 -> 38, 16,384 169 -> 112 (315 ops: 106 -> 122)
 #ifndef ACE_SPREAD_MAX_PLAIN
 #define ACE_SPREAD_MAX_PLAIN 4096
+#endif
+// ... and where the kernel of mid-sized batches can run, whose time hardly grows from 64 to 16,384 plans: up to this many
+// (3,584 / 3,840 / 4,096 plans, us, plan per workgroup -> mid-sized: 315 ops 39 / 41 / 45 -> 43, 523 ops 57 / 60 / 65 -> 67,
+// 821 ops 79 / 82 / 89 -> 81, 1,251 ops 104 / 106 / 119 -> 107).
+#ifndef ACE_SPREAD_MAX_MID
+#define ACE_SPREAD_MAX_MID 3840
 #endif
 #ifndef ACE_SPREAD_MAX_RECORDS
 #define ACE_SPREAD_MAX_RECORDS 8192
@@ -718,6 +730,11 @@ template <bool BD, bool RANGED, bool WIN, bool DEFER> static int allow_big_lds()
     return ACE_OK;
 }
 
+template <int L> static int allow_duo_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<L>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    return ACE_OK;
+}
+
 // Per op position, what the assembly form of the op loop (ace_score_loop_asm.inc) reads with scalar loads: the LDS
 // address of the position's row at its hot sub-table and at its collective-cost tables, the LDS address of the
 // 32-bit pair-kind block of the (this op, next op) pair, and two flags (bit 0: the rule "ordinary op followed by a layer
@@ -1018,6 +1035,8 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = allow_big_lds<false, false, false, false>()) || (rc = allow_big_lds<false, false, true, false>()) ||
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
+        (rc = allow_duo_lds<64>()) || (rc = allow_duo_lds<128>()) || (rc = allow_duo_lds<256>()) ||
+        (rc = allow_duo_lds<512>()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
         ace_destroy(h);
         return rc;
@@ -1109,8 +1128,27 @@ static void launch_spread(const AceKernelArgs &a, hipStream_t s) {
     else launch_spread_c<BD, RANGED, false>(a, s);
 }
 
+// Workgroup size of the kernel of mid-sized batches for this call, or 0: plain scoring of a batch that leaves the large kernel
+// short of wavefronts, of tables the assembly loops can run on.
+static int duo_lanes(const ace_handle_t *h, const AceKernelArgs &a) {
+    if (a.range || a.stage_out || !a.stage_ws || h->n_windows > 1 || !a.pos4 || !a.g.lut2a_lds_off || a.flat_rows16 <= 0) return 0;
+    const int L = ace_duo_lanes(a.g.P);
+    return L && ace_duo_lds(a.g, h->lds_bytes, L) <= kMaxLds ? L : 0;
+}
+template <int L>
+static void launch_duo_l(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    hipLaunchKernelGGL((ace_duo_kernel<L>), dim3((unsigned)((a.g.P + L - 1) / L)), dim3(kDuoBlock), ace_duo_lds(a.g, h->lds_bytes, L), s, a);
+}
+static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    if (L == 64) launch_duo_l<64>(h, a, s);
+    else if (L == 128) launch_duo_l<128>(h, a, s);
+    else if (L == 256) launch_duo_l<256>(h, a, s);
+    else launch_duo_l<512>(h, a, s);
+}
+
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    if (a.pos_spread && a.g.P <= (a.stage_out ? ACE_SPREAD_MAX_RECORDS : ACE_SPREAD_MAX_PLAIN)) {
+    const int mid = duo_lanes(h, a);
+    if (a.pos_spread && a.g.P <= (a.stage_out ? ACE_SPREAD_MAX_RECORDS : mid ? ACE_SPREAD_MAX_MID : ACE_SPREAD_MAX_PLAIN)) {
         if (a.range) launch_spread<true, true>(a, s);
         else if (a.stage_out) launch_spread<true, false>(a, s);
         else launch_spread<false, false>(a, s);
@@ -1119,6 +1157,7 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
     if (a.range) launch_score_w<true, true>(h, a, s);
     else if (a.stage_out) launch_score_w<true, false>(h, a, s);
     else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
+    else if (mid) launch_duo(mid, h, a, s);
     else if (a.stage_ws) launch_score_b<false, false, false, true>(h, a, s);
     else launch_score_w<false, false>(h, a, s);
 }

@@ -225,6 +225,7 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
     uint64_t rk_all;            // per stage (4 bits each): the stage size as the pair-kind tables index it
     uint64_t diag_next, rk_next;   // diags / rk_all shifted down by the stages handed out so far
     uint32_t ws_stride;         // DEFER: 16-byte units between two stages of one plan in the workspace
+    uint32_t ws_piece;          // ... between the 16-byte pieces of a record (replay)
     uint32_t ws_off;            // DEFER: 16-byte units from the plan's first slot to the slot of the current stage (fits: see ensure_stage_ws)
     uint64_t glogs_next;        // DEFER: glogs shifted down by the stages handed out so far
     uint32_t lut2_lane;         // DEFER: LDS address of the offset pairs of this plan's micro-batch size
@@ -247,6 +248,7 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
         status = 0;
         lastclose = false; replay_row = 0; replay_code = 0; r_next = 0; pair_prev = 0; row_ids = nullptr;
         ws_stride = ACE_WS_REC / 2;
+        ws_piece = 1;
         ws_off = 0;
         fwd = bwd = rcs = W = A = saved = run = peak = rfm = rbm = rs_f = rs_b = mc = 0.0;
         id_fwd = id_bwd = id_in = 0.0;
@@ -395,7 +397,7 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
         const int sl = s2 < ACE_MAX_STAGES ? s2 : ACE_MAX_STAGES - 1;
         const ace_d2 *p = reinterpret_cast<const ace_d2 *>(ws) + (size_t)((uint32_t)sl * ws_stride);
 #pragma unroll
-        for (int j = 0; j < 5; ++j) rec.r[j] = p[j];
+        for (int j = 0; j < 5; ++j) rec.r[j] = p[(uint32_t)j * ws_piece];
     }
 
     // `live`: the plan has a stage s2 (else the record is whatever the slot held: entry 0 of row 0 is looked up, and
@@ -468,6 +470,46 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
         }
     replayed:
         s = n_st;               // (the evaluation walked s again; result() checks the count of the op loop)
+    }
+
+    // The stashed stages first, first + step, ... (< n_st) alone: `take(s, t)` gets the time of each, max_mem becomes the
+    // largest of their memories.  What links a stage to the one before it (the row and code of its first op) is read from
+    // that one's record.  Three records in flight, as above.
+    template <class Take>
+    ACE_HD void replay_some(const AceGeom &g, const AceLds &lds, const double *ws, int first, int step, int n_st, uint32_t code0, uint32_t row0,
+                            Take take) {
+        Record r[3];
+        uint64_t link[3];
+        auto fetch = [&](int s2, int k) {
+            replay_load(ws, s2, r[k]);
+            link[k] = 0;
+            if (s2 > 0) {
+                const ace_d2 *p = reinterpret_cast<const ace_d2 *>(ws) + (size_t)((uint32_t)(s2 - 1) * ws_stride + 4u * ws_piece);
+                __builtin_memcpy(&link[k], &p->y, 8);
+            }
+        };
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            if (first + k * step < n_st) fetch(first + k * step, k);
+        for (int base = first; base < ACE_MAX_STAGES; base += 3 * step) {
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                const int s2 = base + k * step;
+                if (!ACE_WAVE_ANY(s2 < n_st)) return;
+                if (s2 < n_st) {
+                    const uint32_t hi = (uint32_t)(link[k] >> 32);
+                    replay_row = s2 > 0 ? hi >> 24 : row0;
+                    replay_code = s2 > 0 ? ((uint32_t)link[k] >> (8u * (hi & 3u))) & 7u : code0;
+                    Lookups lx;
+                    replay_lookups(g, lds, r[k], s2, true, lx);
+                    replay_take(g, r[k], lx, s2);
+                    if (s2 + 3 * step < n_st) fetch(s2 + 3 * step, k);
+                    sum_t = 0.0;
+                    finish_tail(g, lds, 0u, lx.c_last, lx.oe, nullptr);
+                    take(s2, sum_t);
+                }
+            }
+        }
     }
 
     // Address of output_size[ops[-1]][mbs[-1]][tp[0]][algo[-1]] (sic, aceso_cost_model.py:321-326) in the row at `lastrow`:

@@ -93,6 +93,41 @@ template <int BLOCK> ACE_HD void stage_rows_flat(const AceKernelArgs &a, unsigne
     for (; j < n; j += BLOCK) dst[j] = src[j];
 }
 
+// The small tables to LDS (whole workgroup); DEFER: in the assembly loops' forms too.
+template <int BLOCK, bool DEFER> ACE_HD void stage_small_tables(const AceKernelArgs &a, unsigned char *lds_raw, int tid) {
+    // pair kinds and the (micro-batch, stage gpus) LUT
+    // (four pair kinds per lane and turn: the table is a multiple of 64 bytes)
+    for (int j = tid; j < (a.rk_bytes >> 2); j += BLOCK) {
+        const uint32_t r4 = reinterpret_cast<const uint32_t *>(a.pair_kinds)[j];
+        reinterpret_cast<uint32_t *>(lds_raw + a.g.rk_lds_off)[j] = r4;
+        if (DEFER && a.g.pk32_lds_off) {
+            uint32_t e[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t r = (r4 >> (8 * q)) & 0xffu;
+                e[q] = ((r & 15u) << a.g.z_shift) | (((r >> 4) << a.g.z_shift) << 16);
+            }
+            // (entries 4j .. 4j + 3 of block j / 16; the blocks are ACE_PK32_BLOCK words apart)
+            uint32_t *dst = reinterpret_cast<uint32_t *>(lds_raw + a.g.pk32_lds_off) + (4 * j + (j >> 4) * (int)(ACE_PK32_BLOCK - 64u));
+#pragma unroll
+            for (int q = 0; q < 4; ++q) dst[q] = e[q];
+        }
+    }
+    for (int j = tid; j < a.stg_words; j += BLOCK) {
+        const uint32_t w = a.stage_lut[j];
+        reinterpret_cast<uint32_t *>(lds_raw + a.g.stg_lds_off)[j] = w;
+        // entry j = micro-batch index * 16 + log2(stage size): byte offset of the stage's diag inside the cost sub-tables,
+        // and the pair-kind block of the stage size relative to it (what PlanState::start_fast hands to the op loop)
+        const uint32_t glog = (uint32_t)j & 15u;
+        const uint32_t z_v = (w & 15u) * (uint32_t)a.g.C * 8u;
+        const uint32_t gl = glog < (uint32_t)a.g.n_glog ? glog : 0u, rk = gl << 6;
+        reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2_lds_off)[j] = ace_u2{z_v, rk - z_v};
+        // (the assembly loop adds the pair-kind block offset to the op pair's own index, not to the diag's, and its blocks
+        // are ACE_PK32_BLOCK words apart)
+        if (DEFER && a.g.lut2a_lds_off) reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2a_lds_off)[j] = ace_u2{z_v, gl * ACE_PK32_BLOCK};
+    }
+}
+
 // Copy the rows window `w` needs from global memory into LDS (whole workgroup).
 template <int BLOCK> ACE_HD void stage_window(const AceKernelArgs &a, unsigned char *lds_raw, int w, int tid) {
     const int rb = a.win_row_begin[w], re = a.win_row_begin[w + 1];
@@ -259,37 +294,7 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
     const ace_u4 h = a.hdr[pl];
     ace_u4 cw = a.codes[(size_t)grp_begin * g.P + pl];
 
-    // small tables: pair kinds and the (micro-batch, stage gpus) LUT; without windows, every row
-    // (four pair kinds per lane and turn: the table is a multiple of 64 bytes)
-    for (int j = tid; j < (a.rk_bytes >> 2); j += BLOCK) {
-        const uint32_t r4 = reinterpret_cast<const uint32_t *>(a.pair_kinds)[j];
-        reinterpret_cast<uint32_t *>(lds_raw + a.g.rk_lds_off)[j] = r4;
-        if (DEFER && a.g.pk32_lds_off) {
-            uint32_t e[4];
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t r = (r4 >> (8 * q)) & 0xffu;
-                e[q] = ((r & 15u) << a.g.z_shift) | (((r >> 4) << a.g.z_shift) << 16);
-            }
-            // (entries 4j .. 4j + 3 of block j / 16; the blocks are ACE_PK32_BLOCK words apart)
-            uint32_t *dst = reinterpret_cast<uint32_t *>(lds_raw + a.g.pk32_lds_off) + (4 * j + (j >> 4) * (int)(ACE_PK32_BLOCK - 64u));
-#pragma unroll
-            for (int q = 0; q < 4; ++q) dst[q] = e[q];
-        }
-    }
-    for (int j = tid; j < a.stg_words; j += BLOCK) {
-        const uint32_t w = a.stage_lut[j];
-        reinterpret_cast<uint32_t *>(lds_raw + a.g.stg_lds_off)[j] = w;
-        // entry j = micro-batch index * 16 + log2(stage size): byte offset of the stage's diag inside the cost sub-tables,
-        // and the pair-kind block of the stage size relative to it (what PlanState::start_fast hands to the op loop)
-        const uint32_t glog = (uint32_t)j & 15u;
-        const uint32_t z_v = (w & 15u) * (uint32_t)a.g.C * 8u;
-        const uint32_t gl = glog < (uint32_t)a.g.n_glog ? glog : 0u, rk = gl << 6;
-        reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2_lds_off)[j] = ace_u2{z_v, rk - z_v};
-        // (the assembly loop adds the pair-kind block offset to the op pair's own index, not to the diag's, and its blocks
-        // are ACE_PK32_BLOCK words apart)
-        if (DEFER && a.g.lut2a_lds_off) reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2a_lds_off)[j] = ace_u2{z_v, gl * ACE_PK32_BLOCK};
-    }
+    stage_small_tables<BLOCK, DEFER>(a, lds_raw, tid);
     // (the assembly op loop over windowed rows fetches its windows itself, in a layout of its own)
 #ifndef ACE_HOST_EMU
     const bool asm_loop = DEFER && lds_base == 0u && a.pos4 && a.g.lut2a_lds_off && (!WIN || (BLOCK == 1024 && a.win_dma));

@@ -1,0 +1,64 @@
+"""The kernel of mid-sized batches (superscaler_amd/csrc/ace_duo.h: a plan walked by several lanes of different wavefronts).
+
+On the GPU: around the batch sizes at which the launcher changes the workgroup, every plan against the C oracle, statuses of
+malformed plans against the emulation.  On the CPU: the committed op loop is what its generator writes."""
+import importlib.util
+import os
+import re
+
+import numpy as np
+import pytest
+
+from superscaler_amd import synth
+from superscaler_amd.plan import PlanBatch
+from tests.helpers import c_oracle_scores, emu_score
+from tests.test_small_batches import SETTINGS, WORKLOADS, tables_for, with_recompute
+
+CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "superscaler_amd", "csrc")
+
+
+def test_committed_duo_loop_is_the_generators_output():
+    spec = importlib.util.spec_from_file_location("gen_duo_loop_asm", os.path.join(CSRC, "gen_duo_loop_asm.py"))
+    gen = importlib.util.module_from_spec(spec)
+    spec.loader.exec_module(gen)
+    text = gen.render()
+    with open(os.path.join(CSRC, "ace_duo_loop_asm.inc")) as f:
+        assert f.read() == text
+    # the operands of the statement live below v28 / s24, the stack registers are s32 / s33
+    body = text.split("#define ACE_DUO_ASM_CLOBBERS")[0]
+    for kind, low, high in (("v", 28, 127), ("s", 24, 99)):
+        for m in re.finditer(rf"\b{kind}(\d+)\b|\b{kind}\[(\d+):(\d+)\]", body):
+            a, b = int(m.group(1) or m.group(2)), int(m.group(1) or m.group(3))
+            assert low <= a <= b <= high and not (kind == "s" and a <= 33 and b >= 32), m.group(0)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,mode,sizes", [("gpt3_13b", "plain", (3840, 3841, 16385)), ("t5_770m", "min", (8191,)), ("gpt3_175b", "noreserved", (4999,)),
+                                             ("gpt3_1_3b", "min", (16384,)), ("gpt_wide_stages", "plain", (5000, 32768, 32769, 65537)),
+                                             ("gpt_16ops", "noreserved", (65536, 131072, 131073)), ("gpt_3tp", "min", (20001, 100001)),
+                                             ("t5_1layer", "plain", (16383, 70000))])
+def test_mid_sized_batches_on_the_gpu(name, mode, sizes):
+    from superscaler_amd.evaluator import PlanEvaluator
+    w = WORKLOADS[name]
+    tables = tables_for(w, **SETTINGS[mode])
+    assert tables.n_windows == 1
+    ev = PlanEvaluator(tables)
+    for n in sizes:
+        print(f"[case] {name} {mode} plans={n}", flush=True)
+        batch = with_recompute(synth.make_plans(w, tables, n_plans=n, seed_offset=n), 0.6, n)
+        it, pk, fe, st = ev.score_host(batch)
+        cit, cpk, cfe, cer = c_oracle_scores(tables, batch, threads=8)
+        assert not cer.any() and (st == 0).all()
+        assert np.array_equal(it, cit) and np.array_equal(pk, cpk) and np.array_equal(fe, cfe)
+    # malformed plans among good ones: status and NaN as everywhere
+    bad = PlanBatch(batch.codes.copy(), batch.hdr.copy())
+    bad.codes[0, 0] &= 0xEF                 # no stage start in front
+    bad.codes[1, 1:] |= 16                  # a stage per op
+    bad.hdr[2, 0] = 40                      # more stages than there may be
+    bad.hdr[3, 0] |= 0xff00                 # no such micro-batch size
+    got = [x.cpu().numpy() for x in ev.score(ev.upload(bad, validate=False))[:4]]
+    want = emu_score(tables, bad.slice(0, 64))
+    for g, x in zip(got, want):
+        assert x is None or np.array_equal(g[:64], x, equal_nan=True)
+    assert np.array_equal(got[0][64:], it[64:]) and np.array_equal(got[1][64:], pk[64:])
+    ev.close()
