@@ -141,8 +141,17 @@ class CostModel:
         batch = self.encode(configs)
         it, pk, fe, st, rec = self.evaluator.score_host(batch, breakdown=True)
         self._raise_for_status(st)
-        for p, cfg in enumerate(configs):
-            self._fill_breakdown(cfg, rec[p])
+        self._fill_all(configs, rec)
+
+    def _fill_all(self, configs, rec):
+        """_fill_breakdown for every plan of a list: natively, except the plan objects that are left to the Python code."""
+        args, fill, p = self.settings, load_objects().fill_all, 0
+        while True:
+            p = fill(configs, rec, p, args.memory_limit, args.memory_main_params, args.memory_optimizer, args.consider_reserved_space)
+            if p >= len(configs):
+                return
+            self._fill_breakdown(configs[p], rec[p])
+            p += 1
 
     def _fill_breakdown(self, config, rec, print_time=False, print_memory=False):
         """aceso_cost_model.py:541-672 from the kernel's per-stage records."""

@@ -1,11 +1,11 @@
 // Plan objects <-> arrays: the parts of a predict_time_breakdown call that walk Python objects (module superscaler_amd._ace_objects).
 //
 //   encode(...)  AcesoConfig-like objects -> code rows and headers (PlanBatch.from_configs)
-//   fill(...)    stage records -> the lists that predict_time_breakdown leaves on a plan object (CostModel._fill_breakdown)
+//   fill(...), fill_all(...)    stage records -> the lists that predict_time_breakdown leaves on a plan object (CostModel._fill_breakdown)
 //
-// Both handle what a search hands over -- lists of small ints -- and leave everything else (other types, other lengths,
+// They handle what a search hands over -- lists of small ints -- and leave everything else (other types, other lengths,
 // values outside the profile database, divisions by zero) to the Python code, which raises what it always raised: encode
-// returns the index of the first plan it did not take, fill returns False.  The floating-point operations of fill are
+// and fill_all return the index of the first plan they did not take, fill returns False.  The floating-point operations of fill are
 // those of the Python code, one IEEE operation each in the same order (the file is compiled with contraction off), and
 // sums of lists go through builtins.sum.
 //
@@ -178,19 +178,10 @@ bool list_sum(const double *v, long n, double *out) {
     return !PyErr_Occurred();
 }
 
-// fill(config, records (double[16][18] buffer), memory_limit, main_params, optimizer, consider_reserved)
-PyObject *fill(PyObject *, PyObject *args) {
-    PyObject *cfg;
-    Py_buffer buf;
-    double max_mem, main_params, optimizer;
-    int reserved_on;
-    if (!PyArg_ParseTuple(args, "Oy*dddp", &cfg, &buf, &max_mem, &main_params, &optimizer, &reserved_on)) return nullptr;
-    double rec[kMaxStages][kRec];
-    const bool have = buf.len >= (Py_ssize_t)sizeof(rec);
-    if (have) memcpy(rec, buf.buf, sizeof(rec));
-    PyBuffer_Release(&buf);
+// One plan from its records: 1, 0 (left to the Python code) or -1 (an exception is set).
+int fill_one(PyObject *cfg, const double (*rec)[kRec], double max_mem, double main_params, double optimizer, int reserved_on) {
     long S = 0, global = 0, micro = 0;
-    bool ok = have && int_attr(cfg, s_num_stages, &S) && S >= 1 && S <= kMaxStages && int_attr(cfg, s_global_bs, &global) &&
+    bool ok = int_attr(cfg, s_num_stages, &S) && S >= 1 && S <= kMaxStages && int_attr(cfg, s_global_bs, &global) &&
               int_attr(cfg, s_micro_bs, &micro) && micro > 0 && global >= 0;
     Ref stages(ok ? PyObject_GetAttr(cfg, s_stages) : nullptr);
     ok = ok && stages && PyList_Check(stages.p) && PyList_GET_SIZE(stages.p) >= S;
@@ -238,7 +229,7 @@ PyObject *fill(PyObject *, PyObject *args) {
     ok = ok && list_sum(t, S, &sum_stage) && list_sum(gpu, S, &sum_gpu);
     if (!ok) {
         if (PyErr_Occurred()) PyErr_Clear();
-        Py_RETURN_FALSE;
+        return 0;
     }
     const double nb1 = (double)(global / micro - 1);
     double times[kMaxStages], idle[kMaxStages];
@@ -261,12 +252,57 @@ PyObject *fill(PyObject *, PyObject *args) {
         PyObject_SetAttr(cfg, s_total_gpu_time, total.p) != 0 || !set_list(cfg, s_breakdown_ideal_time_per_gpu, ideal, S) ||
         !set_list(cfg, s_breakdown_eff_loss_time_per_gpu, loss, S) || !set_list(cfg, s_breakdown_recomp_time_per_gpu, recomp_l, S) ||
         !set_list(cfg, s_efficient_time_list, idle, S))
+        return -1;
+    return 1;
+}
+
+// fill(config, records (double[16][18] buffer), memory_limit, main_params, optimizer, consider_reserved): whether it did
+PyObject *fill(PyObject *, PyObject *args) {
+    PyObject *cfg;
+    Py_buffer buf;
+    double max_mem, main_params, optimizer;
+    int reserved_on;
+    if (!PyArg_ParseTuple(args, "Oy*dddp", &cfg, &buf, &max_mem, &main_params, &optimizer, &reserved_on)) return nullptr;
+    double rec[kMaxStages][kRec];
+    const bool have = buf.len >= (Py_ssize_t)sizeof(rec);
+    if (have) memcpy(rec, buf.buf, sizeof(rec));
+    PyBuffer_Release(&buf);
+    const int rc = have ? fill_one(cfg, rec, max_mem, main_params, optimizer, reserved_on) : 0;
+    if (rc < 0) return nullptr;
+    return PyBool_FromLong(rc);
+}
+
+// fill_all(configs (a sequence), records (double[n][16][18] buffer), start, memory_limit, main_params, optimizer, consider_reserved):
+// the plans from `start` on; returns the index of the first one not taken (all of them: their number)
+PyObject *fill_all(PyObject *, PyObject *args) {
+    PyObject *configs;
+    Py_buffer buf;
+    Py_ssize_t p;
+    double max_mem, main_params, optimizer;
+    int reserved_on;
+    if (!PyArg_ParseTuple(args, "Oy*ndddp", &configs, &buf, &p, &max_mem, &main_params, &optimizer, &reserved_on)) return nullptr;
+    Ref seq(PySequence_Fast(configs, "fill_all: a sequence of plans"));
+    const Py_ssize_t have = buf.len / (Py_ssize_t)(sizeof(double) * kMaxStages * kRec);
+    int rc = seq && p >= 0 ? 1 : -1;
+    for (; rc == 1 && p < PySequence_Fast_GET_SIZE(seq.p); ++p) {
+        double rec[kMaxStages][kRec];                        // (a copy: the buffer need not be aligned)
+        rc = p < have;
+        if (!rc) break;
+        memcpy(rec, static_cast<const char *>(buf.buf) + (size_t)p * sizeof(rec), sizeof(rec));
+        rc = fill_one(PySequence_Fast_GET_ITEM(seq.p, p), rec, max_mem, main_params, optimizer, reserved_on);
+        if (rc != 1) break;
+    }
+    PyBuffer_Release(&buf);
+    if (rc < 0) {
+        if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "fill_all: start");
         return nullptr;
-    Py_RETURN_TRUE;
+    }
+    return PyLong_FromSsize_t(p);
 }
 
 PyMethodDef methods[] = {{"encode", encode, METH_VARARGS, "plan objects -> code rows and headers; the index of the first plan not taken"},
                          {"fill", fill, METH_VARARGS, "stage records -> the lists of predict_time_breakdown; whether it did"},
+                         {"fill_all", fill_all, METH_VARARGS, "the same for a list of plans; the index of the first plan not taken"},
                          {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ace_objects", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -69,3 +69,18 @@ def test_other_plan_objects_and_errors_take_the_python_code():
     for error, c in bad:
         with pytest.raises(error):
             PlanBatch.from_configs([good[0], c], tables)
+
+
+def test_a_list_of_plans_is_filled_like_each_of_them():
+    w = odd_workloads()[2]
+    cm = cost_model(w)
+    batch = synth.make_plans(w, cm.tables, n_plans=9, seed_offset=4)
+    rec = emu_score(cm.tables, batch, breakdown=True)[4]
+    one, all_ = ([batch.to_config(p, cm.tables) for p in range(9)] for _ in range(2))
+    for p in (0, 4, 5, 8):
+        one[p].stages = all_[p].stages = tuple(one[p].stages)        # (left to the Python code)
+    for p, c in enumerate(one):
+        cm._fill_breakdown(c, rec[p])
+    cm._fill_all(all_, rec)
+    assert one == all_ and all(c.time_list for c in all_)
+    cm._fill_all([], rec[:0])
