@@ -256,6 +256,23 @@ typedef struct ace_move_draws {
 int ace_build_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
                     int gpus_per_node, const ace_move_draws_t *draws, uint32_t *moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out,
                     int max_templates, int *n_templates_out);
+/* The same, and of the moves (in order) only the n_moves_out whose plan is in none of the sets and not an earlier move's; the
+ * plans' keys (those of ace_apply_moves) are added to sets[0].  n_sets 0: the first move of each descriptor. */
+int ace_new_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
+                  int gpus_per_node, const ace_move_draws_t *draws, ace_keyset_t *const *sets, int n_sets, uint32_t *moves_out,
+                  size_t *n_moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out, int max_templates, int *n_templates_out);
+
+/* One step of a search over single-move neighbours in one call: ace_new_moves, the new plans expanded on the handle's device
+ * (ace_apply_moves), scored (ace_score_batch) and the fastest feasible one picked (ace_topk).  HOST memory in and out; the
+ * handle keeps the buffers, and no other call on it may run meanwhile.  codes_out / hdr_out: the picked plan, if found. */
+typedef struct ace_step_result {
+    size_t n_moves;         /* neighbours scored */
+    int32_t found;          /* one of them is feasible */
+    double iter_ms, peak_mb;
+} ace_step_result_t;
+int ace_search_step(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, const uint32_t *stage_lut, int gpus_per_node,
+                    const ace_move_draws_t *draws, ace_keyset_t *const *sets, int n_sets, double memory_limit, int strict,
+                    uint8_t *codes_out, uint32_t *hdr_out, ace_step_result_t *result, void *stream);
 
 /* Sort keys for grouped storage (ace_batch_t.d_order) of a batch that is already on the device: d_keys[i]
  * (uint64[n_plans]) orders the plans by pipeline depth, deepest first, then by the positions of their first two

@@ -119,10 +119,7 @@ class CostModel:
     def top_k(self, plans, k: int, memory_limit: Optional[float] = None, strict: bool = False):
         """Indices and times of the k fastest feasible plans (ascending, ties -> lower index)."""
         batch = plans if isinstance(plans, PlanBatch) else self.encode(plans)
-        ev = self.evaluator
-        d = ev.upload(batch)
-        it, pk, fe, st = ev.score(d, memory_limit, strict)
-        return ev.read_topk(ev.topk_packed(it, fe, k), k)
+        return self.evaluator.top_k(batch, k, memory_limit, strict)
 
     @staticmethod
     def _raise_for_status(status):

@@ -12,7 +12,7 @@
 #endif
 
 // One 64-bit value per (16-byte word, word index): two rounds of the splitmix64 finaliser.
-ACE_HD unsigned long long plan_key_word(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t idx) {
+ACE_HHD unsigned long long plan_key_word(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t idx) {
     unsigned long long x = ((unsigned long long)b << 32 | a) + 0x9E3779B97F4A7C15ull * (2ull * idx + 1ull);
     unsigned long long y = ((unsigned long long)d << 32 | c) ^ (x >> 29);
     x = (x ^ (x >> 30)) * 0xBF58476D1CE4E5B9ull;
@@ -24,7 +24,7 @@ ACE_HD unsigned long long plan_key_word(uint32_t a, uint32_t b, uint32_t c, uint
 }
 
 // The second half of a plan's 128-bit key: the same construction with other odd multipliers.
-ACE_HD unsigned long long plan_key_word2(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t idx) {
+ACE_HHD unsigned long long plan_key_word2(uint32_t a, uint32_t b, uint32_t c, uint32_t d, uint32_t idx) {
     unsigned long long x = ((unsigned long long)d << 32 | b) + 0xD6E8FEB86659FD93ull * (2ull * idx + 1ull);
     unsigned long long y = ((unsigned long long)c << 32 | a) ^ (x >> 31);
     x = (x ^ (x >> 32)) * 0xFF51AFD7ED558CCDull;

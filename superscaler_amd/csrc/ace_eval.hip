@@ -641,10 +641,23 @@ struct ace_handle {
     ace_u2 *d_rc_pos;          // check_recompute's tables (ace_recompute_prepare), or null
     double *d_rc_act;
     unsigned char *host_in, *host_out;   // page-locked buffers of ace_score_host (null until the first call)
+    struct StepBuffers *step;  // of ace_search_step (null until the first call)
     double *d_stage_ws;        // grow-only workspace for deferred stage tails
     size_t stage_ws_plans;     // capacity in plans
     int stage_ws_fixed;        // ace_reserve(..., fixed): a larger batch is an error instead of a reallocation
 };
+
+struct StepOut { long long idx; double iter_ms, peak_mb; int32_t count; };
+struct StepBuffers {
+    std::vector<uint8_t> t_codes;
+    std::vector<uint32_t> t_hdr;
+    unsigned char *host, *dev;          // page-locked: StepOut, then what goes up; both grow only
+    size_t host_bytes, dev_bytes;
+};
+__global__ void step_out_kernel(const long long *idx, const double *val, const int32_t *count, const double *peak, StepOut *out) {
+    const int32_t n = *count;
+    *out = StepOut{*idx, *val, n > 0 ? peak[*idx] : 0.0, n};
+}
 
 // The bodies of these kernels live in ace_edit_kernels.h (shared with the host build of the tests).
 __global__ __launch_bounds__(256) void apply_moves_kernel(const ace_u4 *tmpl_codes, const ace_u4 *tmpl_hdr, int n_templates,
@@ -1058,6 +1071,11 @@ void ace_destroy(ace_handle_t *h) {
     if (h->host_in) (void)hipHostFree(h->host_in);
     if (h->host_out) (void)hipHostFree(h->host_out);
     if (h->d_stage_ws) (void)hipFree(h->d_stage_ws);
+    if (h->step) {
+        if (h->step->host) (void)hipHostFree(h->step->host);
+        if (h->step->dev) (void)hipFree(h->step->dev);
+        delete h->step;
+    }
     delete h;
 }
 
@@ -1623,14 +1641,132 @@ int ace_keyset_keys(const ace_keyset_t *s, uint64_t *keys_out) {
     return ACE_OK;
 }
 
+static bool moves_args(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
+                       int gpus_per_node, const ace_move_draws_t *draws, uint32_t *moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out,
+                       int *n_templates_out) {
+    return codes && hdr && stage_lut && draws && moves_out && t_codes_out && t_hdr_out && n_templates_out && num_ops > 0 &&
+           num_ops < 65536 && (n_algo == 1 || n_algo == 2) && n_tp > 0 && n_tp <= 4 && n_mbs > 0 && gpus_per_node > 0;
+}
+
 int ace_build_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
                     int gpus_per_node, const ace_move_draws_t *draws, uint32_t *moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out,
                     int max_templates, int *n_templates_out) {
-    if (!codes || !hdr || !stage_lut || !draws || !moves_out || !t_codes_out || !t_hdr_out || !n_templates_out || num_ops <= 0 ||
-        num_ops >= 65536 || (n_algo != 1 && n_algo != 2) || n_tp <= 0 || n_tp > 4 || n_mbs <= 0 || gpus_per_node <= 0)
+    if (!moves_args(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, draws, moves_out, t_codes_out, t_hdr_out, n_templates_out))
         return ACE_EINVAL;
     return ace_build_moves_body(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, *draws, moves_out, t_codes_out, t_hdr_out,
                                 max_templates, n_templates_out);
+}
+
+int ace_new_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,
+                  int gpus_per_node, const ace_move_draws_t *draws, ace_keyset_t *const *sets, int n_sets, uint32_t *moves_out,
+                  size_t *n_moves_out, uint8_t *t_codes_out, uint32_t *t_hdr_out, int max_templates, int *n_templates_out) {
+    const AceKeySet *in[4];
+    if (!moves_args(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, draws, moves_out, t_codes_out, t_hdr_out, n_templates_out) ||
+        !n_moves_out || !key_sets(sets, n_sets, in))
+        return ACE_EINVAL;
+    try {
+        AceKeySet *s[4];
+        for (int i = 0; i < n_sets; ++i) s[i] = key_set(sets[i]);
+        return ace_new_moves_body(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, *draws, s, n_sets, moves_out, n_moves_out,
+                                  t_codes_out, t_hdr_out, max_templates, n_templates_out);
+    } catch (const std::bad_alloc &) {
+        return ACE_ENOMEM;
+    }
+}
+
+static int search_step(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, const uint32_t *stage_lut, int gpus_per_node,
+                       const ace_move_draws_t *draws, ace_keyset_t *const *sets, int n_sets, double memory_limit, int strict,
+                       uint8_t *codes_out, uint32_t *hdr_out, ace_step_result_t *res, hipStream_t s) {
+    const AceGeom &g = h->geom;
+    const size_t N = (size_t)g.N, G = (size_t)g.G, n = draws->n;
+    const int S = (int)(hdr[0] & 0xffu), cap = 3 + S * (S > 0 ? S - 1 : 0);
+    if (!h->step) h->step = new StepBuffers();
+    StepBuffers &b = *h->step;
+    b.t_codes.resize((size_t)cap * N);
+    b.t_hdr.resize((size_t)cap * 4);
+    // page-locked: [StepOut][moves][template headers][template code rows, padded]
+    const size_t host_need = 64 + 16 * n + (size_t)cap * 16 * (1 + G);
+    if (b.host_bytes < host_need) {
+        if (b.host) ACE_HIP(hipHostFree(b.host));
+        b.host = nullptr;
+        b.host_bytes = 0;
+        ACE_HIP(hipHostMalloc((void **)&b.host, host_need, hipHostMallocDefault));
+        b.host_bytes = host_need;
+    }
+    unsigned char *up = b.host + 64;
+    uint32_t *moves = reinterpret_cast<uint32_t *>(up);
+    int T = 0;
+    size_t m = 0;
+    int rc = ace_new_moves(codes, hdr, g.N, g.n_algo, g.n_tp, g.n_mbs, stage_lut, gpus_per_node, draws, sets, n_sets, moves, &m,
+                           b.t_codes.data(), b.t_hdr.data(), cap, &T);
+    if (rc) return rc;
+    res->n_moves = m;
+    if (!m) return ACE_OK;
+    const size_t off_hdr = 16 * m, off_codes = off_hdr + 16 * (size_t)T, up_bytes = off_codes + (size_t)T * G * 16;
+    memcpy(up + off_hdr, b.t_hdr.data(), 16 * (size_t)T);
+    memset(up + off_codes, 0, (size_t)T * G * 16);
+    for (int t = 0; t < T; ++t) memcpy(up + off_codes + (size_t)t * G * 16, b.t_codes.data() + (size_t)t * N, N);
+    // device: what went up, the plans, their scores, the pick
+    size_t at = 0;
+    auto take = [&](size_t bytes) { const size_t o = at; at += (bytes + 255) & ~(size_t)255; return o; };
+    const size_t ws = ace_topk_workspace_bytes(m, 1);
+    const size_t o_up = take(up_bytes), o_codes = take(G * m * 16), o_hdr = take(16 * m), o_it = take(8 * m), o_pk = take(8 * m),
+                 o_fe = take(m), o_top = take(24), o_ws = take(ws);
+    if (b.dev_bytes < at) {
+        if (b.dev) ACE_HIP(hipFree(b.dev));
+        b.dev = nullptr;
+        b.dev_bytes = 0;
+        ACE_HIP(hipMalloc((void **)&b.dev, at + at / 4));
+        b.dev_bytes = at + at / 4;
+    }
+    unsigned char *d = b.dev;
+    ACE_HIP(hipMemcpyAsync(d + o_up, up, up_bytes, hipMemcpyHostToDevice, s));
+    double *it = reinterpret_cast<double *>(d + o_it), *pk = reinterpret_cast<double *>(d + o_pk), *val = reinterpret_cast<double *>(d + o_top + 8);
+    int64_t *idx = reinterpret_cast<int64_t *>(d + o_top);
+    int32_t *count = reinterpret_cast<int32_t *>(d + o_top + 16);
+    const ace_batch_t batch{d + o_codes, reinterpret_cast<const uint32_t *>(d + o_hdr), nullptr, m, nullptr};
+    if ((rc = ace_apply_moves(d + o_up + off_codes, reinterpret_cast<const uint32_t *>(d + o_up + off_hdr), T,
+                              reinterpret_cast<const uint32_t *>(d + o_up), m, g.N, g.n_algo, d + o_codes,
+                              reinterpret_cast<uint32_t *>(d + o_hdr), nullptr, s)) ||
+        (rc = ace_score_batch(h, &batch, memory_limit, strict, it, pk, d + o_fe, nullptr, nullptr, s)) ||
+        (rc = ace_topk(h, it, d + o_fe, m, 1, idx, val, count, d + o_ws, ws, s)))
+        return rc;
+    StepOut *out = reinterpret_cast<StepOut *>(b.host);
+    hipLaunchKernelGGL(step_out_kernel, dim3(1), dim3(1), 0, s, (const long long *)idx, val, count, pk, out);
+    ACE_HIP(hipGetLastError());
+    ACE_HIP(hipStreamSynchronize(s));
+    if (out->count > 0 && out->idx >= 0 && (size_t)out->idx < m) {
+        const uint32_t *mv = moves + 4 * out->idx;
+        const size_t t = mv[0] & 0xffffu;
+        memcpy(codes_out, b.t_codes.data() + t * N, N);
+        memcpy(hdr_out, b.t_hdr.data() + 4 * t, 16);
+        ace_apply_move(mv, g.N, g.n_algo, codes_out);
+        res->found = 1;
+        res->iter_ms = out->iter_ms;
+        res->peak_mb = out->peak_mb;
+    }
+    return ACE_OK;
+}
+
+int ace_search_step(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, const uint32_t *stage_lut, int gpus_per_node,
+                    const ace_move_draws_t *draws, ace_keyset_t *const *sets, int n_sets, double memory_limit, int strict,
+                    uint8_t *codes_out, uint32_t *hdr_out, ace_step_result_t *result, void *stream) {
+    if (!h || !codes || !hdr || !stage_lut || !draws || !codes_out || !hdr_out || !result || draws->n == 0 || draws->n > 0x7fffffffull ||
+        h->geom.N >= 65536)
+        return ACE_EINVAL;
+    *result = ace_step_result_t{0, 0, 0.0, 0.0};
+    int dev = -1;
+    ACE_HIP(hipGetDevice(&dev));
+    if (dev != h->device) ACE_HIP(hipSetDevice(h->device));
+    int rc;
+    try {
+        rc = search_step(h, codes, hdr, stage_lut, gpus_per_node, draws, sets, n_sets, memory_limit, strict, codes_out, hdr_out, result,
+                         (hipStream_t)stream);
+    } catch (const std::bad_alloc &) {
+        rc = ACE_ENOMEM;
+    }
+    if (dev != h->device) ACE_HIP(hipSetDevice(dev));
+    return rc;
 }
 
 }  // extern "C"

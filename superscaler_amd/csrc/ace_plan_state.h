@@ -30,6 +30,7 @@
 #include <cstdlib>
 #include <cstring>
 #define ACE_HD inline
+#define ACE_HHD inline
 #define ACE_WAVE_ANY(x) (x)
 struct AceLds {
     const unsigned char *base;
@@ -55,6 +56,7 @@ static inline uint32_t ace_lds_base(const unsigned char *) { return 0u; }   // h
 static inline double ace_max(double a, double b) { return a > b ? a : b; }
 #else
 #define ACE_HD __device__ __forceinline__
+#define ACE_HHD __host__ __device__ __forceinline__
 #define ACE_WAVE_ANY(x) __any(x)
 // LDS reads take the absolute LDS byte address.  The address of the workgroup's LDS array is a
 // link-time constant (zero when the kernel has no other LDS variables) that the compiler cannot fold

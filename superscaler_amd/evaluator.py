@@ -19,7 +19,7 @@ EXPORTS = ["ace_abi_version", "ace_strerror", "ace_last_hip_error", "ace_create"
            "ace_score_batch", "ace_score_batch_static", "ace_reserve", "ace_topk_workspace_bytes", "ace_topk", "ace_time_score_kernel", "ace_apply_moves",
            "ace_recompute_groups", "ace_recompute_select", "ace_group_keys", "ace_gather_plans",
            "ace_keyset_create", "ace_keyset_destroy", "ace_keyset_size", "ace_keyset_add", "ace_keyset_unseen", "ace_keyset_claim",
-           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves", "ace_recompute_prepare", "ace_recompute_batch",
+           "ace_keyset_move", "ace_keyset_keys", "ace_build_moves", "ace_new_moves", "ace_search_step", "ace_recompute_prepare", "ace_recompute_batch",
            "ace_pack_plans", "ace_unpack_plans", "ace_check_plans", "ace_score_host", "ace_pack_host"]
 
 
@@ -39,6 +39,10 @@ class AceMoveDrawsStruct(ctypes.Structure):
                 ("x", ctypes.c_void_p * 6), ("y", ctypes.c_void_p * 6)]
 
 
+class AceStepResultStruct(ctypes.Structure):
+    _fields_ = [("n_moves", ctypes.c_size_t), ("found", ctypes.c_int32), ("iter_ms", ctypes.c_double), ("peak_mb", ctypes.c_double)]
+
+
 ACE_ETOOBIG = -2
 
 
@@ -54,6 +58,7 @@ def load_library():
     if not os.path.exists(_LIB_PATH):
         raise AceError(f"{_LIB_PATH} is missing: build it with `python -m superscaler_amd.build` "
                        "(there is no CPU fallback for plan scoring)")
+    import torch  # noqa: F401  (its HIP runtime has to be the one the library binds to, also where the first call is a host one)
     lib = ctypes.CDLL(_LIB_PATH)
     lib.ace_abi_version.restype = ctypes.c_int
     lib.ace_strerror.restype = ctypes.c_char_p
@@ -114,6 +119,10 @@ def load_library():
     lib.ace_recompute_prepare.argtypes = [vp] * 4
     lib.ace_recompute_batch.argtypes = [vp, ctypes.POINTER(AceBatchStruct), ctypes.c_double, ctypes.c_double] + [vp] * 4
     ci = ctypes.c_int
+    lib.ace_search_step.argtypes = [vp, vp, vp, vp, ci, ctypes.POINTER(AceMoveDrawsStruct), ctypes.POINTER(vp), ci, ctypes.c_double, ci, vp, vp,
+                                    ctypes.POINTER(AceStepResultStruct), vp]
+    lib.ace_new_moves.argtypes = [vp, vp, ci, ci, ci, ci, vp, ci, ctypes.POINTER(AceMoveDrawsStruct), ctypes.POINTER(vp), ci, vp, ctypes.POINTER(sz),
+                                  vp, vp, ci, ctypes.POINTER(ci)]
     lib.ace_build_moves.argtypes = [vp, vp, ci, ci, ci, ci, vp, ci, ctypes.POINTER(AceMoveDrawsStruct), vp, vp, vp, ci, ctypes.POINTER(ci)]
     if lib.ace_abi_version() != ABI_VERSION:
         raise AceError("libace_eval.so has a different ABI version")
@@ -229,9 +238,9 @@ def rows_to_device(batch: PlanBatch, device, staging=None):
     return rows, hdr
 
 
-def pack_rows(rows, hdr, check=None):
+def pack_rows(rows, hdr, check=None, findings=None):
     """Code rows [P, N] on the device -> [ceil(N / 16), P, 16] (plan-minor, sixteen ops per 16-byte word, zero padded);
-    `check` as in DeviceBatch."""
+    `check` and `findings` as in DeviceBatch."""
     import torch
     P, N = rows.shape
     G = (N + 15) // 16
@@ -240,12 +249,12 @@ def pack_rows(rows, hdr, check=None):
     lib = load_library()
     codes = torch.empty((G, P, 16), dtype=torch.uint8, device=rows.device)
     n_mbs, n_codes = check or (0, 8)
-    flags = torch.zeros(1, dtype=torch.int32, device=rows.device) if check else None
+    flags = None if not check else torch.zeros(1, dtype=torch.int32, device=rows.device) if findings is None else findings
     with torch.cuda.device(rows.device):
         _check(lib, lib.ace_pack_plans(rows.data_ptr(), P, N, hdr.data_ptr() if check else None, n_mbs, n_codes, codes.data_ptr(),
                                        flags.data_ptr() if check else None,
                                        torch.cuda.current_stream(rows.device).cuda_stream), "ace_pack_plans")
-    if check:
+    if check and findings is None:
         msg = finding(int(flags.item()))
         if msg:
             raise ValueError(msg)
@@ -256,7 +265,7 @@ class DeviceBatch:
     """A PlanBatch resident in HBM in the layout the kernel streams."""
 
     def __init__(self, batch: PlanBatch, device="cuda:0", ranges: Optional[np.ndarray] = None, staging=None,
-                 group_by_depth: bool = False, check=None):
+                 group_by_depth: bool = False, check=None, findings=None):
         """`staging`: a pinned uint8 host tensor of at least P * N + 16 * P bytes; the plans then go through
         it and the copy to the device does not block the host (the caller must not reuse the tensor
         before that copy has completed).
@@ -264,7 +273,8 @@ class DeviceBatch:
         first two stage boundaries, with the permutation alongside (`order`), so that the lanes of a
         wavefront close their stages together; results still come back in the caller's order.
         `check`: (micro-batch sizes, codes) of the tables; the plans' structure is then checked on the way
-        (ValueError)."""
+        (ValueError).  `findings`: a zeroed device int32 that takes what the check finds instead; the caller reads it,
+        with what it reads anyway."""
         import torch
         P, N = batch.codes.shape
         order = None
@@ -279,7 +289,7 @@ class DeviceBatch:
             r = np.ascontiguousarray(ranges, dtype=np.uint32)
             assert r.shape == (P, 2)
             ranges = torch.from_numpy(r.view(np.int32)).to(device)
-        self._set(pack_rows(rows, hdr, check), hdr, N, ranges, order)
+        self._set(pack_rows(rows, hdr, check, findings), hdr, N, ranges, order)
 
     def _set(self, codes, hdr, num_ops, ranges, order):
         self.n_plans, self.num_ops = int(hdr.shape[0]), int(num_ops)
@@ -319,6 +329,7 @@ class PlanEvaluator:
         self._topk_ws = None
         self._rc_ready = None
         self._graphs_alive = 0
+        self._copy_stream = None
 
     def close(self):
         if getattr(self, "handle", None):
@@ -332,9 +343,9 @@ class PlanEvaluator:
             pass
 
     def upload(self, batch: PlanBatch, validate: bool = True, ranges: Optional[np.ndarray] = None,
-               staging=None, group_by_depth: bool = False) -> DeviceBatch:
+               staging=None, group_by_depth: bool = False, findings=None) -> DeviceBatch:
         """`validate` checks the encoding on the host first (a clear message instead of per-plan status
-        bytes; the kernel itself is safe for any byte content).  `group_by_depth`: see DeviceBatch."""
+        bytes; the kernel itself is safe for any byte content).  `group_by_depth`, `findings`: see DeviceBatch."""
         check = None
         if validate and ranges is None:
             # (small batches are checked before they go anywhere; for others the check rides on the device's packing of the
@@ -344,7 +355,7 @@ class PlanEvaluator:
             if msg:
                 raise ValueError(msg)
             check = None if small else (len(self.tables.db.mbs_list), self.tables.C)
-        return DeviceBatch(batch, self.device, ranges, staging, group_by_depth, check)
+        return DeviceBatch(batch, self.device, ranges, staging, group_by_depth, check, findings)
 
     def pinned_plan_batch(self, n_plans: int) -> PlanBatch:
         """An empty PlanBatch (codes uint8 [n_plans, N], hdr uint32 [n_plans, 4]) whose arrays live in page-locked host
@@ -362,6 +373,12 @@ class PlanEvaluator:
     def device_context(self):
         """Context manager that makes this evaluator's GPU the current one (for raw library calls)."""
         return self._torch.cuda.device(self.device)
+
+    def copy_stream(self):
+        """A stream for copies beside the kernels, the same one every time (the allocator keeps memory by stream)."""
+        if self._copy_stream is None:
+            self._copy_stream = self._torch.cuda.Stream(self.device)
+        return self._copy_stream
 
     def _stream(self):
         return ctypes.c_void_p(self._torch.cuda.current_stream(self.device).cuda_stream)
@@ -405,15 +422,16 @@ class PlanEvaluator:
         buf = self.topk_packed(iter_ms, feasible, k)
         return buf[:8 * k].view(torch.int64), buf[8 * k:16 * k].view(torch.float64), buf[16 * k:16 * k + 4].view(torch.int32)
 
-    def topk_packed(self, iter_ms, feasible, k: int):
-        """topk() in one device buffer (indices, times, count: one copy brings all of them to the host)."""
+    def topk_packed(self, iter_ms, feasible, k: int, out=None):
+        """topk() in one device buffer (indices, times, count: one copy brings all of them to the host); `out`: that buffer
+        (uint8, at least 16 * k + 4)."""
         torch = self._torch
         n = iter_ms.numel()
         need = self.lib.ace_topk_workspace_bytes(n, k)
         if self._topk_ws is None or self._topk_ws.numel() < need:
             # (a captured step keeps its own reference to the workspace it recorded, so the old one stays alive for it)
             self._topk_ws = torch.empty(need, dtype=torch.uint8, device=self.device)
-        buf = torch.empty(16 * k + 8, dtype=torch.uint8, device=self.device)
+        buf = torch.empty(16 * k + 8, dtype=torch.uint8, device=self.device) if out is None else out
         at = buf.data_ptr()
         with torch.cuda.device(self.device):
             rc = self.lib.ace_topk(self.handle, iter_ms.data_ptr(), feasible.data_ptr(), n, k, at, at + 8 * k, at + 16 * k,
@@ -424,9 +442,22 @@ class PlanEvaluator:
     @staticmethod
     def read_topk(buf, k: int):
         """topk_packed's result on the host: (indices, times) of the feasible ones."""
-        host = buf.cpu().numpy()
+        host = buf if isinstance(buf, np.ndarray) else buf.cpu().numpy()
         n = int(host[16 * k:16 * k + 4].view(np.int32)[0])
         return host[:8 * k].view(np.int64)[:n], host[8 * k:16 * k].view(np.float64)[:n]
+
+    def top_k(self, batch: PlanBatch, k: int, memory_limit: Optional[float] = None, strict: bool = False):
+        """(indices, times) of the k fastest feasible plans of a host batch.  Everything is asked for before anything is read:
+        what the structural check of the plans has found comes back with the result (scoring is safe for any bytes)."""
+        torch = self._torch
+        buf = torch.zeros(16 * k + 16, dtype=torch.uint8, device=self.device)
+        d = self.upload(batch, findings=buf[16 * k + 8:16 * k + 12].view(torch.int32))
+        it, pk, fe, st = self.score(d, memory_limit, strict)
+        host = self.topk_packed(it, fe, k, buf).cpu().numpy()
+        msg = finding(int(host[16 * k + 8:16 * k + 12].view(np.int32)[0]))
+        if msg:
+            raise ValueError(msg)
+        return self.read_topk(host, k)
 
     def capture_step(self, dbatch: DeviceBatch, k: int, memory_limit: Optional[float] = None, strict: bool = False):
         """Score + top-k of a resident batch recorded once in a HIP graph (the library's launches record into a
@@ -460,7 +491,7 @@ class PlanEvaluator:
         feasible plans over all batches (ascending, ties -> lower global index) and the number of
         plans seen."""
         torch = self._torch
-        copy_stream = torch.cuda.Stream(device=self.device)
+        copy_stream = self.copy_stream()
         main = torch.cuda.current_stream(self.device)
         best_idx = np.empty(0, dtype=np.int64)
         best_val = np.empty(0, dtype=np.float64)
@@ -528,6 +559,20 @@ class PlanEvaluator:
         _check(self.lib, rc, "ace_apply_moves")
         d = DeviceBatch.from_device(codes, hdr, N)
         return (d, keys) if with_keys else d
+
+    def search_step(self, plan: PlanBatch, draws: AceMoveDrawsStruct, sets=()):
+        """One step of a search in one library call (ace_search_step): the new ones among the drawn moves on plan 0 of `plan`
+        expanded, scored and the fastest feasible one picked: (plan, iteration ms, peak MB), or None.  `sets`: handles of
+        the visited sets (empty: only repeated moves are dropped)."""
+        t, best = self.tables, AceStepResultStruct()
+        row, hdr = np.ascontiguousarray(plan.codes[0]), np.ascontiguousarray(plan.hdr[0])
+        codes_out, hdr_out = np.empty((1, len(row)), dtype=np.uint8), np.empty((1, 4), dtype=np.uint32)
+        handles = (ctypes.c_void_p * max(1, len(sets)))(*sets)
+        _check(self.lib, self.lib.ace_search_step(self.handle, row.ctypes.data, hdr.ctypes.data, t.stage_lut.ctypes.data,
+                                                  t.settings.num_gpus_per_node, ctypes.byref(draws), handles, len(sets),
+                                                  float(t.settings.memory_limit), 0, codes_out.ctypes.data, hdr_out.ctypes.data,
+                                                  ctypes.byref(best), self._stream()), "ace_search_step")
+        return (PlanBatch(codes_out, hdr_out), best.iter_ms, best.peak_mb) if best.found else None
 
     def prepare_recompute(self, no_recompute: np.ndarray) -> bool:
         """Upload what check_recompute needs beside the tables (once); False if the op graph is too long for the kernel."""

@@ -8,6 +8,7 @@ scored by one kernel launch.  The search policy of the reference (aceso_policy.p
 reproduced: `hill_climb` is a plain best-neighbour descent used to exercise the batched path.
 """
 import ctypes
+from concurrent.futures import ThreadPoolExecutor
 from typing import Tuple
 
 import numpy as np
@@ -94,9 +95,28 @@ def _draw_moves(n: int, S: int, tables: CompiledTables, rng: np.random.Generator
     return out
 
 
-def _build_moves(base: PlanBatch, tables: CompiledTables, draws) -> Tuple[PlanBatch, np.ndarray]:
-    """The drawn moves on base plan 0 as (templates, moves): the library's ace_build_moves."""
-    from .evaluator import AceMoveDrawsStruct, _check, load_library
+def _draws_struct(draws):
+    """_draw_moves's result as the library takes it (an AceMoveDrawsStruct that keeps the arrays it points to)."""
+    from .evaluator import AceMoveDrawsStruct
+    d = AceMoveDrawsStruct()
+    d.n = draws["n"]
+    d.keep = []
+    for name in ("rows", "x", "y"):
+        to = getattr(d, name)
+        for k, a in enumerate(draws[name]):
+            a = np.ascontiguousarray(a, dtype=np.int64)
+            d.keep.append(a)
+            to[k] = a.ctypes.data
+            if name == "rows":
+                d.count[k] = len(a)
+    return d
+
+
+def _build_moves(base: PlanBatch, tables: CompiledTables, draws, sets=None) -> Tuple[PlanBatch, np.ndarray]:
+    """The drawn moves on base plan 0 as (templates, moves): the library's ace_build_moves.  With `sets` (_KeySets, a list)
+    those whose plan none of them has, the first of each, their keys added to sets[0] (an empty list: the first of each
+    descriptor): ace_new_moves."""
+    from .evaluator import _check, load_library
     lib = load_library()
     N, M, n = tables.graph.num_ops, len(tables.db.mbs_list), draws["n"]
     if N >= 65536:
@@ -106,20 +126,17 @@ def _build_moves(base: PlanBatch, tables: CompiledTables, draws) -> Tuple[PlanBa
     t_codes, t_hdr = np.empty((cap, N), dtype=np.uint8), np.empty((cap, 4), dtype=np.uint32)
     moves = np.empty((n, 4), dtype=np.uint32)
     row, hdr = np.ascontiguousarray(base.codes[0]), np.ascontiguousarray(base.hdr[0])
-    d = AceMoveDrawsStruct()
-    d.n = n
-    keep = []
-    for name in ("rows", "x", "y"):
-        for k, a in enumerate(draws[name]):
-            a = np.ascontiguousarray(a, dtype=np.int64)
-            keep.append(a)
-            getattr(d, name)[k] = a.ctypes.data
-            if name == "rows":
-                d.count[k] = len(a)
+    d = _draws_struct(draws)
     n_templates = ctypes.c_int(0)
-    _check(lib, lib.ace_build_moves(row.ctypes.data, hdr.ctypes.data, N, tables.db.n_algo, len(tables.db.tp_list), M,
-                                    tables.stage_lut.ctypes.data, tables.settings.num_gpus_per_node, ctypes.byref(d), moves.ctypes.data, t_codes.ctypes.data,
-                                    t_hdr.ctypes.data, cap, ctypes.byref(n_templates)), "ace_build_moves")
+    plan = (row.ctypes.data, hdr.ctypes.data, N, tables.db.n_algo, len(tables.db.tp_list), M, tables.stage_lut.ctypes.data,
+            tables.settings.num_gpus_per_node, ctypes.byref(d))
+    dest = (t_codes.ctypes.data, t_hdr.ctypes.data, cap, ctypes.byref(n_templates))
+    if sets is None:
+        _check(lib, lib.ace_build_moves(*plan, moves.ctypes.data, *dest), "ace_build_moves")
+    else:
+        handles, n_moves = (ctypes.c_void_p * max(1, len(sets)))(*[s.handle for s in sets]), ctypes.c_size_t(0)
+        _check(lib, lib.ace_new_moves(*plan, handles, len(sets), moves.ctypes.data, ctypes.byref(n_moves), *dest), "ace_new_moves")
+        moves = moves[:n_moves.value]
     return PlanBatch(t_codes[:n_templates.value], t_hdr[:n_templates.value]), moves
 
 
@@ -446,12 +463,38 @@ class VisitedKeys:
         """unseen(), and those keys marked."""
         # (only what the large set lacks goes to the small one: the two stay disjoint, __len__ is their sum)
         mask = _first_of_each(as_key128(keys), (self._small, self._large), claim=True)
+        self.fold()
+        return mask
+
+    def claim_moves(self, base: PlanBatch, tables: CompiledTables, draws) -> Tuple[PlanBatch, np.ndarray]:
+        """_build_moves, of the moves those whose plan is unseen, and these marked."""
+        made = _build_moves(base, tables, draws, [self._small, self._large])
+        self.fold()
+        return made
+
+    def handles(self):
+        """The native sets for the library's calls that look keys up in both and add to the small one (then call fold())."""
+        return [self._small.handle, self._large.handle]
+
+    def fold(self) -> None:
         if len(self._small) > self.SMALL_LIMIT:
             self._large.take(self._small)
-        return mask
 
     def mark(self, keys: np.ndarray) -> None:
         self.claim(keys)
+
+
+def _best_recomputed(cm, d, below: float):
+    """check_recompute's choice for every plan of a device batch, then (plan, iteration ms, peak MB) of the fastest feasible one
+    if that is faster than `below`."""
+    ev = cm.evaluator
+    d = cm.update_recompute_device(d)
+    it, pk, fe, st = ev.score(d)
+    idx, val = ev.read_topk(ev.topk_packed(it, fe, 1), 1)
+    if not len(idx) or float(val[0]) >= below:
+        return None
+    best = int(idx[0])
+    return ev.download(d, ev._torch.tensor([best], device=d.hdr.device)), float(val[0]), float(pk[best].item())
 
 
 def hill_climb(cm, start: PlanBatch, steps: int, n_neighbours: int, seed: int = 0, max_move: int = 8,
@@ -464,8 +507,8 @@ def hill_climb(cm, start: PlanBatch, steps: int, n_neighbours: int, seed: int = 
     replaced by check_recompute's choice before it is scored, as the reference's primitives do
     (aceso_prims.py:107-108).  With `device_moves` the neighbours never exist on the host: the move
     descriptors (16 bytes each) are expanded by the library on the device and only the winner is
-    rebuilt here; `visited` is then a VisitedKeys (128-bit keys of the plan bytes, computed by the
-    same kernel, before any recompute bits are re-chosen) and `greedy_recompute` runs check_recompute's
+    rebuilt here; `visited` is then a VisitedKeys (128-bit keys of the plan bytes, derived from the
+    descriptors, before any recompute bits are re-chosen) and `greedy_recompute` runs check_recompute's
     loop on the device as well (CostModel.update_recompute_device).
     Returns (plan, iteration ms, peak MB)."""
     if device_moves and isinstance(visited, VisitedPlans):
@@ -474,47 +517,43 @@ def hill_climb(cm, start: PlanBatch, steps: int, n_neighbours: int, seed: int = 
     tables = cm.tables
     ev = cm.evaluator
     cur = start.slice(0, 1)
-    it, pk, fe, st = ev.score_host(cur)
-    cur_t = float(it[0]) if fe[0] else float("inf")
-    cur_m = float(pk[0])
-    if visited is not None:
-        visited.mark(plan_keys_host(cur) if device_moves else cur)
-    draws = None
+
+    def begin():
+        it, pk, fe, st = ev.score_host(cur)
+        if visited is not None:
+            visited.mark(plan_keys_host(cur) if device_moves else cur)
+        return float(it[0]) if fe[0] else float("inf"), float(pk[0])
+    if device_moves:
+        # The random choices of a step depend on the plan's stage count only, which no move changes: a second thread draws the
+        # next step's meanwhile (a step is one library call, during which the interpreter is free).
+        n_stages = int(cur.hdr[0, 0] & 0xff)
+
+        def draw():
+            draws = _draw_moves(n_neighbours, n_stages, tables, rng, max_move)
+            return draws if greedy_recompute else _draws_struct(draws)
+        with ThreadPoolExecutor(1) as pool:
+            ahead = pool.submit(draw) if steps > 0 else None
+            cur_t, cur_m = begin()
+            for step in range(steps):
+                draws = ahead.result()
+                if step + 1 < steps:
+                    ahead = pool.submit(draw)
+                # (without a visited set equal descriptors are equal plans: one of each is kept.  First occurrences, in the order
+                # they were drawn: among neighbours of equal time the earliest wins, as it does when the duplicates are scored too)
+                if not greedy_recompute:
+                    best = ev.search_step(cur, draws, () if visited is None else visited.handles())
+                    if visited is not None:
+                        visited.fold()
+                else:
+                    templates, moves = _build_moves(cur, tables, draws, []) if visited is None else visited.claim_moves(cur, tables, draws)
+                    best = _best_recomputed(cm, ev.apply_moves(templates, moves), cur_t) if len(moves) else None
+                if best is not None and best[1] < cur_t:
+                    cur, cur_t, cur_m = best
+                if on_step is not None:
+                    on_step(step, cur_t, cur_m)
+        return cur, cur_t, cur_m
+    cur_t, cur_m = begin()
     for step in range(steps):
-        if device_moves:
-            if draws is None:
-                draws = _draw_moves(n_neighbours, int(cur.hdr[0, 0] & 0xff), tables, rng, max_move)
-            templates, moves = _build_moves(cur, tables, draws)
-            draws = None
-            if visited is None:
-                # equal descriptors are equal plans: keep one of each (first occurrences, in the order they were drawn:
-                # among neighbours of equal time the earliest wins, as it does when the duplicates are scored too)
-                moves = moves[_first_of_each(moves)]
-                d = ev.apply_moves(templates, moves)
-            else:
-                d, keys = ev.apply_moves(templates, moves, with_keys=True)
-                keep = np.flatnonzero(visited.claim(keys.cpu().numpy().view(np.uint64)))
-                if len(keep) == 0:
-                    if on_step is not None:
-                        on_step(step, cur_t, cur_m)
-                    continue
-                moves = moves[keep]
-                d = ev.select(d, ev._torch.from_numpy(keep).to(d.hdr.device))
-            if greedy_recompute:
-                d = cm.update_recompute_device(d)
-            it, pk, fe, st = ev.score(d)
-            top = ev.topk_packed(it, fe, 1)
-            if step + 1 < steps:
-                draws = _draw_moves(n_neighbours, int(cur.hdr[0, 0] & 0xff), tables, rng, max_move)
-            idx, val = ev.read_topk(top, 1)
-            if len(idx) and float(val[0]) < cur_t:
-                best_i, cur_t = int(idx[0]), float(val[0])
-                cur_m = float(pk[best_i].item())
-                cur = ev.download(d, ev._torch.tensor([best_i], device=d.hdr.device)) if greedy_recompute else \
-                    apply_moves_host(templates, moves[best_i:best_i + 1], tables.db.n_algo)
-            if on_step is not None:
-                on_step(step, cur_t, cur_m)
-            continue
         nb = make_neighbours(cur, tables, n_neighbours, rng, max_move)
         if visited is not None:
             keep = np.flatnonzero(visited.unseen(nb))

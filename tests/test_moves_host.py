@@ -1,11 +1,11 @@
 """The native host side of the batched search: ace_build_moves (drawn choices -> descriptors) against the rules of
-sample_moves written out row by row, and the key set against a Python set."""
+sample_moves written out row by row, ace_new_moves against the keys of the expanded plans, and the key set against a Python set."""
 import numpy as np
 import pytest
 
 from superscaler_amd import synth
 from superscaler_amd.neighbours import (OP_ALGO_TOGGLE, OP_MIGRATE, OP_RC_TOGGLE, OP_TP_STEP, VisitedKeys, _build_moves, _draw_moves,
-                                        apply_moves_host)
+                                        apply_moves_host, plan_keys_host)
 from superscaler_amd.plan import validate_batch
 from tests.helpers import odd_workloads
 
@@ -67,6 +67,28 @@ def test_drawn_moves_become_the_descriptors_of_the_rules(name):
                 assert moved[what[1]] == -1 and moved[what[2]] == 1 and sum(map(abs, moved)) == 2
 
 
+@pytest.mark.parametrize("name", ["gpt3_1_3b", "t5_770m", "wresnet_1b", "gpt_16ops", "gpt_wide_stages", "t5_1tp"])
+def test_moves_kept_are_those_whose_expanded_plans_are_new(name):
+    w = WORKLOADS[name]
+    tables = synth.make_tables(w)
+    a, b = VisitedKeys(), VisitedKeys()
+    for p in range(5):
+        base = synth.make_plans(w, tables, n_plans=8, seed_offset=50).slice(p % 4, p % 4 + 1)
+        draws = _draw_moves(3000, int(base.hdr[0, 0] & 0xff), tables, np.random.default_rng(p), [8, 40][p % 2])
+        if p == 3:
+            draws["y"][3] = draws["y"][3] * 3 - 3           # (runs that have no bit of their own, and empty ones)
+        templates, moves = _build_moves(base, tables, draws)
+        want = moves[a.claim(plan_keys_host(apply_moves_host(templates, moves, tables.db.n_algo)))]
+        t2, got = b.claim_moves(base, tables, draws)
+        assert np.array_equal(got, want) and np.array_equal(t2.codes, templates.codes) and np.array_equal(t2.hdr, templates.hdr)
+        assert len(a) == len(b) and not a.unseen(b._small.keys()).any()
+        seen, first = set(), []
+        for m in moves.tolist():
+            first.append(tuple(m) not in seen)
+            seen.add(tuple(m))
+        assert np.array_equal(_build_moves(base, tables, draws, [])[1], moves[first])
+
+
 @pytest.mark.parametrize("limit", [10, 65536])
 def test_key_set_behaves_like_a_set(limit):
     import copy
@@ -85,3 +107,30 @@ def test_key_set_behaves_like_a_set(limit):
         assert len(vk) == len(seen) and not vk.unseen(keys).any()
     assert len(copy.deepcopy(vk)) == len(vk) and not copy.deepcopy(vk).unseen(keys).any()
     assert vk.unseen(np.zeros((0, 2), dtype=np.uint64)).tolist() == []
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["gpt3_1_3b", "t5_770m", "wresnet_1b", "gpt_wide_stages"])
+def test_a_step_picks_what_its_parts_pick(name):
+    from superscaler_amd.evaluator import PlanEvaluator
+    from superscaler_amd.neighbours import _draws_struct
+    w = WORKLOADS[name]
+    tables = synth.make_tables(w)
+    ev = PlanEvaluator(tables)
+    a, b = VisitedKeys(), VisitedKeys()
+    for p in range(6):
+        base = synth.make_plans(w, tables, n_plans=8, seed_offset=50).slice(p % 4, p % 4 + 1)
+        draws = _draw_moves([3000, 200, 1][p % 3], int(base.hdr[0, 0] & 0xff), tables, np.random.default_rng(p), 8)
+        for keep in (None, a):
+            templates, moves = _build_moves(base, tables, draws, []) if keep is None else a.claim_moves(base, tables, draws)
+            got = ev.search_step(base, _draws_struct(draws), () if keep is None else b.handles())
+            want = None
+            if len(moves):
+                it, pk, fe, _ = ev.score(ev.apply_moves(templates, moves))
+                idx, val = ev.read_topk(ev.topk_packed(it, fe, 1), 1)
+                if len(idx):
+                    want = (apply_moves_host(templates, moves[idx[:1]], tables.db.n_algo), float(val[0]), float(pk[int(idx[0])].item()))
+            assert (got is None) == (want is None) and len(a) == len(b)
+            if got is not None:
+                assert got[1:] == want[1:] and np.array_equal(got[0].codes, want[0].codes) and np.array_equal(got[0].hdr, want[0].hdr)
+    ev.close()
