@@ -21,17 +21,16 @@
 //   16,384     66.0 -> 47.3   131.3 -> 72.4   136.9 -> 87.0           258.6 -> 117.1
 //   32,768     67.0 -> 53.2   135.3 -> 85.7   140.1 -> 98.5           259.0 -> 160.7
 //   65,536     70.8 -> 65.9   139.5 -> 114.4  142.7 -> 130.1          264.9 -> 228.6
-//  100,000    133.4 -> 76.6   264.7 -> 154.1  273.7 -> 155.3          517.1 -> 354.7
 // Up to 16,384 plans the longest wavefront is what is waited for (about 220 cycles per op, of which 110 are the issue of its
 // 27 instructions), from 65,536 on the SIMDs have two and more wavefronts to issue for all the time.
 #pragma once
 #include "ace_score_loop.h"
 
 // Plans per workgroup: the number that fills the 256 CUs with one workgroup each (the rows take most of a CU's LDS).  Above
-// 512 plans per CU the kernel of large batches has its four wavefronts per SIMD (131,072 plans of 523 ops: 160 us here, 163
-// there): 0.
+// 256 plans per CU the kernel of large batches is the faster one (ace_many.h; 131,072 plans of 523 ops: 141 us, 512 plans per
+// workgroup here 162; 65,536 plans: 114 us here, 134 there): 0.
 inline int ace_duo_lanes(long long plans) {
-    for (int L = 64; L <= 512; L *= 2)
+    for (int L = 64; L <= 256; L *= 2)
         if (plans <= 256ll * L) return L;
     return 0;
 }
@@ -57,20 +56,19 @@ template <int BLOCK> __device__ __forceinline__ void duo_rows(const AceKernelArg
 }
 
 #define ACE_DUO_RUN(TEXT)                                                                                                         \
-    asm volatile(TEXT : [wsnext] "=&v"(wsnext)                                                                                         \
+    asm volatile(TEXT :                                                                                        \
                  : [glogs] "v"(glogs), [lut2] "v"(lut2), [codeoff] "v"(code_off), [recoff] "v"(rec_off), [zerop] "v"(zero_pair),  \
                    [codes] "s"(codes), [pos] "s"(pos), [n_ops] "s"(a.g.N), [recbase] "s"(rec_base),                          \
                    [gstride_lo] "s"((uint32_t)gstride), [gstride_hi] "s"((uint32_t)(gstride >> 32)), [wsstride] "s"(ws_stride),   \
                    [wspiece] "s"(ws_piece), [grp] "s"(grp), [cut] "s"(cut), [recnext] "v"(rec_next)                                 \
                  : ACE_DUO_ASM_CLOBBERS)
 // Walks one part of the lane's plan, from 16-op group `grp` on; the stages that start in front of position `cut` are parked, the
-// first one at `rec_off`, the next at `rec_next` (kNoRecord: nowhere); returns where the next one would have gone.  `role` is the same for the whole wavefront, and all 64
+// first one at `rec_off`, the next at `rec_next` (kNoRecord: nowhere).  `role` is the same for the whole wavefront, and all 64
 // lanes are active.
 constexpr uint32_t kNoRecord = 0x80000000u;
-__device__ __forceinline__ uint32_t duo_loop(const AceKernelArgs &a, uint32_t role, uint32_t grp, uint32_t cut, uint64_t glogs, uint32_t lut2,
+__device__ __forceinline__ void duo_loop(const AceKernelArgs &a, uint32_t role, uint32_t grp, uint32_t cut, uint64_t glogs, uint32_t lut2,
                                          uint32_t code_off, uint32_t zero_pair, const double *rec_base, uint32_t rec_off,
                                          uint32_t rec_next, uint32_t ws_stride, uint32_t ws_piece) {
-    uint32_t wsnext;
     const uint64_t gstride = (uint64_t)(uint32_t)a.g.P * 16u;
     const unsigned char *codes = reinterpret_cast<const unsigned char *>(a.codes) + gstride * grp;
     const ace_u4 *pos = a.pos4 + (size_t)grp * 16u;
@@ -82,7 +80,6 @@ __device__ __forceinline__ uint32_t duo_loop(const AceKernelArgs &a, uint32_t ro
         else if (a.g.flags & ACE_F_RESERVED_MIN) ACE_DUO_RUN(ACE_DUO_ASM_MEMORY_MIN);
         else ACE_DUO_RUN(ACE_DUO_ASM_MEMORY_MAX);
     }
-    return wsnext;
 }
 #undef ACE_DUO_RUN
 
@@ -101,7 +98,6 @@ template <int L> struct DuoDeal;
 template <> struct DuoDeal<64> { static constexpr uint32_t v[3] = {0x00000000u, 0xff543210u, 0x6u}; };
 template <> struct DuoDeal<128> { static constexpr uint32_t v[3] = {0x10101010u, 0x33221100u, 0x44u}; };
 template <> struct DuoDeal<256> { static constexpr uint32_t v[3] = {0x32103210u, 0x11110000u, 0x2222u}; };
-template <> struct DuoDeal<512> { static constexpr uint32_t v[3] = {0x45673210u, 0u, 0x11111111u}; };
 
 // One workgroup: L plans.  The LDS array starts at address 0 (the kernel has no other LDS variables).
 template <int L> __device__ __forceinline__ void ace_duo_body(const AceKernelArgs &a, unsigned char *lds_raw, int tid, long long block) {
@@ -147,7 +143,7 @@ template <int L> __device__ __forceinline__ void ace_duo_body(const AceKernelArg
     // Stages that start in this part (every role counts half of its groups), in the parts before it, and altogether.
     uint32_t own = 0, before = 0, first = 0, n_st = 0;
     if (grp < grp_end) first = a.codes[(size_t)grp * g.P + pl].x & 0x1fu;
-    if (L < 512) {
+    {
         const uint32_t mid = (grp + grp_end + 1u) >> 1, end = role ? grp_end : mid;
         for (uint32_t k0 = role ? mid : grp; k0 < end; k0 += 8u) {
             ace_u4 c[8];
@@ -186,16 +182,14 @@ template <int L> __device__ __forceinline__ void ace_duo_body(const AceKernelArg
     // the part's first position is in stage `before` (it starts there), or in the one before that
     const bool opens = part == 0u || (first & 0x10u) != 0u, any = part == 0u || own != 0u;
     const uint32_t here = before + (opens ? 1u : 0u);                // one more than the index of that stage
-    uint32_t next = 0;
     if (part == 0u) __builtin_amdgcn_s_setprio(3);                  // (the longest walk of a slice: 78.3 -> 72.9 us, 16,384 plans of 523 ops)
     if (grp < grp_end && __any(any)) {
         const uint32_t shift = here > 1u ? 4u * (here - 1u) : 0u;
-        next = duo_loop(a, role, grp, part + 1u < parts ? 16u * grp_end : 0x7fffffffu, shift < 64u ? st.glogs >> shift : 0ull,
+        duo_loop(a, role, grp, part + 1u < parts ? 16u * grp_end : 0x7fffffffu, shift < 64u ? st.glogs >> shift : 0ull,
                  g.lut2a_lds_off + st.bidx * 128u, (uint32_t)pl * 16u, zero_pair, rec_base,
                  opens ? at * 16u + before * kStride : kNoRecord, any ? at * 16u + here * kStride : kNoRecord, kStride, kPiece);
     }
     __builtin_amdgcn_s_setprio(0);
-    if (L == 512) n_st = (next - at * 16u) / kStride - 1u;
     __syncthreads();                                                // all pieces of the records
     // Stage tails: every lane evaluates its role's half of every `parts`-th stage and leaves the stage times / the largest
     // stage memory in places of the records that only this lane reads; then one lane per plan puts the plan together.
@@ -204,41 +198,35 @@ template <int L> __device__ __forceinline__ void ace_duo_body(const AceKernelArg
     st.ws_stride = kStride / 16u;
     st.ws_piece = kPiece / 16u;
     const uint32_t code0 = a.codes[pl].x & 0x1fu, row0 = a.pos_info[0] & 0xffu;
-    double sum = 0.0, mx = 0.0, mem = 0.0;
     if (idle) {
     } else if (role) {
         st.replay_some(g, lds, rec, (int)part, (int)parts, n_live, code0 & 7u, row0, [](int, double) {});
         rec[(size_t)part * (kStride / 8u) + 2u * (kPiece / 8u)] = st.max_mem;
-    } else if (L < 512)
+    } else
         st.replay_some(g, lds, rec, (int)part, (int)parts, n_live, code0 & 7u, row0,
                        [=](int s, double t) { rec[(size_t)s * (kStride / 8u)] = t; });
-    else
-        st.replay_some(g, lds, rec, 0, 1, n_live, code0 & 7u, row0, [&](int, double t) { sum += t; mx = ace_max(mx, t); });
     __syncthreads();
     if (role || part) return;
     // (all loads before the first use: one trip to memory)
-    if (L < 512) {
-        double t[ACE_MAX_STAGES];
+    double t[ACE_MAX_STAGES], sum = 0.0, mx = 0.0, mem = 0.0;
 #pragma unroll
-        for (int s = 0; s < ACE_MAX_STAGES; ++s) {
-            t[s] = 0.0;
-            if (s < n_live) t[s] = rec[(size_t)s * (kStride / 8u)];
-        }
-        double pm[8];
+    for (int s = 0; s < ACE_MAX_STAGES; ++s) {
+        t[s] = 0.0;
+        if (s < n_live) t[s] = rec[(size_t)s * (kStride / 8u)];
+    }
+    double pm[8];
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            pm[k] = 0.0;
-            if (k < (int)parts) pm[k] = rec[(size_t)k * (kStride / 8u) + 2u * (kPiece / 8u)];
-        }
+    for (int k = 0; k < 8; ++k) {
+        pm[k] = 0.0;
+        if (k < (int)parts) pm[k] = rec[(size_t)k * (kStride / 8u) + 2u * (kPiece / 8u)];
+    }
 #pragma unroll
-        for (int s = 0; s < ACE_MAX_STAGES; ++s) {
-            sum += t[s];                                            // (stage times are sums from +0.0: adding 0.0 changes nothing)
-            mx = ace_max(mx, t[s]);
-        }
+    for (int s = 0; s < ACE_MAX_STAGES; ++s) {
+        sum += t[s];                                            // (stage times are sums from +0.0: adding 0.0 changes nothing)
+        mx = ace_max(mx, t[s]);
+    }
 #pragma unroll
-        for (int k = 0; k < 8; ++k) mem = ace_max(mem, pm[k]);
-    } else
-        mem = rec[2u * (kPiece / 8u)];
+    for (int k = 0; k < 8; ++k) mem = ace_max(mem, pm[k]);
     st.s = (int)n_st;
     st.sum_t = sum; st.max_t = mx; st.max_mem = mem;
     if (!(code0 & 0x10u)) st.status = ACE_PLAN_MALFORMED;            // the first op must open a stage

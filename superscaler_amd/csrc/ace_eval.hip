@@ -25,6 +25,7 @@
 #include "ace_score_loop.h"
 #include "ace_spread.h"
 #include "ace_duo.h"
+#include "ace_many.h"
 #include "ace_recompute.h"
 
 // Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans (the
@@ -85,6 +86,11 @@ __global__ __launch_bounds__(kSpreadLanes) void ace_spread_kernel(const AceKerne
 template <int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(const AceKernelArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_duo_body<L>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+}
+// Large batches on the assembly loop with every row resident, see ace_many.h.
+__global__ __launch_bounds__(1024) void ace_many_kernel(const AceKernelArgs a, const uint32_t slices) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    ace_many_body(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -748,6 +754,11 @@ template <int L> static int allow_duo_lds() {
     return ACE_OK;
 }
 
+static int allow_many_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_many_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    return ACE_OK;
+}
+
 // Per op position, what the assembly form of the op loop (ace_score_loop_asm.inc) reads with scalar loads: the LDS
 // address of the position's row at its hot sub-table and at its collective-cost tables, the LDS address of the
 // 32-bit pair-kind block of the (this op, next op) pair, and two flags (bit 0: the rule "ordinary op followed by a layer
@@ -1049,7 +1060,7 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
         (rc = allow_duo_lds<64>()) || (rc = allow_duo_lds<128>()) || (rc = allow_duo_lds<256>()) ||
-        (rc = allow_duo_lds<512>()) ||
+        (rc = allow_many_lds()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
         ace_destroy(h);
         return rc;
@@ -1146,12 +1157,23 @@ static void launch_spread(const AceKernelArgs &a, hipStream_t s) {
     else launch_spread_c<BD, RANGED, false>(a, s);
 }
 
-// Workgroup size of the kernel of mid-sized batches for this call, or 0: plain scoring of a batch that leaves the large kernel
-// short of wavefronts, of tables the assembly loops can run on.
+// Plain scoring on tables that the assembly loops walk with every row resident: the kernels of mid-sized and large batches.
+static bool resident_asm(const ace_handle_t *h, const AceKernelArgs &a) {
+    return !a.range && !a.stage_out && a.stage_ws && h->n_windows == 1 && a.pos4 && a.g.lut2a_lds_off && a.flat_rows16 > 0;
+}
+// Workgroup size of the kernel of mid-sized batches for this call, or 0.
 static int duo_lanes(const ace_handle_t *h, const AceKernelArgs &a) {
-    if (a.range || a.stage_out || !a.stage_ws || h->n_windows > 1 || !a.pos4 || !a.g.lut2a_lds_off || a.flat_rows16 <= 0) return 0;
-    const int L = ace_duo_lanes(a.g.P);
+    const int L = resident_asm(h, a) ? ace_duo_lanes(a.g.P) : 0;
     return L && ace_duo_lds(a.g, h->lds_bytes, L) <= kMaxLds ? L : 0;
+}
+// The kernel of large batches (false: it cannot take this call).
+static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    const uint32_t slices = ace_many_slices(a.g.P), lanes = 64u * slices;
+    const uint32_t deal = a.g.rk_lds_off + 128u + 2u * 1024u, lds = deal > h->lds_bytes ? deal : h->lds_bytes;
+    const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
+    if (!resident_asm(h, a) || a.stage_ws != h->d_stage_ws || lds > kMaxLds || groups * lanes > h->stage_ws_plans) return false;
+    hipLaunchKernelGGL(ace_many_kernel, dim3((unsigned)groups), dim3(1024), lds, s, a, slices);
+    return true;
 }
 template <int L>
 static void launch_duo_l(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
@@ -1160,8 +1182,7 @@ static void launch_duo_l(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
 static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     if (L == 64) launch_duo_l<64>(h, a, s);
     else if (L == 128) launch_duo_l<128>(h, a, s);
-    else if (L == 256) launch_duo_l<256>(h, a, s);
-    else launch_duo_l<512>(h, a, s);
+    else launch_duo_l<256>(h, a, s);
 }
 
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
@@ -1176,6 +1197,7 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
     else if (a.stage_out) launch_score_w<true, false>(h, a, s);
     else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
     else if (mid) launch_duo(mid, h, a, s);
+    else if (launch_many(h, a, s)) return;
     else if (a.stage_ws) launch_score_b<false, false, false, true>(h, a, s);
     else launch_score_w<false, false>(h, a, s);
 }
@@ -1185,7 +1207,8 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
 static int ensure_stage_ws(ace_handle_t *h, AceKernelArgs *a) {
     a->stage_ws = nullptr;
     if (a->range || a->stage_out || (h->n_windows > 1 && !h->d_pos_types) || h->geom.N >= 32768 || (h->geom.flags & ACE_F_COLLECTIVE_MEM)) return ACE_OK;
-    const size_t need = (((size_t)a->g.P + kBlock - 1) / kBlock) * kBlock;
+    // (a block more: the kernel of large batches rounds the share of every CU up)
+    const size_t need = (((size_t)a->g.P + kBlock - 1) / kBlock + 1) * kBlock;
     if (need * ACE_MAX_STAGES * (ACE_WS_REC / 2) > 0xffffffffull) return ACE_OK;   // (a workspace of 64 GiB and more: such batches take the plain kernel)
     if (need > h->stage_ws_plans) {
         if (h->stage_ws_fixed) return ACE_EFIXED;

@@ -1,0 +1,91 @@
+// Scoring of LARGE batches where the assembly op loop runs with every row resident: the kernel of ace_score_loop.h (a plan per
+// lane, sixteen wavefronts per workgroup and CU) with workgroups of as many plans as make an even share.
+//
+// The rows fill a CU's LDS, so the workgroups of a batch run in rounds of 256, and with 1,024 plans each a batch of 200,000
+// leaves a fifth of the CUs idle and the last 37,856 plans of one of 300,000 take a second round of their own.  Here a
+// workgroup takes 64 * slices plans, at most 1,024, so that the rounds the batch needs are all full.  (One workgroup per CU
+// that stages once and walks several rounds, with or without a barrier between them, was slower: 1,048,576 plans of 523 ops
+// 757 / 797 us instead of 729.)  Rows are staged by LDS-direct loads.
+// Measured, us per launch, before -> now:
+//   plans      315 ops          523 ops          821 ops          1,251 ops
+//   100,000   132.4 -> 69.1    263.9 -> 136.5   272.4 -> 139.8   517.1 -> 293.0     (two rounds of 256-lane workgroups before)
+//   131,072    88.9 -> 71.2    163.4 -> 141.4   161.7 -> 142.9   422.6 -> 305.1
+//   200,003    94.3 -> 86.5    174.9 -> 169.1   172.8 -> 170.2   456.6 -> 416.6
+//   300,000   178.0 -> 152.7   338.6 -> 297.2   326.0 -> 310.3   864.7 -> 740.2
+//   600,000   275.3 -> 258.8   525.7 -> 507.6   505.6 -> 497.6  1328.8 -> 1185.7
+// and the same for whole rounds.  What bounds it is the issue of vector instructions (the op loop) up to the batch's last op,
+// and then the records coming back from memory.
+#pragma once
+#include "ace_duo.h"
+
+// Slices of 64 plans per workgroup.
+inline uint32_t ace_many_slices(long long plans) {
+    const long long fullest = ((plans + 63) / 64 + 255) / 256;       // slices of the batch on the fullest CU
+    const long long rounds = (fullest + 15) / 16;
+    return (uint32_t)((fullest + rounds - 1) / rounds);
+}
+
+#ifndef ACE_HOST_EMU
+// One workgroup of 1,024 lanes.
+__device__ __forceinline__ void ace_many_body(const AceKernelArgs &a, uint32_t slices, unsigned char *lds_raw, int tid, long long block) {
+    constexpr int kLanes = 1024;
+    const AceGeom &g = a.g;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6), lane = (uint32_t)tid & 63u;
+    const uint32_t lanes = 64u * slices;
+    duo_rows<kLanes>(a, lds_raw, wave, lane);
+    // Deal: counting sort of the plans by pipeline depth, the deepest first (see ace_score_body), where the small tables go.
+    // Sorted slice q goes to wavefront q in rows of four, every second row reversed: each SIMD gets the same mix.
+    unsigned int *cnt = reinterpret_cast<unsigned int *>(lds_raw + g.rk_lds_off);
+    unsigned short *plan_of = reinterpret_cast<unsigned short *>(lds_raw + g.rk_lds_off + 128);
+    const uint32_t q = (wave & 4u) ? wave ^ 3u : wave;
+    if (tid < 32) cnt[tid] = 0u;
+    const long long slot = block * lanes + tid;
+    uint32_t depth = 0, rank = 0;                                   // (slots past the batch: last)
+    if ((uint32_t)tid < lanes && slot < g.P) {
+        depth = a.hdr[slot].x & 0xffu;
+        depth = depth > 16u ? 16u : depth;
+    }
+    __syncthreads();
+    if ((uint32_t)tid < lanes) rank = atomicAdd(&cnt[16u - depth], 1u);
+    __syncthreads();
+    if ((uint32_t)tid < lanes) {
+        for (uint32_t b = 0; b < 16u - depth; ++b) rank += cnt[b];
+        plan_of[rank] = (unsigned short)tid;
+    }
+    __syncthreads();
+    const uint32_t at = (q << 6) | lane;
+    const long long plan = block * lanes + (q < slices ? (uint32_t)plan_of[at] : 0u);
+    __syncthreads();
+    const bool in_batch = plan < g.P;
+    const long long pl = in_batch ? plan : (long long)g.P - 1;      // plan this lane reads
+    const long long out = a.order ? (long long)a.order[pl] : plan;
+    const bool active = in_batch && out < g.P;
+    const ace_u4 h = a.hdr[pl];
+    const uint32_t first = a.codes[pl].x & 0x1fu;
+    stage_small_tables<kLanes, true>(a, lds_raw, tid);
+    if (g.pace_lds_off && tid < 32) reinterpret_cast<uint32_t *>(lds_raw + g.pace_lds_off)[tid] = 0u;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // the rows
+    __syncthreads();
+    if (q >= slices) return;
+
+    const AceLds lds = ace_make_lds(lds_raw, 0u);
+    PlanState<false, false, true> st;
+    st.init(g, lds, h, ace_u2{0u, 0u});
+    if (!(first & 0x10u)) st.status = ACE_PLAN_MALFORMED;            // the first op must open a stage
+    const uint32_t stride = lanes * (ACE_WS_REC * 8u), rec_off = at * (ACE_WS_REC * 8u);
+    st.ws_stride = stride / 16u;
+    double *rec_base = a.stage_ws + (size_t)block * ACE_MAX_STAGES * lanes * ACE_WS_REC;
+    const int n_st = (int)ace_score_loop_asm<false>(a, g, st.glogs, g.lut2a_lds_off + st.bidx * 128u, (uint32_t)pl * 16u, rec_base, rec_off,
+                                                    stride, 0u, wave);
+    st.replay_all(g, lds, rec_base + rec_off / 8u, n_st, first & 7u, a.pos_info[0] & 0xffu);
+    double iter, peak;
+    uint8_t feas, stat;
+    st.result(g, a.nbm1[st.bidx], iter, peak, feas, stat);
+    if (active) {
+        a.iter_ms[out] = iter;
+        a.peak_mb[out] = peak;
+        a.feasible[out] = feas;
+        if (a.status) a.status[out] = stat;
+    }
+}
+#endif

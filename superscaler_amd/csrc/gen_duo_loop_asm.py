@@ -494,7 +494,6 @@ class Duo:
         o("L_exit_%=:")
         o("s_mov_b64 exec, -1")
         o("s_waitcnt vmcnt(0) lgkmcnt(0)")
-        o(f"v_mov_b32 %[wsnext], {WSNEXT}")
         return self.lines
 
 

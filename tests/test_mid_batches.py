@@ -35,7 +35,7 @@ def test_committed_duo_loop_is_the_generators_output():
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,mode,sizes", [("gpt3_13b", "plain", (3840, 3841, 16385)), ("t5_770m", "min", (8191,)), ("gpt3_175b", "noreserved", (4999,)),
                                              ("gpt3_1_3b", "min", (16384,)), ("gpt_wide_stages", "plain", (5000, 32768, 32769, 65537)),
-                                             ("gpt_16ops", "noreserved", (65536, 131072, 131073)), ("gpt_3tp", "min", (20001, 100001)),
+                                             ("gpt_16ops", "noreserved", (65536,)), ("gpt_3tp", "min", (20001, 100001)),
                                              ("t5_1layer", "plain", (16383, 70000))])
 def test_mid_sized_batches_on_the_gpu(name, mode, sizes):
     from superscaler_amd.evaluator import PlanEvaluator
@@ -61,4 +61,24 @@ def test_mid_sized_batches_on_the_gpu(name, mode, sizes):
     for g, x in zip(got, want):
         assert x is None or np.array_equal(g[:64], x, equal_nan=True)
     assert np.array_equal(got[0][64:], it[64:]) and np.array_equal(got[1][64:], pk[64:])
+    ev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,mode,sizes", [("gpt_16ops", "plain", (65537, 131072, 200001, 262144)), ("gpt_wide_stages", "min", (262145, 300003)),
+                                             ("t5_1layer", "noreserved", (147456, 600001)), ("gpt3_1_3b", "plain", (270000,))])
+def test_large_batches_in_even_shares_on_the_gpu(name, mode, sizes):
+    from superscaler_amd.evaluator import PlanEvaluator
+    w = WORKLOADS[name]
+    tables = tables_for(w, **SETTINGS[mode])
+    ev = PlanEvaluator(tables)
+    base = synth.make_plans(w, tables, n_plans=40000, seed_offset=7)
+    rng = np.random.default_rng(1)
+    for n in sizes:
+        print(f"[case] {name} {mode} plans={n}", flush=True)
+        pick = rng.integers(0, base.n_plans, n)
+        want = c_oracle_scores(tables, base, threads=8)
+        batch = PlanBatch(base.codes[pick], base.hdr[pick])
+        it, pk, fe, st = ev.score_host(batch)
+        assert (st == 0).all() and np.array_equal(it, want[0][pick]) and np.array_equal(pk, want[1][pick]) and np.array_equal(fe, want[2][pick])
     ev.close()
