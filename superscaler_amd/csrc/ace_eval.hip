@@ -87,10 +87,10 @@ template <int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(con
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_duo_body<L>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
-// Large batches on the assembly loop with every row resident, see ace_many.h.
-__global__ __launch_bounds__(1024) void ace_many_kernel(const AceKernelArgs a, const uint32_t slices) {
+// Large batches on the assembly loop, see ace_many.h.
+template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(const AceKernelArgs a, const uint32_t slices) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_many_body(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_many_body<WIN>(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -98,24 +98,17 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
 }
 
 // Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has four workgroups
-// (1,024 plans), that of the kernels with a plan per lane not before 16,384; they cross between 4,096 and 16,384 plans,
-// earlier without stage records (the lane-per-plan kernel defers the stage tails there).  Measured, us per launch,
-// lane per plan -> plan per workgroup (launches back to back: 13 to 20 us is what the host needs for one):
-//   plain    315 ops:    1 plan  49 -> 13, 1,024  65 -> 16, 4,096  66 -> 45;  1,251 ops: 1  169 -> 26, 4,096  254 -> 118
-//   records  523 ops:    1 plan 117 -> 19, 1,024 312 -> 24, 4,096 321 -> 80, 16,384 322 -> 274 (315 ops: 147 -> 194)
-//   queries  523 ops:   64      163 -> 20, 1,024 189 -> 21, 4,096 194 -> 38, 16,384 169 -> 112 (315 ops: 106 -> 122)
-#ifndef ACE_SPREAD_MAX_PLAIN
-#define ACE_SPREAD_MAX_PLAIN 4096
-#endif
-// ... and where the kernel of mid-sized batches can run, whose time hardly grows from 64 to 16,384 plans: up to this many
-// (3,584 / 3,840 / 4,096 plans, us, plan per workgroup -> mid-sized: 315 ops 39 / 41 / 45 -> 43, 523 ops 57 / 60 / 65 -> 67,
-// 821 ops 79 / 82 / 89 -> 81, 1,251 ops 104 / 106 / 119 -> 107).
-#ifndef ACE_SPREAD_MAX_MID
-#define ACE_SPREAD_MAX_MID 3840
-#endif
-#ifndef ACE_SPREAD_MAX_RECORDS
-#define ACE_SPREAD_MAX_RECORDS 8192
-#endif
+// (1,024 plans); that of the others, where a lane or a few walk a plan, hardly does until the chip is full, and they cross
+// where that time is reached.  By what else would take the batch, in us per launch (plan per workgroup / the other):
+//   PLAIN    the mid-sized kernel      3,584 / 3,840 / 4,096 plans: 315 ops 39 41 45 / 43, 523 ops 57 60 65 / 67, 821 ops
+//                                      79 82 89 / 81, 1,251 ops 104 106 119 / 107
+//   WINDOWED large, windowed rows      7,168 / 8,192 plans: 114 ops 39 44 / 42, 176 ops 47 53 / 55
+//   SLOW     no assembly loop (memory of collectives, more than 256 rows)   16,384 plans: 315 ops 150 / 164, 523 ops 254 / 455
+//   RECORDS  stage records             12,288 plans: 315 ops 148 / 146, 523 ops 209 / 322, 134 ops 83 / 172; single-stage
+//            queries                   12,288: 315 ops 93 / 106, 523 ops 89 / 185
+// and at one plan 13 to 26 where a lane needs 49 to 169 (13 to 20 us is what the host needs for a launch).
+constexpr int kSpreadMaxPlain = 3840, kSpreadMaxWindowed = 7680, kSpreadMaxSlow = 16384, kSpreadMaxRecords = 12288;
+constexpr int kSpreadMaxOther = 4096;    // (deferred stage tails on the C++ form of the loop: tables that leave the assembly loop no room)
 
 // ------------------------------------------------------------------------------------------
 // top-k: radix select on the order-preserving 64-bit image of the iteration time, then a
@@ -635,6 +628,7 @@ struct ace_handle {
     ace_u2 *d_pos_spread;      // per position, for the kernel of small batches (null: more ops than it takes)
     uint32_t *d_pos_types;     // d_pos_info with row indices in place of LDS slots (windowed rows, at most 256 of them; else null)
     ace_u4 *d_pos4;            // per position, for the assembly op loop (null when its pair-kind table has no room in LDS)
+    int32_t n_fetch;           // fetch events of d_win_dma
     ace_u4 *d_win_dma;         // windowed rows: what the assembly op loop fetches its windows by (setup_windowed_asm), or null
     AceGeom geom_wa;           // ... and the LDS layout of the kernel that runs it
     uint32_t lds_bytes_wa;
@@ -754,8 +748,8 @@ template <int L> static int allow_duo_lds() {
     return ACE_OK;
 }
 
-static int allow_many_lds() {
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_many_kernel), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+template <bool WIN> static int allow_many_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_many_kernel<WIN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     return ACE_OK;
 }
 
@@ -910,6 +904,7 @@ static int setup_windowed_asm(ace_handle *h, const ace_tables_t *t, size_t pos_e
     int rc = upload((void **)&h->d_win_dma, blob.data(), blob.size() * sizeof(ace_u4));
     if (rc == ACE_OK) rc = upload((void **)&h->d_pos4, p4.data(), p4.size() * sizeof(ace_u4));
     if (rc != ACE_OK) return rc;
+    h->n_fetch = n_ev;
     h->geom_wa = h->geom;
     h->geom_wa.rk_lds_off = 2u * slots * crow;
     h->geom_wa.stg_lds_off = stg_off; h->geom_wa.lut2_lds_off = lut2_off; h->geom_wa.pk32_lds_off = pk32_off; h->geom_wa.pace_lds_off = 0; h->geom_wa.lut2a_lds_off = lut2a_off;
@@ -1060,7 +1055,7 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
         (rc = allow_duo_lds<64>()) || (rc = allow_duo_lds<128>()) || (rc = allow_duo_lds<256>()) ||
-        (rc = allow_many_lds()) ||
+        (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
         ace_destroy(h);
         return rc;
@@ -1105,7 +1100,7 @@ static int fill_args(ace_handle_t *h, const ace_batch_t *b, double memory_limit,
     a->hdr = reinterpret_cast<const ace_u4 *>(b->d_hdr);
     a->range = reinterpret_cast<const ace_u2 *>(b->d_range);
     a->order = b->d_order;
-    a->rows = h->d_rows; a->pos_info = h->d_pos_info; a->pos_types = h->d_pos_types; a->pos4 = h->d_pos4; a->win_dma = h->d_win_dma; a->pos_spread = h->d_pos_spread; a->pair_kinds = h->d_pair_kinds; a->stage_lut = h->d_stage_lut;
+    a->rows = h->d_rows; a->pos_info = h->d_pos_info; a->pos_types = h->d_pos_types; a->pos4 = h->d_pos4; a->win_dma = h->d_win_dma; a->n_fetch = h->n_fetch; a->pos_spread = h->d_pos_spread; a->pair_kinds = h->d_pair_kinds; a->stage_lut = h->d_stage_lut;
     a->nbm1 = h->d_nbm1; a->win_pos = h->d_win_pos; a->win_row_begin = h->d_win_row_begin; a->win_rows = h->d_win_rows;
     a->n_windows = h->n_windows; a->row_doubles = h->row_doubles; a->rk_bytes = h->rk_bytes; a->stg_words = h->stg_words;
     a->flat_rows16 = h->flat_rows16;
@@ -1123,14 +1118,6 @@ static void launch_score_b(const ace_handle_t *h, const AceKernelArgs &a, hipStr
         if (!DEFER)         // (ensure_stage_ws never hands such tables to the deferred kernel)
             hipLaunchKernelGGL((ace_score_kernel<BD, RANGED, WIN, false, kBlock, true>), dim3((unsigned)((P + kBlock - 1) / kBlock)),
                                dim3(kBlock), h->lds_bytes, s, a);
-    } else if (WIN && DEFER && h->d_win_dma) {
-        // the assembly op loop over windowed rows lays LDS out its own way (batches of any size: with the next window
-        // arriving while a window is walked, the large workgroup is the faster one from a single plan on)
-        AceKernelArgs b = a;
-        b.g = h->geom_wa;
-        b.g.P = a.g.P; b.g.mem_limit = a.g.mem_limit; b.g.strict = a.g.strict;
-        hipLaunchKernelGGL((ace_score_kernel<BD, RANGED, WIN, DEFER, kBlock>), dim3((unsigned)((P + kBlock - 1) / kBlock)),
-                           dim3(kBlock), h->lds_bytes_wa, s, b);
     } else if ((P + kBlock - 1) / kBlock < (size_t)kSmallBatchBlocks)
         hipLaunchKernelGGL((ace_score_kernel<BD, RANGED, WIN, DEFER, kSmallBlock>), dim3((unsigned)((P + kSmallBlock - 1) / kSmallBlock)),
                            dim3(kSmallBlock), h->lds_bytes, s, a);
@@ -1168,11 +1155,19 @@ static int duo_lanes(const ace_handle_t *h, const AceKernelArgs &a) {
 }
 // The kernel of large batches (false: it cannot take this call).
 static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    const uint32_t slices = ace_many_slices(a.g.P), lanes = 64u * slices;
-    const uint32_t deal = a.g.rk_lds_off + 128u + 2u * 1024u, lds = deal > h->lds_bytes ? deal : h->lds_bytes;
-    const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
-    if (!resident_asm(h, a) || a.stage_ws != h->d_stage_ws || lds > kMaxLds || groups * lanes > h->stage_ws_plans) return false;
-    hipLaunchKernelGGL(ace_many_kernel, dim3((unsigned)groups), dim3(1024), lds, s, a, slices);
+    const bool win = h->n_windows > 1 && h->d_win_dma && a.stage_ws && !a.range && !a.stage_out;
+    if (!win && !resident_asm(h, a)) return false;
+    AceKernelArgs b = a;
+    if (win) {                                          // (that loop lays LDS out its own way)
+        b.g = h->geom_wa;
+        b.g.P = a.g.P; b.g.mem_limit = a.g.mem_limit; b.g.strict = a.g.strict;
+    }
+    const uint32_t slices = ace_many_slices(a.g.P), lanes = 64u * slices, tables = win ? h->lds_bytes_wa : h->lds_bytes;
+    const uint32_t deal = b.g.rk_lds_off + 128u + 2u * 1024u, lds = deal > tables ? deal : tables;
+    const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes, room = a.stage_ws == h->d_stage_ws ? h->stage_ws_plans : (size_t)ACE_STATIC_MAX_PLANS;
+    if (lds > kMaxLds || groups * lanes > room) return false;
+    if (win) hipLaunchKernelGGL(ace_many_kernel<true>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
+    else hipLaunchKernelGGL(ace_many_kernel<false>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
     return true;
 }
 template <int L>
@@ -1187,7 +1182,8 @@ static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hip
 
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     const int mid = duo_lanes(h, a);
-    if (a.pos_spread && a.g.P <= (a.stage_out ? ACE_SPREAD_MAX_RECORDS : mid ? ACE_SPREAD_MAX_MID : ACE_SPREAD_MAX_PLAIN)) {
+    const int most = a.stage_out ? kSpreadMaxRecords : mid ? kSpreadMaxPlain : !a.stage_ws ? kSpreadMaxSlow : h->d_win_dma ? kSpreadMaxWindowed : kSpreadMaxOther;
+    if (a.pos_spread && a.g.P <= most) {
         if (a.range) launch_spread<true, true>(a, s);
         else if (a.stage_out) launch_spread<true, false>(a, s);
         else launch_spread<false, false>(a, s);
@@ -1195,9 +1191,9 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
     }
     if (a.range) launch_score_w<true, true>(h, a, s);
     else if (a.stage_out) launch_score_w<true, false>(h, a, s);
-    else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
     else if (mid) launch_duo(mid, h, a, s);
     else if (launch_many(h, a, s)) return;
+    else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
     else if (a.stage_ws) launch_score_b<false, false, false, true>(h, a, s);
     else launch_score_w<false, false>(h, a, s);
 }

@@ -37,6 +37,7 @@ struct AceKernelArgs {
     const int32_t *win_row_begin;
     const uint32_t *win_rows;   // pairs (type, lds byte offset)
     const ace_u4 *win_dma;      // what the assembly op loop stages the windows from (see ace_score_loop_asm), or null
+    int32_t n_fetch;            // ... its fetch events
     int32_t n_windows, row_doubles, rk_bytes, stg_words;
     int32_t flat_rows16;        // rows resident and laid out in LDS as they lie in `rows`: their size in 16-byte pieces (else 0)
     double *iter_ms, *peak_mb;
@@ -218,15 +219,13 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
     const bool flat = !WIN && a.flat_rows16 > 0;
     if (flat) rows_first = stage_rows_first<BLOCK>(a, tid);
     long long plan = slot;
-    uint32_t prio = 0;                                              // issue priority of this wavefront in the op loop
 #ifndef ACE_HOST_EMU
     if (!RANGED && BLOCK >= 128) {
         // The lanes of a wavefront walk the ops together, and every op at which one of them closes a stage takes all
         // of them through the stage-end code: so the workgroup deals its plans to its lanes by pipeline depth
         // (counting sort on the depth in the plan header, deepest first; plans of one depth in any order), and the
         // sorted wavefronts to the SIMDs in turn (wavefront w runs on SIMD w % 4) so that each SIMD gets the same
-        // mix.  The wavefronts with the deeper plans get the higher issue priority: they have the most instructions
-        // to issue and would otherwise be the last to finish, alone on their SIMDs.  Only which lane scores which
+        // mix.  Only which lane scores which
         // plan changes: results go to the plan's own index.  (Single-stage queries are left as they come: their
         // length, not a depth, is what would have to be sorted on.)
         unsigned int *cnt = reinterpret_cast<unsigned int *>(lds_raw);                  // 17 bins (nothing is staged yet)
@@ -249,10 +248,6 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
         plan_of[(wave << 6) | (sorted & 63u)] = (unsigned short)tid;
         ACE_SYNC();
         plan = block * BLOCK + plan_of[tid];
-        if (BLOCK >= 1024) {
-            const uint32_t pw = (uint32_t)tid >> 6, qs = (pw & 4u) ? (pw ^ 3u) : pw;       // the sorted slice this wavefront walks
-            prio = __builtin_amdgcn_readfirstlane(3u - (qs >> 2));
-        }
         ACE_SYNC();
     }
 #endif
@@ -295,15 +290,15 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
     ace_u4 cw = a.codes[(size_t)grp_begin * g.P + pl];
 
     stage_small_tables<BLOCK, DEFER>(a, lds_raw, tid);
-    // (the assembly op loop over windowed rows fetches its windows itself, in a layout of its own)
+    // (the assembly op loop over windowed rows: ace_many.h)
 #ifndef ACE_HOST_EMU
-    const bool asm_loop = DEFER && lds_base == 0u && a.pos4 && a.g.lut2a_lds_off && (!WIN || (BLOCK == 1024 && a.win_dma));
+    const bool asm_loop = DEFER && !WIN && lds_base == 0u && a.pos4 && a.g.lut2a_lds_off;
 #else
     const bool asm_loop = false;
 #endif
     if (DEFER && a.g.pace_lds_off && tid < 32) reinterpret_cast<uint32_t *>(lds_raw + a.g.pace_lds_off)[tid] = 0u;
     if (flat) stage_rows_flat<BLOCK>(a, lds_raw, tid, rows_first);
-    else if (!(WIN && asm_loop)) stage_window<BLOCK>(a, lds_raw, w0, tid);       // every row, or the first window's
+    else stage_window<BLOCK>(a, lds_raw, w0, tid);       // every row, or the first window's
     ACE_SYNC();
 
     AceLds lds = ace_make_lds(lds_raw, lds_bytes);
@@ -331,9 +326,9 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
         // the assembly form of the loop below (same operations per plan, same results)
         if (!(cw.x & 0x10u)) st.status = ACE_PLAN_MALFORMED;    // the first op must open a stage
         // (the loop looks each stage's offsets up in LDS, by the stage size's log2)
-        st.s = (int)ace_score_loop_asm<WIN>(a, g, st.glogs, g.lut2a_lds_off + st.bidx * 128u, (uint32_t)pl * 16u,
+        st.s = (int)ace_score_loop_asm<false>(a, g, st.glogs, g.lut2a_lds_off + st.bidx * 128u, (uint32_t)pl * 16u,
                                             a.stage_ws + (size_t)block * ACE_MAX_STAGES * BLOCK * ACE_WS_REC,
-                                            (uint32_t)tid * (ACE_WS_REC * 8u), (uint32_t)BLOCK * (ACE_WS_REC * 8u), prio,
+                                            (uint32_t)tid * (ACE_WS_REC * 8u), (uint32_t)BLOCK * (ACE_WS_REC * 8u), 0u,
                                             (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6));
         grp_stop = grp_begin;
     } else

@@ -66,7 +66,9 @@ def test_mid_sized_batches_on_the_gpu(name, mode, sizes):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,mode,sizes", [("gpt_16ops", "plain", (65537, 131072, 200001, 262144)), ("gpt_wide_stages", "min", (262145, 300003)),
-                                             ("t5_1layer", "noreserved", (147456, 600001)), ("gpt3_1_3b", "plain", (270000,))])
+                                             ("t5_1layer", "noreserved", (147456, 600001)), ("gpt3_1_3b", "plain", (270000,)),
+                                             ("wresnet_1b", "plain", (7680, 7681, 16385, 270001)), ("resnet_1111", "min", (8000, 70000)),
+                                             ("resnet_16gpus", "noreserved", (16384, 33333))])
 def test_large_batches_in_even_shares_on_the_gpu(name, mode, sizes):
     from superscaler_amd.evaluator import PlanEvaluator
     w = WORKLOADS[name]
