@@ -97,17 +97,18 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
     ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 
-// Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has four workgroups
-// (1,024 plans); that of the others, where a lane or a few walk a plan, hardly does until the chip is full, and they cross
+// Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has six workgroups
+// (1,536 plans); that of the others, where a lane or a few walk a plan, hardly does until the chip is full, and they cross
 // where that time is reached.  By what else would take the batch, in us per launch (plan per workgroup / the other):
-//   PLAIN    the mid-sized kernel      3,584 / 3,840 / 4,096 plans: 315 ops 39 41 45 / 43, 523 ops 57 60 65 / 67, 821 ops
-//                                      79 82 89 / 81, 1,251 ops 104 106 119 / 107
-//   WINDOWED large, windowed rows      7,168 / 8,192 plans: 114 ops 39 44 / 42, 176 ops 47 53 / 55
-//   SLOW     no assembly loop (memory of collectives, more than 256 rows)   16,384 plans: 315 ops 150 / 164, 523 ops 254 / 455
-//   RECORDS  stage records             12,288 plans: 315 ops 148 / 146, 523 ops 209 / 322, 134 ops 83 / 172; single-stage
-//            queries                   12,288: 315 ops 93 / 106, 523 ops 89 / 185
-// and at one plan 13 to 26 where a lane needs 49 to 169 (13 to 20 us is what the host needs for a launch).
-constexpr int kSpreadMaxPlain = 3840, kSpreadMaxWindowed = 7680, kSpreadMaxSlow = 16384, kSpreadMaxRecords = 12288;
+//   PLAIN    the mid-sized kernel      4,096 / 4,608 plans: 315 ops 39 42 / 43, 523 ops 58 63 / 67, 821 ops 79 87 / 81,
+//                                      1,251 ops 106 116 / 109
+//   WINDOWED large, windowed rows      7,168 / 8,192 plans: 114 ops 36 40 / 42, 176 ops 57 64 / 55
+//   SLOW     no assembly loop (memory of collectives, more than 256 rows)   16,384 / 20,480 plans: 315 ops 145 179 / 163,
+//            523 ops 214 265 / 460, 114 ops 88 110 / 140
+//   RECORDS  stage records             12,288 / 16,384 plans: 315 ops 125 162 / 146, 523 ops 181 234 / 325, 134 ops 82 106 / 171;
+//            single-stage queries      315 ops 77 99 / 105, 523 ops 73 91 / 182
+// and at one plan 8 to 26 where a lane needs 49 to 169 (13 to 20 us is what the host needs for a launch).
+constexpr int kSpreadMaxPlain = 4096, kSpreadMaxWindowed = 7680, kSpreadMaxSlow = 18432, kSpreadMaxRecords = 14336;
 constexpr int kSpreadMaxOther = 4096;    // (deferred stage tails on the C++ form of the loop: tables that leave the assembly loop no room)
 
 // ------------------------------------------------------------------------------------------
@@ -1135,7 +1136,7 @@ static void launch_score_w(const ace_handle_t *h, const AceKernelArgs &a, hipStr
 template <bool BD, bool RANGED, bool COLL>
 static void launch_spread_c(const AceKernelArgs &a, hipStream_t s) {
     SpreadShared sh;
-    const uint32_t lds = ace_spread_layout(SpreadCols<BD, COLL>::kCols, a.g.G, (uint32_t)a.rk_bytes, nullptr, &sh);
+    const uint32_t lds = ace_spread_layout(SpreadCols<BD, COLL>::kCols, a.g.G, nullptr, &sh);
     hipLaunchKernelGGL((ace_spread_kernel<BD, RANGED, COLL>), dim3((unsigned)a.g.P), dim3(kSpreadLanes), lds, s, a);
 }
 template <bool BD, bool RANGED>

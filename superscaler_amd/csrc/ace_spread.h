@@ -22,7 +22,9 @@
 constexpr int kSpreadLanes = 256;
 constexpr int kSpreadPitch = kSpreadLanes + 2;      // doubles per column: columns start four banks apart
 constexpr int kSpreadMaxOps = 16 * kSpreadLanes;    // a lane holds one 16-op group's stage starts
-constexpr uint32_t kSpreadPairBytes = 8192;         // pair kinds up to this size are staged in LDS (else read where they are)
+// LDS is what limits how many plans are on their way in a CU, and a kernel that mostly waits gains from every one of them: the
+// table of pair kinds (up to 8 KB) is read where it is, and the per-group arrays are as long as the plan.  Six plans per CU
+// instead of four; 3,001 plans, us per launch: 315 ops 35.6 -> 30.1, 523 ops 51.4 -> 45.0, 1,223 ops 89.7 -> 81.1.
 
 // Columns: sums first, maxima after them.
 template <bool BD, bool COLL> struct SpreadCols {
@@ -44,11 +46,10 @@ struct SpreadShared {
     uint32_t *keep;         // [8] ops of the chunk that continue their segment, a bit each
     uint32_t *lut;          // [16] stage_lut of the plan's micro-batch size
     int32_t *bound;         // [18] first op of each stage, num_ops past the last
-    uint16_t *starts;       // [256] stage starts of each 16-op group, a bit each
-    uint16_t *count;        // [256] ... and their number
-    uint16_t *prefix;       // [256] stage starts before the group
+    uint16_t *starts;       // [G] stage starts of each 16-op group, a bit each
+    uint16_t *count;        // [G] ... and their number
+    uint16_t *prefix;       // [G] stage starts before the group
     int32_t *n_stages;
-    const uint8_t *pairs;   // pair kinds, in LDS or where they are
 };
 
 #ifdef ACE_HOST_EMU
@@ -56,7 +57,7 @@ inline
 #else
 __host__ __device__ __forceinline__
 #endif
-uint32_t ace_spread_layout(int cols, int G, uint32_t rk_bytes, unsigned char *lds, SpreadShared *s) {
+uint32_t ace_spread_layout(int cols, int G, unsigned char *lds, SpreadShared *s) {
     uint32_t o = 0;
     auto take = [&](uint32_t bytes) { const uint32_t at = o; o += (bytes + 15u) & ~15u; return lds + at; };
     s->x = reinterpret_cast<double *>(take((uint32_t)(cols * kSpreadPitch + 16) * 8u));
@@ -68,11 +69,10 @@ uint32_t ace_spread_layout(int cols, int G, uint32_t rk_bytes, unsigned char *ld
     s->keep = reinterpret_cast<uint32_t *>(take(32u));
     s->lut = reinterpret_cast<uint32_t *>(take(64u));
     s->bound = reinterpret_cast<int32_t *>(take(72u));
-    s->starts = reinterpret_cast<uint16_t *>(take(512u));
-    s->count = reinterpret_cast<uint16_t *>(take(512u));
-    s->prefix = reinterpret_cast<uint16_t *>(take(512u));
+    s->starts = reinterpret_cast<uint16_t *>(take(2u * (uint32_t)G));
+    s->count = reinterpret_cast<uint16_t *>(take(2u * (uint32_t)G));
+    s->prefix = reinterpret_cast<uint16_t *>(take(2u * (uint32_t)G));
     s->n_stages = reinterpret_cast<int32_t *>(take(4u));
-    s->pairs = take(rk_bytes <= kSpreadPairBytes ? rk_bytes : 0u);
     return o;
 }
 
@@ -148,8 +148,7 @@ template <bool RANGED> ACE_HD void spread_fetch(const AceKernelArgs &a, const Sp
         reinterpret_cast<ace_u4 *>(s.codes)[tid] = ace_u4{w[0], w[1], w[2], w[3]};
         s.starts[tid] = (uint16_t)bits;
         s.count[tid] = (uint16_t)__builtin_popcount(bits);
-    } else
-        s.count[tid] = 0;
+    }
     if (tid == 0) {
         reinterpret_cast<ace_u4 *>(s.codes)[g.G] = ace_u4{0u, 0u, 0u, 0u};
         s.carry[0] = 0.0;
@@ -158,9 +157,6 @@ template <bool RANGED> ACE_HD void spread_fetch(const AceKernelArgs &a, const Sp
     if (tid < 16) s.lut[tid] = a.stage_lut[p.bidx * 16u + (uint32_t)tid];
     if (tid < 8) s.keep[tid] = 0u;
     if (tid < 18) s.bound[tid] = g.N;
-    if ((uint32_t)a.rk_bytes <= kSpreadPairBytes)                    // (a multiple of 64 bytes)
-        for (int j = tid; j < (a.rk_bytes >> 2); j += kSpreadLanes)
-            reinterpret_cast<uint32_t *>(const_cast<uint8_t *>(s.pairs))[j] = reinterpret_cast<const uint32_t *>(a.pair_kinds)[j];
 }
 
 // ---- stages: where each stage begins -----------------------------------------------------------------------------------------
@@ -217,7 +213,7 @@ ACE_HD void spread_load(const AceKernelArgs &a, const SpreadShared &s, const Spr
     r.zf = r.zb = r.mf = r.mb = 0.0;
     if ((g.flags & ACE_F_RESHARDING) && !first) {           // (a stage's first op pays no resharding)
         const uint32_t gl = glog < (uint32_t)g.n_glog ? glog : 0u;
-        const uint32_t id = s.pairs[(prev & 0xffu) * g.rk_kind_stride + gl * 64u + (pbyte & 7u) * 8u + (byte & 7u)];
+        const uint32_t id = a.pair_kinds[(prev & 0xffu) * g.rk_kind_stride + gl * 64u + (pbyte & 7u) * 8u + (byte & 7u)];
         const unsigned char *z = row + g.z_off + e * 8u;
         const uint32_t fo = (id & 15u) << g.z_shift, bo = (id >> 4) << g.z_shift;
         r.zf = *reinterpret_cast<const double *>(z + fo);
@@ -429,8 +425,7 @@ template <bool BD, bool RANGED, bool COLL>
 ACE_HD void ace_spread_body(const AceKernelArgs &a, unsigned char *lds_raw, int tid_, long long plan) {
     typedef SpreadCols<BD, COLL> K;
     SpreadShared s;
-    ace_spread_layout(K::kCols, a.g.G, (uint32_t)a.rk_bytes, lds_raw, &s);
-    if ((uint32_t)a.rk_bytes > kSpreadPairBytes) s.pairs = a.pair_kinds;
+    ace_spread_layout(K::kCols, a.g.G, lds_raw, &s);
 #ifdef ACE_HOST_EMU
     static SpreadLane lane[kSpreadLanes];
     (void)tid_;

@@ -145,7 +145,7 @@ void run_lanes(const AceKernelArgs &a, unsigned char *lds, uint32_t lds_bytes) {
 template <bool BD, bool RANGED, bool COLL>
 void run_spread(const AceKernelArgs &a, GuardedPool &pool) {
     SpreadShared sh;
-    const uint32_t bytes = ace_spread_layout(SpreadCols<BD, COLL>::kCols, a.g.G, (uint32_t)a.rk_bytes, nullptr, &sh);
+    const uint32_t bytes = ace_spread_layout(SpreadCols<BD, COLL>::kCols, a.g.G, nullptr, &sh);
     unsigned char *lds = (unsigned char *)pool.place(nullptr, bytes);
     for (long long p = 0; p < a.g.P; ++p) {
         memset(lds, 0xff, bytes);

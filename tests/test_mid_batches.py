@@ -33,7 +33,7 @@ def test_committed_duo_loop_is_the_generators_output():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("name,mode,sizes", [("gpt3_13b", "plain", (3840, 3841, 16385)), ("t5_770m", "min", (8191,)), ("gpt3_175b", "noreserved", (4999,)),
+@pytest.mark.parametrize("name,mode,sizes", [("gpt3_13b", "plain", (3840, 4096, 4097, 16385)), ("t5_770m", "min", (8191,)), ("gpt3_175b", "noreserved", (4999,)),
                                              ("gpt3_1_3b", "min", (16384,)), ("gpt_wide_stages", "plain", (5000, 32768, 32769, 65537)),
                                              ("gpt_16ops", "noreserved", (65536,)), ("gpt_3tp", "min", (20001, 100001)),
                                              ("t5_1layer", "plain", (16383, 70000))])
