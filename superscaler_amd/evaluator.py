@@ -9,7 +9,7 @@ from typing import Optional
 
 import numpy as np
 
-from .plan import PlanBatch, check_shape, finding, validate_batch
+from .plan import PlanBatch, check_shape, finding, host_arrays, validate_batch
 from .tables import ABI_VERSION, MAX_STAGES, STAGE_REC, AceTablesStruct, CompiledTables
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libace_eval.so")
@@ -580,10 +580,10 @@ class PlanEvaluator:
         expanded, scored and the fastest feasible one picked: (plan, iteration ms, peak MB), or None.  `sets`: handles of
         the visited sets (empty: only repeated moves are dropped)."""
         t, best = self.tables, AceStepResultStruct()
-        row, hdr = np.ascontiguousarray(plan.codes[0]), np.ascontiguousarray(plan.hdr[0])
-        codes_out, hdr_out = np.empty((1, len(row)), dtype=np.uint8), np.empty((1, 4), dtype=np.uint32)
+        codes, hdr = host_arrays(plan.codes[:1], plan.hdr[:1], t.graph.num_ops)
+        codes_out, hdr_out = np.empty_like(codes), np.empty_like(hdr)
         handles = (ctypes.c_void_p * max(1, len(sets)))(*sets)
-        _check(self.lib, self.lib.ace_search_step(self.handle, row.ctypes.data, hdr.ctypes.data, t.stage_lut.ctypes.data,
+        _check(self.lib, self.lib.ace_search_step(self.handle, codes.ctypes.data, hdr.ctypes.data, t.stage_lut.ctypes.data,
                                                   t.settings.num_gpus_per_node, ctypes.byref(draws), handles, len(sets),
                                                   float(t.settings.memory_limit), 0, codes_out.ctypes.data, hdr_out.ctypes.data,
                                                   ctypes.byref(best), self._stream()), "ace_search_step")

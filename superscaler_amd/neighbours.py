@@ -14,7 +14,7 @@ from typing import Tuple
 import numpy as np
 
 from . import opgraph as og
-from .plan import PlanBatch
+from .plan import PlanBatch, host_arrays
 from .tables import CompiledTables
 
 
@@ -121,14 +121,14 @@ def _build_moves(base: PlanBatch, tables: CompiledTables, draws, sets=None) -> T
     N, M, n = tables.graph.num_ops, len(tables.db.mbs_list), draws["n"]
     if N >= 65536:
         raise ValueError("move descriptors hold 16-bit op positions")
-    S = int(base.hdr[0, 0] & 0xff)
+    codes, hdr = host_arrays(base.codes[:1], base.hdr[:1], N)
+    S = int(hdr[0, 0] & 0xff)
     cap = 3 + S * (S - 1)
     t_codes, t_hdr = np.empty((cap, N), dtype=np.uint8), np.empty((cap, 4), dtype=np.uint32)
     moves = np.empty((n, 4), dtype=np.uint32)
-    row, hdr = np.ascontiguousarray(base.codes[0]), np.ascontiguousarray(base.hdr[0])
     d = _draws_struct(draws)
     n_templates = ctypes.c_int(0)
-    plan = (row.ctypes.data, hdr.ctypes.data, N, tables.db.n_algo, len(tables.db.tp_list), M, tables.stage_lut.ctypes.data,
+    plan = (codes.ctypes.data, hdr.ctypes.data, N, tables.db.n_algo, len(tables.db.tp_list), M, tables.stage_lut.ctypes.data,
             tables.settings.num_gpus_per_node, ctypes.byref(d))
     dest = (t_codes.ctypes.data, t_hdr.ctypes.data, cap, ctypes.byref(n_templates))
     if sets is None:

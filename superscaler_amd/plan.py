@@ -261,6 +261,30 @@ class PlanBatch:
         return np.ascontiguousarray(padded.reshape(P, G, 16).transpose(1, 0, 2))
 
 
+_U8, _U32 = np.dtype(np.uint8), np.dtype(np.uint32)
+
+
+def host_arrays(codes, hdr, num_ops: Optional[int] = None):
+    """Code rows and headers of a host batch as native code reads them through raw pointers: uint8 [P, N] (N = `num_ops` if that
+    is given) and uint32 [P, 4], C-contiguous, the arrays themselves where they are that already.  Other integer types are converted
+    by value, one header row stands for all plans; anything else is refused (ValueError, TypeError)."""
+    if codes.ndim != 2 or hdr.ndim != 2 or hdr.shape[1] != 4 or hdr.shape[0] not in (1, codes.shape[0]):
+        raise ValueError(f"code rows [plans, ops] and headers [plans, 4] expected, not {codes.shape} and {hdr.shape}")
+    if num_ops is not None and codes.shape[1] != num_ops:
+        raise ValueError(f"batch has {codes.shape[1]} ops per plan, op graph {num_ops}")
+    if codes.dtype is not _U8 or not codes.flags.c_contiguous:
+        codes = _as_integers(codes, _U8)
+    if hdr.dtype is not _U32 or not hdr.flags.c_contiguous or len(hdr) != len(codes):
+        hdr = _as_integers(np.broadcast_to(hdr, (len(codes), 4)), _U32)
+    return codes, hdr
+
+
+def _as_integers(a, dtype):
+    if a.dtype.kind not in "iub":
+        raise TypeError(f"plans are arrays of integers, not {a.dtype}")
+    return np.ascontiguousarray(a, dtype=dtype)
+
+
 # what the structural check of a batch finds wrong (ace_check_plans / ace_pack_plans), in this order
 FINDINGS = ("num_stages outside 1..16", "stage-start bits disagree with num_stages", "op 0 must start a stage",
             "micro-batch index outside the profile database", "tp/algo code outside the profile database")

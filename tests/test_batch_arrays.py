@@ -1,0 +1,66 @@
+"""What a host batch's arrays may look like where native code reads them: other integer types and layouts are converted, one
+header row stands for all plans, and arrays that are too short (or too long) are refused before anything reads them."""
+import ctypes
+import types
+
+import numpy as np
+import pytest
+
+from superscaler_amd import synth
+from superscaler_amd.evaluator import PlanEvaluator
+from superscaler_amd.neighbours import _draw_moves, _draws_struct, sample_moves
+from superscaler_amd.plan import PlanBatch
+from tests.helpers import odd_workloads
+
+W = odd_workloads()[2]
+TYPES = [np.uint8, np.int8, np.int32, np.int64, np.uint64, ">i4"]
+
+
+def tables_and_plans(n):
+    tables = synth.make_tables(W)
+    return tables, synth.make_plans(W, tables, n_plans=n, seed_offset=3)
+
+
+def forms(batch):
+    """The same plans in other integer types and memory layouts."""
+    for t in TYPES:
+        yield PlanBatch(batch.codes.astype(t), batch.hdr.astype(np.int64 if t != np.uint64 else np.uint64))
+    yield PlanBatch(np.asfortranarray(batch.codes), np.asfortranarray(batch.hdr))
+    yield PlanBatch(np.repeat(batch.codes, 2, axis=1)[:, ::2], np.repeat(batch.hdr, 2, axis=0)[::2])
+
+
+def at(pointer, like):
+    """What stands at `pointer`, as an array like `like`."""
+    return np.frombuffer(ctypes.string_at(pointer, like.nbytes), dtype=like.dtype).reshape(like.shape)
+
+
+def test_moves_are_drawn_from_the_plans_values():
+    tables, batch = tables_and_plans(4)
+    for p in range(4):
+        base = batch.slice(p, p + 1)
+        want = sample_moves(base, tables, 400, np.random.default_rng(p))
+        for b in forms(base):
+            templates, moves = sample_moves(b, tables, 400, np.random.default_rng(p))
+            assert np.array_equal(moves, want[1]) and np.array_equal(templates.codes, want[0].codes) and np.array_equal(templates.hdr, want[0].hdr)
+    N = tables.graph.num_ops
+    for bad in (PlanBatch(base.codes[:, :N - 1], base.hdr), PlanBatch(base.codes, base.hdr[:, :3])):
+        with pytest.raises(ValueError):
+            sample_moves(bad, tables, 400, np.random.default_rng(0))
+    with pytest.raises(TypeError):
+        sample_moves(PlanBatch(base.codes.astype(float), base.hdr), tables, 400, np.random.default_rng(0))
+
+
+def test_a_search_step_reads_the_plans_values():
+    tables, batch = tables_and_plans(1)
+    seen = []
+
+    def ace_search_step(handle, row, hdr, *_):
+        seen.append((at(row, batch.codes[0]), at(hdr, batch.hdr[0])))
+        return 0
+    ev = types.SimpleNamespace(tables=tables, lib=types.SimpleNamespace(ace_search_step=ace_search_step), handle=None, _stream=lambda: None)
+    draws = _draws_struct(_draw_moves(10, int(batch.hdr[0, 0] & 0xff), tables, np.random.default_rng(0)))
+    for b in forms(batch):
+        PlanEvaluator.search_step(ev, b, draws)
+        assert np.array_equal(seen[-1][0], batch.codes[0]) and np.array_equal(seen[-1][1], batch.hdr[0])
+    with pytest.raises(ValueError):
+        PlanEvaluator.search_step(ev, PlanBatch(batch.codes[:, :-1], batch.hdr), draws)
