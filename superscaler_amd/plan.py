@@ -310,7 +310,7 @@ def validate_batch(batch: PlanBatch, tables: CompiledTables) -> Optional[str]:
     if msg:
         return msg
     from .evaluator import load_library
-    codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr)
+    codes, hdr = host_arrays(batch.codes, batch.hdr)
     return finding(load_library().ace_check_plans(codes.ctypes.data, hdr.ctypes.data, codes.shape[0], codes.shape[1],
                                                   len(tables.db.mbs_list), tables.C))
 

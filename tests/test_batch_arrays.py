@@ -6,10 +6,11 @@ import types
 import numpy as np
 import pytest
 
+from superscaler_amd import plan as plan_mod
 from superscaler_amd import synth
 from superscaler_amd.evaluator import PlanEvaluator
 from superscaler_amd.neighbours import _draw_moves, _draws_struct, sample_moves
-from superscaler_amd.plan import PlanBatch
+from superscaler_amd.plan import PlanBatch, validate_batch
 from tests.helpers import odd_workloads
 
 W = odd_workloads()[2]
@@ -64,3 +65,22 @@ def test_a_search_step_reads_the_plans_values():
         assert np.array_equal(seen[-1][0], batch.codes[0]) and np.array_equal(seen[-1][1], batch.hdr[0])
     with pytest.raises(ValueError):
         PlanEvaluator.search_step(ev, PlanBatch(batch.codes[:, :-1], batch.hdr), draws)
+
+
+def test_the_structural_check_wants_a_header_per_plan():
+    tables, batch = tables_and_plans(8)
+    for b in forms(batch):
+        assert validate_batch(b, tables) is None
+    for rows in (0, 4, 7, 9):
+        with pytest.raises(ValueError):
+            validate_batch(PlanBatch(batch.codes, np.resize(batch.hdr, (rows, 4))), tables)
+    for bad in (batch.hdr[:, :3], batch.hdr[:, 0], np.repeat(batch.hdr, 2, axis=1)):
+        with pytest.raises(ValueError):
+            validate_batch(PlanBatch(batch.codes, bad), tables)
+    with pytest.raises(TypeError):
+        validate_batch(PlanBatch(batch.codes.astype(float), batch.hdr), tables)
+    # one header for all of them: checked against every plan's stage starts
+    same = PlanBatch(np.repeat(batch.codes[:1], 8, axis=0), batch.hdr[:1])
+    assert validate_batch(same, tables) is None
+    same.codes[5, 1:] |= 16
+    assert validate_batch(same, tables) == plan_mod.FINDINGS[1]
