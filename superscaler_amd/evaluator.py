@@ -199,7 +199,7 @@ def depth_order(batch: PlanBatch) -> np.ndarray:
 def pack_small_inputs(buf: np.ndarray, batch: PlanBatch, ranges) -> int:
     """Lay a small batch out for the kernel in `buf` (uint8) as ace_score_host does: codes [ceil(N/16)][P][16] (zero padded),
     then the headers uint32 [P][4], then the ranges uint32 [P][2] if given.  Returns the number of bytes used."""
-    codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr, dtype=np.uint32)
+    codes, hdr = host_arrays(batch.codes, batch.hdr)
     rg = None if ranges is None else np.ascontiguousarray(ranges, dtype=np.uint32)
     P, N = codes.shape
     args = (codes.ctypes.data, hdr.ctypes.data, None if rg is None else rg.ctypes.data, P, N)
@@ -226,9 +226,9 @@ def rows_to_device(batch: PlanBatch, device, staging=None):
     pinned = getattr(batch, "pinned_tensors", None)
     if pinned is not None:
         return pinned[0].to(device, non_blocking=True), pinned[1].to(device, non_blocking=True)
-    host_rows = torch.from_numpy(np.ascontiguousarray(batch.codes)).view(-1)
-    host_hdr = torch.from_numpy(np.ascontiguousarray(batch.hdr).view(np.uint8)).view(-1)
-    P, N = batch.codes.shape
+    codes, hdr = host_arrays(batch.codes, batch.hdr)
+    host_rows, host_hdr = torch.from_numpy(codes).view(-1), torch.from_numpy(hdr.view(np.uint8)).view(-1)
+    P, N = codes.shape
     if torch.device(device).type != "cuda":
         return host_rows.view(P, N).to(device), host_hdr.view(torch.int32).view(P, 4).to(device)
     head, size = host_hdr.numel(), host_rows.numel()
@@ -698,7 +698,7 @@ class PlanEvaluator:
         P, N = batch.codes.shape
         breakdown = breakdown or ranges is not None
         n_rec = 1 if ranges is not None else MAX_STAGES          # a single-stage query has one record
-        codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr)
+        codes, hdr = host_arrays(batch.codes, batch.hdr)
         if ranges is not None:
             ranges = np.ascontiguousarray(ranges, dtype=np.uint32)
         times = np.empty((2, P))

@@ -8,7 +8,7 @@ import pytest
 
 from superscaler_amd import plan as plan_mod
 from superscaler_amd import synth
-from superscaler_amd.evaluator import PlanEvaluator
+from superscaler_amd.evaluator import PlanEvaluator, pack_small_inputs, rows_to_device
 from superscaler_amd.neighbours import _draw_moves, _draws_struct, sample_moves
 from superscaler_amd.plan import PlanBatch, validate_batch
 from tests.helpers import odd_workloads
@@ -84,3 +84,47 @@ def test_the_structural_check_wants_a_header_per_plan():
     assert validate_batch(same, tables) is None
     same.codes[5, 1:] |= 16
     assert validate_batch(same, tables) == plan_mod.FINDINGS[1]
+
+
+def fake_evaluator(tables, calls):
+    """A PlanEvaluator whose library only records what it is handed."""
+    import torch
+    ev = PlanEvaluator.__new__(PlanEvaluator)
+    ev.tables, ev.device, ev.handle, ev._torch = tables, torch.device("cuda", 0), None, types.SimpleNamespace(
+        _C=types.SimpleNamespace(_cuda_getCurrentRawStream=lambda device: device))
+
+    def ace_score_host(handle, codes, hdr, ranges, P, *_):
+        shape = (P, tables.graph.num_ops)
+        calls.append((at(codes, np.empty(shape, np.uint8)), at(hdr, np.empty((P, 4), np.uint32)),
+                      None if ranges is None else at(ranges, np.empty((P, 2), np.uint32)), _[-1]))
+        return 0
+    ev.lib = types.SimpleNamespace(ace_score_host=ace_score_host)
+    return ev
+
+
+def test_scores_are_asked_for_the_plans_values():
+    import torch
+    tables, batch = tables_and_plans(8)
+    P, N = batch.codes.shape
+    calls = []
+    ev = fake_evaluator(tables, calls)
+    ranges = np.tile(np.array([[0, N]], dtype=np.uint32), (P, 1))
+    want = np.zeros(1 << 16, dtype=np.uint8)
+    used = pack_small_inputs(want, batch, ranges)
+    one = PlanBatch(np.repeat(batch.codes[:1], P, axis=0), batch.hdr[:1])
+    for b in [*forms(batch), one]:
+        ref = batch if b is not one else PlanBatch(one.codes, np.repeat(one.hdr, P, axis=0))
+        for rg in (None, ranges):
+            ev.score_host(b, ranges=rg)
+            codes, hdr = calls[-1][:2]
+            assert np.array_equal(codes, ref.codes) and np.array_equal(hdr, ref.hdr)
+        rows, hdr = rows_to_device(b, "cpu")
+        assert rows.dtype == torch.uint8 and np.array_equal(rows.numpy(), ref.codes) and np.array_equal(hdr.numpy().view(np.uint32), ref.hdr)
+        if b is not one:
+            got = np.zeros_like(want)
+            assert pack_small_inputs(got, b, ranges) == used and np.array_equal(got, want)
+    for bad in (PlanBatch(batch.codes, batch.hdr[:4]), PlanBatch(batch.codes, batch.hdr[:, :3])):
+        for call in (lambda: ev.score_host(bad), lambda: ev.score_host(bad, ranges=ranges), lambda: rows_to_device(bad, "cpu"),
+                     lambda: pack_small_inputs(np.zeros_like(want), bad, None)):
+            with pytest.raises(ValueError):
+                call()
