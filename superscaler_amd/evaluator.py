@@ -196,12 +196,24 @@ def depth_order(batch: PlanBatch) -> np.ndarray:
     return perm[deal_slots(P)]
 
 
+def host_ranges(ranges, n_plans: int) -> np.ndarray:
+    """The op ranges of single-stage queries as native code reads them: uint32 [n_plans, 2], contiguous; one range stands for all
+    queries, other shapes are refused (ValueError)."""
+    if isinstance(ranges, np.ndarray) and ranges.dtype == np.uint32 and ranges.shape == (n_plans, 2) and ranges.flags.c_contiguous:
+        return ranges
+    out = np.empty((n_plans, 2), dtype=np.uint32)
+    out[...] = ranges
+    return out
+
+
 def pack_small_inputs(buf: np.ndarray, batch: PlanBatch, ranges) -> int:
     """Lay a small batch out for the kernel in `buf` (uint8) as ace_score_host does: codes [ceil(N/16)][P][16] (zero padded),
     then the headers uint32 [P][4], then the ranges uint32 [P][2] if given.  Returns the number of bytes used."""
     codes, hdr = host_arrays(batch.codes, batch.hdr)
-    rg = None if ranges is None else np.ascontiguousarray(ranges, dtype=np.uint32)
     P, N = codes.shape
+    rg = None if ranges is None else host_ranges(ranges, P)
+    if buf.dtype != np.uint8 or not (buf.flags.c_contiguous and buf.flags.writeable):
+        raise ValueError("a contiguous uint8 buffer expected")
     args = (codes.ctypes.data, hdr.ctypes.data, None if rg is None else rg.ctypes.data, P, N)
     lib = load_library()
     if lib.ace_pack_host(*args, None) > buf.nbytes:
@@ -700,7 +712,7 @@ class PlanEvaluator:
         n_rec = 1 if ranges is not None else MAX_STAGES          # a single-stage query has one record
         codes, hdr = host_arrays(batch.codes, batch.hdr)
         if ranges is not None:
-            ranges = np.ascontiguousarray(ranges, dtype=np.uint32)
+            ranges = host_ranges(ranges, P)
         times = np.empty((2, P))
         flags = np.empty((2, P), dtype=np.uint8)
         rec = np.empty((P, n_rec, STAGE_REC)) if breakdown else None

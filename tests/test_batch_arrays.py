@@ -128,3 +128,28 @@ def test_scores_are_asked_for_the_plans_values():
                      lambda: pack_small_inputs(np.zeros_like(want), bad, None)):
             with pytest.raises(ValueError):
                 call()
+
+
+def test_ranges_stand_for_every_query():
+    tables, batch = tables_and_plans(8)
+    P, N = batch.codes.shape
+    calls = []
+    ev = fake_evaluator(tables, calls)
+    per_query = np.stack([np.arange(P), np.arange(P) + 2], axis=1)
+    for rg, want in ((per_query, per_query), (per_query.astype(np.uint32), per_query), (np.asfortranarray(per_query), per_query),
+                     (per_query.tolist(), per_query), ((3, 5), np.tile([[3, 5]], (P, 1))), (np.array([[3, 5]]), np.tile([[3, 5]], (P, 1)))):
+        ev.score_host(batch, ranges=rg)
+        assert np.array_equal(calls[-1][2], want)
+        buf = np.zeros(1 << 16, dtype=np.uint8)
+        used = pack_small_inputs(buf, batch, rg)
+        assert np.array_equal(buf[used - 8 * P:used].view(np.uint32).reshape(P, 2), want)
+    for buf in (np.zeros(1 << 16, dtype=np.int8), np.zeros(1 << 17, dtype=np.uint8)[::2], np.frombuffer(bytes(1 << 16), dtype=np.uint8)):
+        with pytest.raises(ValueError):
+            pack_small_inputs(buf, batch, per_query)
+    made = len(calls)
+    for rg in (per_query[:4], per_query[:0], np.zeros((P, 3)), np.zeros(P), np.zeros((P, 1, 2))):
+        with pytest.raises(ValueError):
+            ev.score_host(batch, ranges=rg)
+        with pytest.raises(ValueError):
+            pack_small_inputs(np.zeros(1 << 16, dtype=np.uint8), batch, rg)
+    assert len(calls) == made
