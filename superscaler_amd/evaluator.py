@@ -382,7 +382,9 @@ class PlanEvaluator:
         """`validate` checks the encoding on the host first (a clear message instead of per-plan status
         bytes; the kernel itself is safe for any byte content).  `group_by_depth`, `findings`: see DeviceBatch."""
         check = None
-        if validate and ranges is None:
+        if validate and ranges is not None:
+            host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)       # (a query's plan need not be a whole one)
+        elif validate:
             # (small batches are checked before they go anywhere; for others the check rides on the device's packing of the
             # plans and costs the read-back of its findings)
             small = batch.codes.size <= self.HOST_CHECK_BYTES
@@ -710,7 +712,7 @@ class PlanEvaluator:
         P, N = batch.codes.shape
         breakdown = breakdown or ranges is not None
         n_rec = 1 if ranges is not None else MAX_STAGES          # a single-stage query has one record
-        codes, hdr = host_arrays(batch.codes, batch.hdr)
+        codes, hdr = host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)
         if ranges is not None:
             ranges = host_ranges(ranges, P)
         times = np.empty((2, P))

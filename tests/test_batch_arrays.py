@@ -153,3 +153,17 @@ def test_ranges_stand_for_every_query():
         with pytest.raises(ValueError):
             pack_small_inputs(np.zeros(1 << 16, dtype=np.uint8), batch, rg)
     assert len(calls) == made
+
+
+def test_queries_have_the_graphs_ops():
+    tables, batch = tables_and_plans(8)
+    calls = []
+    ev = fake_evaluator(tables, calls)
+    ranges = np.tile([[0, 1]], (8, 1))
+    for bad in (PlanBatch(batch.codes[:, :-1], batch.hdr), PlanBatch(np.repeat(batch.codes, 2, axis=1), batch.hdr)):
+        for kw in ({}, {"ranges": ranges}, {"ranges": ranges, "group_by_depth": True}):
+            with pytest.raises(ValueError, match="ops per plan"):
+                ev.score_host(bad, **kw)
+        with pytest.raises(ValueError, match="ops per plan"):
+            ev.upload(bad, ranges=ranges)
+    assert not calls
