@@ -233,7 +233,7 @@ STAGING_SLOTS = 3
 def rows_to_device(batch: PlanBatch, device, staging=None):
     """The code rows (uint8 [P, N]) and headers (int32 [P, 4]) of a host batch on the device, in the host's layout.  Plans in
     page-locked memory (PlanEvaluator.pinned_plan_batch) are read where they are, by copies that may still be under way;
-    others are staged in page-locked memory (`staging`: see DeviceBatch), and may be rewritten after the call."""
+    others are staged in page-locked memory and may be rewritten after the call (`staging`: the memory to use, see DeviceBatch)."""
     import torch
     pinned = getattr(batch, "pinned_tensors", None)
     if pinned is not None:
@@ -244,9 +244,15 @@ def rows_to_device(batch: PlanBatch, device, staging=None):
     if torch.device(device).type != "cuda":
         return host_rows.view(P, N).to(device), host_hdr.view(torch.int32).view(P, 4).to(device)
     head, size = host_hdr.numel(), host_rows.numel()
+    if staging is not None:
+        # (the caller's buffer, whatever its size: nothing waits for the device)
+        stage, stage_hdr = staging[:size].view(P, N), torch.empty((P, 4), dtype=torch.int32, pin_memory=True)
+        stage.copy_(host_rows.view(P, N))
+        stage_hdr.copy_(host_hdr.view(torch.int32).view(P, 4))
+        return stage.to(device, non_blocking=True), stage_hdr.to(device, non_blocking=True)
     if head + size <= STAGING_PIECE:
         # (one transfer for both)
-        stage = torch.empty(head + size, dtype=torch.uint8, pin_memory=True) if staging is None else staging[:head + size]
+        stage = torch.empty(head + size, dtype=torch.uint8, pin_memory=True)
         stage[:head].copy_(host_hdr)
         stage[head:].copy_(host_rows)
         both = stage.to(device, non_blocking=True)
@@ -301,7 +307,7 @@ class DeviceBatch:
 
     def __init__(self, batch: PlanBatch, device="cuda:0", ranges: Optional[np.ndarray] = None, staging=None,
                  group_by_depth: bool = False, check=None, findings=None):
-        """`staging`: a pinned uint8 host tensor of at least P * N + 16 * P bytes; the plans then go through
+        """`staging`: a pinned uint8 host tensor of at least P * N bytes; the plan bytes then go through
         it and the copy to the device does not block the host (the caller must not reuse the tensor
         before that copy has completed).
         `group_by_depth`: store the plans sorted by pipeline depth (deepest first) and position of the
@@ -386,8 +392,9 @@ class PlanEvaluator:
             host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)       # (a query's plan need not be a whole one)
         elif validate:
             # (small batches are checked before they go anywhere; for others the check rides on the device's packing of the
-            # plans and costs the read-back of its findings)
-            small = batch.codes.size <= self.HOST_CHECK_BYTES
+            # plans and costs the read-back of its findings; not where the call must not wait for the device)
+            small = batch.codes.size <= self.HOST_CHECK_BYTES or (findings is None and (
+                staging is not None or self._torch.cuda.is_current_stream_capturing()))
             msg = validate_batch(batch, self.tables) if small else check_shape(batch, self.tables)
             if msg:
                 raise ValueError(msg)
