@@ -359,7 +359,10 @@ class PlanEvaluator:
             raise AceError("no GPU visible: plan scoring runs on the HIP kernels only")
         self.lib = load_library()
         self.tables = tables
+        # (a device without an index: the one that is current now, where the handle comes to live)
         self.device = torch.device(device)
+        if self.device.index is None:
+            self.device = torch.device(self.device.type, torch.cuda.current_device())
         self._torch = torch
         with torch.cuda.device(self.device):
             ts = tables.as_struct()
@@ -727,7 +730,7 @@ class PlanEvaluator:
         rec = np.empty((P, n_rec, STAGE_REC)) if breakdown else None
         rc = self.lib.ace_score_host(self.handle, codes.ctypes.data, hdr.ctypes.data, ranges.ctypes.data if ranges is not None else None, P,
                                      limit, int(strict), times.ctypes.data, flags.ctypes.data, rec.ctypes.data if breakdown else None,
-                                     self._torch._C._cuda_getCurrentRawStream(self.device.index or 0))
+                                     self._torch._C._cuda_getCurrentRawStream(self.device.index))
         if rc == ACE_ETOOBIG:
             return None
         _check(self.lib, rc, "ace_score_host")

@@ -1,5 +1,6 @@
 """What a host batch's arrays may look like where native code reads them: other integer types and layouts are converted, one
 header row stands for all plans, and arrays that are too short (or too long) are refused before anything reads them."""
+import contextlib
 import ctypes
 import types
 
@@ -167,3 +168,25 @@ def test_queries_have_the_graphs_ops():
         with pytest.raises(ValueError, match="ops per plan"):
             ev.upload(bad, ranges=ranges)
     assert not calls
+
+
+def test_a_device_without_an_index_is_the_one_that_was_current(monkeypatch):
+    """The library's handle lives on that one: its stream is the one a call must be ordered on, whatever is current later."""
+    import torch
+    from superscaler_amd import evaluator
+    tables, batch = tables_and_plans(2)
+    calls = []
+    made = types.SimpleNamespace(ace_create=lambda tables, handle: 0, ace_check_plans=evaluator.load_library().ace_check_plans,
+                                 ace_score_host=fake_evaluator(tables, calls).lib.ace_score_host)
+    current = [3]
+    monkeypatch.setattr(evaluator, "load_library", lambda: made)
+    monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: current[0])
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda index: 1000 + index, raising=False)
+    ev = {d: PlanEvaluator(tables, d) for d in ("cuda", "cuda:1", 2, torch.device("cuda"))}
+    current[0] = 0
+    for d, index in (("cuda", 3), ("cuda:1", 1), (2, 2), (torch.device("cuda"), 3)):
+        assert ev[d].device == torch.device("cuda", index)
+        ev[d].score_host(batch)
+        assert calls[-1][3] == 1000 + index
