@@ -84,3 +84,63 @@ def test_a_list_of_plans_is_filled_like_each_of_them():
     cm._fill_all(all_, rec)
     assert one == all_ and all(c.time_list for c in all_)
     cm._fill_all([], rec[:0])
+
+
+class Changing:
+    """A plan object (or stage) whose attribute `when` runs `what` each time it is read; `log` gets every read, and "gone" when the
+    object is."""
+
+    def __init__(self, of, when, what, log):
+        self.__dict__["_in"] = (dict(vars(of)), when, what, log)
+
+    def __getattr__(self, name):
+        attributes, when, what, log = self.__dict__["_in"]
+        log.append(name)
+        if name == when:
+            what()
+        return attributes[name]
+
+    def __setattr__(self, name, value):
+        self.__dict__["_in"][3].append(name)
+
+    def __del__(self):
+        self.__dict__["_in"][3].append("gone")
+
+
+READ_OF_STAGE = {"encode": ["ops", "tp_size", "dp_size", "algo", "recompute_ops"], "fill": ["num_gpus", "num_stages_behind", "recompute_ops"]}
+
+
+@pytest.mark.parametrize("call", ["encode", "fill"])
+@pytest.mark.parametrize("when", [0, 1, 2])
+def test_objects_that_attribute_reads_drop_are_held(call, when):
+    w = odd_workloads()[2]
+    cm = cost_model(w)
+    t, s = cm.tables, cm.settings
+    batch = synth.make_plans(w, t, n_plans=40, seed_offset=4)
+    rec = emu_score(t, batch, breakdown=True)[4]
+    codes, hdr = np.empty((2, t.graph.num_ops), dtype=np.uint8), np.empty((2, 4), dtype=np.uint32)
+
+    def run(configs):
+        if call == "encode":
+            return load_objects().encode(configs, 0, t.graph.num_ops, t.db.n_algo, s.num_gpus_per_node, False, *t.encode_luts, codes, hdr)
+        return load_objects().fill_all(configs, rec[:2], 0, s.memory_limit, s.memory_main_params, s.memory_optimizer, True)
+    p = next(p for p in range(40) if (batch.hdr[p, 0] & 0xff) > 2)
+    # a stage that its own list drops: every attribute is read before it is gone, and the plan is left (its stages are others now)
+    c, log = batch.to_config(p, t), []
+    stages = c.stages
+    read = READ_OF_STAGE[call]
+    stages[0] = Changing(stages[0], read[when], stages.clear, log)
+    assert run([c]) == 0
+    assert log == read + ["gone"]
+    # ... its last stage: nothing is left to refuse
+    c, log = batch.to_config(p, t), []
+    stages = c.stages
+    stages[-1] = Changing(stages[-1], read[when], stages.clear, log)
+    assert run([c]) == 1
+    assert log == read + ["gone"]
+    # a plan that the list of plans drops, and the plans behind it
+    name = ["num_stages", "micro_bs", "stages"][when]
+    log, configs = [], []
+    configs[:] = [Changing(batch.to_config(p, t), name, configs.clear, log), batch.to_config(p, t)]
+    assert run(configs) == 1
+    assert log[-1] == "gone" and log.count("gone") == 1 and len(log) > 3
