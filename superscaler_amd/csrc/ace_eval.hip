@@ -19,6 +19,7 @@
 #include <vector>
 
 #include "ace_edit_kernels.h"
+#include "ace_grid.h"
 #include "ace_keyset.h"
 #include "ace_pack.h"
 #include "ace_moves_host.h"
@@ -92,9 +93,9 @@ template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(cons
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_many_body<WIN>(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
-template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a) {
+template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a, const long long first) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, first + (long long)blockIdx.x);
 }
 
 // Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has six workgroups
@@ -663,8 +664,8 @@ __global__ void step_out_kernel(const long long *idx, const double *val, const i
 // The bodies of these kernels live in ace_edit_kernels.h (shared with the host build of the tests).
 __global__ __launch_bounds__(256) void apply_moves_kernel(const ace_u4 *tmpl_codes, const ace_u4 *tmpl_hdr, int n_templates,
                                                           const ace_u4 *moves, unsigned long long n, int G, int a_shift,
-                                                          ace_u4 *codes_out, ace_u4 *hdr_out, unsigned long long *key_out) {
-    apply_moves_body((unsigned long long)blockIdx.x * 256 + threadIdx.x, tmpl_codes, tmpl_hdr, n_templates, moves, n, G, a_shift,
+                                                          ace_u4 *codes_out, ace_u4 *hdr_out, unsigned long long *key_out, unsigned long long first) {
+    apply_moves_body((first + blockIdx.x) * 256 + threadIdx.x, tmpl_codes, tmpl_hdr, n_templates, moves, n, G, a_shift,
                      codes_out, hdr_out, key_out);
 }
 
@@ -674,18 +675,18 @@ __global__ __launch_bounds__(256) void group_keys_kernel(const ace_u4 *codes, co
 }
 
 __global__ __launch_bounds__(256) void gather_plans_kernel(const ace_u4 *codes_in, const ace_u4 *hdr_in, const uint32_t *perm,
-                                                           unsigned long long n, int G, ace_u4 *codes_out, ace_u4 *hdr_out) {
-    gather_plans_body((unsigned long long)blockIdx.x * 256 + threadIdx.x, codes_in, hdr_in, perm, n, G, codes_out, hdr_out);
+                                                           unsigned long long n, int G, ace_u4 *codes_out, ace_u4 *hdr_out, unsigned long long first) {
+    gather_plans_body((first + blockIdx.x) * 256 + threadIdx.x, codes_in, hdr_in, perm, n, G, codes_out, hdr_out);
 }
 
-__global__ __launch_bounds__(kPackLanes) void pack_plans_kernel(const PackArgs a) {
+__global__ __launch_bounds__(kPackLanes) void pack_plans_kernel(const PackArgs a, const long long first) {
     __shared__ PackShared s;
-    ace_pack_body(a, s, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_pack_body(a, s, (int)threadIdx.x, first + (long long)blockIdx.x);
 }
 
-__global__ __launch_bounds__(kPackLanes) void unpack_plans_kernel(const PackArgs a) {
+__global__ __launch_bounds__(kPackLanes) void unpack_plans_kernel(const PackArgs a, const long long first) {
     __shared__ PackShared s;
-    ace_unpack_body(a, s, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_unpack_body(a, s, (int)threadIdx.x, first + (long long)blockIdx.x);
 }
 
 __global__ void rc_groups_kernel(RcTables t, int n, const int32_t *q_plan, const int32_t *q_lo, const int32_t *q_hi,
@@ -1417,11 +1418,13 @@ int ace_apply_moves(const uint8_t *d_template_codes, const uint32_t *d_template_
     const unsigned long long total = (unsigned long long)n_moves * (unsigned long long)G;
     const unsigned long long blocks = (total + 255) / 256;
     if (blocks > 0x7fffffffull) return ACE_ETOOBIG;
-    hipLaunchKernelGGL(apply_moves_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
-                       reinterpret_cast<const ace_u4 *>(d_template_codes), reinterpret_cast<const ace_u4 *>(d_template_hdr),
-                       n_templates, reinterpret_cast<const ace_u4 *>(d_moves), (unsigned long long)n_moves, G,
-                       n_algo == 2 ? 1 : 0, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<ace_u4 *>(d_hdr_out),
-                       reinterpret_cast<unsigned long long *>(d_keys_out));
+    ace_grid_parts(blocks, 256, [&](uint64_t first, uint32_t groups) {
+        hipLaunchKernelGGL(apply_moves_kernel, dim3(groups), dim3(256), 0, (hipStream_t)stream,
+                           reinterpret_cast<const ace_u4 *>(d_template_codes), reinterpret_cast<const ace_u4 *>(d_template_hdr),
+                           n_templates, reinterpret_cast<const ace_u4 *>(d_moves), (unsigned long long)n_moves, G,
+                           n_algo == 2 ? 1 : 0, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<ace_u4 *>(d_hdr_out),
+                           reinterpret_cast<unsigned long long *>(d_keys_out), (unsigned long long)first);
+    });
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1448,9 +1451,12 @@ int ace_gather_plans(const uint8_t *d_codes_in, const uint32_t *d_hdr_in, const 
     const int G = (num_ops + 15) / 16;
     const unsigned long long blocks = ((unsigned long long)n_plans * G + 255) / 256;
     if (blocks > 0x7fffffffull) return ACE_ETOOBIG;
-    hipLaunchKernelGGL(gather_plans_kernel, dim3((unsigned)blocks), dim3(256), 0, (hipStream_t)stream,
-                       reinterpret_cast<const ace_u4 *>(d_codes_in), reinterpret_cast<const ace_u4 *>(d_hdr_in), d_perm,
-                       (unsigned long long)n_plans, G, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<ace_u4 *>(d_hdr_out));
+    ace_grid_parts(blocks, 256, [&](uint64_t first, uint32_t groups) {
+        hipLaunchKernelGGL(gather_plans_kernel, dim3(groups), dim3(256), 0, (hipStream_t)stream,
+                           reinterpret_cast<const ace_u4 *>(d_codes_in), reinterpret_cast<const ace_u4 *>(d_hdr_in), d_perm,
+                           (unsigned long long)n_plans, G, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<ace_u4 *>(d_hdr_out),
+                           (unsigned long long)first);
+    });
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1462,7 +1468,9 @@ int ace_pack_plans(const uint8_t *d_rows, size_t n_plans, int num_ops, const uin
         return ACE_EINVAL;
     PackArgs a{d_rows, nullptr, nullptr, reinterpret_cast<ace_u4 *>(d_codes_out), reinterpret_cast<const ace_u4 *>(d_hdr), d_flags,
                (long long)n_plans, num_ops, (num_ops + 15) / 16, n_mbs, n_codes};
-    hipLaunchKernelGGL(pack_plans_kernel, dim3((unsigned)((n_plans + kPackPlans - 1) / kPackPlans)), dim3(kPackLanes), 0, (hipStream_t)stream, a);
+    ace_grid_parts((n_plans + kPackPlans - 1) / kPackPlans, kPackLanes, [&](uint64_t first, uint32_t groups) {
+        hipLaunchKernelGGL(pack_plans_kernel, dim3(groups), dim3(kPackLanes), 0, (hipStream_t)stream, a, (long long)first);
+    });
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1473,7 +1481,9 @@ int ace_unpack_plans(const uint8_t *d_codes, size_t n_plans, int num_ops, uint8_
         return ACE_EINVAL;
     PackArgs a{nullptr, d_rows_out, reinterpret_cast<const ace_u4 *>(d_codes), nullptr, nullptr, nullptr, (long long)n_plans, num_ops,
                (num_ops + 15) / 16, 0, 8};
-    hipLaunchKernelGGL(unpack_plans_kernel, dim3((unsigned)((n_plans + kPackPlans - 1) / kPackPlans)), dim3(kPackLanes), 0, (hipStream_t)stream, a);
+    ace_grid_parts((n_plans + kPackPlans - 1) / kPackPlans, kPackLanes, [&](uint64_t first, uint32_t groups) {
+        hipLaunchKernelGGL(unpack_plans_kernel, dim3(groups), dim3(kPackLanes), 0, (hipStream_t)stream, a, (long long)first);
+    });
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1558,10 +1568,10 @@ int ace_recompute_batch(ace_handle_t *h, const ace_batch_t *batch, double memory
     a.peak_backward = peak_backward;
     RcShared s;
     const uint32_t lds = ace_rc_layout(a.k.g.N, a.k.g.G, nullptr, &s);
-    if (a.k.g.flags & ACE_F_COLLECTIVE_MEM)
-        hipLaunchKernelGGL((ace_rc_kernel<true>), dim3((unsigned)a.k.g.P), dim3(kSpreadLanes), lds, (hipStream_t)stream, a);
-    else
-        hipLaunchKernelGGL((ace_rc_kernel<false>), dim3((unsigned)a.k.g.P), dim3(kSpreadLanes), lds, (hipStream_t)stream, a);
+    const auto kernel = a.k.g.flags & ACE_F_COLLECTIVE_MEM ? ace_rc_kernel<true> : ace_rc_kernel<false>;
+    ace_grid_parts((uint64_t)a.k.g.P, kSpreadLanes, [&](uint64_t first, uint32_t groups) {
+        hipLaunchKernelGGL(kernel, dim3(groups), dim3(kSpreadLanes), lds, (hipStream_t)stream, a, (long long)first);
+    });
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }

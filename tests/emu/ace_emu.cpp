@@ -5,6 +5,7 @@
 // library never links or loads this file.
 #define ACE_HOST_EMU 1
 #include "ace_edit_kernels.h"
+#include "ace_grid.h"
 #include "ace_score_loop.h"
 #include "ace_spread.h"
 #include "ace_recompute.h"
@@ -473,4 +474,14 @@ extern "C" int ace_emu_unpack(const uint8_t *codes, long long P, int N, uint8_t 
     }
     memcpy(rows_out, a.rows_out, (size_t)P * N);
     return 0;
+}
+
+// The parts of a grid (ace_grid.h): up to `room` pairs (first workgroup, workgroups) in `out`; returns their number.
+extern "C" int ace_emu_grid_parts(unsigned long long groups, unsigned lanes, unsigned long long *out, int room) {
+    int n = 0;
+    ace_grid_parts(groups, lanes, [&](uint64_t first, uint32_t count) {
+        if (n < room) { out[2 * n] = first; out[2 * n + 1] = count; }
+        ++n;
+    });
+    return n;
 }
