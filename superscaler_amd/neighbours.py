@@ -8,6 +8,7 @@ scored by one kernel launch.  The search policy of the reference (aceso_policy.p
 reproduced: `hill_climb` is a plain best-neighbour descent used to exercise the batched path.
 """
 import ctypes
+import threading
 from concurrent.futures import ThreadPoolExecutor
 from typing import Tuple
 
@@ -419,6 +420,11 @@ class _KeySet:
     def take(self, other: "_KeySet") -> None:
         self._check(self._lib, self._lib.ace_keyset_move(self.handle, other.handle), "ace_keyset_move")
 
+    def copy(self) -> "_KeySet":
+        other = _KeySet()
+        other.add(self.keys())
+        return other
+
     def __getstate__(self):
         return self.keys()
 
@@ -451,34 +457,58 @@ class VisitedKeys:
     def __init__(self):
         self._large = _KeySet()
         self._small = _KeySet()
+        # (library calls run without the interpreter's lock, and the native sets are for one thread at a time)
+        self._lock = threading.RLock()
+
+    def __getstate__(self):
+        state = {k: v for k, v in self.__dict__.items() if k != "_lock"}
+        with self._lock:
+            state.update(_large=self._large.copy(), _small=self._small.copy())
+        return state
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._lock = threading.RLock()
 
     def __len__(self):
-        return len(self._large) + len(self._small)
+        with self._lock:
+            return len(self._large) + len(self._small)
 
     def unseen(self, keys: np.ndarray) -> np.ndarray:
         """Mask of the keys not marked before that do not repeat an earlier entry of `keys`."""
-        return _first_of_each(as_key128(keys), (self._small, self._large))
+        with self._lock:
+            return _first_of_each(as_key128(keys), (self._small, self._large))
 
     def claim(self, keys: np.ndarray) -> np.ndarray:
         """unseen(), and those keys marked."""
-        # (only what the large set lacks goes to the small one: the two stay disjoint, __len__ is their sum)
-        mask = _first_of_each(as_key128(keys), (self._small, self._large), claim=True)
-        self.fold()
-        return mask
+        with self._lock:
+            # (only what the large set lacks goes to the small one: the two stay disjoint, __len__ is their sum)
+            mask = _first_of_each(as_key128(keys), (self._small, self._large), claim=True)
+            self.fold()
+            return mask
 
     def claim_moves(self, base: PlanBatch, tables: CompiledTables, draws) -> Tuple[PlanBatch, np.ndarray]:
         """_build_moves, of the moves those whose plan is unseen, and these marked."""
-        made = _build_moves(base, tables, draws, [self._small, self._large])
-        self.fold()
-        return made
+        with self._lock:
+            made = _build_moves(base, tables, draws, [self._small, self._large])
+            self.fold()
+            return made
+
+    def search_step(self, ev, plan: PlanBatch, draws):
+        """PlanEvaluator.search_step among the neighbours that are unseen, and these marked."""
+        with self._lock:
+            best = ev.search_step(plan, draws, self.handles())
+            self.fold()
+            return best
 
     def handles(self):
         """The native sets for the library's calls that look keys up in both and add to the small one (then call fold())."""
         return [self._small.handle, self._large.handle]
 
     def fold(self) -> None:
-        if len(self._small) > self.SMALL_LIMIT:
-            self._large.take(self._small)
+        with self._lock:
+            if len(self._small) > self.SMALL_LIMIT:
+                self._large.take(self._small)
 
     def mark(self, keys: np.ndarray) -> None:
         self.claim(keys)
@@ -541,9 +571,7 @@ def hill_climb(cm, start: PlanBatch, steps: int, n_neighbours: int, seed: int = 
                 # (without a visited set equal descriptors are equal plans: one of each is kept.  First occurrences, in the order
                 # they were drawn: among neighbours of equal time the earliest wins, as it does when the duplicates are scored too)
                 if not greedy_recompute:
-                    best = ev.search_step(cur, draws, () if visited is None else visited.handles())
-                    if visited is not None:
-                        visited.fold()
+                    best = ev.search_step(cur, draws) if visited is None else visited.search_step(ev, cur, draws)
                 else:
                     templates, moves = _build_moves(cur, tables, draws, []) if visited is None else visited.claim_moves(cur, tables, draws)
                     best = _best_recomputed(cm, ev.apply_moves(templates, moves), cur_t) if len(moves) else None

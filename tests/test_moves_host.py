@@ -109,6 +109,35 @@ def test_key_set_behaves_like_a_set(limit):
     assert vk.unseen(np.zeros((0, 2), dtype=np.uint64)).tolist() == []
 
 
+def test_threads_may_share_a_visited_set():
+    """Every key is claimed once, whichever thread comes first (and copies are whole)."""
+    import copy
+    from concurrent.futures import ThreadPoolExecutor
+    w = WORKLOADS["gpt_wide_stages"]
+    tables = synth.make_tables(w)
+    base = synth.make_plans(w, tables, n_plans=1, seed_offset=50)
+    vk = VisitedKeys()
+    vk.SMALL_LIMIT = 3000
+
+    def work(seed):
+        rng = np.random.default_rng(seed)
+        mine = []
+        for step in range(15):
+            keys = rng.integers(0, 60_000, size=(4000, 1), dtype=np.uint64).repeat(2, axis=1)
+            vk.unseen(keys)
+            mine.append(keys[vk.claim(keys)])
+            draws = _draw_moves(2000, int(base.hdr[0, 0] & 0xff), tables, rng, 8)
+            templates, moves = vk.claim_moves(base, tables, draws)
+            mine.append(plan_keys_host(apply_moves_host(templates, moves, tables.db.n_algo)))
+            if step % 5 == 0:
+                copied = copy.deepcopy(vk)
+                assert not copied.unseen(mine[0]).any() and len(copied) <= len(vk)
+        return np.concatenate(mine)
+    with ThreadPoolExecutor(8) as pool:
+        claimed = np.concatenate(list(pool.map(work, range(8))))
+    assert len(np.unique(claimed, axis=0)) == len(claimed) == len(vk)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", ["gpt3_1_3b", "t5_770m", "wresnet_1b", "gpt_wide_stages"])
 def test_a_step_picks_what_its_parts_pick(name):
