@@ -264,7 +264,7 @@ int ace_new_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_
 
 /* One step of a search over single-move neighbours in one call: ace_new_moves, the new plans expanded on the handle's device
  * (ace_apply_moves), scored (ace_score_batch) and the fastest feasible one picked (ace_topk).  HOST memory in and out; the
- * handle keeps the buffers, and no other call on it may run meanwhile.  codes_out / hdr_out: the picked plan, if found. */
+ * handle keeps the buffers, and calls of several threads take turns.  codes_out / hdr_out: the picked plan, if found. */
 typedef struct ace_step_result {
     size_t n_moves;         /* neighbours scored */
     int32_t found;          /* one of them is feasible */

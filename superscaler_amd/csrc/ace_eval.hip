@@ -647,6 +647,9 @@ struct ace_handle {
     double *d_stage_ws;        // grow-only workspace for deferred stage tails
     size_t stage_ws_plans;     // capacity in plans
     int stage_ws_fixed;        // ace_reserve(..., fixed): a larger batch is an error instead of a reallocation
+    std::mutex host_calls;     // held by ace_score_host and ace_search_step from their first to their last use of host_in, host_out and
+                               // step: the next call, of another thread, must find the transfers of the one before ended
+    std::mutex workspace;      // held from the look at d_stage_ws to the launch that uses it: another thread's larger batch replaces it
 };
 
 struct StepOut { long long idx; double iter_ms, peak_mb; int32_t count; };
@@ -1009,9 +1012,8 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         if ((t->pair_kinds[j] & 15u) >= lim || (uint32_t)(t->pair_kinds[j] >> 4) >= lim) return ACE_EINVAL;
     }
 
-    ace_handle *h = new (std::nothrow) ace_handle();
+    ace_handle *h = new (std::nothrow) ace_handle();       // (all zeros)
     if (!h) return ACE_ENOMEM;
-    memset(h, 0, sizeof(*h));
     AceGeom &g = h->geom;
     g.N = t->num_ops; g.P = 0; g.G = (t->num_ops + 15) / 16;
     g.C = C; g.A_shift = t->n_algo == 2 ? 1 : 0;
@@ -1224,6 +1226,7 @@ extern "C" {
 
 int ace_reserve(ace_handle_t *h, size_t max_plans, int fixed) {
     if (!h || max_plans > 0x7fffffffull) return ACE_EINVAL;
+    std::lock_guard<std::mutex> lock(h->workspace);
     if (max_plans) {
         AceKernelArgs a;
         memset(&a, 0, sizeof(a));
@@ -1243,6 +1246,7 @@ int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_lim
     AceKernelArgs a;
     int rc = fill_args(h, batch, memory_limit, strict, d_iter_ms, d_peak_mb, d_feasible, d_status, d_stage_out, &a);
     if (rc) return rc;
+    std::lock_guard<std::mutex> lock(h->workspace);
     if ((rc = ensure_stage_ws(h, &a))) return rc;
     launch_score(h, a, (hipStream_t)stream);
     ACE_HIP(hipGetLastError());
@@ -1274,6 +1278,7 @@ int ace_score_host(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, c
     const size_t off_hdr = G * P * 16, off_rng = off_hdr + P * 16, n_in = ace_pack_host(nullptr, nullptr, range, P, (int)N, nullptr);
     const size_t off_rec = 16 * P, off_flags = off_rec + rec_bytes, n_out = off_flags + 2 * P;
     if (P > kHostIoBytes || n_in > kHostIoBytes || n_out > kHostIoBytes) return ACE_ETOOBIG;
+    std::lock_guard<std::mutex> lock(h->host_calls);
     int dev = -1;
     ACE_HIP(hipGetDevice(&dev));
     if (dev != h->device) ACE_HIP(hipSetDevice(h->device));
@@ -1332,6 +1337,7 @@ int ace_time_score_kernel(ace_handle_t *h, const ace_batch_t *batch, double memo
     AceKernelArgs a;
     int rc = fill_args(h, batch, memory_limit, strict, d_iter_ms, d_peak_mb, d_feasible, nullptr, nullptr, &a);
     if (rc) return rc;
+    std::lock_guard<std::mutex> lock(h->workspace);
     if ((rc = ensure_stage_ws(h, &a))) return rc;
     hipStream_t s = (hipStream_t)stream;
     hipEvent_t e0, e1;
@@ -1785,6 +1791,7 @@ int ace_search_step(ace_handle_t *h, const uint8_t *codes, const uint32_t *hdr, 
         h->geom.N >= 65536)
         return ACE_EINVAL;
     *result = ace_step_result_t{0, 0, 0.0, 0.0};
+    std::lock_guard<std::mutex> lock(h->host_calls);
     int dev = -1;
     ACE_HIP(hipGetDevice(&dev));
     if (dev != h->device) ACE_HIP(hipSetDevice(h->device));
