@@ -5,6 +5,7 @@ score itself: if the HIP library is missing or no GPU is present it raises.
 """
 import ctypes
 import os
+import threading
 from typing import Optional
 
 import numpy as np
@@ -371,7 +372,7 @@ class PlanEvaluator:
         self.handle = h
         self._deal_cache = {}
         self._topk_ws = None
-        self._rc_ready = None
+        self._rc_ready, self._rc_lock = None, threading.Lock()
         self._graphs_alive = 0
         self._copy_stream = None
 
@@ -615,17 +616,18 @@ class PlanEvaluator:
 
     def prepare_recompute(self, no_recompute: np.ndarray) -> bool:
         """Upload what check_recompute needs beside the tables (once); False if the op graph is too long for the kernel."""
-        if self._rc_ready is None:
-            t = self.tables
-            types = np.ascontiguousarray(t.graph.type_of_pos, dtype=np.int32)
-            act = np.ascontiguousarray(t.db.tables["activations"], dtype=np.float64)
-            norec = np.ascontiguousarray(no_recompute, dtype=np.uint8)
-            with self.device_context():
-                rc = self.lib.ace_recompute_prepare(self.handle, types.ctypes.data, act.ctypes.data, norec.ctypes.data)
-            if rc != ACE_ETOOBIG:
-                _check(self.lib, rc, "ace_recompute_prepare")
-            self._rc_ready = rc == 0
-        return self._rc_ready
+        with self._rc_lock:
+            if self._rc_ready is None:
+                t = self.tables
+                types = np.ascontiguousarray(t.graph.type_of_pos, dtype=np.int32)
+                act = np.ascontiguousarray(t.db.tables["activations"], dtype=np.float64)
+                norec = np.ascontiguousarray(no_recompute, dtype=np.uint8)
+                with self.device_context():
+                    rc = self.lib.ace_recompute_prepare(self.handle, types.ctypes.data, act.ctypes.data, norec.ctypes.data)
+                if rc != ACE_ETOOBIG:
+                    _check(self.lib, rc, "ace_recompute_prepare")
+                self._rc_ready = rc == 0
+            return self._rc_ready
 
     def recompute(self, d: DeviceBatch, memory_limit: float, peak_backward: float):
         """check_recompute's choice for every stage of every plan, after prepare_recompute: (the new batch, status of the

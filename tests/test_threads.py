@@ -1,5 +1,6 @@
 """Several threads with one evaluator: the host calls share page-locked buffers and take turns, and what is made on first use is
 made once."""
+import types
 from concurrent.futures import ThreadPoolExecutor
 
 import numpy as np
@@ -8,6 +9,25 @@ import pytest
 from superscaler_amd import synth
 from superscaler_amd.evaluator import PlanEvaluator
 from tests.test_small_batches import WORKLOADS, stage_queries
+
+
+def test_recompute_is_prepared_once():
+    import contextlib
+    import threading
+    import time
+    tables = synth.make_tables(WORKLOADS["gpt_wide_stages"])
+    calls = []
+
+    def prepare(*_):
+        calls.append(1)
+        time.sleep(0.05)
+        return 0
+    ev = types.SimpleNamespace(tables=tables, handle=None, lib=types.SimpleNamespace(ace_recompute_prepare=prepare), _rc_ready=None,
+                               _rc_lock=threading.Lock(), device_context=contextlib.nullcontext)
+    none = np.zeros(len(tables.db.op_names), dtype=np.uint8)
+    with ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(lambda _: PlanEvaluator.prepare_recompute(ev, none), range(4))) == [True] * 4
+    assert len(calls) == 1
 
 
 @pytest.mark.gpu
