@@ -1,7 +1,10 @@
-// The scoring kernel's op loop, as a function of (workgroup, lane): the GPU kernel in ace_eval.hip
+// The scoring kernel's op loop in C++, as a function of (workgroup, lane): the GPU kernel in ace_eval.hip
 // is a one-line wrapper around ace_score_body(), and a host build (ACE_HOST_EMU, one lane per
 // "workgroup") runs the very same loop on the CPU with every array behind guard pages, so that an
 // index error shows up as a host fault in the CPU test-suite instead of a memory fault on the GPU.
+// On the GPU it takes what no other kernel does: larger batches of stage records and single-stage queries, and plain scoring on
+// tables that the assembly loops do not walk (memory of collectives, windowed rows too short to be fetched, rows that leave the
+// loops' tables no room in LDS or lie there in another order).
 #pragma once
 #include "ace_plan_state.h"
 
@@ -94,14 +97,14 @@ template <int BLOCK> ACE_HD void stage_rows_flat(const AceKernelArgs &a, unsigne
     for (; j < n; j += BLOCK) dst[j] = src[j];
 }
 
-// The small tables to LDS (whole workgroup); DEFER: in the assembly loops' forms too.
-template <int BLOCK, bool DEFER> ACE_HD void stage_small_tables(const AceKernelArgs &a, unsigned char *lds_raw, int tid) {
+// The small tables to LDS (whole workgroup); ASM: in the assembly loops' forms too.
+template <int BLOCK, bool ASM> ACE_HD void stage_small_tables(const AceKernelArgs &a, unsigned char *lds_raw, int tid) {
     // pair kinds and the (micro-batch, stage gpus) LUT
     // (four pair kinds per lane and turn: the table is a multiple of 64 bytes)
     for (int j = tid; j < (a.rk_bytes >> 2); j += BLOCK) {
         const uint32_t r4 = reinterpret_cast<const uint32_t *>(a.pair_kinds)[j];
         reinterpret_cast<uint32_t *>(lds_raw + a.g.rk_lds_off)[j] = r4;
-        if (DEFER && a.g.pk32_lds_off) {
+        if (ASM && a.g.pk32_lds_off) {
             uint32_t e[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
@@ -125,7 +128,7 @@ template <int BLOCK, bool DEFER> ACE_HD void stage_small_tables(const AceKernelA
         reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2_lds_off)[j] = ace_u2{z_v, rk - z_v};
         // (the assembly loop adds the pair-kind block offset to the op pair's own index, not to the diag's, and its blocks
         // are ACE_PK32_BLOCK words apart)
-        if (DEFER && a.g.lut2a_lds_off) reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2a_lds_off)[j] = ace_u2{z_v, gl * ACE_PK32_BLOCK};
+        if (ASM && a.g.lut2a_lds_off) reinterpret_cast<ace_u2 *>(lds_raw + a.g.lut2a_lds_off)[j] = ace_u2{z_v, gl * ACE_PK32_BLOCK};
     }
 }
 
@@ -213,7 +216,6 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
     const uint32_t lds_base = ace_lds_base(lds_raw);
     g.hot_off += lds_base; g.start_off += lds_base; g.out_off += lds_base; g.z_off += lds_base;
     g.rk_lds_off += lds_base; g.stg_lds_off += lds_base; g.lut2_lds_off += lds_base;
-    if (g.lut2a_lds_off) g.lut2a_lds_off += lds_base;
     const long long slot = block * BLOCK + tid;                     // this lane's place in the batch (and in the workspace)
     AceRowsFirst rows_first;
     const bool flat = !WIN && a.flat_rows16 > 0;
@@ -289,14 +291,7 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
     const ace_u4 h = a.hdr[pl];
     ace_u4 cw = a.codes[(size_t)grp_begin * g.P + pl];
 
-    stage_small_tables<BLOCK, DEFER>(a, lds_raw, tid);
-    // (the assembly op loop over windowed rows: ace_many.h)
-#ifndef ACE_HOST_EMU
-    const bool asm_loop = DEFER && !WIN && lds_base == 0u && a.pos4 && a.g.lut2a_lds_off;
-#else
-    const bool asm_loop = false;
-#endif
-    if (DEFER && a.g.pace_lds_off && tid < 32) reinterpret_cast<uint32_t *>(lds_raw + a.g.pace_lds_off)[tid] = 0u;
+    stage_small_tables<BLOCK, false>(a, lds_raw, tid);
     if (flat) stage_rows_flat<BLOCK>(a, lds_raw, tid, rows_first);
     else stage_window<BLOCK>(a, lds_raw, w0, tid);       // every row, or the first window's
     ACE_SYNC();
@@ -320,22 +315,9 @@ ACE_HD void ace_score_body(const AceKernelArgs &a, unsigned char *lds_raw, uint3
     int w = w0 + 1;
     int next_win = WIN ? a.win_pos[w] : 0x7fffffff;
     const uint32_t first_code = cw.x & 7u;
-    int grp_stop = grp_end;
-#ifndef ACE_HOST_EMU
-    if (asm_loop) {
-        // the assembly form of the loop below (same operations per plan, same results)
-        if (!(cw.x & 0x10u)) st.status = ACE_PLAN_MALFORMED;    // the first op must open a stage
-        // (the loop looks each stage's offsets up in LDS, by the stage size's log2)
-        st.s = (int)ace_score_loop_asm<false>(a, g, st.glogs, g.lut2a_lds_off + st.bidx * 128u, (uint32_t)pl * 16u,
-                                            a.stage_ws + (size_t)block * ACE_MAX_STAGES * BLOCK * ACE_WS_REC,
-                                            (uint32_t)tid * (ACE_WS_REC * 8u), (uint32_t)BLOCK * (ACE_WS_REC * 8u), 0u,
-                                            (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6));
-        grp_stop = grp_begin;
-    } else
-#endif
     if (!RANGED) st.begin(g, lds, 0, cw.x & 0xffu, a.pos_info[0]);
     uint32_t pinfo = grp_begin ? a.pos_info[(grp_begin << 4) - 1] : 0u;    // descriptor of the previous group's last position
-    for (int grp = grp_begin; grp < grp_stop; ++grp) {
+    for (int grp = grp_begin; grp < grp_end; ++grp) {
         const int base = grp << 4;
         // the sixteen position descriptors of this group: scalar loads (the array is padded)
         const ace_u4 *ip = reinterpret_cast<const ace_u4 *>(a.pos_info + base);

@@ -68,7 +68,9 @@ def test_mid_sized_batches_on_the_gpu(name, mode, sizes):
 @pytest.mark.parametrize("name,mode,sizes", [("gpt_16ops", "plain", (65537, 131072, 200001, 262144)), ("gpt_wide_stages", "min", (262145, 300003)),
                                              ("t5_1layer", "noreserved", (147456, 600001)), ("gpt3_1_3b", "plain", (270000,)),
                                              ("wresnet_1b", "plain", (7680, 7681, 16385, 270001)), ("resnet_1111", "min", (8000, 70000)),
-                                             ("resnet_16gpus", "noreserved", (16384, 33333))])
+                                             ("resnet_16gpus", "noreserved", (16384, 33333)),
+                                             # (no assembly loop: windowed rows of short parts, by 256 and by 1,024 lanes)
+                                             ("resnet_2tp", "plain", (4096, 4097, 131073))])
 def test_large_batches_in_even_shares_on_the_gpu(name, mode, sizes):
     from superscaler_amd.evaluator import PlanEvaluator
     w = WORKLOADS[name]
@@ -83,4 +85,33 @@ def test_large_batches_in_even_shares_on_the_gpu(name, mode, sizes):
         batch = PlanBatch(base.codes[pick], base.hdr[pick])
         it, pk, fe, st = ev.score_host(batch)
         assert (st == 0).all() and np.array_equal(it, want[0][pick]) and np.array_equal(pk, want[1][pick]) and np.array_equal(fe, want[2][pick])
+    ev.close()
+
+
+def with_rows_in_another_order(tables, seed):
+    """The same tables with the resident rows in other LDS slots."""
+    import copy
+    t = copy.copy(tables)
+    n = len(t.win_rows)
+    assert t.n_windows == 1 and np.array_equal(t.win_rows[:, 1], np.arange(n) * t.rows.shape[1] * 8)
+    slot = np.random.default_rng(seed).permutation(n).astype(np.uint32)
+    t.win_rows = np.stack([t.win_rows[:, 0], slot * np.uint32(t.rows.shape[1] * 8)], axis=1)
+    info = t.pos_info
+    t.pos_info = (info & np.uint32(0xffff0000)) | slot[info & 0xff] | slot[(info >> 8) & 0xff] << np.uint32(8)
+    return t
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,sizes", [("gpt_wide_stages", (100, 4097, 131073)), ("t5_1layer", (5000,))])
+def test_rows_in_another_order_on_the_gpu(name, sizes):
+    from superscaler_amd.evaluator import PlanEvaluator
+    w = WORKLOADS[name]
+    tables = tables_for(w)
+    ev = PlanEvaluator(with_rows_in_another_order(tables, 3))
+    for n in sizes:
+        print(f"[case] {name} plans={n}", flush=True)
+        batch = synth.make_plans(w, tables, n_plans=n, seed_offset=n)
+        it, pk, fe, st = ev.score_host(batch)
+        want = c_oracle_scores(tables, batch, threads=8)
+        assert (st == 0).all() and np.array_equal(it, want[0]) and np.array_equal(pk, want[1]) and np.array_equal(fe, want[2])
     ev.close()
