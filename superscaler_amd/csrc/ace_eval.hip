@@ -100,17 +100,21 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
 
 // Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has six workgroups
 // (1,536 plans); that of the others, where a lane or a few walk a plan, hardly does until the chip is full, and they cross
-// where that time is reached.  By what else would take the batch, in us per launch (plan per workgroup / the other):
-//   PLAIN    the mid-sized kernel      4,096 / 4,608 plans: 315 ops 39 42 / 43, 523 ops 58 63 / 67, 821 ops 79 87 / 81,
-//                                      1,251 ops 106 116 / 109
-//   WINDOWED large, windowed rows      7,168 / 8,192 plans: 114 ops 36 40 / 42, 176 ops 57 64 / 55
-//   SLOW     no assembly loop (memory of collectives, more than 256 rows)   16,384 / 20,480 plans: 315 ops 145 179 / 163,
-//            523 ops 214 265 / 460, 114 ops 88 110 / 140
-//   RECORDS  stage records             12,288 / 16,384 plans: 315 ops 125 162 / 146, 523 ops 181 234 / 325, 134 ops 82 106 / 171;
-//            single-stage queries      315 ops 77 99 / 105, 523 ops 73 91 / 182
+// where that time is reached.  That place depends on the graph: both times grow with the ops, but not alike.  A path has one
+// limit all the same, at or below the first crossing of the graphs measured for it, so a graph that crosses later has a jump
+// there.  By what else would take the batch, in us per launch at the limit and where the graph crosses (plan per workgroup / the other):
+//   PLAIN    the mid-sized kernel                    limit  4,096: 315 ops  37 / 42, crosses at  4,800 plans; 523 ops  56 /  66,  5,000;
+//                                                                  821 ops  78 / 81,  4,300; 1,251 ops 104 / 111,  4,400
+//   WINDOWED large, windowed rows                    limit  7,680: 118 ops  34 / 41, crosses at  9,800 plans; 134 ops 37 / 46, 10,000; 174 ops 41 / 53, 10,450
+//   SLOW     no assembly loop (memory of collectives, more than 256 rows)
+//                                                    limit 18,432: 315 ops 161 / 161, 18,400; 523 ops 238 / 459, above 24,576 (313 / 460);
+//                                                                  134 ops  97 / 140, above 24,576 (128 / 140)
+//   RECORDS  stage records                           limit 14,336: 315 ops 134 / 136, 14,500; 523 ops 199 / 316, 23,000; 134 ops 81 / 148, above 24,576
+//            single-stage queries                           14,336: 315 ops  85 / 103, 18,000; 523 ops 80 / 179, 134 ops 53 / 124, both above 24,576
+//   OTHER    the C++ loop with deferred stage tails  limit  4,096:  62 ops  18 / 41, 11,500; 134 ops  22 / 83, 20,000
 // and at one plan 8 to 26 where a lane needs 49 to 169 (13 to 20 us is what the host needs for a launch).
 constexpr int kSpreadMaxPlain = 4096, kSpreadMaxWindowed = 7680, kSpreadMaxSlow = 18432, kSpreadMaxRecords = 14336;
-constexpr int kSpreadMaxOther = 4096;    // (deferred stage tails on the C++ form of the loop: tables that leave the assembly loop no room)
+constexpr int kSpreadMaxOther = 4096;    // (tables that no assembly loop walks: windowed rows too short to be fetched, no room in LDS)
 
 // ------------------------------------------------------------------------------------------
 // top-k: radix select on the order-preserving 64-bit image of the iteration time, then a
