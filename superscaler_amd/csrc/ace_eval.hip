@@ -1,14 +1,18 @@
 // MI355X (gfx950) batched plan evaluator: kernels and C ABI (see include/ace_eval.h).
 //
-// Scoring kernel: one plan per lane.  All lanes of a workgroup walk the op sequence in
-// lockstep, so the op type at each step is wave-uniform: the row of profiled values for
-// that type sits in LDS at a scalar base address and each lane only adds its own
-// (micro-batch, tp, algo) offset -- at most n_tp*n_algo distinct, consecutive entries per
-// sub-table, i.e. LDS reads without bank conflicts.  Plan bytes are stored plan-minor
-// ([16-op group][plan][16 bytes]) so a wavefront's load covers 1 KiB of consecutive HBM.
-// Every plan's sums run sequentially in op order in fp64, which reproduces the reference's
-// Python floats bit for bit.  When the rows of all op types do not fit in LDS the op
-// sequence is cut into windows and the workgroup restages the rows at each window boundary.
+// Scoring, by the size of the batch (launch_score holds the rule):
+//   ace_spread.h      small batches, and most batches of stage records and single-stage queries: a plan per workgroup, its ops
+//                     over the lanes
+//   ace_duo.h         mid-sized batches, every row resident: a plan walked by several lanes
+//   ace_many.h        large batches: a plan per lane
+//   ace_score_loop.h  what these leave, in C++: a plan per lane
+// With a plan per lane, all lanes of a workgroup walk the op sequence in lockstep, so the op type at each step is wave-uniform:
+// the row of profiled values for that type sits in LDS at a scalar base address and each lane only adds its own (micro-batch,
+// tp, algo) offset -- at most n_tp*n_algo distinct, consecutive entries per sub-table, i.e. LDS reads without bank conflicts.
+// Plan bytes are stored plan-minor ([16-op group][plan][16 bytes]) so a wavefront's load covers 1 KiB of consecutive HBM.
+// When the rows of all op types do not fit in LDS the op sequence is cut into windows, whose rows are staged in turn.
+// Whatever the kernel, every plan's sums run sequentially in op order in fp64, which reproduces the reference's Python floats
+// bit for bit.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>

@@ -10,7 +10,7 @@ from typing import Optional
 
 import numpy as np
 
-from .plan import PlanBatch, check_shape, finding, host_arrays, validate_batch
+from .plan import PlanBatch, check_plans, check_shape, finding, host_arrays, validate_batch
 from .tables import ABI_VERSION, MAX_STAGES, STAGE_REC, AceTablesStruct, CompiledTables
 
 _LIB_PATH = os.path.join(os.path.dirname(os.path.abspath(__file__)), "libace_eval.so")
@@ -197,14 +197,17 @@ def depth_order(batch: PlanBatch) -> np.ndarray:
     return perm[deal_slots(P)]
 
 
+_U32 = np.dtype(np.uint32)
+
+
 def host_ranges(ranges, n_plans: int) -> np.ndarray:
     """The op ranges of single-stage queries as native code reads them: uint32 [n_plans, 2], contiguous; one range stands for all
     queries, other shapes are refused (ValueError)."""
-    if isinstance(ranges, np.ndarray) and ranges.dtype == np.uint32 and ranges.shape == (n_plans, 2) and ranges.flags.c_contiguous:
-        return ranges
-    out = np.empty((n_plans, 2), dtype=np.uint32)
-    out[...] = ranges
-    return out
+    r = np.ascontiguousarray(ranges, _U32)
+    if r.shape != (n_plans, 2):
+        r, one = np.empty((n_plans, 2), dtype=_U32), r
+        r[...] = one
+    return r
 
 
 def pack_small_inputs(buf: np.ndarray, batch: PlanBatch, ranges) -> int:
@@ -512,7 +515,7 @@ class PlanEvaluator:
         capturing stream as they are; nothing in them clears memory with a memset node).  Returns a StepGraph:
         `replay()` runs the recorded launches again on the batch's current bytes and returns the same output
         tensors ((iter_ms, peak_mb, feasible, status), (indices, times, count)).  For a batch that is scored
-        again and again after edits in place; the seventeen launches of a step then cost one submission."""
+        again and again after edits in place; the launches of a step (scoring, one or two of the top-k for k <= 256) then cost one submission."""
         return StepGraph(self, dbatch, k, memory_limit, strict)
 
     def time_score_kernel(self, dbatch: DeviceBatch, reps: int, memory_limit: Optional[float] = None) -> float:
@@ -721,16 +724,21 @@ class PlanEvaluator:
 
     def _score_small(self, batch: PlanBatch, limit: float, strict: bool, breakdown: bool, ranges):
         """score_host for a batch whose inputs and outputs fit the library's page-locked buffers; None if they do not."""
-        P, N = batch.codes.shape
+        P = batch.codes.shape[0]
         breakdown = breakdown or ranges is not None
         n_rec = 1 if ranges is not None else MAX_STAGES          # a single-stage query has one record
         codes, hdr = host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)
+        codes_at, hdr_at = codes.ctypes.data, hdr.ctypes.data
         if ranges is not None:
             ranges = host_ranges(ranges, P)
+        else:
+            msg = check_plans(self.lib, codes_at, hdr_at, P, self.tables) if P else check_shape(batch, self.tables)
+            if msg:
+                raise ValueError(msg)
         times = np.empty((2, P))
         flags = np.empty((2, P), dtype=np.uint8)
         rec = np.empty((P, n_rec, STAGE_REC)) if breakdown else None
-        rc = self.lib.ace_score_host(self.handle, codes.ctypes.data, hdr.ctypes.data, ranges.ctypes.data if ranges is not None else None, P,
+        rc = self.lib.ace_score_host(self.handle, codes_at, hdr_at, ranges.ctypes.data if ranges is not None else None, P,
                                      limit, int(strict), times.ctypes.data, flags.ctypes.data, rec.ctypes.data if breakdown else None,
                                      self._torch._C._cuda_getCurrentRawStream(self.device.index))
         if rc == ACE_ETOOBIG:
@@ -743,10 +751,6 @@ class PlanEvaluator:
     def score_host(self, batch: PlanBatch, memory_limit=None, strict=False, breakdown=False, ranges=None,
                    group_by_depth: bool = False):
         if not group_by_depth and batch.n_plans <= 4096 and batch.codes.size < self.SMALL_IO_BYTES:
-            if ranges is None:
-                msg = validate_batch(batch, self.tables)
-                if msg:
-                    raise ValueError(msg)
             limit = float(self.tables.settings.memory_limit if memory_limit is None else memory_limit)
             out = self._score_small(batch, limit, strict, breakdown, ranges)
             if out is not None:

@@ -268,21 +268,16 @@ def host_arrays(codes, hdr, num_ops: Optional[int] = None):
     """Code rows and headers of a host batch as native code reads them through raw pointers: uint8 [P, N] (N = `num_ops` if that
     is given) and uint32 [P, 4], C-contiguous, the arrays themselves where they are that already.  Other integer types are converted
     by value, one header row stands for all plans; anything else is refused (ValueError, TypeError)."""
-    if codes.ndim != 2 or hdr.ndim != 2 or hdr.shape[1] != 4 or hdr.shape[0] not in (1, codes.shape[0]):
-        raise ValueError(f"code rows [plans, ops] and headers [plans, 4] expected, not {codes.shape} and {hdr.shape}")
-    if num_ops is not None and codes.shape[1] != num_ops:
-        raise ValueError(f"batch has {codes.shape[1]} ops per plan, op graph {num_ops}")
-    if codes.dtype is not _U8 or not codes.flags.c_contiguous:
-        codes = _as_integers(codes, _U8)
-    if hdr.dtype is not _U32 or not hdr.flags.c_contiguous or len(hdr) != len(codes):
-        hdr = _as_integers(np.broadcast_to(hdr, (len(codes), 4)), _U32)
-    return codes, hdr
-
-
-def _as_integers(a, dtype):
-    if a.dtype.kind not in "iub":
-        raise TypeError(f"plans are arrays of integers, not {a.dtype}")
-    return np.ascontiguousarray(a, dtype=dtype)
+    shape = codes.shape
+    if len(shape) != 2 or hdr.shape != (shape[0], 4):
+        if len(shape) != 2 or hdr.shape != (1, 4):
+            raise ValueError(f"code rows [plans, ops] and headers [plans, 4] expected, not {shape} and {hdr.shape}")
+        hdr = np.broadcast_to(hdr, (shape[0], 4))
+    if num_ops is not None and shape[1] != num_ops:
+        raise ValueError(f"batch has {shape[1]} ops per plan, op graph {num_ops}")
+    if (codes.dtype is not _U8 or hdr.dtype is not _U32) and (codes.dtype.kind not in "iub" or hdr.dtype.kind not in "iub"):
+        raise TypeError(f"plans are arrays of integers, not {codes.dtype} and {hdr.dtype}")
+    return np.ascontiguousarray(codes, _U8), np.ascontiguousarray(hdr, _U32)
 
 
 # what the structural check of a batch finds wrong (ace_check_plans / ace_pack_plans), in this order
@@ -311,8 +306,12 @@ def validate_batch(batch: PlanBatch, tables: CompiledTables) -> Optional[str]:
         return msg
     from .evaluator import load_library
     codes, hdr = host_arrays(batch.codes, batch.hdr)
-    return finding(load_library().ace_check_plans(codes.ctypes.data, hdr.ctypes.data, codes.shape[0], codes.shape[1],
-                                                  len(tables.db.mbs_list), tables.C))
+    return check_plans(load_library(), codes.ctypes.data, hdr.ctypes.data, len(codes), tables)
+
+
+def check_plans(lib, codes_at: int, hdr_at: int, n_plans: int, tables: CompiledTables) -> Optional[str]:
+    """validate_batch for arrays that host_arrays gave, by their addresses."""
+    return finding(lib.ace_check_plans(codes_at, hdr_at, n_plans, tables.graph.num_ops, len(tables.db.mbs_list), tables.C))
 
 
 # model_size -> (num_layers, seq_len, hidden, ffn_hidden, heads, kv_channels, vocab)  (aceso_utils.py:27-34)

@@ -9,7 +9,7 @@ import pytest
 
 from superscaler_amd import plan as plan_mod
 from superscaler_amd import synth
-from superscaler_amd.evaluator import PlanEvaluator, pack_small_inputs, rows_to_device
+from superscaler_amd.evaluator import PlanEvaluator, load_library, pack_small_inputs, rows_to_device
 from superscaler_amd.neighbours import _draw_moves, _draws_struct, sample_moves
 from superscaler_amd.plan import PlanBatch, validate_batch
 from tests.helpers import odd_workloads
@@ -99,7 +99,7 @@ def fake_evaluator(tables, calls):
         calls.append((at(codes, np.empty(shape, np.uint8)), at(hdr, np.empty((P, 4), np.uint32)),
                       None if ranges is None else at(ranges, np.empty((P, 2), np.uint32)), _[-1]))
         return 0
-    ev.lib = types.SimpleNamespace(ace_score_host=ace_score_host)
+    ev.lib = types.SimpleNamespace(ace_score_host=ace_score_host, ace_check_plans=load_library().ace_check_plans)
     return ev
 
 
@@ -176,8 +176,8 @@ def test_a_device_without_an_index_is_the_one_that_was_current(monkeypatch):
     from superscaler_amd import evaluator
     tables, batch = tables_and_plans(2)
     calls = []
-    made = types.SimpleNamespace(ace_create=lambda tables, handle: 0, ace_check_plans=evaluator.load_library().ace_check_plans,
-                                 ace_score_host=fake_evaluator(tables, calls).lib.ace_score_host)
+    made = fake_evaluator(tables, calls).lib
+    made.ace_create = lambda tables, handle: 0
     current = [3]
     monkeypatch.setattr(evaluator, "load_library", lambda: made)
     monkeypatch.setattr(torch.cuda, "is_available", lambda: True)
