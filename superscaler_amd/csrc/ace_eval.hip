@@ -361,6 +361,8 @@ __global__ __launch_bounds__(1024) void topk_finish(TopkState *st, Cand *less, C
 // Bound by the latency of the two selections (about three dozen workgroup barriers each), not by reading the input.
 // Launches back to back (10 us is what the host needs for a call), us, against a sampled bound, a filter pass and one
 // selection: k = 64, 4,096 entries 23 -> 10, 262,144 entries 27 -> 17, 2^20 entries 34 -> 23; k = 256, 2^20 entries 80 -> 40.
+// (Behind the scoring kernel, its inputs not in a cache any more, kernel trace: 262,144 entries 8.5 + 8.9, 2^20 entries 15.4 + 15.1;
+// the three launches before took 8.7 + 11.6 + 13.9 there.)
 // ------------------------------------------------------------------------------------------
 constexpr int kShortMaxK = 256;
 constexpr unsigned kShortMaxEntries = 16384;     // entries one workgroup selects from: sixteen per lane
