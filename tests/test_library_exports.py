@@ -58,6 +58,28 @@ def test_missing_library_fails_loudly(monkeypatch):
         evaluator.load_library()
 
 
+def test_host_side_work_on_plans_names_the_build_command_without_the_libraries(monkeypatch):
+    """Encoding, the structural check, move descriptors and visited sets are native; tables, plans and plan files are not."""
+    import sys
+    import numpy as np
+    import superscaler_amd
+    from superscaler_amd.neighbours import VisitedKeys, sample_moves
+    from superscaler_amd.plan import PlanBatch, validate_batch
+    monkeypatch.setattr(evaluator, "_lib", None)
+    monkeypatch.setattr(evaluator, "_objects", None)
+    monkeypatch.setattr(evaluator, "_LIB_PATH", "/nonexistent/libace_eval.so")
+    monkeypatch.setitem(sys.modules, "superscaler_amd._ace_objects", None)
+    monkeypatch.delattr(superscaler_amd, "_ace_objects", raising=False)
+    w = synth.WORKLOADS["gpt3_1_3b"]
+    tables = synth.make_tables(w)
+    batch = synth.make_plans(w, tables, n_plans=2)
+    config = batch.to_config(0, tables)
+    for call in (lambda: PlanBatch.from_configs([config], tables), lambda: validate_batch(batch, tables),
+                 lambda: sample_moves(batch, tables, 10, np.random.default_rng(0)), VisitedKeys):
+        with pytest.raises(evaluator.AceError, match="python -m superscaler_amd.build"):
+            call()
+
+
 def test_no_gpu_means_no_scoring():
     import torch
     if torch.cuda.is_available():
