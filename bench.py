@@ -25,8 +25,8 @@ HBM_PEAK_GBPS = 8000.0
 # the same pass; vector instructions per op and wavefront = SQ_INSTS_VALU / SQ_WAVES / ops; 14 of them are the
 # reference's own fp64 arithmetic (nine adds / multiply-adds, five maxima).
 PROFILE_COUNTERS = {
-    ("gpt3_13b", 523): {"source": "profiles/score_kernel_gpt3_13b.md", "library": "b570eaebab746de3", "traffic_bytes_per_plan": 1715.0,
-                        "valu_per_op_per_wavefront": 35.1, "valu_busy": 0.78},
+    ("gpt3_13b", 523): {"source": "profiles/score_kernel_gpt3_13b.md", "library": "bc5cb87df14fc94c", "traffic_bytes_per_plan": 1722.0,
+                        "valu_per_op_per_wavefront": 35.0, "valu_busy": 0.78},
 }
 # the other configured workloads, timed after the headline measurement (kernel only, HIP events on the launch stream)
 OTHER_WORKLOADS = ("gpt3_1_3b", "t5_770m", "wresnet_1b", "gpt3_175b")
@@ -73,11 +73,17 @@ def cpu_baseline(tables, batch, threads):
             "c_port_single_core_sample": f"first {n1} plans, {dt_one:.2f} s, 1 thread"}
 
 
-def kernel_name(tables):
-    """The instantiation plain scoring of a large batch runs (the library's choice, ensure_stage_ws in ace_eval.hip)."""
-    deferred = tables.graph.num_ops < 65536 and (tables.n_windows == 1 or tables.rows.shape[0] <= 256)
-    return "ace_score_kernel<BD=false,RANGED=false,WIN=%s,DEFER=%s>" % ("true" if tables.n_windows > 1 else "false",
-                                                                          "true" if deferred else "false")
+def kernel_name(tables, n_plans):
+    """The kernel that plain scoring of a batch runs (the library's choice, launch_score in ace_eval.hip), for tables that its
+    assembly loops walk, as the configured workloads' are."""
+    windowed = tables.n_windows > 1
+    if windowed and tables.rows.shape[0] > 256:
+        return "ace_score_kernel<WIN=true>"
+    if n_plans <= (7680 if windowed else 4096):
+        return "ace_spread_kernel"
+    if not windowed and n_plans <= 65536:
+        return "ace_duo_kernel"
+    return "ace_many_kernel<WIN=%s>" % ("true" if windowed else "false")
 
 
 def other_workloads(steps):
@@ -97,7 +103,7 @@ def other_workloads(steps):
         ms = ev.time_score_kernel(d, reps=max(steps, 20))
         bpp = 3 * d.num_ops + 19
         gbps = bpp * d.n_plans / (ms * 1e-3) / 1e9
-        out[name] = {"kernel": kernel_name(tables), "ops": d.num_ops, "plans": d.n_plans, "kernel_ms": ms,
+        out[name] = {"kernel": kernel_name(tables, d.n_plans), "ops": d.num_ops, "plans": d.n_plans, "kernel_ms": ms,
                      "plans_per_s_kernel": d.n_plans / (ms * 1e-3), "algorithmic_bytes_per_plan": bpp,
                      "achieved_GBps": gbps, "frac": gbps / HBM_PEAK_GBPS}
         ev.close()
@@ -225,7 +231,7 @@ def main():
                                     f"PP in {w.pp_choices}, mbs in {w.mbs_list}, recompute p={w.recompute_p}, "
                                     f"memory cap {w.memory_limit:.0f} MB, global batch {w.global_batch}, top-{args.topk}",
                         "step": "score kernel + device-wide top-k, inputs resident in HBM",
-                        "layout": "plans in the generator's order (each workgroup of the kernel deals its 1,024 plans to "
+                        "layout": "plans in the generator's order (each workgroup of the kernel deals its plans, up to 1,024, to "
                                   "its lanes by pipeline depth; nothing is reordered beforehand)",
                         "feasible_plans": n_feasible, "best_iter_ms": best, "plan_generation_s": round(gen_s, 1)},
                        **secondary),
@@ -234,7 +240,7 @@ def main():
                      "traffic": counters["traffic_bytes_per_plan"] * P if counters else None,
                      "traffic_source": f'{counters["source"]} (library sources {counters["library"]})' if counters else counters_note,
                      "algorithmic_bytes": algo_bytes,
-                     "kernel": kernel_name(tables), "kernel_ms": kern_ms,
+                     "kernel": kernel_name(tables, P), "kernel_ms": kern_ms,
                      "algorithmic_bytes_per_plan": 3 * N + 19,
                      "bytes_moved_per_plan": d.bytes_moved_per_plan + 17,
                      "achieved_on_bytes_moved": moved_bytes / (kern_ms * 1e-3) / 1e9,
