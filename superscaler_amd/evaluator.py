@@ -434,11 +434,18 @@ class PlanEvaluator:
     def _stream(self):
         return ctypes.c_void_p(self._torch.cuda.current_stream(self.device).cuda_stream)
 
+    def _fits(self, d: DeviceBatch):
+        """The kernels read as many 16-op groups of every plan as the op graph has."""
+        groups = (self.tables.graph.num_ops + 15) // 16
+        if d.codes.numel() < groups * d.n_plans * 16:
+            raise ValueError(f"{d.n_plans} plans of {groups} 16-op groups expected, the batch's codes have {d.codes.numel()} bytes")
+
     def score(self, dbatch: DeviceBatch, memory_limit: Optional[float] = None, strict: bool = False,
               breakdown: bool = False, out=None):
         """Launch the scoring kernel; returns device tensors (iter_ms, peak_mb, feasible, status[, stage records
         [P, 16, STAGE_REC]; [P, 1, STAGE_REC] for single-stage queries])."""
         torch = self._torch
+        self._fits(dbatch)
         P = dbatch.n_plans
         limit = float(self.tables.settings.memory_limit if memory_limit is None else memory_limit)
         if out is None:
@@ -522,6 +529,7 @@ class PlanEvaluator:
         """Average scoring-kernel duration in ms over `reps` back-to-back launches (hipEvents on the
         launch stream)."""
         torch = self._torch
+        self._fits(dbatch)
         P = dbatch.n_plans
         limit = float(self.tables.settings.memory_limit if memory_limit is None else memory_limit)
         it = torch.empty(P, dtype=torch.float64, device=self.device)
@@ -608,6 +616,8 @@ class PlanEvaluator:
         expanded, scored and the fastest feasible one picked: (plan, iteration ms, peak MB), or None.  `sets`: handles of
         the visited sets (empty: only repeated moves are dropped)."""
         t, best = self.tables, AceStepResultStruct()
+        if t.graph.num_ops >= 65536:
+            raise ValueError("move descriptors hold 16-bit op positions")
         codes, hdr = host_arrays(plan.codes[:1], plan.hdr[:1], t.graph.num_ops)
         codes_out, hdr_out = np.empty_like(codes), np.empty_like(hdr)
         handles = (ctypes.c_void_p * max(1, len(sets)))(*sets)

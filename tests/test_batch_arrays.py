@@ -190,3 +190,28 @@ def test_a_device_without_an_index_is_the_one_that_was_current(monkeypatch):
         assert ev[d].device == torch.device("cuda", index)
         ev[d].score_host(batch)
         assert calls[-1][3] == 1000 + index
+
+
+def test_device_batches_hold_the_graphs_ops():
+    """A batch that was not checked when it was made (from_device, upload(validate=False)): fewer 16-op groups than the graph has
+    would be read past their end."""
+    import torch
+    from superscaler_amd.evaluator import DeviceBatch
+    from superscaler_amd.neighbours import _draw_moves, _draws_struct
+    tables, batch = tables_and_plans(4)
+    calls = []
+    ev = fake_evaluator(tables, calls)
+    P, N = batch.codes.shape
+    assert 16 < N < 32
+    hdr = torch.from_numpy(batch.hdr.view(np.int32))
+    small = DeviceBatch.from_device(torch.zeros((1, P, 16), dtype=torch.uint8), hdr, 16)
+    short = DeviceBatch.from_device(torch.zeros((2, P - 1, 16), dtype=torch.uint8), hdr, N)
+    for d in (small, short):
+        for call in (lambda: ev.score(d), lambda: ev.time_score_kernel(d, 1), lambda: ev.recompute(d, 1e4, 0.0)):
+            with pytest.raises(ValueError, match="16-op groups"):
+                call()
+    # op positions of a search's moves have 16 bits
+    ev.tables = types.SimpleNamespace(graph=types.SimpleNamespace(num_ops=65536), settings=tables.settings, stage_lut=tables.stage_lut)
+    with pytest.raises(ValueError, match="16-bit"):
+        ev.search_step(PlanBatch(np.zeros((1, 65536), dtype=np.uint8), batch.hdr[:1]),
+                       _draws_struct(_draw_moves(1, 1, tables, np.random.default_rng(0))))
