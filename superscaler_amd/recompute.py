@@ -203,7 +203,9 @@ def update_recompute_device(cm, dbatch):
     n_types = len(tables.db.op_names)
     norec = ((np.asarray(tables.graph.flags)[:n_types] & og.F_NO_RECOMPUTE) != 0).astype(np.uint8)
     if hasattr(ev, "recompute") and ev.prepare_recompute(norec):
-        out, status, flags = ev.recompute(dbatch, args.memory_limit, args.peak_mem_in_backward)
+        # (the plans are whole ones, also where the batch carries the ranges of single-stage queries)
+        whole = dbatch if dbatch.ranges is None else DeviceBatch.from_device(dbatch.codes, dbatch.hdr, N)
+        out, status, flags = ev.recompute(whole, args.memory_limit, args.peak_mem_in_backward)
         count, first, grid, bad = flags.tolist()
         if count or first:
             raise ValueError("malformed encoding: stage bits do not match the stage counts")

@@ -101,6 +101,9 @@ def test_one_launch_on_the_gpu(name, mode, n):
     for limit in limits(ref, batch):
         cm.settings.memory_limit = ref.settings.memory_limit = limit
         assert np.array_equal(cm.update_recompute_arrays(batch).codes, update_recompute_arrays(ref, batch).codes)
+    # (ranges that a batch carries for single-stage queries do not matter: every stage of the whole plans is looked at)
+    ranged = cm.evaluator.upload(batch, ranges=np.tile(np.array([[0, 1]], dtype=np.uint32), (n, 1)))
+    assert np.array_equal(cm.evaluator.download(cm.update_recompute_device(ranged)).codes, update_recompute_arrays(ref, batch).codes)
     bad = PlanBatch(batch.codes.copy(), batch.hdr.copy())
     bad.hdr[0, 0] += 1
     with pytest.raises(ValueError):
