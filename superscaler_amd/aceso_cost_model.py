@@ -143,6 +143,8 @@ class CostModel:
     def _fill_all(self, configs, rec):
         """_fill_breakdown for every plan of a list: natively, except the plan objects that are left to the Python code."""
         args, fill, p = self.settings, load_objects().fill_all, 0
+        if not isinstance(configs, (list, tuple)):
+            configs = list(configs)
         while True:
             p = fill(configs, rec, p, args.memory_limit, args.memory_main_params, args.memory_optimizer, args.consider_reserved_space)
             if p >= len(configs):

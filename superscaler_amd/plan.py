@@ -167,6 +167,8 @@ class PlanBatch:
         single-stage queries do (aceso_cost_model.py:494-495)."""
         from .evaluator import load_objects
         db, N, P = tables.db, tables.graph.num_ops, len(configs)
+        if not isinstance(configs, (list, tuple)):
+            configs = list(configs)
         mbs, tp_lut = tables.encode_luts
         codes = np.empty((P, N), dtype=np.uint8)
         hdr = np.empty((P, 4), dtype=np.uint32)

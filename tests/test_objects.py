@@ -1,5 +1,6 @@
 """The native walk over plan objects (superscaler_amd/csrc/ace_objects.cpp) against the Python code it stands in for: the same
 arrays and lists for a search's plans, the same arrays and errors for everything it leaves to that code."""
+import collections
 import copy
 
 import numpy as np
@@ -84,6 +85,23 @@ def test_a_list_of_plans_is_filled_like_each_of_them():
     cm._fill_all(all_, rec)
     assert one == all_ and all(c.time_list for c in all_)
     cm._fill_all([], rec[:0])
+
+
+def test_plans_come_in_any_collection():
+    w = odd_workloads()[2]
+    cm = cost_model(w)
+    batch = synth.make_plans(w, cm.tables, n_plans=5, seed_offset=4)
+    configs = [batch.to_config(p, cm.tables) for p in range(5)]
+    configs[2].stages[0].tp_size = tuple(configs[2].stages[0].tp_size)      # (left to the Python code)
+    configs[3].stages = tuple(configs[3].stages)
+    rec = emu_score(cm.tables, batch, breakdown=True)[4]
+    for some in (dict(enumerate(configs)).values(), collections.deque(configs)):
+        got = PlanBatch.from_configs(some, cm.tables)
+        assert np.array_equal(got.codes, batch.codes) and np.array_equal(got.hdr, batch.hdr)
+        cm._fill_all(some, rec)
+        assert all(c.time_list for c in configs)
+        for c in configs:
+            c.time_list = []
 
 
 class Changing:
