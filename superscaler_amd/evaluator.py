@@ -213,7 +213,7 @@ def host_ranges(ranges, n_plans: int) -> np.ndarray:
 def pack_small_inputs(buf: np.ndarray, batch: PlanBatch, ranges) -> int:
     """Lay a small batch out for the kernel in `buf` (uint8) as ace_score_host does: codes [ceil(N/16)][P][16] (zero padded),
     then the headers uint32 [P][4], then the ranges uint32 [P][2] if given.  Returns the number of bytes used."""
-    codes, hdr = host_arrays(batch.codes, batch.hdr)
+    codes, hdr = host_arrays(batch.codes, batch.hdr, integers=False)
     P, N = codes.shape
     rg = None if ranges is None else host_ranges(ranges, P)
     if buf.dtype != np.uint8 or not (buf.flags.c_contiguous and buf.flags.writeable):
@@ -396,7 +396,7 @@ class PlanEvaluator:
         bytes; the kernel itself is safe for any byte content).  `group_by_depth`, `findings`: see DeviceBatch."""
         check = None
         if validate and ranges is not None:
-            host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)       # (a query's plan need not be a whole one)
+            host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)       # (a query's plan need not be a whole one: no check of it)
         elif validate:
             # (small batches are checked before they go anywhere; for others the check rides on the device's packing of the
             # plans and costs the read-back of its findings; not where the call must not wait for the device)
@@ -737,7 +737,8 @@ class PlanEvaluator:
         P = batch.codes.shape[0]
         breakdown = breakdown or ranges is not None
         n_rec = 1 if ranges is not None else MAX_STAGES          # a single-stage query has one record
-        codes, hdr = host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops)
+        # (a query's plan is not checked: it never had to be of integers)
+        codes, hdr = host_arrays(batch.codes, batch.hdr, self.tables.graph.num_ops, integers=ranges is None)
         codes_at, hdr_at = codes.ctypes.data, hdr.ctypes.data
         if ranges is not None:
             ranges = host_ranges(ranges, P)

@@ -266,10 +266,10 @@ class PlanBatch:
 _U8, _U32 = np.dtype(np.uint8), np.dtype(np.uint32)
 
 
-def host_arrays(codes, hdr, num_ops: Optional[int] = None):
+def host_arrays(codes, hdr, num_ops: Optional[int] = None, integers: bool = True):
     """Code rows and headers of a host batch as native code reads them through raw pointers: uint8 [P, N] (N = `num_ops` if that
-    is given) and uint32 [P, 4], C-contiguous, the arrays themselves where they are that already.  Other integer types are converted
-    by value, one header row stands for all plans; anything else is refused (ValueError, TypeError)."""
+    is given) and uint32 [P, 4], C-contiguous, the arrays themselves where they are that already.  Other integer types (`integers`
+    false: all types) are converted by value, one header row stands for all plans; anything else is refused (ValueError, TypeError)."""
     shape = codes.shape
     if len(shape) != 2 or hdr.shape != (shape[0], 4):
         if len(shape) != 2 or hdr.shape != (1, 4):
@@ -277,7 +277,7 @@ def host_arrays(codes, hdr, num_ops: Optional[int] = None):
         hdr = np.broadcast_to(hdr, (shape[0], 4))
     if num_ops is not None and shape[1] != num_ops:
         raise ValueError(f"batch has {shape[1]} ops per plan, op graph {num_ops}")
-    if (codes.dtype is not _U8 or hdr.dtype is not _U32) and (codes.dtype.kind not in "iub" or hdr.dtype.kind not in "iub"):
+    if integers and (codes.dtype is not _U8 or hdr.dtype is not _U32) and (codes.dtype.kind not in "iub" or hdr.dtype.kind not in "iub"):
         raise TypeError(f"plans are arrays of integers, not {codes.dtype} and {hdr.dtype}")
     return np.ascontiguousarray(codes, _U8), np.ascontiguousarray(hdr, _U32)
 

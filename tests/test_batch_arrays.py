@@ -215,3 +215,13 @@ def test_device_batches_hold_the_graphs_ops():
     with pytest.raises(ValueError, match="16-bit"):
         ev.search_step(PlanBatch(np.zeros((1, 65536), dtype=np.uint8), batch.hdr[:1]),
                        _draws_struct(_draw_moves(1, 1, tables, np.random.default_rng(0))))
+
+
+def test_queries_of_other_types_are_converted():
+    tables, batch = tables_and_plans(8)
+    calls = []
+    ev = fake_evaluator(tables, calls)
+    ev.score_host(PlanBatch(batch.codes.astype(float), batch.hdr.astype(float)), ranges=(0, 3))
+    assert np.array_equal(calls[-1][0], batch.codes) and np.array_equal(calls[-1][1], batch.hdr)
+    with pytest.raises(TypeError):
+        ev.score_host(PlanBatch(batch.codes.astype(float), batch.hdr))
