@@ -289,6 +289,8 @@ def pack_rows(rows, hdr, check=None, findings=None):
     import torch
     P, N = rows.shape
     G = (N + 15) // 16
+    if P == 0:
+        return torch.empty((G, 0, 16), dtype=torch.uint8, device=rows.device)
     if rows.device.type != "cuda":
         return torch.nn.functional.pad(rows, (0, G * 16 - N)).view(P, G, 16).permute(1, 0, 2).contiguous()
     lib = load_library()
@@ -443,7 +445,8 @@ class PlanEvaluator:
     def score(self, dbatch: DeviceBatch, memory_limit: Optional[float] = None, strict: bool = False,
               breakdown: bool = False, out=None):
         """Launch the scoring kernel; returns device tensors (iter_ms, peak_mb, feasible, status[, stage records
-        [P, 16, STAGE_REC]; [P, 1, STAGE_REC] for single-stage queries])."""
+        [P, 16, STAGE_REC]; [P, 1, STAGE_REC] for single-stage queries]).  Where `status` is not 0 the scores are NaN and
+        the records hold no particular values."""
         torch = self._torch
         self._fits(dbatch)
         P = dbatch.n_plans
@@ -670,6 +673,8 @@ class PlanEvaluator:
             raise ValueError("download: the batch is stored in grouped order (group_by_depth)")
         torch = self._torch
         P, N = d.n_plans, d.num_ops
+        if P == 0:
+            return PlanBatch(np.empty((0, N), dtype=np.uint8), np.empty((0, 4), dtype=np.uint32))
         both = torch.empty(16 * P + P * N, dtype=torch.uint8, device=self.device)
         both[:16 * P].copy_(d.hdr.view(torch.uint8).view(-1))
         with self.device_context():

@@ -225,3 +225,18 @@ def test_queries_of_other_types_are_converted():
     assert np.array_equal(calls[-1][0], batch.codes) and np.array_equal(calls[-1][1], batch.hdr)
     with pytest.raises(TypeError):
         ev.score_host(PlanBatch(batch.codes.astype(float), batch.hdr))
+
+
+@pytest.mark.gpu
+def test_empty_batches_on_the_gpu():
+    import torch
+    tables, batch = tables_and_plans(8)
+    ev = PlanEvaluator(tables)
+    empty = ev.upload(batch.slice(0, 0), validate=False)
+    assert empty.n_plans == 0 and empty.codes.shape == (2, 0, 16) and empty.hdr.shape == (0, 4)
+    with pytest.raises(ValueError):
+        ev.upload(batch.slice(0, 0))
+    d = ev.upload(batch)
+    none = ev.download(d, torch.zeros(0, dtype=torch.int64, device="cuda"))
+    assert none.codes.shape == (0, tables.graph.num_ops) and none.hdr.shape == (0, 4) and none.hdr.dtype == np.uint32
+    ev.close()
