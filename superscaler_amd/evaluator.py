@@ -4,6 +4,7 @@
 score itself: if the HIP library is missing or no GPU is present it raises.
 """
 import ctypes
+import operator
 import os
 import threading
 from typing import Optional
@@ -479,7 +480,7 @@ class PlanEvaluator:
 
     def topk(self, iter_ms, feasible, k: int):
         """Device-wide top-k: (indices int64[k], times f64[k], count)."""
-        torch = self._torch
+        torch, k = self._torch, operator.index(k)
         buf = self.topk_packed(iter_ms, feasible, k)
         return buf[:8 * k].view(torch.int64), buf[8 * k:16 * k].view(torch.float64), buf[16 * k:16 * k + 4].view(torch.int32)
 
@@ -487,7 +488,7 @@ class PlanEvaluator:
         """topk() in one device buffer (indices, times, count: one copy brings all of them to the host); `out`: that buffer
         (uint8, at least 16 * k + 4)."""
         torch = self._torch
-        n = iter_ms.numel()
+        n, k = iter_ms.numel(), operator.index(k)
         need = self.lib.ace_topk_workspace_bytes(n, k)
         if self._topk_ws is None or self._topk_ws.numel() < need:
             # (a captured step keeps its own reference to the workspace it recorded, so the old one stays alive for it)
@@ -510,7 +511,7 @@ class PlanEvaluator:
     def top_k(self, batch: PlanBatch, k: int, memory_limit: Optional[float] = None, strict: bool = False):
         """(indices, times) of the k fastest feasible plans of a host batch.  Everything is asked for before anything is read:
         what the structural check of the plans has found comes back with the result (scoring is safe for any bytes)."""
-        torch = self._torch
+        torch, k = self._torch, operator.index(k)
         buf = torch.zeros(16 * k + 16, dtype=torch.uint8, device=self.device)
         d = self.upload(batch, findings=buf[16 * k + 8:16 * k + 12].view(torch.int32))
         it, pk, fe, st = self.score(d, memory_limit, strict)

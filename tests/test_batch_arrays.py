@@ -228,7 +228,7 @@ def test_queries_of_other_types_are_converted():
 
 
 @pytest.mark.gpu
-def test_empty_batches_on_the_gpu():
+def test_empty_batches_and_other_integers_on_the_gpu():
     import torch
     tables, batch = tables_and_plans(8)
     ev = PlanEvaluator(tables)
@@ -239,4 +239,11 @@ def test_empty_batches_on_the_gpu():
     d = ev.upload(batch)
     none = ev.download(d, torch.zeros(0, dtype=torch.int64, device="cuda"))
     assert none.codes.shape == (0, tables.graph.num_ops) and none.hdr.shape == (0, 4) and none.hdr.dtype == np.uint32
+    want = ev.top_k(batch, 3)
+    for k in (np.int64(3), np.uint8(3)):
+        got = ev.top_k(batch, k)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        assert ev.score_stream([batch], k)[0].tolist() == want[0].tolist()
+    with pytest.raises(TypeError):
+        ev.top_k(batch, 3.0)
     ev.close()
