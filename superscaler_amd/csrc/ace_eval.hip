@@ -1264,9 +1264,9 @@ int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_lim
 }
 
 size_t ace_pack_host(const uint8_t *codes, const uint32_t *hdr, const uint32_t *range, size_t n_plans, int num_ops, uint8_t *out) {
-    const size_t P = n_plans, N = (size_t)num_ops, G = (N + 15) / 16, off_hdr = G * P * 16, off_rng = off_hdr + P * 16;
+    const size_t P = n_plans, N = num_ops > 0 ? (size_t)num_ops : 0, G = (N + 15) / 16, off_hdr = G * P * 16, off_rng = off_hdr + P * 16;
     if (out) {
-        for (size_t p = 0; p < P; ++p) {
+        for (size_t p = 0; p < P && G; ++p) {
             const uint8_t *row = codes + p * N;
             for (size_t g = 0; g + 1 < G; ++g) memcpy(out + (g * P + p) * 16, row + g * 16, 16);
             unsigned char last[16] = {0};

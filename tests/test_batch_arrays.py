@@ -156,6 +156,13 @@ def test_ranges_stand_for_every_query():
     assert len(calls) == made
 
 
+def test_plans_without_ops_have_no_code_words():
+    buf = np.full(4096, 7, dtype=np.uint8)
+    b = PlanBatch(np.zeros((3, 0), dtype=np.uint8), np.arange(12, dtype=np.uint32).reshape(3, 4))
+    assert pack_small_inputs(buf[1024:], b, None) == 48
+    assert np.array_equal(buf[1024:1072].view(np.uint32), np.arange(12)) and (buf[:1024] == 7).all() and (buf[1072:] == 7).all()
+
+
 def test_queries_have_the_graphs_ops():
     tables, batch = tables_and_plans(8)
     calls = []
