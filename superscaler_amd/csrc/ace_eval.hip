@@ -60,6 +60,15 @@ constexpr int kMaxDevices = 64;
 double *g_static_ptr[kMaxDevices];     // device address of `scratch` by device ordinal; filled once per device
 std::mutex g_static_mutex;
 
+// f() where host memory may run out (no exception leaves a C entry)
+template <class F> static int or_enomem(F f) {
+    try {
+        return f();
+    } catch (const std::bad_alloc &) {
+        return ACE_ENOMEM;
+    }
+}
+
 #define ACE_HIP(call)                                                                          \
     do {                                                                                       \
         hipError_t e_ = (call);                                                                \
@@ -1057,14 +1066,14 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = upload((void **)&h->d_rows, t->rows, (size_t)t->num_types * row_bytes, (size_t)t->num_types * row_bytes + 4096u)) ||
         (rc = upload((void **)&h->d_pos_info, t->pos_info, (size_t)(t->num_ops + 1) * 4, pos_entries * 4)) ||
         (rc = upload_pos4(h, t, pos_entries, pk32_off)) ||
-        (rc = upload_pos_types(h, t, pos_entries)) || (rc = upload_pos_spread(h, t, pos_entries)) ||
+        (rc = upload_pos_types(h, t, pos_entries)) || (rc = or_enomem([&] { return upload_pos_spread(h, t, pos_entries); })) ||
         (rc = upload((void **)&h->d_pair_kinds, t->pair_kinds, (size_t)rk_bytes)) ||
         (rc = upload((void **)&h->d_stage_lut, t->stage_lut, (size_t)stg_words * 4)) ||
         (rc = upload((void **)&h->d_nbm1, t->nb_minus_1, (size_t)t->n_mbs * 8)) ||
         (rc = upload((void **)&h->d_win_pos, t->win_pos, (size_t)(t->n_windows + 1) * 4)) ||
         (rc = upload((void **)&h->d_win_row_begin, t->win_row_begin, (size_t)(t->n_windows + 1) * 4)) ||
         (rc = upload((void **)&h->d_win_rows, t->win_rows, (size_t)n_win_rows * 8)) ||
-        (rc = setup_windowed_asm(h, t, pos_entries, rk_bytes, stg_words)) ||
+        (rc = or_enomem([&] { return setup_windowed_asm(h, t, pos_entries, rk_bytes, stg_words); })) ||
         (rc = allow_big_lds<false, false, false, false>()) || (rc = allow_big_lds<false, false, true, false>()) ||
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
@@ -1553,7 +1562,8 @@ int ace_recompute_prepare(ace_handle_t *h, const int32_t *type_of_pos, const dou
     if (lds > kMaxLds) return ACE_ETOOBIG;
     ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_rc_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_rc_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
-    std::vector<ace_u2> pos((size_t)N);
+    std::vector<ace_u2> pos;
+    if (or_enomem([&] { return pos.resize((size_t)N), ACE_OK; })) return ACE_ENOMEM;
     ace_rc_positions(type_of_pos, no_recompute, N, h->num_types, pos.data());
     if (h->d_rc_pos) (void)hipFree(h->d_rc_pos);
     if (h->d_rc_act) (void)hipFree(h->d_rc_act);
@@ -1699,8 +1709,10 @@ int ace_build_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int 
                     int max_templates, int *n_templates_out) {
     if (!moves_args(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, draws, moves_out, t_codes_out, t_hdr_out, n_templates_out))
         return ACE_EINVAL;
-    return ace_build_moves_body(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, *draws, moves_out, t_codes_out, t_hdr_out,
-                                max_templates, n_templates_out);
+    return or_enomem([&] {
+        return ace_build_moves_body(codes, hdr, num_ops, n_algo, n_tp, n_mbs, stage_lut, gpus_per_node, *draws, moves_out, t_codes_out,
+                                    t_hdr_out, max_templates, n_templates_out);
+    });
 }
 
 int ace_new_moves(const uint8_t *codes, const uint32_t *hdr, int num_ops, int n_algo, int n_tp, int n_mbs, const uint32_t *stage_lut,

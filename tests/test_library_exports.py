@@ -89,6 +89,33 @@ def test_no_gpu_means_no_scoring():
         evaluator.PlanEvaluator(tables)
 
 
+OUT_OF_MEMORY = """
+import ctypes, resource
+import numpy as np
+from superscaler_amd import evaluator
+lib = evaluator.load_library()
+d = evaluator.AceMoveDrawsStruct()
+d.n = 1
+codes, hdr, out = np.full(16, 16, dtype=np.uint8), np.array([1, 0, 0, 0], dtype=np.uint32), np.zeros(4096, dtype=np.uint32)
+codes[1:] = 0
+n = ctypes.c_int(0)
+used = int(open("/proc/self/statm").read().split()[0]) * resource.getpagesize()
+resource.setrlimit(resource.RLIMIT_AS, (used + (1 << 28), used + (1 << 28)))
+# (a table of 2^30 micro-batch sizes: 16 GiB that are asked for before anything is read)
+rc = lib.ace_build_moves(codes.ctypes.data, hdr.ctypes.data, 16, 2, 4, 1 << 30, out.ctypes.data, 8, ctypes.byref(d), out.ctypes.data, out.ctypes.data,
+                         out.ctypes.data, 3, ctypes.byref(n))
+print("code", rc)
+"""
+
+
+def test_a_call_that_runs_out_of_memory_returns_a_code():
+    import subprocess
+    import sys
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    proc = subprocess.run([sys.executable, "-c", OUT_OF_MEMORY], cwd=root, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+    assert proc.returncode == 0 and "code -4" in proc.stdout, (proc.returncode, proc.stdout[-500:])
+
+
 def test_header_is_plain_c_and_matches_the_library(tmp_path):
     """include/ace_eval.h compiles as C99 on its own, and a C program that takes the address of every
     declared function links against the library (the declarations and the exports agree)."""
