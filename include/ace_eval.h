@@ -128,10 +128,9 @@ typedef struct ace_batch {
     const uint32_t *d_order;   /* NULL, or uint32[n_plans]: slot i of d_codes / d_hdr / d_range holds the caller's plan
                                   d_order[i], and every result of that plan (d_iter_ms, d_peak_mb, d_feasible,
                                   d_status, d_stage_out) is written at index d_order[i].  Lets the caller store the
-                                  plans in the order that suits the kernel -- lanes of a wavefront that close their
-                                  stages at the same ops do not wait for each other, so grouping plans by pipeline
-                                  depth (deepest first) and first stage boundaries is worth about a seventh of the
-                                  kernel time on mixed batches -- and still get results in its own order.  Must be
+                                  plans in another order than it wants its results in.  (The kernels group a
+                                  workgroup's plans by pipeline depth themselves: storing a whole batch by depth and
+                                  first stage boundaries is worth one percent of the kernel time on mixed batches.)  Must be
                                   a permutation of 0 .. n_plans - 1 (entries >= n_plans are skipped). */
 } ace_batch_t;
 
@@ -151,6 +150,7 @@ void ace_destroy(ace_handle_t *h);
  *  d_stage_out: NULL, or double[n_plans][ACE_MAX_STAGES][ACE_STAGE_REC] receiving the per-stage
  *  quantities predict_time_breakdown / predict_stage_time / predict_stage_memory are made of; for a
  *  batch of single-stage queries (batch->d_range) one record each: double[n_plans][ACE_STAGE_REC].
+ *  The records of a plan whose status is not ACE_PLAN_OK hold no particular values.
  * Plain scoring (no d_stage_out, no d_range) uses a workspace owned by the handle (80 bytes per plan
  * and stage, allocated on first use and grown when a larger batch arrives: that call allocates, unless
  * ace_reserve() sized or fixed it beforehand), so scoring calls on one handle must be stream-ordered with
