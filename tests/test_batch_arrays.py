@@ -91,6 +91,7 @@ def fake_evaluator(tables, calls):
     """A PlanEvaluator whose library only records what it is handed."""
     import torch
     ev = PlanEvaluator.__new__(PlanEvaluator)
+    ev._plan_bytes = 16 * ((tables.graph.num_ops + 15) // 16)
     ev.tables, ev.device, ev.handle, ev._torch = tables, torch.device("cuda", 0), None, types.SimpleNamespace(
         _C=types.SimpleNamespace(_cuda_getCurrentRawStream=lambda device: device))
 
