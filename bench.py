@@ -83,7 +83,7 @@ def kernel_name(tables, n_plans):
         return "ace_spread_kernel"
     if not windowed and n_plans <= 65536:
         return "ace_duo_kernel"
-    return "ace_many_kernel<WIN=%s>" % ("true" if windowed else "false")
+    return "ace_many_kernel<WIN=true>" if windowed else "ace_dense_kernel"
 
 
 def other_workloads(steps):

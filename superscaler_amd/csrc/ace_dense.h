@@ -1,0 +1,485 @@
+// Scoring of LARGE batches over dense tables: a plan per lane, like ace_many.h, but what an op costs a lane beside the
+// reference's own additions is as little as could be found: two v_dot4_u32_u8 for all addresses, one 8-byte LDS read per value,
+// one 16-byte read for both collectives' costs, and records that are stored in whole cache lines (gen_dense_loop_asm.py).  The
+// tables take less than half of a CU's LDS in the form below, so two workgroups of eight wavefronts share a CU, and one evaluates
+// its stage tails or stages its tables while the other walks.
+// From 65,537 plans on, where the tables fit this form: 40 (resharding off) or 64 entries per row, and 80 KB.
+// Measured, us per launch, ace_many.h -> here:
+//   plans      315 ops           523 ops           821 ops, no resharding   1,251 ops, 16 stages
+//   65,537     64.2 ->  58.9     130.1 -> 117.5    134.7 -> 113.9           285.1 -> 235.2
+//   100,000    65.5 ->  60.1     131.4 -> 120.9    135.8 -> 116.2           287.8 -> 238.8
+//   262,144   102.4 ->  88.6     176.9 -> 149.5    167.0 -> 148.7           461.0 -> 398.3
+//   1,048,576                    694.0 -> 555.9
+//   (523 ops, 1,048,576 plans, all of one stage: 447 -> 357, all of sixteen: 1,456 -> 981)
+// What bounds it is the issue of vector instructions: about 30 per op and wavefront of the mix of depths (35 before), and the issue
+// of everything else beside them; with fewer than four wavefronts per SIMD the latency of a step.  One workgroup of 1,024 lanes per
+// CU instead: 594 us where two of 512 took 567.
+//
+// The dense tables, one block that is copied to LDS address 0 on:
+//   pairs   16 bytes {forward, backward} ms of resharding, every distinct pair once, {0, 0} first
+//   rows    per op type used: five arrays of `entries` doubles (ACE_DENSE_ARRAY bytes each): forward, backward, weights,
+//           activations, and the ranks of the two reserved sizes (16 bits each) among all that occur; indexed diag * C + code
+//           as the table compiler's rows are
+//   slabs   per distinct (pair kind, next op's type): blocks of [code][next code] 16-bit addresses into `pairs`, one block per
+//           distinct (diag, stage size)
+//   lut     per (micro-batch size, stage size): LDS address of the diag's entries in the first row, of its block in the first slab
+//   stages  the stage LUT as it is
+// and what the evaluation of the stage tails looks up (from global memory those were six gathers per stage, 1 ns per lane and CU
+// each: 115 of 760 us per 1,048,576 plans of 523 ops):
+//   reserved sizes by rank; per (row, diag * C + code) and per (row, output entry) a 16-bit LDS address of the distinct
+//   {input MB, intra-node ms, inter-node ms} and {output intra, inter}
+// With two algorithms and four tp sizes most codes in use are even, and diags four apart lie 256 bytes apart: from the fourth on
+// they lie 8 bytes further, so that their even codes read different banks.  Blocks of a slab are 132 bytes apart for the same reason.
+// What a code byte reads that names no profiled entry (codes past the last tp size) is what it reads in the table compiler's
+// rows: the tables are filled by those addresses.
+#pragma once
+#include <algorithm>
+#include <cstring>
+#include <map>
+#include <utility>
+#include <vector>
+
+#include "ace_score_loop.h"
+
+constexpr uint32_t kDenseLds = 80u * 1024u;    // LDS of a workgroup: two per CU
+constexpr int kDenseLanes = 512;
+
+struct AceDenseArgs {
+    const ace_u4 *image;        // the tables
+    const ace_u4 *pos;          // [16 * G + 16] per position: dot4 scalars of the row and of the slab, record word, flags (as pos4)
+    uint32_t image16;           // size of the image in 16-byte pieces
+    uint32_t lut_off, stg_off, rf_off, rb_off, in_off, out_off;   // LDS offsets
+    uint32_t in_entries, out_entries;   // 16-bit addresses per row
+    uint32_t kv;                // constant byte(s) of the code words
+    uint32_t row0;              // row of the first op
+};
+
+// What the library keeps of it (built on the host).
+struct AceDenseTables {
+    std::vector<unsigned char> image;
+    std::vector<ace_u4> pos;
+    AceDenseArgs args{};        // (offsets)
+    uint32_t array = 0;
+    bool ok = false;
+};
+
+// LDS behind the image: the deal's bins and permutation, the arrival counters.
+inline uint32_t ace_dense_lds(uint32_t image_bytes) { return ((image_bytes + 15u) & ~15u) + 128u + 2u * (uint32_t)kDenseLanes + 128u; }
+
+// Fills `d` from tables whose rows are all resident (d.ok false: they do not fit this form).
+inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseTables &d) {
+    d = AceDenseTables();
+    const int N = t->num_ops, C = t->n_tp * t->n_algo, ND = t->n_diag;
+    if (t->n_windows != 1 || (t->flags & ACE_F_COLLECTIVE_MEM) || t->num_types > 256 || N >= 32768) return;
+    const bool rsh = (t->flags & ACE_F_RESHARDING) != 0;
+    const uint32_t entries = (uint32_t)(ND * C + 8), array = entries <= 40u ? 320u : entries <= 64u ? 520u : 0u;
+    if (!array) return;
+    auto diag_entry = [&](uint32_t dg) { return dg * (uint32_t)C + (C == 8 && t->n_algo == 2 && dg >= 4u ? 1u : 0u); };
+    const size_t n_rows_all = (size_t)t->num_types * (size_t)t->row_doubles;
+    auto at = [&](size_t type, size_t off) {                       // a double of a row, or of what follows it in memory
+        const size_t i = type * (size_t)t->row_doubles + off;
+        return i < n_rows_all ? t->rows[i] : 0.0;
+    };
+    std::vector<uint32_t> types(pos_entries);
+    ace_pos_types(t, types.data(), pos_entries);
+    // rows in use, in the order of their types
+    std::vector<int> row_of(256, -1);
+    std::vector<uint32_t> used;
+    for (int i = 0; i < N; ++i) row_of[types[i] & 0xffu] = 0;
+    for (uint32_t ty = 0; ty < 256u; ++ty)
+        if (row_of[ty] == 0) { row_of[ty] = (int)used.size(); used.push_back(ty); }
+    // ranks of the reserved sizes: what a running maximum from 0.0 can become (0.0: rank 0)
+    std::vector<double> reserved_fwd, reserved_bwd, *const values[2] = {&reserved_fwd, &reserved_bwd};
+    for (int w = 0; w < 2; ++w) {
+        std::vector<double> &v = *values[w];
+        for (uint32_t ty : used)
+            for (uint32_t e = 0; e < entries; ++e) {
+                const double x = at(ty, (size_t)t->hot_off + e * 6u + 4u + (size_t)w);
+                if (x > 0.0) v.push_back(x);
+            }
+        v.push_back(0.0);
+        std::sort(v.begin(), v.end());
+        v.erase(std::unique(v.begin(), v.end()), v.end());
+        if (v.size() > 65536u) return;
+    }
+    auto rank = [&](int w, double x) {
+        return x > 0.0 ? (uint32_t)(std::lower_bound(values[w]->begin(), values[w]->end(), x) - values[w]->begin()) : 0u;
+    };
+    // pairs, slabs, blocks
+    std::vector<std::pair<uint64_t, uint64_t>> pairs{{0u, 0u}};
+    std::map<std::pair<uint64_t, uint64_t>, uint32_t> pair_at{{{0u, 0u}, 0u}};
+    std::vector<uint32_t> slab_of(pos_entries, 0u);                // per position, of the (this op, next op) pair
+    std::vector<uint32_t> block_of((size_t)t->n_mbs * 16u, 0u);
+    std::vector<std::vector<uint16_t>> slabs;                      // [slab][block * 64 + code * 8 + next code]
+    size_t n_blocks = 1;
+    constexpr uint32_t kBlock = 132u;
+    if (rsh) {
+        std::vector<std::pair<uint32_t, uint32_t>> kinds, stages;   // (pair kind, next type); (diag, stage size as the pair kinds index it)
+        std::vector<uint32_t> kind_of(N, 0u), stage_of((size_t)t->n_mbs * 16u);
+        auto index = [](std::vector<std::pair<uint32_t, uint32_t>> &v, std::pair<uint32_t, uint32_t> x) {
+            const auto it = std::find(v.begin(), v.end(), x);
+            if (it != v.end()) return (uint32_t)(it - v.begin());
+            v.push_back(x);
+            return (uint32_t)v.size() - 1u;
+        };
+        for (int i = 0; i + 1 < N; ++i) kind_of[i] = index(kinds, {(t->pos_info[i] >> 16) & 0xffu, types[i + 1] & 0xffu});
+        if (kinds.empty()) kinds.push_back({0u, types[0] & 0xffu});
+        for (uint32_t j = 0; j < (uint32_t)t->n_mbs * 16u; ++j)
+            stage_of[j] = index(stages, {t->stage_lut[j] & 15u, (j & 15u) < (uint32_t)t->n_glog ? j & 15u : 0u});
+        // a stage's block over all kinds at once: equal ones are kept once
+        std::vector<std::vector<uint16_t>> columns;
+        std::vector<uint32_t> column_of;
+        for (const auto &st : stages) {
+            std::vector<uint16_t> col;
+            for (const auto &k : kinds)
+                for (uint32_t cc = 0; cc < 64u; ++cc) {
+                    const uint32_t id = t->pair_kinds[((size_t)k.first * t->n_glog + st.second) * 64u + cc];
+                    const size_t e = (size_t)t->z_off + st.first * (uint32_t)C + (cc & 7u);
+                    std::pair<uint64_t, uint64_t> p;
+                    const double f = at(k.second, e + (size_t)(id & 15u) * t->z_table_doubles), b = at(k.second, e + (size_t)(id >> 4) * t->z_table_doubles);
+                    memcpy(&p.first, &f, 8);
+                    memcpy(&p.second, &b, 8);
+                    const auto ins = pair_at.insert({p, (uint32_t)pairs.size()});
+                    if (ins.second) pairs.push_back(p);
+                    if (pairs.size() > 4096u) return;               // (16-bit LDS addresses)
+                    col.push_back((uint16_t)(ins.first->second * 16u));
+                }
+            uint32_t c = (uint32_t)(std::find(columns.begin(), columns.end(), col) - columns.begin());
+            if (c == columns.size()) columns.push_back(col);
+            column_of.push_back(c);
+        }
+        n_blocks = columns.size();
+        for (size_t j = 0; j < block_of.size(); ++j) block_of[j] = column_of[stage_of[j]];
+        // ... and equal slabs
+        std::vector<uint32_t> slab_of_kind;
+        for (size_t k = 0; k < kinds.size(); ++k) {
+            std::vector<uint16_t> s;
+            for (const auto &col : columns) s.insert(s.end(), col.begin() + k * 64u, col.begin() + (k + 1u) * 64u);
+            uint32_t at_slab = (uint32_t)(std::find(slabs.begin(), slabs.end(), s) - slabs.begin());
+            if (at_slab == slabs.size()) slabs.push_back(s);
+            slab_of_kind.push_back(at_slab);
+        }
+        for (int i = 0; i + 1 < N; ++i) slab_of[i] = slab_of_kind[kind_of[i]];
+    }
+    // the constant byte K and how far apart rows and slabs lie: multiples of it, at most 255 for the last one
+    const uint32_t n_rows = (uint32_t)used.size(), n_slabs = (uint32_t)slabs.size(), slab_bytes = (uint32_t)n_blocks * kBlock;
+    uint32_t K = 0, row_pitch = array * 5u, slab_pitch = 0;
+    if (rsh) {
+        uint64_t best = ~0ull;
+        for (uint32_t k = 8; k <= 248u; k += 8u) {
+            const uint32_t u = (array * 5u + k - 1u) / k, v = (slab_bytes + k - 1u) / k;
+            if ((n_rows - 1u) * u > 255u || (n_slabs - 1u) * v > 255u) continue;
+            const uint64_t size = (uint64_t)n_rows * u * k + (uint64_t)n_slabs * v * k;
+            if (size < best) { best = size; K = k; row_pitch = u * k; slab_pitch = v * k; }
+        }
+        if (!K) return;
+    } else if ((n_rows - 1u) * row_pitch > 248u * 255u + 247u) return;   // (two constant bytes: 248 and 8)
+    AceDenseArgs &g = d.args;
+    g.kv = rsh ? K << 24 : (248u << 24) | (8u << 16);
+    // what the evaluation looks up: distinct {input MB, intra, inter} and {output intra, inter}, their place per row and entry
+    typedef std::vector<uint64_t> Bits;
+    std::vector<Bits> values_in, values_out;
+    auto place_of = [&](std::vector<Bits> &v, uint32_t ty, size_t off, size_t n) {
+        Bits b(n);
+        for (size_t k = 0; k < n; ++k) {
+            const double x = at(ty, off + k);
+            memcpy(&b[k], &x, 8);
+        }
+        const size_t i = (size_t)(std::find(v.begin(), v.end(), b) - v.begin());
+        if (i == v.size()) v.push_back(b);
+        return (uint32_t)i;
+    };
+    g.in_entries = entries;
+    g.out_entries = (uint32_t)(t->n_mbs * t->n_tp + 8) * (uint32_t)t->n_algo;    // (a code past the last tp size: up to index 7)
+    std::vector<uint32_t> in_of, out_of;
+    for (uint32_t ty : used) {
+        for (uint32_t e = 0; e < g.in_entries; ++e) in_of.push_back(place_of(values_in, ty, (size_t)t->start_off + e * 3u, 3));
+        for (uint32_t e = 0; e < g.out_entries; ++e) out_of.push_back(place_of(values_out, ty, (size_t)t->out_off + e * 2u, 2));
+    }
+    // the image (what 16-bit addresses name lies in front)
+    uint32_t end = 0;
+    auto take = [&](size_t bytes, uint32_t align) {
+        const uint32_t off = (end + align - 1u) / align * align;
+        end = off + (uint32_t)bytes;
+        return off;
+    };
+    take(pairs.size() * 16u, 16u);
+    const uint32_t vout_off = take(values_out.size() * 16u, 16u), vin_off = take(values_in.size() * 24u, 8u);
+    if (end > 65536u) return;
+    const uint32_t rows_off = take((size_t)n_rows * row_pitch, 16u), slabs_off = take((size_t)n_slabs * slab_pitch, 16u);
+    g.lut_off = take((size_t)t->n_mbs * 128u, 128u);
+    g.stg_off = take((size_t)t->n_mbs * 64u, 4u);
+    g.rf_off = take(reserved_fwd.size() * 8u, 8u);
+    g.rb_off = take(reserved_bwd.size() * 8u, 8u);
+    g.in_off = take(in_of.size() * 2u, 2u);
+    g.out_off = take(out_of.size() * 2u, 2u);
+    const uint32_t bytes = take(0, 16u);
+    if (ace_dense_lds(bytes) > kDenseLds) return;
+    g.image16 = bytes / 16u;
+    d.image.assign(bytes, 0);
+    auto put = [&](uint32_t off, const void *p, size_t n) { if (n) memcpy(d.image.data() + off, p, n); };
+    for (size_t i = 0; i < pairs.size(); ++i) {
+        put((uint32_t)i * 16u, &pairs[i].first, 8);
+        put((uint32_t)i * 16u + 8u, &pairs[i].second, 8);
+    }
+    for (size_t i = 0; i < values_out.size(); ++i) put(vout_off + (uint32_t)i * 16u, values_out[i].data(), 16);
+    for (size_t i = 0; i < values_in.size(); ++i) put(vin_off + (uint32_t)i * 24u, values_in[i].data(), 24);
+    for (size_t i = 0; i < in_of.size(); ++i) {
+        const uint16_t a16 = (uint16_t)(vin_off + in_of[i] * 24u);
+        put(g.in_off + (uint32_t)i * 2u, &a16, 2);
+    }
+    for (size_t i = 0; i < out_of.size(); ++i) {
+        const uint16_t a16 = (uint16_t)(vout_off + out_of[i] * 16u);
+        put(g.out_off + (uint32_t)i * 2u, &a16, 2);
+    }
+    put(g.rf_off, reserved_fwd.data(), reserved_fwd.size() * 8u);
+    put(g.rb_off, reserved_bwd.data(), reserved_bwd.size() * 8u);
+    for (uint32_t r = 0; r < n_rows; ++r)
+        for (uint32_t dg = 0; dg <= (uint32_t)ND; ++dg)
+            for (uint32_t c = 0; c < 8u; ++c) {
+                // (a code past the last one reads what follows its diag's entries)
+                const uint32_t e = dg * (uint32_t)C + c, to = rows_off + r * row_pitch + (diag_entry(dg) + c) * 8u;
+                if (c >= (uint32_t)C && dg < (uint32_t)ND) continue;
+                double v[6];
+                for (uint32_t k = 0; k < 6u; ++k) v[k] = at(used[r], (size_t)t->hot_off + e * 6u + k);
+                for (uint32_t k = 0; k < 4u; ++k) put(to + k * array, &v[k], 8);
+                const uint32_t both = rank(0, v[4]) | (rank(1, v[5]) << 16);
+                put(to + 4u * array, &both, 4);
+            }
+    for (uint32_t s = 0; s < n_slabs; ++s)
+        for (uint32_t b = 0; b < (uint32_t)n_blocks; ++b) put(slabs_off + s * slab_pitch + b * kBlock, slabs[s].data() + b * 64u, 128);
+    for (uint32_t j = 0; j < (uint32_t)t->n_mbs * 16u; ++j) {
+        const ace_u2 z{rows_off + diag_entry(t->stage_lut[j] & 15u) * 8u, slabs_off + block_of[j] * kBlock};
+        put(g.lut_off + j * 8u, &z, 8);
+        put(g.stg_off + j * 4u, &t->stage_lut[j], 4);
+    }
+    // positions
+    d.pos.assign(pos_entries, ace_u4{0u, 0u, 0u, 0u});
+    for (size_t i = 0; i < pos_entries; ++i) {
+        const bool odd = (i & 1u) != 0u, in = i < (size_t)N;
+        const uint32_t info = in ? t->pos_info[i] : 0u;
+        const uint32_t row = in ? (uint32_t)row_of[types[i] & 0xffu] : 0u, place = row * row_pitch, slab = in ? slab_of[i] : 0u;
+        const uint32_t last = in ? (uint32_t)row_of[types[i] & 0xffu] : 0u, next = in ? (uint32_t)row_of[(types[i] >> 8) & 0xffu] : 0u;
+        ace_u4 &p = d.pos[i];
+        p.x = (odd ? 8u << 8 : 8u) | (rsh ? (place / K) << 24 : ((place / 248u) << 24) | (((place % 248u) / 8u) << 16));
+        p.y = rsh ? (odd ? (16u << 8) | (2u << 16) : 16u | (2u << 8)) | ((slab * (slab_pitch / K)) << 24) : 0u;
+        // record word: codes of the stage's last op and of the next one in bytes 0 and 1 (odd positions with resharding: 1
+        // and 2, bit 11 set), rows of both in the other two
+        p.z = rsh && odd ? last | (next << 24) | (1u << 11) : (last << 16) | (next << 24);
+        p.w = (((info >> 24) & 1u) ^ 1u) | (((info >> 25) & 1u) << 1);
+    }
+    d.array = array;
+    g.row0 = (uint32_t)row_of[types[0] & 0xffu];
+    d.ok = true;
+}
+
+// What a record word says.
+struct DenseMeta { uint32_t c_last, c_next, row_last, row_next; };
+ACE_HD DenseMeta dense_meta(uint32_t m) {
+    const bool odd = (m >> 11) & 1u;
+    const uint32_t w = odd ? m >> 8 : m;
+    return DenseMeta{w & 7u, (w >> 8) & 7u, (odd ? m : m >> 16) & 0xffu, m >> 24};
+}
+
+// Slices of 64 plans per workgroup, so that the rounds of two workgroups per CU that the batch needs are all full.
+inline uint32_t ace_dense_slices(long long plans) {
+    const long long most = kDenseLanes / 64, fullest = ((plans + 63) / 64 + 511) / 512;
+    const long long rounds = (fullest + most - 1) / most;
+    return (uint32_t)((fullest + rounds - 1) / rounds);
+}
+
+// A wavefront's part of the workspace: the records of its plans' stages in the order in which they were stored, as five pieces of up
+// to 1,024 times 16 bytes -- {fwd + bwd, recompute}, {resharding forward, backward}, {weights, activations}, {saved, peak},
+// {ranks, record word, record word of the stage before, place} --, and behind them what each came to: {ms, MB} at [stage][lane].
+// A place is stage * 128 + lane * 2.
+constexpr uint32_t kDensePiece = 64u * ACE_MAX_STAGES * 16u, kDenseResults = 5u * kDensePiece, kDenseWave = 6u * kDensePiece;
+static_assert(kDensePiece == 16384u, "as the loop has it");
+constexpr uint32_t kDensePlan = kDenseWave / 64u;                // workspace bytes per plan
+
+typedef PlanState<false, false, true> DenseState;
+struct DenseRecord { ace_d2 r[4]; ace_u4 tail; };
+ACE_HD void dense_load(const unsigned char *ws, uint32_t i, DenseRecord &rec) {
+#pragma unroll
+    for (uint32_t j = 0; j < 4u; ++j) rec.r[j] = *reinterpret_cast<const ace_d2 *>(ws + j * kDensePiece + i * 16u);
+    rec.tail = *reinterpret_cast<const ace_u4 *>(ws + 4u * kDensePiece + i * 16u);
+}
+
+#ifdef ACE_HOST_EMU
+ACE_HD uint32_t dense_shfl(uint32_t x, uint32_t) { return x; }   // (wavefronts of one lane)
+constexpr uint32_t kDenseWidth = 1;
+#else
+ACE_HD uint32_t dense_shfl(uint32_t x, uint32_t lane) { return (uint32_t)__shfl((int)x, (int)lane, 64); }
+constexpr uint32_t kDenseWidth = 64;
+#endif
+
+// One record: time and memory of its stage, in st.sum_t and st.max_mem.  `own`: the lane's own plan (its header's words reach the
+// lanes that evaluate its stages through dense_shfl).
+ACE_HD void dense_stage(const AceDenseArgs &d, const AceGeom &g, const AceLds &lds, const DenseState &own, const DenseRecord &rec, DenseState &st) {
+    const uint32_t lane = (rec.tail.w >> 1) & 63u, s = rec.tail.w >> 7;
+    const uint32_t sb = dense_shfl((uint32_t)own.S | (own.bidx << 8), lane);
+    const uint32_t glogs = dense_shfl((uint32_t)own.glogs, lane), glogs_hi = dense_shfl((uint32_t)(own.glogs >> 32), lane);
+    st.cross = dense_shfl(own.cross, lane);
+    st.S = (int)(sb & 0xffu);
+    st.s = (int)s;
+    const uint32_t glog = ((s & 8u ? glogs_hi : glogs) >> (4u * (s & 7u))) & 15u;
+    const DenseMeta m = dense_meta(rec.tail.y), before = dense_meta(rec.tail.z);
+    const uint32_t lut = lds.ld<uint32_t>(d.stg_off + ((sb >> 8) * 16u + glog) * 4u);
+    st.mrow = lut >> 16;
+    st.t_first = before.c_next >> g.A_shift;
+    const uint32_t e = ace_mul24(lut & 15u, (uint32_t)g.C) + before.c_next, o = DenseState::out_entry_addr(g, 0u, m.c_last, st.t_first, st.mrow) >> 4;
+    const uint32_t in = lds.ld<uint16_t>(d.in_off + (ace_mul24(before.row_next, d.in_entries) + e) * 2u);
+    const uint32_t out = lds.ld<uint16_t>(d.out_off + (ace_mul24(m.row_last, d.out_entries) + o) * 2u);
+    st.rfm = lds.ld<double>(d.rf_off + (rec.tail.x & 0xffffu) * 8u);
+    st.rbm = lds.ld<double>(d.rb_off + (rec.tail.x >> 16) * 8u);
+    st.inputs = lds.ld<double>(in);
+    st.in_comm = lds.ld<double>(in + (((st.cross >> s) & 1u) ? 16u : 8u));
+    const ace_d2 oe = lds.ld<ace_d2>(out);
+    st.out_cross = (st.cross >> (16u + s)) & 1u;
+    // (fwd + bwd is added up already, and the peak closed)
+    st.fwd = rec.r[0].x; st.bwd = 0.0; st.rcs = rec.r[0].y; st.rs_f = rec.r[1].x; st.rs_b = rec.r[1].y; st.W = rec.r[2].x; st.A = rec.r[2].y;
+    st.saved = rec.r[3].x; st.peak = rec.r[3].y; st.run = 0.0; st.lastclose = false;
+    st.sum_t = 0.0; st.max_t = 0.0; st.max_mem = 0.0;
+    st.finish_tail(g, lds, 0u, m.c_last, oe, nullptr);
+}
+
+// The tails of all stages of a wavefront's plans, a record per lane whoever's it is (all lanes are busy whatever the depths of the
+// plans), the next two rounds' records on their way; then each lane puts its own plan together, stage times in order.
+ACE_HD void dense_replay(const AceDenseArgs &d, const AceGeom &g, const AceLds &lds, DenseState &own, unsigned char *ws, uint32_t lane,
+                         uint32_t stored, int n_st) {
+    DenseRecord r[3];
+    auto fetch = [&](uint32_t round, DenseRecord &rec) {
+        const uint32_t i = round * kDenseWidth + lane;
+        dense_load(ws, i < stored ? i : stored - 1u, rec);
+    };
+    if (stored == 0u) return;                                      // (plans of more stages than there may be)
+    const uint32_t rounds = (stored + kDenseWidth - 1u) / kDenseWidth;
+    fetch(0, r[0]);
+    fetch(1, r[1]);
+    fetch(2, r[2]);
+    for (uint32_t base = 0; base < rounds; base += 3u) {
+#pragma unroll
+        for (uint32_t k = 0; k < 3u; ++k) {
+            const uint32_t round = base + k;
+            if (round >= rounds) break;
+            DenseState st;
+            dense_stage(d, g, lds, own, r[k], st);
+            const uint32_t place = r[k].tail.w;
+            if (round + 3u < rounds) fetch(round + 3u, r[k]);
+            if (round * kDenseWidth + lane < stored)
+                *reinterpret_cast<ace_d2 *>(ws + kDenseResults + (place >> 7) * 1024u + ((place >> 1) & 63u) * 16u) = ace_d2{st.sum_t, st.max_mem};
+        }
+    }
+#ifndef ACE_HOST_EMU
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#endif
+    const int n = n_st < ACE_MAX_STAGES ? n_st : ACE_MAX_STAGES;
+    for (int base = 0; base < ACE_MAX_STAGES; base += 4) {
+        if (!ACE_ANY(base < n)) return;
+        ace_d2 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] = base + k < n ? *reinterpret_cast<const ace_d2 *>(ws + kDenseResults + (uint32_t)(base + k) * 1024u + lane * 16u) : ace_d2{0.0, 0.0};
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (base + k < n) {
+                own.sum_t += v[k].x;
+                own.max_t = ace_max(own.max_t, v[k].x);
+                own.max_mem = ace_max(own.max_mem, v[k].y);
+            }
+    }
+}
+
+#ifndef ACE_HOST_EMU
+#include "ace_dense_loop_asm.inc"
+
+// The op loop: returns the number of stages of the lane's plan, and in `stored` that of the wavefront's records; `ws`: the
+// wavefront's part of the workspace.  Arrays of the rows lie A bytes apart.
+template <int A>
+__device__ __forceinline__ uint32_t dense_loop(const AceKernelArgs &a, const AceDenseArgs &d, uint64_t glogs, uint32_t lut2, uint64_t zvrk, uint32_t code_off,
+                                               const unsigned char *ws, uint32_t lane, uint32_t meta0, uint32_t pace, uint32_t pace_mask, uint32_t &stored) {
+    uint32_t placed;
+    const uint64_t gstride = (uint64_t)(uint32_t)a.g.P * 16u;
+    const uint32_t gs_lo = (uint32_t)gstride, gs_hi = (uint32_t)(gstride >> 32);
+#define ACE_DENSE_RUN(TEXT)                                                                                                       \
+    asm volatile(TEXT : [placed] "=&v"(placed), [stored] "=&v"(stored)                                                           \
+                 : [glogs] "v"(glogs), [lut2] "v"(lut2), [zvrk] "v"(zvrk), [codeoff] "v"(code_off), [place] "v"(lane * 2u), [meta0] "v"(meta0), \
+                   [codes] "s"(a.codes), [pos] "s"(d.pos), [n_ops] "s"(a.g.N), [recbase] "s"(ws),                               \
+                   [gstride_lo] "s"(gs_lo), [gstride_hi] "s"(gs_hi), [pace] "s"(pace), [pacemask] "s"(pace_mask),                \
+                   [kv] "s"(d.kv), [a1] "n"(A), [a2] "n"(2 * A), [a3] "n"(3 * A), [a4] "n"(4 * A)                                \
+                 : ACE_DENSE_ASM_CLOBBERS)
+    if (a.g.flags & ACE_F_RESHARDING) ACE_DENSE_RUN(ACE_DENSE_ASM_RSH1);
+    else ACE_DENSE_RUN(ACE_DENSE_ASM_RSH0);
+#undef ACE_DENSE_RUN
+    return placed >> 7;
+}
+
+// One workgroup; its LDS array starts at address 0 (the kernel has no other LDS variables).
+template <int A> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
+                                                                int tid, long long block) {
+    constexpr int kLanes = kDenseLanes;
+    const AceGeom &g0 = a.g;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6), lane = (uint32_t)tid & 63u;
+    const uint32_t lanes = 64u * slices;
+    {
+        typedef const void __attribute__((address_space(1))) *gptr;
+        typedef void __attribute__((address_space(3))) *lptr;
+        for (uint32_t at = wave * 64u; at < d.image16; at += kLanes)
+            if (at + lane < d.image16) __builtin_amdgcn_global_load_lds((gptr)(d.image + at + lane), (lptr)(lds_raw + at * 16u), 16, 0, 0);
+    }
+    // Deal: counting sort of the plans by pipeline depth, the deepest first (see ace_score_body); sorted slice q goes to
+    // wavefront q in rows of four, every second row reversed: each SIMD gets the same mix.
+    unsigned int *cnt = reinterpret_cast<unsigned int *>(lds_raw + d.image16 * 16u);
+    unsigned short *plan_of = reinterpret_cast<unsigned short *>(cnt + 32);
+    uint32_t *pace = reinterpret_cast<uint32_t *>(plan_of + kLanes);
+    const uint32_t q = (wave & 4u) ? wave ^ 3u : wave;
+    if (tid < 32) { cnt[tid] = 0u; pace[tid] = 0u; }
+    const long long slot = block * lanes + tid;
+    uint32_t depth = 0, rank = 0;                                   // (slots past the batch: last)
+    if ((uint32_t)tid < lanes && slot < g0.P) {
+        depth = a.hdr[slot].x & 0xffu;
+        depth = depth > 16u ? 16u : depth;
+    }
+    __syncthreads();
+    if ((uint32_t)tid < lanes) rank = atomicAdd(&cnt[16u - depth], 1u);
+    __syncthreads();
+    if ((uint32_t)tid < lanes) {
+        for (uint32_t b = 0; b < 16u - depth; ++b) rank += cnt[b];
+        plan_of[rank] = (unsigned short)tid;
+    }
+    __syncthreads();
+    const uint32_t at = (q << 6) | lane;
+    const long long plan = block * lanes + (q < slices ? (uint32_t)plan_of[at] : 0u);
+    const bool in_batch = plan < g0.P;
+    const long long pl = in_batch ? plan : (long long)g0.P - 1;     // plan this lane reads
+    const long long out = a.order ? (long long)a.order[pl] : plan;
+    const bool active = in_batch && out < g0.P;
+    const ace_u4 h = a.hdr[pl];
+    const uint32_t first = a.codes[pl].x & 0x1fu;
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // the tables
+    __syncthreads();
+    if (q >= slices) return;
+
+    AceGeom g = g0;
+    g.out_off = 0u;                                                 // (what the evaluation indexes the outputs' addresses by)
+    const AceLds lds = ace_make_lds(lds_raw, 0u);
+    DenseState st;
+    st.init(g, lds, h, ace_u2{0u, 0u});
+    if (!(first & 0x10u)) st.status = ACE_PLAN_MALFORMED;            // the first op must open a stage
+    const uint32_t lut = d.lut_off + st.bidx * 128u;
+    unsigned char *ws = reinterpret_cast<unsigned char *>(a.stage_ws) + ((size_t)block * slices + q) * kDenseWave;
+    const uint64_t zvrk = lds.ld<uint64_t>(lut + ((uint32_t)st.glogs & 15u) * 8u);
+    uint32_t stored;
+    const int n_st = (int)dense_loop<A>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.row0 << 24),
+                                        d.image16 * 16u + 128u + 2u * kLanes + (wave & 3u) * 32u, 1u, stored);
+    dense_replay(d, g, lds, st, ws, lane, (uint32_t)__builtin_amdgcn_readfirstlane((int)stored), n_st);
+    st.s = n_st;                                                    // (result() checks the count of the op loop)
+    double iter, peak;
+    uint8_t feas, stat;
+    st.result(g, a.nbm1[st.bidx], iter, peak, feas, stat);
+    if (active) {
+        a.iter_ms[out] = iter;
+        a.peak_mb[out] = peak;
+        a.feasible[out] = feas;
+        if (a.status) a.status[out] = stat;
+    }
+}
+#endif

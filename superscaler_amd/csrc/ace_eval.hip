@@ -4,7 +4,8 @@
 //   ace_spread.h      small batches, and most batches of stage records and single-stage queries: a plan per workgroup, its ops
 //                     over the lanes
 //   ace_duo.h         mid-sized batches, every row resident: a plan walked by several lanes
-//   ace_many.h        large batches: a plan per lane
+//   ace_dense.h       large batches: a plan per lane, over tables in a denser form
+//   ace_many.h        large batches on other tables: a plan per lane
 //   ace_score_loop.h  what these leave, in C++: a plan per lane
 // With a plan per lane, all lanes of a workgroup walk the op sequence in lockstep, so the op type at each step is wave-uniform:
 // the row of profiled values for that type sits in LDS at a scalar base address and each lane only adds its own (micro-batch,
@@ -31,6 +32,7 @@
 #include "ace_spread.h"
 #include "ace_duo.h"
 #include "ace_many.h"
+#include "ace_dense.h"
 #include "ace_recompute.h"
 
 // Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans (the
@@ -105,6 +107,11 @@ template <int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(con
 template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(const AceKernelArgs a, const uint32_t slices) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_many_body<WIN>(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+}
+// ... over dense tables, see ace_dense.h.
+template <int A> __global__ __launch_bounds__(kDenseLanes, 4) void ace_dense_kernel(const AceKernelArgs a, const AceDenseArgs d, const uint32_t slices) {
+    extern __shared__ __align__(16) unsigned char lds_raw[];
+    ace_dense_body<A>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a, const long long first) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -653,6 +660,8 @@ struct ace_handle {
     ace_u4 *d_win_dma;         // windowed rows: what the assembly op loop fetches its windows by (setup_windowed_asm), or null
     AceGeom geom_wa;           // ... and the LDS layout of the kernel that runs it
     uint32_t lds_bytes_wa;
+    AceDenseArgs dense;        // tables of ace_dense.h (device addresses; image null: they do not fit that form)
+    uint32_t dense_array;
     uint8_t *d_pair_kinds;
     uint32_t *d_stage_lut;
     double *d_nbm1;
@@ -774,6 +783,11 @@ template <int L> static int allow_duo_lds() {
 
 template <bool WIN> static int allow_many_lds() {
     ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_many_kernel<WIN>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    return ACE_OK;
+}
+
+template <int A> static int allow_dense_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<A>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
     return ACE_OK;
 }
 
@@ -936,6 +950,19 @@ static int setup_windowed_asm(ace_handle *h, const ace_tables_t *t, size_t pos_e
     return ACE_OK;
 }
 
+// The dense tables, where the handle's fit that form.
+static int setup_dense(ace_handle *h, const ace_tables_t *t, size_t pos_entries) {
+    AceDenseTables d;
+    ace_dense_build(t, pos_entries, d);
+    if (!d.ok) return ACE_OK;
+    h->dense = d.args;
+    int rc = upload((void **)&h->dense.pos, d.pos.data(), d.pos.size() * sizeof(ace_u4));
+    if (rc == ACE_OK) rc = upload((void **)&h->dense.image, d.image.data(), d.image.size());
+    if (rc != ACE_OK) return rc;
+    h->dense_array = d.array;
+    return ACE_OK;
+}
+
 // The device address of `scratch` on the current device (looked up once per device).
 static int static_scratch_ptr(double **out) {
     int dev = -1;
@@ -1074,11 +1101,12 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = upload((void **)&h->d_win_row_begin, t->win_row_begin, (size_t)(t->n_windows + 1) * 4)) ||
         (rc = upload((void **)&h->d_win_rows, t->win_rows, (size_t)n_win_rows * 8)) ||
         (rc = or_enomem([&] { return setup_windowed_asm(h, t, pos_entries, rk_bytes, stg_words); })) ||
+        (rc = or_enomem([&] { return setup_dense(h, t, pos_entries); })) ||
         (rc = allow_big_lds<false, false, false, false>()) || (rc = allow_big_lds<false, false, true, false>()) ||
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
         (rc = allow_duo_lds<64>()) || (rc = allow_duo_lds<128>()) || (rc = allow_duo_lds<256>()) ||
-        (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) ||
+        (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) || (rc = allow_dense_lds<320>()) || (rc = allow_dense_lds<520>()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
         ace_destroy(h);
         return rc;
@@ -1093,6 +1121,8 @@ void ace_destroy(ace_handle_t *h) {
     (void)hipFree(h->d_pair_kinds);
     if (h->d_pos4) (void)hipFree(h->d_pos4);
     if (h->d_win_dma) (void)hipFree(h->d_win_dma);
+    for (const void *p : {(const void *)h->dense.image, (const void *)h->dense.pos})
+        if (p) (void)hipFree(const_cast<void *>(p));
     (void)hipFree(h->d_stage_lut); (void)hipFree(h->d_nbm1); (void)hipFree(h->d_win_pos);
     (void)hipFree(h->d_win_row_begin); (void)hipFree(h->d_win_rows);
     if (h->d_rc_pos) (void)hipFree(h->d_rc_pos);
@@ -1193,6 +1223,16 @@ static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream
     else hipLaunchKernelGGL(ace_many_kernel<false>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
     return true;
 }
+// ... over dense tables (ace_dense.h has both sides measured: from the first batch on that the kernel of mid-sized ones leaves).
+static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    if (!h->dense.image || a.range || a.stage_out || !a.stage_ws) return false;
+    const uint32_t slices = ace_dense_slices(a.g.P), lanes = 64u * slices, lds = ace_dense_lds(h->dense.image16 * 16u);
+    const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
+    if (a.stage_ws != h->d_stage_ws || groups * lanes > h->stage_ws_plans) return false;    // (the static scratch holds no such records)
+    if (h->dense_array == 320u) hipLaunchKernelGGL(ace_dense_kernel<320>, dim3((unsigned)groups), dim3(kDenseLanes), lds, s, a, h->dense, slices);
+    else hipLaunchKernelGGL(ace_dense_kernel<520>, dim3((unsigned)groups), dim3(kDenseLanes), lds, s, a, h->dense, slices);
+    return true;
+}
 template <int L>
 static void launch_duo_l(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     hipLaunchKernelGGL((ace_duo_kernel<L>), dim3((unsigned)((a.g.P + L - 1) / L)), dim3(kDuoBlock), ace_duo_lds(a.g, h->lds_bytes, L), s, a);
@@ -1215,7 +1255,7 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
     if (a.range) launch_score_w<true, true>(h, a, s);
     else if (a.stage_out) launch_score_w<true, false>(h, a, s);
     else if (mid) launch_duo(mid, h, a, s);
-    else if (launch_many(h, a, s)) return;
+    else if (launch_dense(h, a, s) || launch_many(h, a, s)) return;
     else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
     else if (a.stage_ws) launch_score_b<false, false, false, true>(h, a, s);
     else launch_score_w<false, false>(h, a, s);
@@ -1234,7 +1274,7 @@ static int ensure_stage_ws(ace_handle_t *h, AceKernelArgs *a) {
         if (h->d_stage_ws) ACE_HIP(hipFree(h->d_stage_ws));
         h->d_stage_ws = nullptr;
         h->stage_ws_plans = 0;
-        ACE_HIP(hipMalloc((void **)&h->d_stage_ws, need * ACE_MAX_STAGES * ACE_WS_REC * sizeof(double)));
+        ACE_HIP(hipMalloc((void **)&h->d_stage_ws, need * (h->dense.image ? (size_t)kDensePlan : ACE_MAX_STAGES * ACE_WS_REC * sizeof(double))));
         h->stage_ws_plans = need;
     }
     a->stage_ws = h->d_stage_ws;

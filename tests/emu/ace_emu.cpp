@@ -7,6 +7,7 @@
 #include "ace_edit_kernels.h"
 #include "ace_grid.h"
 #include "ace_score_loop.h"
+#include "ace_dense.h"
 #include "ace_spread.h"
 #include "ace_recompute.h"
 #include "ace_pack.h"
@@ -106,6 +107,102 @@ extern "C" int ace_emu_score(const ace_tables_t *t, const uint8_t *codes /* [P][
     return 0;
 }
 
+
+// ------------------------------------------------------------------------------------------
+// The dense tables (ace_dense.h): built as the library builds them and walked as the assembly loop walks them -- one dot product per
+// address, ranks, parked records -- with every read checked against the image.  Returns 1 if the tables do not fit that form.
+// ------------------------------------------------------------------------------------------
+extern "C" int ace_emu_dense(const ace_tables_t *t, const uint8_t *codes /* [P][N] */, const uint32_t *hdr, long long P, double memory_limit,
+                             int strict, double *iter_ms, double *peak_mb, uint8_t *feasible, uint8_t *status, int32_t *shape /* [4] */) {
+    const int N = t->num_ops;
+    const size_t pos_entries = (size_t)((N + 15) / 16) * 16 + 16;
+    AceDenseTables d;
+    ace_dense_build(t, pos_entries, d);
+    if (!d.ok) return 1;
+    shape[0] = (int32_t)d.image.size(); shape[1] = (int32_t)d.array; shape[2] = (int32_t)(d.args.rb_off - d.args.rf_off) / 8; shape[3] = (int32_t)d.args.kv;
+    const bool rsh = (t->flags & ACE_F_RESHARDING) != 0;
+    AceGeom g;
+    memset(&g, 0, sizeof(g));
+    g.N = N; g.P = (int32_t)P; g.C = t->n_tp * t->n_algo; g.A_shift = t->n_algo == 2 ? 1 : 0;
+    g.n_mbs = t->n_mbs; g.n_tp = t->n_tp; g.n_algo = t->n_algo; g.n_glog = t->n_glog;
+    g.hot_off = t->hot_off * 8u; g.start_off = t->start_off * 8u; g.out_off = t->out_off * 8u; g.z_off = t->z_off * 8u;
+    g.row_bytes = (uint32_t)t->row_doubles * 8u;
+    g.flags = t->flags; g.main_params = t->main_params; g.optimizer = t->optimizer;
+    g.mem_limit = memory_limit; g.strict = strict ? 1 : 0;
+    const AceDenseArgs &da = d.args;
+    const AceLds lds{d.image.data(), (uint32_t)d.image.size()};
+    g.out_off = 0u;
+    auto dot = [](uint32_t a, uint32_t b, uint32_t c) {
+        for (int k = 0; k < 4; ++k) c += ((a >> (8 * k)) & 255u) * ((b >> (8 * k)) & 255u);
+        return c;
+    };
+    for (long long p = 0; p < P; ++p) {
+        auto code = [&](int i) { return i < N ? (uint32_t)(codes[(size_t)p * N + i] & 0x1fu) : i == N ? 0x10u : 0u; };
+        ace_u4 h;
+        memcpy(&h, hdr + 4 * p, 16);
+        DenseState st;
+        st.init(g, lds, h, ace_u2{0u, 0u});
+        if (!(code(0) & 0x10u)) st.status = ACE_PLAN_MALFORMED;
+        std::vector<unsigned char> ws(kDenseWave, 0xff);                // (a wavefront of one lane)
+        uint64_t glogs = st.glogs;
+        auto stage = [&]() {
+            const ace_u2 z = lds.ld<ace_u2>(da.lut_off + st.bidx * 128u + ((uint32_t)glogs & 15u) * 8u);
+            glogs >>= 4;
+            return z;
+        };
+        ace_u2 z = stage();
+        double fwd = 0, bwd = 0, rcs = 0, rsf = 0, rsb = 0, w = 0, act = 0, saved = 0, peak = 0, run = 0;
+        uint32_t rf = 0, rb = 0, cost = 0, before = (code(0) & 7u) << 8 | da.row0 << 24;
+        int n_st = 0;
+        for (int i = 0; i < N; ++i) {
+            const uint32_t b = code(i), nb = code(i + 1);
+            const ace_u4 &pos = d.pos[i];
+            uint32_t word = 0;                                          // codes from the even position on, behind them the constant(s)
+            for (int k = 0; k < (rsh ? 3 : 2); ++k) word |= (code((i & ~1) + k) & 7u) << (8 * k);
+            word |= da.kv;
+            const uint32_t e = dot(word, pos.x, z.x);
+            const double v[4] = {lds.ld<double>(e), lds.ld<double>(e + d.array), lds.ld<double>(e + 2 * d.array), lds.ld<double>(e + 3 * d.array)};
+            const uint32_t ranks = lds.ld<uint32_t>(e + 4 * d.array);
+            fwd += v[0]; bwd += v[1]; w += v[2]; act += v[3];
+            if (rsh) {
+                const ace_d2 c = lds.ld<ace_d2>(cost);
+                rsf += c.x; rsb += c.y;
+                cost = lds.ld<uint16_t>(dot(word, pos.y, z.y));
+            }
+            const bool last = (nb >> 4) & 1u, rc = (b >> 3) & 1u, pair = rc && ((nb >> 3) & 1u) && !last, keep = pair && (pos.w & 1u);
+            if (last && !(i > 0 && (d.pos[i - 1].w & 2u))) run = 0.0;
+            if (!last) {
+                rf = (ranks & 0xffffu) > rf ? ranks & 0xffffu : rf;
+                rb = (ranks >> 16) > rb ? ranks >> 16 : rb;
+            }
+            if (rc) rcs += v[0];
+            if (pair) run += v[3];
+            if (keep) saved += v[3];
+            else { peak = ace_max(peak, run); run = 0.0; }
+            if (!last) continue;
+            if (n_st < ACE_MAX_STAGES) {
+                const double vals[8] = {fwd + bwd, rcs, rsf, rsb, w, act, saved, peak};
+                for (uint32_t j = 0; j < 4u; ++j) memcpy(ws.data() + j * kDensePiece + (uint32_t)n_st * 16u, vals + 2 * j, 16);
+                const uint32_t even = (b & 7u) | (nb & 7u) << 8, odd = (b & 7u) << 8 | (nb & 7u) << 16;
+                const uint32_t word = (rsh && (i & 1) ? odd : even) | pos.z;
+                const ace_u4 tail{rf | rb << 16, word, before, (uint32_t)n_st * 128u};
+                memcpy(ws.data() + 4u * kDensePiece + (uint32_t)n_st * 16u, &tail, 16);
+                before = word;
+            }
+            ++n_st;
+            fwd = bwd = rcs = rsf = rsb = w = act = saved = peak = run = 0.0;
+            rf = rb = cost = 0;
+            z = stage();
+        }
+        dense_replay(da, g, lds, st, ws.data(), 0u, (uint32_t)(n_st < ACE_MAX_STAGES ? n_st : ACE_MAX_STAGES), n_st);
+        st.s = n_st;
+        uint8_t feas, stat;
+        st.result(g, t->nb_minus_1[st.bidx], iter_ms[p], peak_mb[p], feas, stat);
+        feasible[p] = feas;
+        status[p] = stat;
+    }
+    return 0;
+}
 
 // ------------------------------------------------------------------------------------------
 // The kernel's own op loop (ace_score_loop.h) on the CPU, one lane per "workgroup", with every

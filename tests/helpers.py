@@ -55,7 +55,7 @@ def emu_lib():
     if _emu is None:
         so = os.path.join(ROOT, "tests", "emu", "libace_emu.so")
         src = os.path.join(ROOT, "tests", "emu", "ace_emu.cpp")
-        hdrs = [os.path.join(ROOT, "superscaler_amd", "csrc", h) for h in ("ace_plan_state.h", "ace_score_loop.h", "ace_spread.h", "ace_recompute.h", "ace_pack.h", "ace_grid.h")]
+        hdrs = [os.path.join(ROOT, "superscaler_amd", "csrc", h) for h in ("ace_plan_state.h", "ace_score_loop.h", "ace_spread.h", "ace_recompute.h", "ace_pack.h", "ace_grid.h", "ace_dense.h")]
         if (not os.path.exists(so)) or os.path.getmtime(so) < max(os.path.getmtime(f) for f in [src] + hdrs):
             subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC",
                             "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "superscaler_amd", "csrc"),
@@ -87,6 +87,23 @@ def emu_score(tables, batch, memory_limit=None, strict=False, breakdown=False, r
                            rec.ctypes.data_as(ctypes.c_void_p) if breakdown else None)
     assert rc == 0
     return it, pk, fe, st, rec
+
+
+def emu_dense_score(tables, batch):
+    """The dense tables of large batches (csrc/ace_dense.h) as the library builds them, walked like the assembly loop walks them;
+    None where the tables do not fit that form."""
+    lib = emu_lib()
+    ts = tables.as_struct()
+    P = batch.n_plans
+    codes, hdr = np.ascontiguousarray(batch.codes), np.ascontiguousarray(batch.hdr)
+    it = np.zeros(P); pk = np.zeros(P)
+    fe = np.zeros(P, dtype=np.uint8); st = np.zeros(P, dtype=np.uint8)
+    shape = np.zeros(4, dtype=np.int32)
+    vp = ctypes.c_void_p
+    rc = lib.ace_emu_dense(ctypes.byref(ts), codes.ctypes.data_as(vp), hdr.ctypes.data_as(vp), ctypes.c_longlong(P),
+                           ctypes.c_double(tables.settings.memory_limit), 0, it.ctypes.data_as(vp), pk.ctypes.data_as(vp),
+                           fe.ctypes.data_as(vp), st.ctypes.data_as(vp), shape.ctypes.data_as(vp))
+    return None if rc else (it, pk, fe, st, shape)
 
 
 def kernel_layout(codes):
