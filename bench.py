@@ -77,13 +77,11 @@ def kernel_name(tables, n_plans):
     """The kernel that plain scoring of a batch runs (the library's choice, launch_score in ace_eval.hip), for tables that its
     assembly loops walk, as the configured workloads' are."""
     windowed = tables.n_windows > 1
-    if windowed and tables.rows.shape[0] > 256:
-        return "ace_score_kernel<WIN=true>"
-    if n_plans <= (7680 if windowed else 4096):
+    if n_plans <= (6144 if windowed else 4096):
         return "ace_spread_kernel"
     if not windowed and n_plans <= 65536:
         return "ace_duo_kernel"
-    return "ace_many_kernel<WIN=true>" if windowed else "ace_dense_kernel"
+    return "ace_dense_kernel<WIN=%s>" % ("true" if windowed else "false")
 
 
 def other_workloads(steps):

@@ -3,7 +3,7 @@
 // one 16-byte read for both collectives' costs, and records that are stored in whole cache lines (gen_dense_loop_asm.py).  The
 // tables take less than half of a CU's LDS in the form below, so two workgroups of eight wavefronts share a CU, and one evaluates
 // its stage tails or stages its tables while the other walks.
-// From 65,537 plans on, where the tables fit this form: 40 (resharding off) or 64 entries per row, and 80 KB.
+// Rows resident (they fit 80 KB with the rest): from 65,537 plans on.  Rows in windows: from what the kernel of small batches leaves.
 // Measured, us per launch, ace_many.h -> here:
 //   plans      315 ops           523 ops           821 ops, no resharding   1,251 ops, 16 stages
 //   65,537     64.2 ->  58.9     130.1 -> 117.5    134.7 -> 113.9           285.1 -> 235.2
@@ -11,13 +11,15 @@
 //   262,144   102.4 ->  88.6     176.9 -> 149.5    167.0 -> 148.7           461.0 -> 398.3
 //   1,048,576                    694.0 -> 555.9
 //   (523 ops, 1,048,576 plans, all of one stage: 447 -> 357, all of sixteen: 1,456 -> 981)
+//   windowed rows: 134 ops, 7,681 plans 45.7 -> 32.6, 65,536 55.4 -> 41.1, 131,072 63.7 -> 48.0, 262,144 92.6 -> 72.9, 300,000 132.7 -> 99.9;
+//   230 ops, 262,144 plans 121.7 -> 88.0; 270 ops in 270 types (the C++ loop before), 100,000 plans 455.8 -> 66.0, 500,000 475.8 -> 196.6
 // What bounds it is the issue of vector instructions: about 30 per op and wavefront of the mix of depths (35 before), and the issue
 // of everything else beside them; with fewer than four wavefronts per SIMD the latency of a step.  One workgroup of 1,024 lanes per
 // CU instead: 594 us where two of 512 took 567.
 //
 // The dense tables, one block that is copied to LDS address 0 on:
 //   pairs   16 bytes {forward, backward} ms of resharding, every distinct pair once, {0, 0} first
-//   rows    per op type used: five arrays of `entries` doubles (ACE_DENSE_ARRAY bytes each): forward, backward, weights,
+//   rows    per op type used: five arrays of doubles (one of the sizes kDenseArrays each): forward, backward, weights,
 //           activations, and the ranks of the two reserved sizes (16 bits each) among all that occur; indexed diag * C + code
 //           as the table compiler's rows are
 //   slabs   per distinct (pair kind, next op's type): blocks of [code][next code] 16-bit addresses into `pairs`, one block per
@@ -26,10 +28,12 @@
 //   stages  the stage LUT as it is
 // and what the evaluation of the stage tails looks up (from global memory those were six gathers per stage, 1 ns per lane and CU
 // each: 115 of 760 us per 1,048,576 plans of 523 ops):
-//   reserved sizes by rank; per (row, diag * C + code) and per (row, output entry) a 16-bit LDS address of the distinct
-//   {input MB, intra-node ms, inter-node ms} and {output intra, inter}
+//   reserved sizes by rank; per (op type, diag * C + code) and per (op type, output entry) a 16-bit LDS address of the distinct
+//   {input MB, intra-node ms, inter-node ms} and {output intra, inter}; types that agree in all of them share one list
 // With two algorithms and four tp sizes most codes in use are even, and diags four apart lie 256 bytes apart: from the fourth on
 // they lie 8 bytes further, so that their even codes read different banks.  Blocks of a slab are 132 bytes apart for the same reason.
+// Rows that do not all fit go through windows (as many ops as the rows of half the space behind the rest serve, a multiple of four),
+// consecutive windows in alternate halves, fetched by the loop itself; everything else stays resident.
 // What a code byte reads that names no profiled entry (codes past the last tp size) is what it reads in the table compiler's
 // rows: the tables are filled by those addresses.
 #pragma once
@@ -43,51 +47,67 @@
 
 constexpr uint32_t kDenseLds = 80u * 1024u;    // LDS of a workgroup: two per CU
 constexpr int kDenseLanes = 512;
+// ... windowed rows: one per CU, so that a window holds more ops (134 ops, two workgroups of 512 lanes per CU with windows of 8 ops against
+// one of 1,024 with 20: 65,536 plans 44.9 / 41.1 us, 262,144 69.4 / 72.9, 300,000 104.6 / 99.9)
+constexpr uint32_t kDenseWinLds = 160u * 1024u;
+constexpr int kDenseWinLanes = 1024;
+constexpr uint32_t kDenseArrays[4] = {320u, 520u, 584u, 968u};   // bytes of an array of a row: up to 40, 64, 72, 120 entries (and the eight bytes further)
 
 struct AceDenseArgs {
     const ace_u4 *image;        // the tables
     const ace_u4 *pos;          // [16 * G + 16] per position: dot4 scalars of the row and of the slab, record word, flags (as pos4)
+    const unsigned char *events;        // windowed rows: fetch records, 48 bytes per event and wavefront (see dense_events)
+    uint32_t n_events;
     uint32_t image16;           // size of the image in 16-byte pieces
     uint32_t lut_off, stg_off, rf_off, rb_off, in_off, out_off;   // LDS offsets
-    uint32_t in_entries, out_entries;   // 16-bit addresses per row
+    uint32_t in_entries, out_entries;   // 16-bit addresses per list
+    uint32_t half, lut_half;    // windowed rows: from the first half of the rows, of the offsets' table, to the second
     uint32_t kv;                // constant byte(s) of the code words
-    uint32_t row0;              // row of the first op
+    uint32_t first_in;          // list of the first op
 };
 
 // What the library keeps of it (built on the host).
 struct AceDenseTables {
     std::vector<unsigned char> image;
     std::vector<ace_u4> pos;
+    std::vector<unsigned char> rows;            // windowed: every row, `row_pitch` bytes each ...
+    std::vector<std::vector<uint32_t>> windows; // ... the rows of each window in the order of their slots
+    std::vector<int> window_start;
+    uint32_t row_pitch = 0, rows_off = 0;
     AceDenseArgs args{};        // (offsets)
-    uint32_t array = 0;
+    uint32_t array = 0, lds = 0;
     bool ok = false;
 };
 
-// LDS behind the image: the deal's bins and permutation, the arrival counters.
-inline uint32_t ace_dense_lds(uint32_t image_bytes) { return ((image_bytes + 15u) & ~15u) + 128u + 2u * (uint32_t)kDenseLanes + 128u; }
+// LDS behind the image: the deal's bins and permutation, and the arrival counters; windowed, the rows lie there afterwards.
+inline uint32_t ace_dense_scratch(int lanes) { return 128u + 2u * (uint32_t)lanes + 128u; }
 
-// Fills `d` from tables whose rows are all resident (d.ok false: they do not fit this form).
-inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseTables &d) {
+// Fills `d` (d.ok false: the tables do not fit this form).  `lds`: how much of it a workgroup of `lanes` lanes may take.
+inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed, uint32_t lds, int lanes, AceDenseTables &d) {
     d = AceDenseTables();
     const int N = t->num_ops, C = t->n_tp * t->n_algo, ND = t->n_diag;
-    if (t->n_windows != 1 || (t->flags & ACE_F_COLLECTIVE_MEM) || t->num_types > 256 || N >= 32768) return;
+    if ((t->flags & ACE_F_COLLECTIVE_MEM) || N >= 32768) return;
     const bool rsh = (t->flags & ACE_F_RESHARDING) != 0;
-    const uint32_t entries = (uint32_t)(ND * C + 8), array = entries <= 40u ? 320u : entries <= 64u ? 520u : 0u;
-    if (!array) return;
-    auto diag_entry = [&](uint32_t dg) { return dg * (uint32_t)C + (C == 8 && t->n_algo == 2 && dg >= 4u ? 1u : 0u); };
+    const uint32_t entries = (uint32_t)(ND * C + 8), array = entries <= 40u ? kDenseArrays[0] : entries <= 64u ? kDenseArrays[1] : entries <= 72u ? kDenseArrays[2] : kDenseArrays[3];
+    if (entries > 120u) return;
+    auto diag_entry = [&](uint32_t dg) { return dg * (uint32_t)C + (C == 8 && t->n_algo == 2 && array != kDenseArrays[0] && dg >= 4u ? 1u : 0u); };
     const size_t n_rows_all = (size_t)t->num_types * (size_t)t->row_doubles;
     auto at = [&](size_t type, size_t off) {                       // a double of a row, or of what follows it in memory
         const size_t i = type * (size_t)t->row_doubles + off;
         return i < n_rows_all ? t->rows[i] : 0.0;
     };
-    std::vector<uint32_t> types(pos_entries);
-    ace_pos_types(t, types.data(), pos_entries);
-    // rows in use, in the order of their types
-    std::vector<int> row_of(256, -1);
-    std::vector<uint32_t> used;
-    for (int i = 0; i < N; ++i) row_of[types[i] & 0xffu] = 0;
-    for (uint32_t ty = 0; ty < 256u; ++ty)
-        if (row_of[ty] == 0) { row_of[ty] = (int)used.size(); used.push_back(ty); }
+    // the op type of each position; those in use, in the order of their numbers
+    std::vector<uint32_t> types(N), used;
+    for (int i = 0, w = 0; i < N; ++i) {
+        while (w + 1 < t->n_windows && t->win_pos[w + 1] <= i) ++w;
+        const uint32_t slot_off = (t->pos_info[i] & 0xffu) * (uint32_t)t->row_doubles * 8u;
+        for (int r = t->win_row_begin[w]; r < t->win_row_begin[w + 1]; ++r)
+            if (t->win_rows[2 * r + 1] == slot_off) types[i] = t->win_rows[2 * r];
+    }
+    std::vector<int> row_of(t->num_types, -1);
+    for (int i = 0; i < N; ++i) row_of[types[i]] = 0;
+    for (int ty = 0; ty < t->num_types; ++ty)
+        if (row_of[ty] == 0) { row_of[ty] = (int)used.size(); used.push_back((uint32_t)ty); }
     // ranks of the reserved sizes: what a running maximum from 0.0 can become (0.0: rank 0)
     std::vector<double> reserved_fwd, reserved_bwd, *const values[2] = {&reserved_fwd, &reserved_bwd};
     for (int w = 0; w < 2; ++w) {
@@ -122,8 +142,8 @@ inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseT
             v.push_back(x);
             return (uint32_t)v.size() - 1u;
         };
-        for (int i = 0; i + 1 < N; ++i) kind_of[i] = index(kinds, {(t->pos_info[i] >> 16) & 0xffu, types[i + 1] & 0xffu});
-        if (kinds.empty()) kinds.push_back({0u, types[0] & 0xffu});
+        for (int i = 0; i + 1 < N; ++i) kind_of[i] = index(kinds, {(t->pos_info[i] >> 16) & 0xffu, types[i + 1]});
+        if (kinds.empty()) kinds.push_back({0u, types[0]});
         for (uint32_t j = 0; j < (uint32_t)t->n_mbs * 16u; ++j)
             stage_of[j] = index(stages, {t->stage_lut[j] & 15u, (j & 15u) < (uint32_t)t->n_glog ? j & 15u : 0u});
         // a stage's block over all kinds at once: equal ones are kept once
@@ -161,21 +181,8 @@ inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseT
         }
         for (int i = 0; i + 1 < N; ++i) slab_of[i] = slab_of_kind[kind_of[i]];
     }
-    // the constant byte K and how far apart rows and slabs lie: multiples of it, at most 255 for the last one
-    const uint32_t n_rows = (uint32_t)used.size(), n_slabs = (uint32_t)slabs.size(), slab_bytes = (uint32_t)n_blocks * kBlock;
-    uint32_t K = 0, row_pitch = array * 5u, slab_pitch = 0;
-    if (rsh) {
-        uint64_t best = ~0ull;
-        for (uint32_t k = 8; k <= 248u; k += 8u) {
-            const uint32_t u = (array * 5u + k - 1u) / k, v = (slab_bytes + k - 1u) / k;
-            if ((n_rows - 1u) * u > 255u || (n_slabs - 1u) * v > 255u) continue;
-            const uint64_t size = (uint64_t)n_rows * u * k + (uint64_t)n_slabs * v * k;
-            if (size < best) { best = size; K = k; row_pitch = u * k; slab_pitch = v * k; }
-        }
-        if (!K) return;
-    } else if ((n_rows - 1u) * row_pitch > 248u * 255u + 247u) return;   // (two constant bytes: 248 and 8)
+    // what the evaluation looks up comes first (it decides how much room the rows have)
     AceDenseArgs &g = d.args;
-    g.kv = rsh ? K << 24 : (248u << 24) | (8u << 16);
     // what the evaluation looks up: distinct {input MB, intra, inter} and {output intra, inter}, their place per row and entry
     typedef std::vector<uint64_t> Bits;
     std::vector<Bits> values_in, values_out;
@@ -191,11 +198,52 @@ inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseT
     };
     g.in_entries = entries;
     g.out_entries = (uint32_t)(t->n_mbs * t->n_tp + 8) * (uint32_t)t->n_algo;    // (a code past the last tp size: up to index 7)
-    std::vector<uint32_t> in_of, out_of;
+    std::vector<std::vector<uint32_t>> in_lists, out_lists;
+    std::vector<uint32_t> in_of, out_of;                            // per row: its list
+    auto list_of = [](std::vector<std::vector<uint32_t>> &v, const std::vector<uint32_t> &x) {
+        const size_t i = (size_t)(std::find(v.begin(), v.end(), x) - v.begin());
+        if (i == v.size()) v.push_back(x);
+        return (uint32_t)i;
+    };
     for (uint32_t ty : used) {
-        for (uint32_t e = 0; e < g.in_entries; ++e) in_of.push_back(place_of(values_in, ty, (size_t)t->start_off + e * 3u, 3));
-        for (uint32_t e = 0; e < g.out_entries; ++e) out_of.push_back(place_of(values_out, ty, (size_t)t->out_off + e * 2u, 2));
+        std::vector<uint32_t> in, out;
+        for (uint32_t e = 0; e < g.in_entries; ++e) in.push_back(place_of(values_in, ty, (size_t)t->start_off + e * 3u, 3));
+        for (uint32_t e = 0; e < g.out_entries; ++e) out.push_back(place_of(values_out, ty, (size_t)t->out_off + e * 2u, 2));
+        in_of.push_back(list_of(in_lists, in));
+        out_of.push_back(list_of(out_lists, out));
     }
+    if (in_lists.size() > 256u || out_lists.size() > 256u) return;   // (eight bits each in a record word)
+    // the constant byte K and how far apart rows and slabs lie: multiples of it, at most 255 for the last one; rows: as many as
+    // `slots` (windowed: in each half)
+    const uint32_t n_slabs = (uint32_t)slabs.size(), slab_bytes = (uint32_t)n_blocks * kBlock;
+    const size_t lists = (in_lists.size() * g.in_entries + out_lists.size() * g.out_entries) * 2u;
+    uint32_t K = 0, row_pitch = 0, slab_pitch = 0, slots = windowed ? 31u : (uint32_t)used.size();
+    auto fits = [&](uint32_t n) {                                   // n rows: K and the pitches, the smallest in all
+        K = 0;
+        uint64_t best = ~0ull;
+        if (!rsh) {                                                 // (two constant bytes: 248 and 8)
+            row_pitch = (array * 5u + 15u) & ~15u;
+            if ((n - 1u) * row_pitch > 248u * 255u + 247u) return false;
+            K = 248u;
+            best = (uint64_t)n * row_pitch * (windowed ? 2u : 1u);
+        } else
+            for (uint32_t k = 8; k <= 248u; k += 8u) {
+                uint32_t u = (array * 5u + k - 1u) / k;
+                const uint32_t v = (slab_bytes + k - 1u) / k;
+                u += windowed && ((u * k) & 15u) ? 1u : 0u;            // (fetched in pieces of 16 bytes)
+                if ((n - 1u) * u > 255u || (n_slabs - 1u) * v > 255u) continue;
+                const uint64_t size = (uint64_t)n * u * k * (windowed ? 2u : 1u) + (uint64_t)n_slabs * v * k;
+                if (size < best) { best = size; K = k; row_pitch = u * k; slab_pitch = v * k; }
+            }
+        const uint64_t rest = pairs.size() * 16u + values_out.size() * 16u + values_in.size() * 24u + (size_t)t->n_mbs * (windowed ? 320u : 192u) +
+                              (reserved_fwd.size() + reserved_bwd.size()) * 8u + lists + 256u;
+        return K != 0u && best + rest + (windowed ? 0u : ace_dense_scratch(lanes)) <= lds;
+    };
+    if (windowed)
+        while (slots >= 4u && (!fits(slots) || slots * ((row_pitch + 1023u) / 1024u) > 4u * (uint32_t)lanes / 64u)) --slots;   // (four loads per event and wavefront)
+    if (slots < 4u && windowed) return;
+    if (!fits(slots)) return;
+    g.kv = rsh ? K << 24 : (248u << 24) | (8u << 16);
     // the image (what 16-bit addresses name lies in front)
     uint32_t end = 0;
     auto take = [&](size_t bytes, uint32_t align) {
@@ -206,16 +254,47 @@ inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseT
     take(pairs.size() * 16u, 16u);
     const uint32_t vout_off = take(values_out.size() * 16u, 16u), vin_off = take(values_in.size() * 24u, 8u);
     if (end > 65536u) return;
-    const uint32_t rows_off = take((size_t)n_rows * row_pitch, 16u), slabs_off = take((size_t)n_slabs * slab_pitch, 16u);
-    g.lut_off = take((size_t)t->n_mbs * 128u, 128u);
+    const uint32_t slabs_off = take((size_t)n_slabs * slab_pitch, 16u);
+    g.lut_half = (uint32_t)t->n_mbs * 128u;
+    g.lut_off = take((size_t)g.lut_half * (windowed ? 2u : 1u), 128u);
     g.stg_off = take((size_t)t->n_mbs * 64u, 4u);
     g.rf_off = take(reserved_fwd.size() * 8u, 8u);
     g.rb_off = take(reserved_bwd.size() * 8u, 8u);
-    g.in_off = take(in_of.size() * 2u, 2u);
-    g.out_off = take(out_of.size() * 2u, 2u);
-    const uint32_t bytes = take(0, 16u);
-    if (ace_dense_lds(bytes) > kDenseLds) return;
+    g.in_off = take(in_lists.size() * g.in_entries * 2u, 2u);
+    g.out_off = take(out_lists.size() * g.out_entries * 2u, 2u);
+    const uint32_t n_rows = (uint32_t)used.size(), rows_off = take(windowed ? 0u : (size_t)n_rows * row_pitch, 16u), bytes = take(0, 16u);
+    g.half = slots * row_pitch;
+    d.lds = bytes + (windowed ? std::max(2u * g.half, ace_dense_scratch(lanes)) : ace_dense_scratch(lanes));
+    if (d.lds > lds) return;
+    d.row_pitch = row_pitch;
+    d.rows_off = rows_off;
     g.image16 = bytes / 16u;
+    // windows: a multiple of four ops each (or up to the last op), of at most `slots` different rows
+    std::vector<uint32_t> place(N, 0u);                             // of each position's row, from the first one (of its half) on
+    if (windowed) {
+        for (int i = 0; i < N;) {
+            std::vector<uint32_t> seen;
+            size_t good_n = 0;
+            int good = -1;
+            for (int j = i; j < N;) {
+                const uint32_t r = (uint32_t)row_of[types[j]];
+                if (std::find(seen.begin(), seen.end(), r) == seen.end()) {
+                    if (seen.size() >= slots) break;
+                    seen.push_back(r);
+                }
+                ++j;
+                if (j == N || (j & 3) == 0) { good = j; good_n = seen.size(); }
+            }
+            if (good < 0) return;
+            seen.resize(good_n);
+            for (int j = i; j < good; ++j) place[j] = (uint32_t)(std::find(seen.begin(), seen.end(), (uint32_t)row_of[types[j]]) - seen.begin()) * row_pitch;
+            d.window_start.push_back(i);
+            d.windows.push_back(seen);
+            i = good;
+        }
+        if (d.windows.size() < 2u) return;
+    } else
+        for (int i = 0; i < N; ++i) place[i] = (uint32_t)row_of[types[i]] * row_pitch;
     d.image.assign(bytes, 0);
     auto put = [&](uint32_t off, const void *p, size_t n) { if (n) memcpy(d.image.data() + off, p, n); };
     for (size_t i = 0; i < pairs.size(); ++i) {
@@ -224,66 +303,110 @@ inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseT
     }
     for (size_t i = 0; i < values_out.size(); ++i) put(vout_off + (uint32_t)i * 16u, values_out[i].data(), 16);
     for (size_t i = 0; i < values_in.size(); ++i) put(vin_off + (uint32_t)i * 24u, values_in[i].data(), 24);
-    for (size_t i = 0; i < in_of.size(); ++i) {
-        const uint16_t a16 = (uint16_t)(vin_off + in_of[i] * 24u);
-        put(g.in_off + (uint32_t)i * 2u, &a16, 2);
-    }
-    for (size_t i = 0; i < out_of.size(); ++i) {
-        const uint16_t a16 = (uint16_t)(vout_off + out_of[i] * 16u);
-        put(g.out_off + (uint32_t)i * 2u, &a16, 2);
-    }
+    auto put_lists = [&](uint32_t off, const std::vector<std::vector<uint32_t>> &v, uint32_t base, uint32_t size) {
+        for (const auto &list : v)
+            for (uint32_t x : list) {
+                const uint16_t a16 = (uint16_t)(base + x * size);
+                put(off, &a16, 2);
+                off += 2u;
+            }
+    };
+    put_lists(g.in_off, in_lists, vin_off, 24u);
+    put_lists(g.out_off, out_lists, vout_off, 16u);
     put(g.rf_off, reserved_fwd.data(), reserved_fwd.size() * 8u);
     put(g.rb_off, reserved_bwd.data(), reserved_bwd.size() * 8u);
-    for (uint32_t r = 0; r < n_rows; ++r)
+    if (windowed) d.rows.assign((size_t)n_rows * row_pitch, 0);
+    unsigned char *rows = windowed ? d.rows.data() : d.image.data() + rows_off;
+    for (size_t r = 0; r < n_rows; ++r)
         for (uint32_t dg = 0; dg <= (uint32_t)ND; ++dg)
             for (uint32_t c = 0; c < 8u; ++c) {
                 // (a code past the last one reads what follows its diag's entries)
-                const uint32_t e = dg * (uint32_t)C + c, to = rows_off + r * row_pitch + (diag_entry(dg) + c) * 8u;
+                const uint32_t e = dg * (uint32_t)C + c;
+                unsigned char *to = rows + r * row_pitch + (diag_entry(dg) + c) * 8u;
                 if (c >= (uint32_t)C && dg < (uint32_t)ND) continue;
                 double v[6];
                 for (uint32_t k = 0; k < 6u; ++k) v[k] = at(used[r], (size_t)t->hot_off + e * 6u + k);
-                for (uint32_t k = 0; k < 4u; ++k) put(to + k * array, &v[k], 8);
+                for (uint32_t k = 0; k < 4u; ++k) memcpy(to + k * array, &v[k], 8);
                 const uint32_t both = rank(0, v[4]) | (rank(1, v[5]) << 16);
-                put(to + 4u * array, &both, 4);
+                memcpy(to + 4u * array, &both, 4);
             }
     for (uint32_t s = 0; s < n_slabs; ++s)
         for (uint32_t b = 0; b < (uint32_t)n_blocks; ++b) put(slabs_off + s * slab_pitch + b * kBlock, slabs[s].data() + b * 64u, 128);
     for (uint32_t j = 0; j < (uint32_t)t->n_mbs * 16u; ++j) {
         const ace_u2 z{rows_off + diag_entry(t->stage_lut[j] & 15u) * 8u, slabs_off + block_of[j] * kBlock};
         put(g.lut_off + j * 8u, &z, 8);
+        const ace_u2 other{z.x + g.half, z.y};
+        if (windowed) put(g.lut_off + g.lut_half + j * 8u, &other, 8);
         put(g.stg_off + j * 4u, &t->stage_lut[j], 4);
     }
     // positions
     d.pos.assign(pos_entries, ace_u4{0u, 0u, 0u, 0u});
     for (size_t i = 0; i < pos_entries; ++i) {
         const bool odd = (i & 1u) != 0u, in = i < (size_t)N;
-        const uint32_t info = in ? t->pos_info[i] : 0u;
-        const uint32_t row = in ? (uint32_t)row_of[types[i] & 0xffu] : 0u, place = row * row_pitch, slab = in ? slab_of[i] : 0u;
-        const uint32_t last = in ? (uint32_t)row_of[types[i] & 0xffu] : 0u, next = in ? (uint32_t)row_of[(types[i] >> 8) & 0xffu] : 0u;
+        const uint32_t info = in ? t->pos_info[i] : 0u, at_row = in ? place[i] : 0u, slab = in ? slab_of[i] : 0u;
+        const uint32_t last = in ? out_of[row_of[types[i]]] : 0u, next = in && i + 1 < (size_t)N ? in_of[row_of[types[i + 1]]] : 0u;
         ace_u4 &p = d.pos[i];
-        p.x = (odd ? 8u << 8 : 8u) | (rsh ? (place / K) << 24 : ((place / 248u) << 24) | (((place % 248u) / 8u) << 16));
+        p.x = (odd ? 8u << 8 : 8u) | (rsh ? (at_row / K) << 24 : ((at_row / 248u) << 24) | (((at_row % 248u) / 8u) << 16));
         p.y = rsh ? (odd ? (16u << 8) | (2u << 16) : 16u | (2u << 8)) | ((slab * (slab_pitch / K)) << 24) : 0u;
         // record word: codes of the stage's last op and of the next one in bytes 0 and 1 (odd positions with resharding: 1
-        // and 2, bit 11 set), rows of both in the other two
+        // and 2, bit 11 set), the last op's list of outputs and the next one's of inputs in the other two
         p.z = rsh && odd ? last | (next << 24) | (1u << 11) : (last << 16) | (next << 24);
         p.w = (((info >> 24) & 1u) ^ 1u) | (((info >> 25) & 1u) << 1);
     }
     d.array = array;
-    g.row0 = (uint32_t)row_of[types[0] & 0xffu];
+    g.first_in = in_of[row_of[types[0]]];
     d.ok = true;
 }
 
+// Every row resident if they fit beside a second workgroup on the CU, else in windows.
+inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseTables &d) {
+    if (t->n_windows == 1) dense_build(t, pos_entries, false, kDenseLds, kDenseLanes, d);
+    if (!d.ok) dense_build(t, pos_entries, true, kDenseWinLds, kDenseWinLanes, d);
+}
+
+// Windowed rows: the fetch records, per event and wavefront 48 bytes = {first position of the window after the one being entered,
+// bit 0: wait for the fetch (else it completes before the next event) | number of loads << 8, address of the rows} and four
+// LDS-direct loads {byte offset in the rows, LDS address} of 1 KB each.  Events: 0 fetches window 0 and waits, 1 fetches window 1,
+// and entering window w >= 1 fetches window w + 1 (the last one fetches window w - 1 again, into the half nobody reads).
+inline std::vector<uint32_t> dense_events(const AceDenseTables &d, uint64_t rows_at) {
+    const int n_w = (int)d.windows.size();
+    const uint32_t waves = (uint32_t)kDenseWinLanes / 64u;
+    std::vector<uint32_t> out((size_t)(n_w + 1) * waves * 12u, 0u);
+    for (int e = 0; e <= n_w; ++e) {
+        const int entering = e < 2 ? 0 : e - 1;                        // the window walked after this event
+        int fetch = e == 0 ? 0 : entering + 1;
+        if (fetch >= n_w) fetch = entering - 1;
+        std::vector<ace_u2> loads;
+        for (size_t s = 0; s < d.windows[fetch].size(); ++s)
+            for (uint32_t off = 0; off < d.row_pitch; off += 1024u) {
+                // (the last load of a row ends with it: it may overlap the one before it)
+                const uint32_t o = off + 1024u <= d.row_pitch ? off : d.row_pitch - 1024u;
+                loads.push_back(ace_u2{d.windows[fetch][s] * d.row_pitch + o, d.rows_off + (fetch & 1 ? d.args.half : 0u) + (uint32_t)s * d.row_pitch + o});
+            }
+        for (uint32_t v = 0; v < waves; ++v) {
+            uint32_t *rec = &out[((size_t)e * waves + v) * 12u], n = 0;
+            for (size_t c = v; c < loads.size(); c += waves, ++n) { rec[4 + 2 * n] = loads[c].x; rec[5 + 2 * n] = loads[c].y; }
+            rec[0] = entering + 1 < n_w ? (uint32_t)d.window_start[entering + 1] : 0x7fffffffu;
+            rec[1] = (e == 0 ? 1u : 0u) | (n << 8);
+            rec[2] = (uint32_t)rows_at;
+            rec[3] = (uint32_t)(rows_at >> 32);
+        }
+    }
+    return out;
+}
+
 // What a record word says.
-struct DenseMeta { uint32_t c_last, c_next, row_last, row_next; };
+struct DenseMeta { uint32_t c_last, c_next, out_list, in_list; };
 ACE_HD DenseMeta dense_meta(uint32_t m) {
     const bool odd = (m >> 11) & 1u;
     const uint32_t w = odd ? m >> 8 : m;
     return DenseMeta{w & 7u, (w >> 8) & 7u, (odd ? m : m >> 16) & 0xffu, m >> 24};
 }
 
-// Slices of 64 plans per workgroup, so that the rounds of two workgroups per CU that the batch needs are all full.
-inline uint32_t ace_dense_slices(long long plans) {
-    const long long most = kDenseLanes / 64, fullest = ((plans + 63) / 64 + 511) / 512;
+// Slices of 64 plans per workgroup (`most`: as many as it has wavefronts), so that the rounds of `places` workgroups that the batch
+// needs are all full.
+inline uint32_t ace_dense_slices(long long plans, long long most, long long places) {
+    const long long fullest = ((plans + 63) / 64 + places - 1) / places;
     const long long rounds = (fullest + most - 1) / most;
     return (uint32_t)((fullest + rounds - 1) / rounds);
 }
@@ -327,8 +450,8 @@ ACE_HD void dense_stage(const AceDenseArgs &d, const AceGeom &g, const AceLds &l
     st.mrow = lut >> 16;
     st.t_first = before.c_next >> g.A_shift;
     const uint32_t e = ace_mul24(lut & 15u, (uint32_t)g.C) + before.c_next, o = DenseState::out_entry_addr(g, 0u, m.c_last, st.t_first, st.mrow) >> 4;
-    const uint32_t in = lds.ld<uint16_t>(d.in_off + (ace_mul24(before.row_next, d.in_entries) + e) * 2u);
-    const uint32_t out = lds.ld<uint16_t>(d.out_off + (ace_mul24(m.row_last, d.out_entries) + o) * 2u);
+    const uint32_t in = lds.ld<uint16_t>(d.in_off + (ace_mul24(before.in_list, d.in_entries) + e) * 2u);
+    const uint32_t out = lds.ld<uint16_t>(d.out_off + (ace_mul24(m.out_list, d.out_entries) + o) * 2u);
     st.rfm = lds.ld<double>(d.rf_off + (rec.tail.x & 0xffffu) * 8u);
     st.rbm = lds.ld<double>(d.rb_off + (rec.tail.x >> 16) * 8u);
     st.inputs = lds.ld<double>(in);
@@ -393,29 +516,58 @@ ACE_HD void dense_replay(const AceDenseArgs &d, const AceGeom &g, const AceLds &
 
 // The op loop: returns the number of stages of the lane's plan, and in `stored` that of the wavefront's records; `ws`: the
 // wavefront's part of the workspace.  Arrays of the rows lie A bytes apart.
-template <int A>
+template <int A, bool WIN>
 __device__ __forceinline__ uint32_t dense_loop(const AceKernelArgs &a, const AceDenseArgs &d, uint64_t glogs, uint32_t lut2, uint64_t zvrk, uint32_t code_off,
-                                               const unsigned char *ws, uint32_t lane, uint32_t meta0, uint32_t pace, uint32_t pace_mask, uint32_t &stored) {
+                                               const unsigned char *ws, uint32_t lane, uint32_t meta0, uint32_t pace, uint32_t prio, uint32_t wave, uint32_t &stored) {
     uint32_t placed;
     const uint64_t gstride = (uint64_t)(uint32_t)a.g.P * 16u;
     const uint32_t gs_lo = (uint32_t)gstride, gs_hi = (uint32_t)(gstride >> 32);
-#define ACE_DENSE_RUN(TEXT)                                                                                                       \
+#define ACE_DENSE_RUN(TEXT, ...)                                                                                                  \
     asm volatile(TEXT : [placed] "=&v"(placed), [stored] "=&v"(stored)                                                           \
-                 : [glogs] "v"(glogs), [lut2] "v"(lut2), [zvrk] "v"(zvrk), [codeoff] "v"(code_off), [place] "v"(lane * 2u), [meta0] "v"(meta0), \
-                   [codes] "s"(a.codes), [pos] "s"(d.pos), [n_ops] "s"(a.g.N), [recbase] "s"(ws),                               \
-                   [gstride_lo] "s"(gs_lo), [gstride_hi] "s"(gs_hi), [pace] "s"(pace), [pacemask] "s"(pace_mask),                \
-                   [kv] "s"(d.kv), [a1] "n"(A), [a2] "n"(2 * A), [a3] "n"(3 * A), [a4] "n"(4 * A)                                \
+                 : [glogs] "v"(glogs), [lut2] "v"(lut2), [zvrk] "v"(zvrk), [codeoff] "v"(code_off), [place] "v"(lane * 2u),      \
+                   [meta0] "v"(meta0), [codes] "s"(a.codes), [pos] "s"(d.pos), [n_ops] "s"(a.g.N), [recbase] "s"(ws),            \
+                   [gstride_lo] "s"(gs_lo), [gstride_hi] "s"(gs_hi), [kv] "s"(d.kv), [a1] "n"(A), [a2] "n"(2 * A),               \
+                   [a3] "n"(3 * A), [a4] "n"(4 * A), __VA_ARGS__                                                                  \
                  : ACE_DENSE_ASM_CLOBBERS)
-    if (a.g.flags & ACE_F_RESHARDING) ACE_DENSE_RUN(ACE_DENSE_ASM_RSH1);
-    else ACE_DENSE_RUN(ACE_DENSE_ASM_RSH0);
+#define ACE_DENSE_RESIDENT [pace] "s"(pace), [pacemask] "s"(1u)
+#define ACE_DENSE_WINDOWED [prio] "s"(prio), [dma] "s"(d.events), [eventsize] "s"((uint32_t)(kDenseWinLanes / 64) * 48u), \
+                           [waveoff] "s"(wave * 48u), [half] "s"(d.half), [luthalf] "s"(d.lut_half)
+    if (WIN) {
+        if (a.g.flags & ACE_F_RESHARDING) ACE_DENSE_RUN(ACE_DENSE_ASM_WIN_RSH1, ACE_DENSE_WINDOWED);
+        else ACE_DENSE_RUN(ACE_DENSE_ASM_WIN_RSH0, ACE_DENSE_WINDOWED);
+    } else {
+        if (a.g.flags & ACE_F_RESHARDING) ACE_DENSE_RUN(ACE_DENSE_ASM_RSH1, ACE_DENSE_RESIDENT);
+        else ACE_DENSE_RUN(ACE_DENSE_ASM_RSH0, ACE_DENSE_RESIDENT);
+    }
 #undef ACE_DENSE_RUN
+#undef ACE_DENSE_RESIDENT
+#undef ACE_DENSE_WINDOWED
     return placed >> 7;
 }
 
+// Windowed rows: the fetches of a wavefront without plans, in step with the loops of the others (fetch_event of
+// gen_dense_loop_asm.py).  As many events as they have: every barrier is met.
+__device__ __forceinline__ void dense_fetch(const AceDenseArgs &d, unsigned char *lds_raw, uint32_t wave, uint32_t lane) {
+    typedef const void __attribute__((address_space(1))) *gptr;
+    typedef void __attribute__((address_space(3))) *lptr;
+    for (uint32_t e = 0; e < d.n_events; ++e) {
+        const uint32_t *rec = reinterpret_cast<const uint32_t *>(d.events + (e * (uint32_t)(kDenseWinLanes / 64) + wave) * 48u);
+        const unsigned char *rows = reinterpret_cast<const unsigned char *>(((uint64_t)rec[3] << 32) | rec[2]);
+        const uint32_t n = (rec[1] >> 8) & 15u, wait = rec[1] & 1u;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n s_barrier" ::: "memory");
+        for (uint32_t k = 0; k < n; ++k) {
+            const uint32_t from = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec[4 + 2 * k]), to = (uint32_t)__builtin_amdgcn_readfirstlane((int)rec[5 + 2 * k]);
+            __builtin_amdgcn_global_load_lds((gptr)(rows + from + lane * 16u), (lptr)(lds_raw + to), 16, 0, 0);
+        }
+        if (wait) asm volatile("s_waitcnt vmcnt(0)\n s_barrier" ::: "memory");
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+}
+
 // One workgroup; its LDS array starts at address 0 (the kernel has no other LDS variables).
-template <int A> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
+template <int A, bool WIN> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
                                                                 int tid, long long block) {
-    constexpr int kLanes = kDenseLanes;
+    constexpr int kLanes = WIN ? kDenseWinLanes : kDenseLanes;
     const AceGeom &g0 = a.g;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6), lane = (uint32_t)tid & 63u;
     const uint32_t lanes = 64u * slices;
@@ -431,7 +583,7 @@ template <int A> __device__ __forceinline__ void ace_dense_body(const AceKernelA
     unsigned short *plan_of = reinterpret_cast<unsigned short *>(cnt + 32);
     uint32_t *pace = reinterpret_cast<uint32_t *>(plan_of + kLanes);
     const uint32_t q = (wave & 4u) ? wave ^ 3u : wave;
-    if (tid < 32) { cnt[tid] = 0u; pace[tid] = 0u; }
+    if (tid < 32) { cnt[tid] = 0u; if (!WIN) pace[tid] = 0u; }
     const long long slot = block * lanes + tid;
     uint32_t depth = 0, rank = 0;                                   // (slots past the batch: last)
     if ((uint32_t)tid < lanes && slot < g0.P) {
@@ -456,7 +608,10 @@ template <int A> __device__ __forceinline__ void ace_dense_body(const AceKernelA
     const uint32_t first = a.codes[pl].x & 0x1fu;
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                 // the tables
     __syncthreads();
-    if (q >= slices) return;
+    if (q >= slices) {
+        if (WIN) dense_fetch(d, lds_raw, wave, lane);
+        return;
+    }
 
     AceGeom g = g0;
     g.out_off = 0u;                                                 // (what the evaluation indexes the outputs' addresses by)
@@ -468,8 +623,10 @@ template <int A> __device__ __forceinline__ void ace_dense_body(const AceKernelA
     unsigned char *ws = reinterpret_cast<unsigned char *>(a.stage_ws) + ((size_t)block * slices + q) * kDenseWave;
     const uint64_t zvrk = lds.ld<uint64_t>(lut + ((uint32_t)st.glogs & 15u) * 8u);
     uint32_t stored;
-    const int n_st = (int)dense_loop<A>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.row0 << 24),
-                                        d.image16 * 16u + 128u + 2u * kLanes + (wave & 3u) * 32u, 1u, stored);
+    // (windowed rows: the deeper its plans, the higher a wavefront's issue priority)
+    const uint32_t prio = (uint32_t)__builtin_amdgcn_readfirstlane((int)(3u - q * 4u / (uint32_t)(kLanes / 64)));
+    const int n_st = (int)dense_loop<A, WIN>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.first_in << 24),
+                                             d.image16 * 16u + 128u + 2u * kLanes + (wave & 3u) * 32u, prio, wave, stored);
     dense_replay(d, g, lds, st, ws, lane, (uint32_t)__builtin_amdgcn_readfirstlane((int)stored), n_st);
     st.s = n_st;                                                    // (result() checks the count of the op loop)
     double iter, peak;

@@ -4,8 +4,8 @@
 //   ace_spread.h      small batches, and most batches of stage records and single-stage queries: a plan per workgroup, its ops
 //                     over the lanes
 //   ace_duo.h         mid-sized batches, every row resident: a plan walked by several lanes
-//   ace_dense.h       large batches: a plan per lane, over tables in a denser form
-//   ace_many.h        large batches on other tables: a plan per lane
+//   ace_dense.h       large batches: a plan per lane, over tables in a denser form, rows resident or in windows
+//   ace_many.h        large batches on tables that do not fit that form: a plan per lane
 //   ace_score_loop.h  what these leave, in C++: a plan per lane
 // With a plan per lane, all lanes of a workgroup walk the op sequence in lockstep, so the op type at each step is wave-uniform:
 // the row of profiled values for that type sits in LDS at a scalar base address and each lane only adds its own (micro-batch,
@@ -109,9 +109,10 @@ template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(cons
     ace_many_body<WIN>(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // ... over dense tables, see ace_dense.h.
-template <int A> __global__ __launch_bounds__(kDenseLanes, 4) void ace_dense_kernel(const AceKernelArgs a, const AceDenseArgs d, const uint32_t slices) {
+template <int A, bool WIN> __global__ __launch_bounds__(WIN ? kDenseWinLanes : kDenseLanes, 4)
+void ace_dense_kernel(const AceKernelArgs a, const AceDenseArgs d, const uint32_t slices) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_dense_body<A>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_dense_body<A, WIN>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a, const long long first) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -125,7 +126,8 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
 // there.  By what else would take the batch, in us per launch at the limit and where the graph crosses (plan per workgroup / the other):
 //   PLAIN    the mid-sized kernel                    limit  4,096: 315 ops  37 / 42, crosses at  4,800 plans; 523 ops  56 /  66,  5,000;
 //                                                                  821 ops  78 / 81,  4,300; 1,251 ops 104 / 111,  4,400
-//   WINDOWED large, windowed rows                    limit  7,680: 118 ops  34 / 41, crosses at  9,800 plans; 134 ops 37 / 46, 10,000; 174 ops 41 / 53, 10,450
+//   WINDOWED large, windowed rows (dense tables)     limit  6,144: 118 ops  29 / 30, crosses at  6,700 plans; 134 ops 31 / 33, 6,600; 182 ops 35 / 39, 7,150;
+//                                                                  230 ops  40 / 44, 7,050; 270 ops 48 / 49, 6,150
 //   SLOW     no assembly loop (memory of collectives, more than 256 rows)
 //                                                    limit 18,432: 315 ops 161 / 161, 18,400; 523 ops 238 / 459, above 24,576 (313 / 460);
 //                                                                  134 ops  97 / 140, above 24,576 (128 / 140)
@@ -133,8 +135,8 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
 //            single-stage queries                           14,336: 315 ops  85 / 103, 18,000; 523 ops 80 / 179, 134 ops 53 / 124, both above 24,576
 //   OTHER    the C++ loop with deferred stage tails  limit  4,096:  62 ops  18 / 41, 11,500; 134 ops  22 / 83, 20,000
 // and at one plan 8 to 26 where a lane needs 49 to 169 (13 to 20 us is what the host needs for a launch).
-constexpr int kSpreadMaxPlain = 4096, kSpreadMaxWindowed = 7680, kSpreadMaxSlow = 18432, kSpreadMaxRecords = 14336;
-constexpr int kSpreadMaxOther = 4096;    // (tables that no assembly loop walks: windowed rows too short to be fetched, no room in LDS)
+constexpr int kSpreadMaxPlain = 4096, kSpreadMaxWindowed = 6144, kSpreadMaxSlow = 18432, kSpreadMaxRecords = 14336;
+constexpr int kSpreadMaxOther = 4096;    // (tables that no assembly loop walks)
 
 // ------------------------------------------------------------------------------------------
 // top-k: radix select on the order-preserving 64-bit image of the iteration time, then a
@@ -661,7 +663,8 @@ struct ace_handle {
     AceGeom geom_wa;           // ... and the LDS layout of the kernel that runs it
     uint32_t lds_bytes_wa;
     AceDenseArgs dense;        // tables of ace_dense.h (device addresses; image null: they do not fit that form)
-    uint32_t dense_array;
+    uint32_t dense_array, dense_lds;
+    unsigned char *d_dense_rows;   // ... windowed: the rows
     uint8_t *d_pair_kinds;
     uint32_t *d_stage_lut;
     double *d_nbm1;
@@ -787,7 +790,8 @@ template <bool WIN> static int allow_many_lds() {
 }
 
 template <int A> static int allow_dense_lds() {
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<A>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<A, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<A, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseWinLds));
     return ACE_OK;
 }
 
@@ -958,7 +962,15 @@ static int setup_dense(ace_handle *h, const ace_tables_t *t, size_t pos_entries)
     h->dense = d.args;
     int rc = upload((void **)&h->dense.pos, d.pos.data(), d.pos.size() * sizeof(ace_u4));
     if (rc == ACE_OK) rc = upload((void **)&h->dense.image, d.image.data(), d.image.size());
+    if (rc == ACE_OK && !d.windows.empty()) {
+        rc = upload((void **)&h->d_dense_rows, d.rows.data(), d.rows.size());
+        if (rc != ACE_OK) return rc;
+        const std::vector<uint32_t> ev = dense_events(d, (uint64_t)(uintptr_t)h->d_dense_rows);
+        rc = upload((void **)&h->dense.events, ev.data(), ev.size() * 4);
+        h->dense.n_events = (uint32_t)d.windows.size() + 1u;
+    }
     if (rc != ACE_OK) return rc;
+    h->dense_lds = d.lds;
     h->dense_array = d.array;
     return ACE_OK;
 }
@@ -1106,7 +1118,8 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
         (rc = allow_duo_lds<64>()) || (rc = allow_duo_lds<128>()) || (rc = allow_duo_lds<256>()) ||
-        (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) || (rc = allow_dense_lds<320>()) || (rc = allow_dense_lds<520>()) ||
+        (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) || (rc = allow_dense_lds<kDenseArrays[0]>()) || (rc = allow_dense_lds<kDenseArrays[1]>()) ||
+        (rc = allow_dense_lds<kDenseArrays[2]>()) || (rc = allow_dense_lds<kDenseArrays[3]>()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
         ace_destroy(h);
         return rc;
@@ -1121,7 +1134,7 @@ void ace_destroy(ace_handle_t *h) {
     (void)hipFree(h->d_pair_kinds);
     if (h->d_pos4) (void)hipFree(h->d_pos4);
     if (h->d_win_dma) (void)hipFree(h->d_win_dma);
-    for (const void *p : {(const void *)h->dense.image, (const void *)h->dense.pos})
+    for (const void *p : {(const void *)h->dense.image, (const void *)h->dense.pos, (const void *)h->dense.events, (const void *)h->d_dense_rows})
         if (p) (void)hipFree(const_cast<void *>(p));
     (void)hipFree(h->d_stage_lut); (void)hipFree(h->d_nbm1); (void)hipFree(h->d_win_pos);
     (void)hipFree(h->d_win_row_begin); (void)hipFree(h->d_win_rows);
@@ -1223,14 +1236,22 @@ static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream
     else hipLaunchKernelGGL(ace_many_kernel<false>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
     return true;
 }
-// ... over dense tables (ace_dense.h has both sides measured: from the first batch on that the kernel of mid-sized ones leaves).
+template <int A>
+static void launch_dense_a(const ace_handle_t *h, const AceKernelArgs &a, size_t groups, uint32_t slices, hipStream_t s) {
+    if (h->dense.events) hipLaunchKernelGGL((ace_dense_kernel<A, true>), dim3((unsigned)groups), dim3(kDenseWinLanes), h->dense_lds, s, a, h->dense, slices);
+    else hipLaunchKernelGGL((ace_dense_kernel<A, false>), dim3((unsigned)groups), dim3(kDenseLanes), h->dense_lds, s, a, h->dense, slices);
+}
+// ... over dense tables (ace_dense.h and the table above kSpreadMaxPlain have both sides measured).
 static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     if (!h->dense.image || a.range || a.stage_out || !a.stage_ws) return false;
-    const uint32_t slices = ace_dense_slices(a.g.P), lanes = 64u * slices, lds = ace_dense_lds(h->dense.image16 * 16u);
+    const bool win = h->dense.events != nullptr;
+    const uint32_t slices = win ? ace_dense_slices(a.g.P, kDenseWinLanes / 64, 256) : ace_dense_slices(a.g.P, kDenseLanes / 64, 512), lanes = 64u * slices;
     const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
     if (a.stage_ws != h->d_stage_ws || groups * lanes > h->stage_ws_plans) return false;    // (the static scratch holds no such records)
-    if (h->dense_array == 320u) hipLaunchKernelGGL(ace_dense_kernel<320>, dim3((unsigned)groups), dim3(kDenseLanes), lds, s, a, h->dense, slices);
-    else hipLaunchKernelGGL(ace_dense_kernel<520>, dim3((unsigned)groups), dim3(kDenseLanes), lds, s, a, h->dense, slices);
+    if (h->dense_array == kDenseArrays[0]) launch_dense_a<kDenseArrays[0]>(h, a, groups, slices, s);
+    else if (h->dense_array == kDenseArrays[1]) launch_dense_a<kDenseArrays[1]>(h, a, groups, slices, s);
+    else if (h->dense_array == kDenseArrays[2]) launch_dense_a<kDenseArrays[2]>(h, a, groups, slices, s);
+    else launch_dense_a<kDenseArrays[3]>(h, a, groups, slices, s);
     return true;
 }
 template <int L>
@@ -1245,7 +1266,7 @@ static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hip
 
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     const int mid = duo_lanes(h, a);
-    const int most = a.stage_out ? kSpreadMaxRecords : mid ? kSpreadMaxPlain : !a.stage_ws ? kSpreadMaxSlow : h->d_win_dma ? kSpreadMaxWindowed : kSpreadMaxOther;
+    const int most = a.stage_out ? kSpreadMaxRecords : mid ? kSpreadMaxPlain : !a.stage_ws ? kSpreadMaxSlow : h->d_win_dma || h->dense.image ? kSpreadMaxWindowed : kSpreadMaxOther;
     if (a.pos_spread && a.g.P <= most) {
         if (a.range) launch_spread<true, true>(a, s);
         else if (a.stage_out) launch_spread<true, false>(a, s);
@@ -1265,7 +1286,7 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
 // per-plan workspace; the handle keeps one and grows it on demand.
 static int ensure_stage_ws(ace_handle_t *h, AceKernelArgs *a) {
     a->stage_ws = nullptr;
-    if (a->range || a->stage_out || (h->n_windows > 1 && !h->d_pos_types) || h->geom.N >= 32768 || (h->geom.flags & ACE_F_COLLECTIVE_MEM)) return ACE_OK;
+    if (a->range || a->stage_out || (h->n_windows > 1 && !h->d_pos_types && !h->dense.image) || h->geom.N >= 32768 || (h->geom.flags & ACE_F_COLLECTIVE_MEM)) return ACE_OK;
     // (a block more: the kernel of large batches rounds the share of every CU up)
     const size_t need = (((size_t)a->g.P + kBlock - 1) / kBlock + 1) * kBlock;
     if (need * ACE_MAX_STAGES * (ACE_WS_REC / 2) > 0xffffffffull) return ACE_OK;   // (a workspace of 64 GiB and more: such batches take the plain kernel)

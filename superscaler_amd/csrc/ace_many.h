@@ -1,6 +1,7 @@
 // Scoring of LARGE batches where the assembly op loop runs: the kernel of ace_score_loop.h (a plan per lane, up to sixteen
-// wavefronts per workgroup and CU) with workgroups of as many plans as make an even share.  Every row resident: from 65,537
-// plans on, where the tables do not fit the dense form (ace_dense.h).  Windowed rows: whatever the kernel of small batches leaves.
+// wavefronts per workgroup and CU) with workgroups of as many plans as make an even share.  For tables that do not fit the dense
+// form (ace_dense.h): more distinct costs or sizes than its lists hold.  Every row resident: from 65,537 plans on.  Windowed rows:
+// whatever the kernel of small batches leaves.
 //
 // The rows fill a CU's LDS, so the workgroups of a batch run in rounds of 256, and with 1,024 plans each a batch of 200,000
 // leaves a fifth of the CUs idle and the last 37,856 plans of one of 300,000 take a second round of their own.  Here a

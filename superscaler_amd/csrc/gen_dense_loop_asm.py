@@ -28,7 +28,12 @@ lone wavefront needs five to six cycles for either.  So a step has one wait (for
 Masks compared a step ahead, or the rule for layer starts as a branch, were 3 % slower; the table offsets of the next stage set in a
 part of their own in front of the sums (so that the reads go out earlier) 1.5 %.
 
-One text per (resharding on / off).  Register use: v28-v127 and s24-s99 belong to the loop; operands live below.
+The "_WIN" texts are for rows that do not fit in LDS together: windows of rows in alternate halves of the rows' space.  At a window's
+first position all wavefronts of the workgroup meet at a barrier, after which each issues its share of the LDS-direct loads of the
+window AFTER the one being entered (fetch_event; the records come from ace_dense.h), which arrive while the workgroup walks a whole
+window.  A lane's offsets are those of the half in use: they and the table they come from change sides with the window.
+
+One text per (rows resident / windowed, resharding on / off).  Register use: v28-v127 and s24-s99 belong to the loop; operands live below.
 """
 import os
 
@@ -74,7 +79,7 @@ def D(y):                                   # per 4-op word: codes 0 1 2 + const
     return dict(a01=f"v{b}", a23=f"v{b + 1}", r8=f"v{b + 2}")
 
 
-ZVRK, ZV, RK, NZVRK = "v[118:119]", "v118", "v119", "v[120:121]"
+ZVRK, ZV, RK, NZVRK, NZV = "v[118:119]", "v118", "v119", "v[120:121]", "v120"
 GLOGS, GLOGS_LO = "v[122:123]", "v122"       # log2 of the sizes of the plan's stages to come, 4 bits each, the next one at bit 3
 LUT2, PACE = "v124", "v125"
 T1, T2, T3 = "v126", "v127", "v73"
@@ -93,6 +98,9 @@ SOFF = ("0", "s53", "s57", "s60", "s61")     # where each piece of the wavefront
 
 K78, VMN, NGRP, MASK, PLANT, PREVFL = "s44", "s50", "s51", "s52", "s56", "s62"
 S0, S1, S2, S23 = "s96", "s97", "s98", "s[98:99]"
+# windowed rows: the next window's first position, the next fetch event, "a window was entered since the next group's code words
+# were asked for", how far the other half of the rows (of the offsets table) lies from the current one
+NEXTWIN, EVT, ARRIVED, HALF, LUTHALF, DMAPTR, DMAOFF = "s34", "s35", "s55", "s54", "s57", "s[60:61]", "s63"
 
 
 def P(y, q):                                # position entry: dot4 scalars of the op's row and of its pair, record word, flags
@@ -105,8 +113,10 @@ def PBUF(y):
 
 
 class Dense:
-    def __init__(self, rsh):
-        self.rsh, self.lines = rsh, []
+    def __init__(self, rsh, win=False):
+        self.rsh, self.win, self.lines = rsh, win, []
+        # (windowed rows: no scalar register is left to keep them in)
+        self.soff = ("0", "s97", "s98", "s99", DMAOFF) if win else SOFF
 
     def o(self, s):
         self.lines.append(s)
@@ -143,7 +153,10 @@ class Dense:
         self.o(f"v_mbcnt_lo_u32_b32 {T1}, s48, {RINGV}")
         self.o(f"v_mbcnt_hi_u32_b32 {T1}, s49, {T1}")
         self.o(f"v_lshlrev_b32 {T1}, 4, {T1}")
-        for regs, off in zip(PIECES, SOFF):
+        if self.win:
+            for i in range(1, 5):
+                self.o(f"s_mov_b32 {self.soff[i]}, {16384 * i}")
+        for regs, off in zip(PIECES, self.soff):
             self.o(f"buffer_store_dwordx4 {regs}, {T1}, {SRD}, {off} offen")
         self.o(f"s_bcnt1_i32_b64 {S0}, {ROOM}")
         self.o("s_mov_b64 exec, -1")
@@ -165,6 +178,53 @@ class Dense:
         if self.rsh:
             self.o(f"ds_read_u16 {R(1 - x1)}, {T2}")           # where the cost of the (k1, k1 + 1) pair is
 
+    def fetch_event(self, L, pq):
+        """Windowed rows, one fetch event: the wavefront's record {first position of the window after the one being entered,
+        bit 0: wait for the fetch | number of loads << 8, address of the rows} and four loads {byte offset in the rows, LDS
+        address} (through s[pq:pq+7]); all wavefronts of the workgroup meet, then each issues its loads (LDS-direct, 1 KB each)."""
+        self.o(f"s_mul_i32 {DMAOFF}, {EVT}, %[eventsize]")
+        self.o(f"s_add_u32 {DMAOFF}, {DMAOFF}, %[waveoff]")
+        self.o(f"s_load_dwordx4 s[96:99], {DMAPTR}, {DMAOFF}")
+        self.o(f"s_add_u32 {DMAOFF}, {DMAOFF}, 16")
+        self.o(f"s_load_dwordx8 s[{pq}:{pq + 7}], {DMAPTR}, {DMAOFF}")
+        self.o("s_waitcnt vmcnt(0) lgkmcnt(0)")             # this wavefront's reads of the old rows and its loads so far have landed
+        self.o("s_barrier")
+        self.o(f"s_mov_b32 {ARRIVED}, 1")                   # (so have the next group's code words, if they were asked for)
+        self.o(f"s_add_u32 {EVT}, {EVT}, 1")
+        self.o(f"v_mbcnt_lo_u32_b32 {T1}, -1, 0")
+        self.o(f"v_mbcnt_hi_u32_b32 {T1}, -1, {T1}")
+        self.o(f"v_lshlrev_b32 {T1}, 4, {T1}")
+        self.o(f"s_bfe_u32 {DMAOFF}, s97, 0x40008")         # number of loads
+        for j in range(4):
+            self.o(f"s_cmp_le_u32 {DMAOFF}, {j}")
+            self.o(f"s_cbranch_scc1 L_fd_{L}")
+            self.o(f"s_mov_b32 m0, s{pq + 2 * j + 1}")
+            self.o(f"v_add_u32_e32 {T2}, s{pq + 2 * j}, {T1}")
+            self.o("s_nop 0")
+            self.o(f"global_load_lds_dwordx4 {T2}, s[98:99]")
+        self.o(f"L_fd_{L}:")
+        self.o(f"s_mov_b32 {NEXTWIN}, s96")
+        self.o("s_bitcmp1_b32 s97, 0")
+        self.o(f"s_cbranch_scc0 L_fa_{L}")
+        self.o("s_waitcnt vmcnt(0)")
+        self.o("s_barrier")
+        self.o(f"L_fa_{L}:")
+
+    def window_switch(self, k1, L, y):
+        """Windowed rows: if op k1 of the group (a multiple of four) is the first of the next window, the next fetch event; the
+        lanes' offsets go over to the other half."""
+        self.c("rows of the next window, if it starts with the next op")
+        self.o(f"s_add_u32 {S0}, {POSBASE}, {k1}")
+        self.o(f"s_cmp_eq_u32 {S0}, {NEXTWIN}")
+        self.o(f"s_cbranch_scc0 L_nw_{L}")
+        self.fetch_event(L, 64 + 16 * y)                    # (the first two position entries of this word are done with)
+        self.o(f"v_add_u32_e32 {ZV}, {HALF}, {ZV}")
+        self.o(f"v_add_u32_e32 {NZV}, {HALF}, {NZV}")
+        self.o(f"v_add_u32_e32 {LUT2}, {LUTHALF}, {LUT2}")
+        self.o(f"s_sub_u32 {HALF}, 0, {HALF}")
+        self.o(f"s_sub_u32 {LUTHALF}, 0, {LUTHALF}")
+        self.o(f"L_nw_{L}:")
+
     def slot(self, k):
         j, b = k >> 2, k & 3
         y, x, k1 = j & 1, k & 1, k + 1
@@ -174,7 +234,7 @@ class Dense:
         L = f"{k}_%="
         self.c(f"================ op {k} of the group")
         if b == 2:
-            if k == 2:
+            if k == 2 and not self.win:
                 self.c("pacing: the wavefronts of a SIMD that entered this group last get the issue priority, those ahead yield")
                 self.o(f"v_readfirstlane_b32 {S0}, {PACE}")
                 self.o(f"s_and_b32 {S0}, {S0}, %[pacemask]")
@@ -250,6 +310,8 @@ class Dense:
         self.o(f"s_cmp_eq_u32 {S0}, %[n_ops]")
         self.o("s_cbranch_scc1 L_exit_%=")
         self.o(f"L_ne_{L}:")
+        if self.win and b == 3:
+            self.window_switch(k1, L, y)
         self.addresses(k1)
         self.o(f"v_pk_max_u16 {RANK}, {RANK}, {RANKS(x)}")
         self.o("s_nop 0" if self.rsh else "s_nop 1")
@@ -296,6 +358,11 @@ class Dense:
 
     def next_group_words(self):
         self.c("the next group's code words have arrived (zeros after the last group): padding and end-of-plan mark")
+        if self.win:
+            # (not if a window was entered since the words were asked for: they were waited for there, and the window
+            # loads now in flight need not be)
+            self.o(f"s_cmp_eq_u32 {ARRIVED}, 1")
+            self.o("s_cbranch_scc1 L_arr_%=")
         # (vector-memory instructions complete in the order they were issued: only what was issued before the load and
         # the load itself have to be waited for, not the record stores of the last few ops)
         for n in (15, 10, 5):
@@ -309,9 +376,22 @@ class Dense:
             if n != 5:
                 self.o("s_branch L_vmd_%=")
         self.o("L_vmd_%=:")
+        if self.win:
+            self.o("L_arr_%=:")
         self.o(f"s_sub_i32 {LEFT}, %[n_ops], {POSBASE}")
         self.o(f"s_sub_i32 {LEFT}, {LEFT}, 16")
         self.apply_masks(NEXT, "nx")
+
+    def pace_count(self):
+        self.c("pacing: count this wavefront into this group's arrival counter of its SIMD (the count before it: its rank there)")
+        self.o(f"s_and_b32 {S0}, {GRP}, 7")
+        self.o(f"s_lshl_b32 {S0}, {S0}, 2")
+        self.o(f"s_add_u32 {S0}, {S0}, %[pace]")
+        self.o(f"v_mov_b32 {T3}, {S0}")
+        self.o(f"v_mov_b32 {T2}, 1")
+        self.o("s_mov_b64 exec, 1")
+        self.o(f"ds_add_rtn_u32 {PACE}, {T3}, {T2}")
+        self.o("s_mov_b64 exec, -1")
 
     def build(self):
         o, c = self.o, self.c
@@ -329,8 +409,9 @@ class Dense:
         o("s_mov_b32 s27, 0x00020000")
         o(f"s_mov_b32 {KC}, 0x{'00070707' if self.rsh else '00000707'}")
         o(f"s_mov_b64 {PEND}, 0")
-        for i in range(1, 5):
-            o(f"s_mov_b32 {SOFF[i]}, {16384 * i}")
+        if not self.win:
+            for i in range(1, 5):
+                o(f"s_mov_b32 {SOFF[i]}, {16384 * i}")
         o(f"s_movk_i32 {LASTPLACE}, {16 * 128}")
         o(f"v_mov_b32 {P_META}, %[meta0]")
         o(f"v_mov_b32 {RINGV}, 0")
@@ -343,6 +424,21 @@ class Dense:
         o(f"s_mov_b32 {GRP}, 0")
         o(f"s_mov_b32 {POSBASE}, 0")
         o(f"s_mov_b32 {PREVFL}, 0")
+        if self.win:
+            c("issue priority of this wavefront: the deeper its plans, the higher (the others wait for it at every window)")
+            for lvl in (3, 2, 1):
+                o(f"s_cmp_eq_u32 %[prio], {lvl}")
+                o(f"s_cbranch_scc0 L_np{lvl}_%=")
+                o(f"s_setprio {lvl}")
+                o(f"L_np{lvl}_%=:")
+            o(f"s_mov_b64 {DMAPTR}, %[dma]")
+            o(f"s_mov_b32 {HALF}, %[half]")
+            o(f"s_mov_b32 {LUTHALF}, %[luthalf]")
+            o(f"s_mov_b32 {ARRIVED}, 0")
+            o(f"s_mov_b32 {EVT}, 0")
+            c("window 0 (waited for), then window 1")
+            self.fetch_event("s0_%=", 80)
+            self.fetch_event("s1_%=", 80)
         o(f"global_load_dwordx4 v[104:107], %[codeoff], {CPTR}")
         o(f"s_load_dwordx16 {PBUF(0)}, {PPTR}, 0")
         for r in (FWD, BWD, RUN, PEAK, RCS, RSF, RSB, W_, A_, SAVED, P_RSF, P_RSB):
@@ -375,15 +471,10 @@ class Dense:
             o(f"v_mov_b32 {r}, 0")
         o("L_loaded_%=:")
         o(f"s_mov_b32 {VMN}, 0")
-        c("pacing: count this wavefront into this group's arrival counter of its SIMD (the count before it: its rank there)")
-        o(f"s_and_b32 {S0}, {GRP}, 7")
-        o(f"s_lshl_b32 {S0}, {S0}, 2")
-        o(f"s_add_u32 {S0}, {S0}, %[pace]")
-        o(f"v_mov_b32 {T3}, {S0}")
-        o(f"v_mov_b32 {T2}, 1")
-        o("s_mov_b64 exec, 1")
-        o(f"ds_add_rtn_u32 {PACE}, {T3}, {T2}")
-        o("s_mov_b64 exec, -1")
+        if self.win:
+            o(f"s_mov_b32 {ARRIVED}, 0")
+        else:
+            self.pace_count()
         for k in range(16):
             self.slot(k)
         c("---- next group")
@@ -416,11 +507,12 @@ def c_string(lines):
 def render():
     """The text of ace_dense_loop_asm.inc."""
     parts = ["// Generated by gen_dense_loop_asm.py -- do not edit.  gfx950 assembly of the op loop over the dense tables,",
-             "// one text per (resharding on / off); see the generator for the design.", "#pragma once", ""]
-    for rsh in (1, 0):
-        parts.append(f"#define ACE_DENSE_ASM_RSH{rsh} \\")
-        parts.append(c_string(Dense(bool(rsh)).build()))
-        parts.append("")
+             "// one text per (rows resident / windowed, resharding on / off); see the generator for the design.", "#pragma once", ""]
+    for win in (0, 1):
+        for rsh in (1, 0):
+            parts.append(f"#define ACE_DENSE_ASM{'_WIN' if win else ''}_RSH{rsh} \\")
+            parts.append(c_string(Dense(bool(rsh), bool(win)).build()))
+            parts.append("")
     clob = ", ".join(f'"v{i}"' for i in range(28, 128)) + ", " + ", ".join(f'"s{i}"' for i in range(24, 100) if i not in (32, 33))   # (s32 / s33 are the ABI's stack registers)
     parts.append(f"#define ACE_DENSE_ASM_CLOBBERS {clob}, \"vcc\", \"scc\", \"memory\"")
     parts.append("")

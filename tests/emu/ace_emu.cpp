@@ -130,7 +130,10 @@ extern "C" int ace_emu_dense(const ace_tables_t *t, const uint8_t *codes /* [P][
     g.flags = t->flags; g.main_params = t->main_params; g.optimizer = t->optimizer;
     g.mem_limit = memory_limit; g.strict = strict ? 1 : 0;
     const AceDenseArgs &da = d.args;
-    const AceLds lds{d.image.data(), (uint32_t)d.image.size()};
+    // (windowed rows: both halves behind the image; a window's rows are put there before its first op, everything else is poisoned)
+    std::vector<unsigned char> mem(std::max<size_t>(d.lds, d.image.size()), 0xff);
+    memcpy(mem.data(), d.image.data(), d.image.size());
+    const AceLds lds{mem.data(), (uint32_t)(d.windows.empty() ? d.image.size() : d.rows_off + 2u * da.half)};
     g.out_off = 0u;
     auto dot = [](uint32_t a, uint32_t b, uint32_t c) {
         for (int k = 0; k < 4; ++k) c += ((a >> (8 * k)) & 255u) * ((b >> (8 * k)) & 255u);
@@ -152,15 +155,24 @@ extern "C" int ace_emu_dense(const ace_tables_t *t, const uint8_t *codes /* [P][
         };
         ace_u2 z = stage();
         double fwd = 0, bwd = 0, rcs = 0, rsf = 0, rsb = 0, w = 0, act = 0, saved = 0, peak = 0, run = 0;
-        uint32_t rf = 0, rb = 0, cost = 0, before = (code(0) & 7u) << 8 | da.row0 << 24;
+        uint32_t rf = 0, rb = 0, cost = 0, before = (code(0) & 7u) << 8 | da.first_in << 24;
         int n_st = 0;
+        size_t win = 0;
+        uint32_t half = 0;
         for (int i = 0; i < N; ++i) {
+            if (win < d.windows.size() && d.window_start[win] == i) {
+                half = win & 1 ? da.half : 0u;
+                memset(mem.data() + d.rows_off, 0xff, 2u * da.half);
+                for (size_t s = 0; s < d.windows[win].size(); ++s)
+                    memcpy(mem.data() + d.rows_off + half + s * d.row_pitch, d.rows.data() + (size_t)d.windows[win][s] * d.row_pitch, d.row_pitch);
+                ++win;
+            }
             const uint32_t b = code(i), nb = code(i + 1);
             const ace_u4 &pos = d.pos[i];
             uint32_t word = 0;                                          // codes from the even position on, behind them the constant(s)
             for (int k = 0; k < (rsh ? 3 : 2); ++k) word |= (code((i & ~1) + k) & 7u) << (8 * k);
             word |= da.kv;
-            const uint32_t e = dot(word, pos.x, z.x);
+            const uint32_t e = dot(word, pos.x, z.x) + half;
             const double v[4] = {lds.ld<double>(e), lds.ld<double>(e + d.array), lds.ld<double>(e + 2 * d.array), lds.ld<double>(e + 3 * d.array)};
             const uint32_t ranks = lds.ld<uint32_t>(e + 4 * d.array);
             fwd += v[0]; bwd += v[1]; w += v[2]; act += v[3];

@@ -4,6 +4,7 @@ On the CPU: the tables as the library builds them, walked like the assembly loop
 reserved sizes, parked records), against the C oracle and, for codes that name no profiled entry, against the per-plan state
 machine; the committed loop text is what its generator writes.  On the GPU: every plan against the C oracle at the sizes where the
 division into workgroups changes, and malformed plans among good ones."""
+import dataclasses
 import importlib.util
 import os
 import re
@@ -17,8 +18,9 @@ from tests.helpers import c_oracle_scores, emu_dense_score, emu_score
 from tests.test_small_batches import SETTINGS, WORKLOADS, tables_for, with_recompute
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "superscaler_amd", "csrc")
-#: the tables that fit (the others: rows in windows, more entries per row, memory of collectives)
-DENSE = {"gpt3_1_3b", "gpt3_13b", "gpt3_175b", "t5_770m", "gpt_1tp_1mbs", "gpt_16ops", "gpt_wide_stages", "gpt_3tp", "t5_1layer", "t5_1tp"}
+#: the tables that fit (not: memory of collectives)
+DENSE = {"gpt3_1_3b", "gpt3_13b", "gpt3_175b", "t5_770m", "gpt_1tp_1mbs", "gpt_16ops", "gpt_wide_stages", "gpt_3tp", "t5_1layer", "t5_1tp",
+         "wresnet_1b", "resnet_1111", "resnet_16gpus", "resnet_2tp", "gpt_6mbs_64gpus"}
 
 
 def test_committed_dense_loop_is_the_generators_output():
@@ -79,10 +81,14 @@ def test_dense_tables_score_like_the_oracle(name, mode):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,mode,sizes", [("gpt_wide_stages", "plain", (65537, 131073, 262145)), ("t5_1tp", "min", (65600, 262144)),
-                                             ("gpt_3tp", "noreserved", (70001,)), ("gpt3_1_3b", "min", (65537,)), ("t5_770m", "plain", (98304,))])
+                                             ("gpt_3tp", "noreserved", (70001,)), ("gpt3_1_3b", "min", (65537,)), ("t5_770m", "plain", (98304,)),
+                                             # (rows in windows)
+                                             ("wresnet_1b", "min", (6145, 16385, 262145)), ("resnet_1111", "plain", (65537,)),
+                                             ("resnet_16gpus", "noreserved", (6200,)), ("gpt_6mbs_64gpus", "plain", (70001,)), ("270 types", "plain", (20001,))])
 def test_large_batches_over_dense_tables_on_the_gpu(name, mode, sizes):
     from superscaler_amd.evaluator import PlanEvaluator
-    w = WORKLOADS[name]
+    # (more op types than fit eight bits)
+    w = WORKLOADS[name] if name in WORKLOADS else dataclasses.replace(WORKLOADS["wresnet_1b"], resnet_blocks=(3, 4, 23, 3))
     tables = tables_for(w, **SETTINGS[mode])
     assert emu_dense_score(tables, synth.make_plans(w, tables, n_plans=1)) is not None
     ev = PlanEvaluator(tables)
