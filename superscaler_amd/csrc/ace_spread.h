@@ -60,7 +60,7 @@ __host__ __device__ __forceinline__
 uint32_t ace_spread_layout(int cols, int G, unsigned char *lds, SpreadShared *s) {
     uint32_t o = 0;
     auto take = [&](uint32_t bytes) { const uint32_t at = o; o += (bytes + 15u) & ~15u; return lds + at; };
-    s->x = reinterpret_cast<double *>(take((uint32_t)(cols * kSpreadPitch + 16) * 8u));
+    s->x = reinterpret_cast<double *>(take((uint32_t)(cols * kSpreadPitch + 32) * 8u));
     s->fin = reinterpret_cast<double *>(take((uint32_t)(cols * ACE_MAX_STAGES) * 8u));
     s->stage_ms = reinterpret_cast<double *>(take(ACE_MAX_STAGES * 8u));
     s->stage_mb = reinterpret_cast<double *>(take(ACE_MAX_STAGES * 8u));
@@ -131,7 +131,7 @@ template <bool RANGED> ACE_HD SpreadPlan spread_plan(const AceKernelArgs &a, lon
 }
 
 // ---- fetch: the plan's bytes and the small tables into LDS, stage starts per 16-op group -----------------------------------
-template <bool RANGED> ACE_HD void spread_fetch(const AceKernelArgs &a, const SpreadShared &s, const SpreadPlan &p, long long plan, int tid) {
+template <bool RANGED> ACE_HD void spread_fetch(const AceKernelArgs &a, const SpreadShared &s, const SpreadPlan &p, long long plan, int cols, int tid) {
     const AceGeom &g = a.g;
     if (tid < g.G) {
         const ace_u4 cw = a.codes[(size_t)tid * g.P + plan];
@@ -157,6 +157,7 @@ template <bool RANGED> ACE_HD void spread_fetch(const AceKernelArgs &a, const Sp
     if (tid < 16) s.lut[tid] = a.stage_lut[p.bidx * 16u + (uint32_t)tid];
     if (tid < 8) s.keep[tid] = 0u;
     if (tid < 18) s.bound[tid] = g.N;
+    if (tid < cols) s.x[tid * kSpreadPitch + kSpreadLanes] = 0.0;
 }
 
 // ---- stages: where each stage begins -----------------------------------------------------------------------------------------
@@ -301,6 +302,48 @@ template <bool BD, bool COLL> ACE_HD void spread_seg(const SpreadShared &s, int 
     if (tid == kSpreadLanes - 1) s.carry[parity ^ 1] = (r.flags & SF_KEEP) ? spread_run(s, act, carry, tid) : 0.0;
 }
 
+// The values lo .. hi - 1 of a column (16-byte aligned; the one at kSpreadLanes is 0.0) added to `acc` in order (SUM), or their
+// maximum with it.  A dependent addition takes a lone wavefront 3.5 ns, any other instruction about three, an LDS read 23: so
+// values come in pairs, sixteen on their way while sixteen are added, in two sets of registers that take turns (nothing is
+// moved), and the rest of a column as a block whose places past its end read the 0.0 (which changes neither a sum nor a maximum
+// here: both start at +0.0).  Eight at a time, moved from set to set: 821 ops of one stage 25.4 us, now SPREAD_NOW.
+template <bool SUM> ACE_HD double spread_next(double acc, double v) { return SUM ? acc + v : ace_max(acc, v); }
+template <bool SUM> ACE_HD double spread_column(const double *x, double acc, int lo, int hi) {
+    int k = lo;
+    if ((k & 1) && k < hi) acc = spread_next<SUM>(acc, x[k++]);
+    if (k + 16 <= hi) {
+        const ace_d2 *p = reinterpret_cast<const ace_d2 *>(x + k);
+        ace_d2 v[8], u[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = p[j];
+        for (;;) {
+            // (reads past the column's end stay inside the columns and are not used)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) u[j] = p[8 + j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc = spread_next<SUM>(spread_next<SUM>(acc, v[j].x), v[j].y);
+            k += 16;
+            if (k + 16 > hi) break;
+            p += 16;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) v[j] = p[j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) acc = spread_next<SUM>(spread_next<SUM>(acc, u[j].x), u[j].y);
+            k += 16;
+            if (k + 16 > hi) break;
+        }
+    }
+    while (k < hi) {
+        double v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = x[k + j < hi ? k + j : kSpreadLanes];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) acc = spread_next<SUM>(acc, v[j]);
+        k += 8;
+    }
+    return acc;
+}
+
 // ---- chain: this chunk's share of the (stage, accumulator) of the lane ------------------------------------------------------
 template <bool BD, bool RANGED, bool COLL>
 ACE_HD void spread_chain(const SpreadShared &s, const SpreadPlan &p, int c0, int tid, SpreadLane &r) {
@@ -314,29 +357,7 @@ ACE_HD void spread_chain(const SpreadShared &s, const SpreadPlan &p, int c0, int
     lo = (lo > c0 ? lo : c0) - c0;
     hi = (hi < c0 + kSpreadLanes ? hi : c0 + kSpreadLanes) - c0;
     const double *x = s.x + col * kSpreadPitch;
-    double acc = r.acc;
-    // eight values in flight while eight are added (reads past the stage's end stay inside the columns and are not used)
-    int k = lo;
-    if (k + 8 <= hi) {
-        double v[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = x[k + j];
-        for (; k + 8 <= hi; k += 8) {
-            double u[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) u[j] = x[k + 8 + j];
-            if (sums) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc += v[j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc = ace_max(acc, v[j]);
-            }
-#pragma unroll
-            for (int j = 0; j < 8; ++j) v[j] = u[j];
-        }
-    }
-    for (; k < hi; ++k) acc = sums ? acc + x[k] : ace_max(acc, x[k]);
+    const double acc = sums ? spread_column<true>(x, r.acc, lo, hi) : spread_column<false>(x, r.acc, lo, hi);
     r.acc = acc;
     s.fin[col * ACE_MAX_STAGES + stage] = acc;
 }
@@ -441,7 +462,7 @@ ACE_HD void ace_spread_body(const AceKernelArgs &a, unsigned char *lds_raw, int 
     const bool active = out < a.g.P;
     const size_t rec_doubles = RANGED ? (size_t)ACE_STAGE_REC : (size_t)(ACE_MAX_STAGES * ACE_STAGE_REC);
     double *rec = (BD && a.stage_out && active) ? a.stage_out + (size_t)out * rec_doubles : nullptr;
-    SPREAD_PHASE((spread_fetch<RANGED>(a, s, p, plan, tid)));
+    SPREAD_PHASE((spread_fetch<RANGED>(a, s, p, plan, K::kCols, tid)));
     if (!RANGED) { SPREAD_PHASE(spread_stages(a, s, tid)); }
     SPREAD_NOWAIT((r.acc = 0.0, spread_load<BD, RANGED, COLL>(a, s, p, p.lo, tid, r)));
     int parity = 0;
