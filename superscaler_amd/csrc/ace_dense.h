@@ -56,6 +56,7 @@ constexpr uint32_t kDenseArrays[4] = {320u, 520u, 584u, 968u};   // bytes of an 
 struct AceDenseArgs {
     const ace_u4 *image;        // the tables
     const ace_u4 *pos;          // [16 * G + 16] per position: dot4 scalars of the row and of the slab, record word, flags (as pos4)
+    const ace_u2 *pos_duo;      // ... as the roles of ace_duo.h have it: the two scalars; then the row's and the record word with the flags at bit 12
     const unsigned char *events;        // windowed rows: fetch records, 48 bytes per event and wavefront (see dense_events)
     uint32_t n_events;
     uint32_t image16;           // size of the image in 16-byte pieces
@@ -70,6 +71,7 @@ struct AceDenseArgs {
 struct AceDenseTables {
     std::vector<unsigned char> image;
     std::vector<ace_u4> pos;
+    std::vector<ace_u2> pos_duo;
     std::vector<unsigned char> rows;            // windowed: every row, `row_pitch` bytes each ...
     std::vector<std::vector<uint32_t>> windows; // ... the rows of each window in the order of their slots
     std::vector<int> window_start;
@@ -341,6 +343,7 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     }
     // positions
     d.pos.assign(pos_entries, ace_u4{0u, 0u, 0u, 0u});
+    d.pos_duo.assign(2u * pos_entries, ace_u2{0u, 0u});
     for (size_t i = 0; i < pos_entries; ++i) {
         const bool odd = (i & 1u) != 0u, in = i < (size_t)N;
         const uint32_t info = in ? t->pos_info[i] : 0u, at_row = in ? place[i] : 0u, slab = in ? slab_of[i] : 0u;
@@ -352,6 +355,8 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
         // and 2, bit 11 set), the last op's list of outputs and the next one's of inputs in the other two
         p.z = rsh && odd ? last | (next << 24) | (1u << 11) : (last << 16) | (next << 24);
         p.w = (((info >> 24) & 1u) ^ 1u) | (((info >> 25) & 1u) << 1);
+        d.pos_duo[i] = ace_u2{p.x, p.y};
+        d.pos_duo[pos_entries + i] = ace_u2{p.x, p.z | (p.w << 12)};
     }
     d.array = array;
     g.first_in = in_of[row_of[types[0]]];
@@ -435,18 +440,11 @@ ACE_HD uint32_t dense_shfl(uint32_t x, uint32_t lane) { return (uint32_t)__shfl(
 constexpr uint32_t kDenseWidth = 64;
 #endif
 
-// One record: time and memory of its stage, in st.sum_t and st.max_mem.  `own`: the lane's own plan (its header's words reach the
-// lanes that evaluate its stages through dense_shfl).
-ACE_HD void dense_stage(const AceDenseArgs &d, const AceGeom &g, const AceLds &lds, const DenseState &own, const DenseRecord &rec, DenseState &st) {
-    const uint32_t lane = (rec.tail.w >> 1) & 63u, s = rec.tail.w >> 7;
-    const uint32_t sb = dense_shfl((uint32_t)own.S | (own.bidx << 8), lane);
-    const uint32_t glogs = dense_shfl((uint32_t)own.glogs, lane), glogs_hi = dense_shfl((uint32_t)(own.glogs >> 32), lane);
-    st.cross = dense_shfl(own.cross, lane);
-    st.S = (int)(sb & 0xffu);
+// One record: time and memory of its stage (number `s`, 2^glog GPUs), in st.sum_t and st.max_mem.
+ACE_HD void dense_tail(const AceDenseArgs &d, const AceGeom &g, const AceLds &lds, uint32_t bidx, uint32_t glog, uint32_t s, const DenseRecord &rec, DenseState &st) {
     st.s = (int)s;
-    const uint32_t glog = ((s & 8u ? glogs_hi : glogs) >> (4u * (s & 7u))) & 15u;
     const DenseMeta m = dense_meta(rec.tail.y), before = dense_meta(rec.tail.z);
-    const uint32_t lut = lds.ld<uint32_t>(d.stg_off + ((sb >> 8) * 16u + glog) * 4u);
+    const uint32_t lut = lds.ld<uint32_t>(d.stg_off + (bidx * 16u + glog) * 4u);
     st.mrow = lut >> 16;
     st.t_first = before.c_next >> g.A_shift;
     const uint32_t e = ace_mul24(lut & 15u, (uint32_t)g.C) + before.c_next, o = DenseState::out_entry_addr(g, 0u, m.c_last, st.t_first, st.mrow) >> 4;
@@ -463,6 +461,16 @@ ACE_HD void dense_stage(const AceDenseArgs &d, const AceGeom &g, const AceLds &l
     st.saved = rec.r[3].x; st.peak = rec.r[3].y; st.run = 0.0; st.lastclose = false;
     st.sum_t = 0.0; st.max_t = 0.0; st.max_mem = 0.0;
     st.finish_tail(g, lds, 0u, m.c_last, oe, nullptr);
+}
+
+// ... of the loop here.  `own`: the lane's own plan (its header's words reach the lanes that evaluate its stages through dense_shfl).
+ACE_HD void dense_stage(const AceDenseArgs &d, const AceGeom &g, const AceLds &lds, const DenseState &own, const DenseRecord &rec, DenseState &st) {
+    const uint32_t lane = (rec.tail.w >> 1) & 63u, s = rec.tail.w >> 7;
+    const uint32_t sb = dense_shfl((uint32_t)own.S | (own.bidx << 8), lane);
+    const uint32_t glogs = dense_shfl((uint32_t)own.glogs, lane), glogs_hi = dense_shfl((uint32_t)(own.glogs >> 32), lane);
+    st.cross = dense_shfl(own.cross, lane);
+    st.S = (int)(sb & 0xffu);
+    dense_tail(d, g, lds, sb >> 8, ((s & 8u ? glogs_hi : glogs) >> (4u * (s & 7u))) & 15u, s, rec, st);
 }
 
 // The tails of all stages of a wavefront's plans, a record per lane whoever's it is (all lanes are busy whatever the depths of the
@@ -564,6 +572,14 @@ __device__ __forceinline__ void dense_fetch(const AceDenseArgs &d, unsigned char
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
 }
 
+// The tables, to LDS address 0 on, by the LANES lanes of the workgroup: 1 KB per wavefront and load, all in flight at once.
+template <int LANES> __device__ __forceinline__ void dense_stage_image(const AceDenseArgs &d, unsigned char *lds_raw, uint32_t wave, uint32_t lane) {
+    typedef const void __attribute__((address_space(1))) *gptr;
+    typedef void __attribute__((address_space(3))) *lptr;
+    for (uint32_t at = wave * 64u; at < d.image16; at += LANES)
+        if (at + lane < d.image16) __builtin_amdgcn_global_load_lds((gptr)(d.image + at + lane), (lptr)(lds_raw + at * 16u), 16, 0, 0);
+}
+
 // One workgroup; its LDS array starts at address 0 (the kernel has no other LDS variables).
 template <int A, bool WIN> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
                                                                 int tid, long long block) {
@@ -571,12 +587,7 @@ template <int A, bool WIN> __device__ __forceinline__ void ace_dense_body(const 
     const AceGeom &g0 = a.g;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6), lane = (uint32_t)tid & 63u;
     const uint32_t lanes = 64u * slices;
-    {
-        typedef const void __attribute__((address_space(1))) *gptr;
-        typedef void __attribute__((address_space(3))) *lptr;
-        for (uint32_t at = wave * 64u; at < d.image16; at += kLanes)
-            if (at + lane < d.image16) __builtin_amdgcn_global_load_lds((gptr)(d.image + at + lane), (lptr)(lds_raw + at * 16u), 16, 0, 0);
-    }
+    dense_stage_image<kLanes>(d, lds_raw, wave, lane);
     // Deal: counting sort of the plans by pipeline depth, the deepest first (see ace_score_body); sorted slice q goes to
     // wavefront q in rows of four, every second row reversed: each SIMD gets the same mix.
     unsigned int *cnt = reinterpret_cast<unsigned int *>(lds_raw + d.image16 * 16u);

@@ -99,9 +99,9 @@ __global__ __launch_bounds__(kSpreadLanes) void ace_spread_kernel(const AceKerne
     ace_spread_body<BD, RANGED, COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // Mid-sized batches: several lanes per plan, see ace_duo.h.
-template <int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(const AceKernelArgs a) {
+template <int A, int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(const AceKernelArgs a, const AceDenseArgs d) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_duo_body<L>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_duo_body<A, L>(a, d, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // Large batches on the assembly loop, see ace_many.h.
 template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(const AceKernelArgs a, const uint32_t slices) {
@@ -124,8 +124,8 @@ template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kern
 // where that time is reached.  That place depends on the graph: both times grow with the ops, but not alike.  A path has one
 // limit all the same, at or below the first crossing of the graphs measured for it, so a graph that crosses later has a jump
 // there.  By what else would take the batch, in us per launch at the limit and where the graph crosses (plan per workgroup / the other):
-//   PLAIN    the mid-sized kernel                    limit  4,096: 315 ops  37 / 42, crosses at  4,800 plans; 523 ops  56 /  66,  5,000;
-//                                                                  821 ops  78 / 81,  4,300; 1,251 ops 104 / 111,  4,400
+//   PLAIN    the mid-sized kernel                    limit  4,096: 315 ops  30 / 32, crosses at  4,300 plans; 523 ops  44 /  50,  4,650;
+//                                                                  821 ops  56 / 67,  5,000; 1,251 ops  82 /  81,  4,050
 //   WINDOWED large, windowed rows (dense tables)     limit  6,144: 118 ops  29 / 30, crosses at  6,700 plans; 134 ops 31 / 33, 6,600; 182 ops 35 / 39, 7,150;
 //                                                                  230 ops  40 / 44, 7,050; 270 ops 48 / 49, 6,150
 //   SLOW     no assembly loop (memory of collectives, more than 256 rows)
@@ -779,8 +779,10 @@ template <bool BD, bool RANGED, bool WIN, bool DEFER> static int allow_big_lds()
     return ACE_OK;
 }
 
-template <int L> static int allow_duo_lds() {
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<L>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+template <int A> static int allow_duo_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<A, 64>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<A, 128>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<A, 256>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     return ACE_OK;
 }
 
@@ -961,6 +963,7 @@ static int setup_dense(ace_handle *h, const ace_tables_t *t, size_t pos_entries)
     if (!d.ok) return ACE_OK;
     h->dense = d.args;
     int rc = upload((void **)&h->dense.pos, d.pos.data(), d.pos.size() * sizeof(ace_u4));
+    if (rc == ACE_OK) rc = upload((void **)&h->dense.pos_duo, d.pos_duo.data(), d.pos_duo.size() * sizeof(ace_u2));
     if (rc == ACE_OK) rc = upload((void **)&h->dense.image, d.image.data(), d.image.size());
     if (rc == ACE_OK && !d.windows.empty()) {
         rc = upload((void **)&h->d_dense_rows, d.rows.data(), d.rows.size());
@@ -1117,7 +1120,8 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = allow_big_lds<false, false, false, false>()) || (rc = allow_big_lds<false, false, true, false>()) ||
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
-        (rc = allow_duo_lds<64>()) || (rc = allow_duo_lds<128>()) || (rc = allow_duo_lds<256>()) ||
+        (rc = allow_duo_lds<kDenseArrays[0]>()) || (rc = allow_duo_lds<kDenseArrays[1]>()) || (rc = allow_duo_lds<kDenseArrays[2]>()) ||
+        (rc = allow_duo_lds<kDenseArrays[3]>()) ||
         (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) || (rc = allow_dense_lds<kDenseArrays[0]>()) || (rc = allow_dense_lds<kDenseArrays[1]>()) ||
         (rc = allow_dense_lds<kDenseArrays[2]>()) || (rc = allow_dense_lds<kDenseArrays[3]>()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
@@ -1134,7 +1138,7 @@ void ace_destroy(ace_handle_t *h) {
     (void)hipFree(h->d_pair_kinds);
     if (h->d_pos4) (void)hipFree(h->d_pos4);
     if (h->d_win_dma) (void)hipFree(h->d_win_dma);
-    for (const void *p : {(const void *)h->dense.image, (const void *)h->dense.pos, (const void *)h->dense.events, (const void *)h->d_dense_rows})
+    for (const void *p : {(const void *)h->dense.image, (const void *)h->dense.pos, (const void *)h->dense.pos_duo, (const void *)h->dense.events, (const void *)h->d_dense_rows})
         if (p) (void)hipFree(const_cast<void *>(p));
     (void)hipFree(h->d_stage_lut); (void)hipFree(h->d_nbm1); (void)hipFree(h->d_win_pos);
     (void)hipFree(h->d_win_row_begin); (void)hipFree(h->d_win_rows);
@@ -1216,8 +1220,7 @@ static bool resident_asm(const ace_handle_t *h, const AceKernelArgs &a) {
 }
 // Workgroup size of the kernel of mid-sized batches for this call, or 0.
 static int duo_lanes(const ace_handle_t *h, const AceKernelArgs &a) {
-    const int L = resident_asm(h, a) ? ace_duo_lanes(a.g.P) : 0;
-    return L && ace_duo_lds(a.g, h->lds_bytes, L) <= kMaxLds ? L : 0;
+    return h->dense.image && !h->dense.events && !a.range && !a.stage_out && a.stage_ws ? ace_duo_lanes(a.g.P) : 0;
 }
 // The kernel of large batches (false: it cannot take this call).
 static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
@@ -1254,14 +1257,19 @@ static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
     else launch_dense_a<kDenseArrays[3]>(h, a, groups, slices, s);
     return true;
 }
-template <int L>
-static void launch_duo_l(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    hipLaunchKernelGGL((ace_duo_kernel<L>), dim3((unsigned)((a.g.P + L - 1) / L)), dim3(kDuoBlock), ace_duo_lds(a.g, h->lds_bytes, L), s, a);
+template <int A>
+static void launch_duo_a(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    const dim3 groups((unsigned)((a.g.P + L - 1) / L));
+    const uint32_t lds = h->dense.image16 * 16u + ace_duo_scratch(L);
+    if (L == 64) hipLaunchKernelGGL((ace_duo_kernel<A, 64>), groups, dim3(kDuoBlock), lds, s, a, h->dense);
+    else if (L == 128) hipLaunchKernelGGL((ace_duo_kernel<A, 128>), groups, dim3(kDuoBlock), lds, s, a, h->dense);
+    else hipLaunchKernelGGL((ace_duo_kernel<A, 256>), groups, dim3(kDuoBlock), lds, s, a, h->dense);
 }
 static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    if (L == 64) launch_duo_l<64>(h, a, s);
-    else if (L == 128) launch_duo_l<128>(h, a, s);
-    else launch_duo_l<256>(h, a, s);
+    if (h->dense_array == kDenseArrays[0]) launch_duo_a<kDenseArrays[0]>(L, h, a, s);
+    else if (h->dense_array == kDenseArrays[1]) launch_duo_a<kDenseArrays[1]>(L, h, a, s);
+    else if (h->dense_array == kDenseArrays[2]) launch_duo_a<kDenseArrays[2]>(L, h, a, s);
+    else launch_duo_a<kDenseArrays[3]>(L, h, a, s);
 }
 
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {

@@ -30,6 +30,16 @@ inline uint32_t ace_many_slices(long long plans) {
 }
 
 #ifndef ACE_HOST_EMU
+// The rows, as one block from LDS address 0 on (a.flat_rows16 > 0): 1 KB per wavefront and load.
+template <int BLOCK> __device__ __forceinline__ void many_rows(const AceKernelArgs &a, unsigned char *lds_raw, uint32_t wave, uint32_t lane) {
+    typedef const void __attribute__((address_space(1))) *gptr;
+    typedef void __attribute__((address_space(3))) *lptr;
+    const uint32_t n = (uint32_t)a.flat_rows16;
+    const unsigned char *src = reinterpret_cast<const unsigned char *>(a.rows);
+    for (uint32_t at = wave * 64u; at < n; at += BLOCK)
+        if (at + lane < n) __builtin_amdgcn_global_load_lds((gptr)(src + (size_t)(at + lane) * 16u), (lptr)(lds_raw + at * 16u), 16, 0, 0);
+}
+
 // Windowed rows: the fetches of a wavefront without plans, in step with the loops of the others (see fetch_event of
 // gen_score_loop_asm.py and setup_windowed_asm).  As many events as they have: every barrier is met.
 __device__ __forceinline__ void many_fetch(const AceKernelArgs &a, unsigned char *lds_raw, uint32_t wave, uint32_t lane) {
@@ -57,7 +67,7 @@ template <bool WIN> __device__ __forceinline__ void ace_many_body(const AceKerne
     const AceGeom &g = a.g;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6), lane = (uint32_t)tid & 63u;
     const uint32_t lanes = 64u * slices;
-    if (!WIN) duo_rows<kLanes>(a, lds_raw, wave, lane);
+    if (!WIN) many_rows<kLanes>(a, lds_raw, wave, lane);
     // Deal: counting sort of the plans by pipeline depth, the deepest first (see ace_score_body), where the small tables go.
     // Sorted slice q goes to wavefront q in rows of four, every second row reversed: each SIMD gets the same mix.
     // (Windowed rows: the deeper its plans, the higher a wavefront's issue priority -- it has the most instructions to issue and

@@ -474,46 +474,6 @@ template <bool BD, bool RANGED, bool DEFER = false, bool COLL = false, bool GROW
         s = n_st;               // (the evaluation walked s again; result() checks the count of the op loop)
     }
 
-    // The stashed stages first, first + step, ... (< n_st) alone: `take(s, t)` gets the time of each, max_mem becomes the
-    // largest of their memories.  What links a stage to the one before it (the row and code of its first op) is read from
-    // that one's record.  Three records in flight, as above.
-    template <class Take>
-    ACE_HD void replay_some(const AceGeom &g, const AceLds &lds, const double *ws, int first, int step, int n_st, uint32_t code0, uint32_t row0,
-                            Take take) {
-        Record r[3];
-        uint64_t link[3];
-        auto fetch = [&](int s2, int k) {
-            replay_load(ws, s2, r[k]);
-            link[k] = 0;
-            if (s2 > 0) {
-                const ace_d2 *p = reinterpret_cast<const ace_d2 *>(ws) + (size_t)((uint32_t)(s2 - 1) * ws_stride + 4u * ws_piece);
-                __builtin_memcpy(&link[k], &p->y, 8);
-            }
-        };
-#pragma unroll
-        for (int k = 0; k < 3; ++k)
-            if (first + k * step < n_st) fetch(first + k * step, k);
-        for (int base = first; base < ACE_MAX_STAGES; base += 3 * step) {
-#pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const int s2 = base + k * step;
-                if (!ACE_WAVE_ANY(s2 < n_st)) return;
-                if (s2 < n_st) {
-                    const uint32_t hi = (uint32_t)(link[k] >> 32);
-                    replay_row = s2 > 0 ? hi >> 24 : row0;
-                    replay_code = s2 > 0 ? ((uint32_t)link[k] >> (8u * (hi & 3u))) & 7u : code0;
-                    Lookups lx;
-                    replay_lookups(g, lds, r[k], s2, true, lx);
-                    replay_take(g, r[k], lx, s2);
-                    if (s2 + 3 * step < n_st) fetch(s2 + 3 * step, k);
-                    sum_t = 0.0;
-                    finish_tail(g, lds, 0u, lx.c_last, lx.oe, nullptr);
-                    take(s2, sum_t);
-                }
-            }
-        }
-    }
-
     // Address of output_size[ops[-1]][mbs[-1]][tp[0]][algo[-1]] (sic, aceso_cost_model.py:321-326) in the row at `lastrow`:
     // `c_last` the last op's code, `tf` the tp index of the stage's first op, `mr` the stage's row of micro-batch indices.
     ACE_HD static uint32_t out_entry_addr(const AceGeom &g, uint32_t lastrow, uint32_t c_last, uint32_t tf, uint32_t mr) {

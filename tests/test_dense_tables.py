@@ -36,7 +36,16 @@ def test_committed_dense_loop_is_the_generators_output():
         for m in re.finditer(rf"\b{kind}(\d+)\b|\b{kind}\[(\d+):(\d+)\]", body):
             a, b = int(m.group(1) or m.group(2)), int(m.group(1) or m.group(3))
             assert low <= a <= b <= high and not (kind == "s" and a <= 33 and b >= 32), m.group(0)
-    # a dot product is read three issue slots later at the earliest
+    dot_products_are_read_late_enough(body)
+
+
+def test_duo_loops_dot_products_are_read_late_enough():
+    with open(os.path.join(CSRC, "ace_duo_loop_asm.inc")) as f:
+        dot_products_are_read_late_enough(f.read().split("#define ACE_DUO_ASM_CLOBBERS")[0])
+
+
+def dot_products_are_read_late_enough(body):
+    """A dot product is read three issue slots later at the earliest."""
     lines = [ln.strip(' "\\').replace("\\n", "") for ln in body.splitlines()]
     ops = [ln for ln in lines if ln and not ln.startswith((";", "#", "//")) and not ln.endswith(":")]
     for i, ln in enumerate(ops):
