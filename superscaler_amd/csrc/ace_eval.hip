@@ -372,15 +372,16 @@ __global__ __launch_bounds__(1024) void topk_finish(TopkState *st, Cand *less, C
 
 // ------------------------------------------------------------------------------------------
 // top-k, short form (k <= 256): workgroups of 1,024 lanes select the k best of a stretch of the input each, one workgroup the
-// k best of what they found (up to 16,384 entries: that workgroup alone).  A selection keeps its entries in registers: radix
-// select on the 96-bit order (key, index) -- so ties fall to the lower index --, starting below the bits that all keys
-// share, cut short as soon as the bucket that holds the k-th entry is small enough to be ranked as it is.  Exact for any
-// input, whatever its order and however many keys are equal: no bound is guessed and no list can overflow.
-// Bound by the latency of the two selections (about three dozen workgroup barriers each), not by reading the input.
-// Launches back to back (10 us is what the host needs for a call), us, against a sampled bound, a filter pass and one
-// selection: k = 64, 4,096 entries 23 -> 10, 262,144 entries 27 -> 17, 2^20 entries 34 -> 23; k = 256, 2^20 entries 80 -> 40.
-// (Behind the scoring kernel, its inputs not in a cache any more, kernel trace: 262,144 entries 8.5 + 8.9, 2^20 entries 15.4 + 15.1;
-// the three launches before took 8.7 + 11.6 + 13.9 there.)
+// k best of what they found (up to 16,384 entries: that workgroup alone).  A selection keeps its entries in registers.  Up to
+// kBoundMaxK it bounds the k-th key by the best ones of the lanes and ranks what lies below (short_bound); where that is too much, and
+// for larger k, it is a radix select on the 96-bit order (key, index) -- so ties fall to the lower index --, starting below the bits that
+// all keys share, cut short as soon as the bucket that holds the k-th entry is small enough to be ranked as it is.  Exact for any
+// input, whatever its order and however many keys are equal: no list that overflows is used.
+// Bound by the latency of the two selections -- their own code's way into the instruction cache, a trip to memory, the barriers --, not
+// by reading the input.  Kernel trace behind the scoring kernel, us, radix select alone -> with the bound, k = 64: 4,096 entries
+// 9.1 -> 6.0; 65,536 entries 9.3 + 7.3 -> 6.7 + 4.6; 262,144 entries 8.6 + 8.9 -> 6.8 + 5.6; 2^20 entries 16.0 + 16.6 -> 11.4 + 8.5; k = 1,
+// 8,192 entries 9.8 -> 4.8.  Where the times spread over more powers of two (lognormal), a call, us: k = 64, 262,144 entries 37 -> 15, k = 160
+// 50 -> 34.
 // ------------------------------------------------------------------------------------------
 constexpr int kShortMaxK = 256;
 constexpr unsigned kShortMaxEntries = 16384;     // entries one workgroup selects from: sixteen per lane
@@ -443,10 +444,77 @@ struct ShortShared {
         Cand bucket[kShortBucket];               // after the passes
     };
     Cand win[kShortMaxK];
+    __align__(16) unsigned int mins[256];        // short_bound
     unsigned int wsum[20];
     unsigned long long wref[16];
-    unsigned int nfin, cur, nwin, nbucket;
+    unsigned int nfin, cur, nwin, nbucket, bound;
 };
+
+// Few entries that hold the k smallest (k <= kBoundMaxK) of the workgroup's, into s.bucket in no order; returns how many (more than
+// kShortBucket: too many, s.bucket is not filled).  Every four neighbouring lanes give the smallest of their entries' leading 32 bits; the
+// k-th smallest of these 256 bounds the k-th key, and what lies at or below it is taken: of random keys in random order some
+// 256 ln(256 / (256 - k)).  That is 251 for k = 160, and ranking them costs their square: a call for 4,096 / 262,144 entries takes
+// 15 / 34 us there (radix select: 26 / 47), with k = 200 29 / 60 (27 / 48).
+// What a selection of 4,096 entries waits for is its own code, run once: some 250 cycles for every 64 bytes of it.  So this is
+// short and has three barriers; the radix selection below takes what it cannot (many equal keys, the best ones all together).
+constexpr int kBoundMaxK = 160;
+template <int kPer>
+__device__ __forceinline__ unsigned int short_bound(ShortShared &s, const unsigned long long (&rk)[kPer], const unsigned int (&ri)[kPer], int k) {
+    const unsigned int tid = threadIdx.x;
+    unsigned int mn = ~0u;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const unsigned int h = (unsigned int)(rk[q] >> 32);
+        mn = h < mn ? h : mn;
+    }
+    unsigned int o = (unsigned int)__builtin_amdgcn_mov_dpp((int)mn, 0xb1, 0xf, 0xf, true);      // (lane ^ 1)
+    mn = o < mn ? o : mn;
+    o = (unsigned int)__builtin_amdgcn_mov_dpp((int)mn, 0x4e, 0xf, 0xf, true);                   // (lane ^ 2)
+    mn = o < mn ? o : mn;
+    if (!(tid & 3u)) s.mins[tid >> 2] = mn;
+    if (tid == 0) { s.nbucket = 0; s.bound = 0; }
+    __syncthreads();
+    unsigned int rank = 0;
+    const ace_u4 *m = reinterpret_cast<const ace_u4 *>(s.mins) + (tid & 3u);
+#pragma unroll 4
+    for (unsigned int j = 0; j < 64u; j += 4u) {
+        const ace_u4 v = m[j];
+        rank += (v.x < mn ? 1u : 0u) + (v.y < mn ? 1u : 0u) + (v.z < mn ? 1u : 0u) + (v.w < mn ? 1u : 0u);
+    }
+    rank += (unsigned int)__builtin_amdgcn_mov_dpp((int)rank, 0xb1, 0xf, 0xf, true);
+    rank += (unsigned int)__builtin_amdgcn_mov_dpp((int)rank, 0x4e, 0xf, 0xf, true);
+    if (!(tid & 3u) && rank < (unsigned int)k) atomicMax(&s.bound, mn);
+    __syncthreads();
+    const unsigned int bound = s.bound;
+#pragma unroll
+    for (int q = 0; q < kPer; ++q)
+        if ((unsigned int)(rk[q] >> 32) <= bound && rk[q] != kInfKey) {
+            const unsigned int p = atomicAdd(&s.nbucket, 1u);
+            if (p < kShortBucket) s.bucket[p] = Cand{rk[q], (long long)ri[q]};
+        }
+    __syncthreads();
+    const unsigned int cnt = s.nbucket;
+    if (cnt > kShortBucket) __syncthreads();                   // (read by all before the radix selection clears it)
+    return cnt;
+}
+
+// `take(rank, entry)` for every entry of `list` (LDS, cnt <= 512 entries): as many neighbouring lanes compare an entry with a part of the
+// others each as there are lanes for it (at most sixteen).
+template <class Take> __device__ __forceinline__ void short_ranked(const Cand *list, unsigned int cnt, Take take) {
+    const unsigned int shift = cnt <= 64u ? 4u : cnt <= 128u ? 3u : cnt <= 256u ? 2u : 1u, parts = 1u << shift;
+    const unsigned int i = threadIdx.x >> shift;
+    if (i >= cnt) return;
+    const Cand me = list[i];
+    unsigned int rank = 0;
+#pragma unroll 2
+    for (unsigned int j = threadIdx.x & (parts - 1u); j < cnt; j += parts) {
+        const Cand o = list[j];
+        rank += o.key < me.key || (o.key == me.key && o.idx < me.idx) ? 1u : 0u;
+    }
+#pragma unroll 1
+    for (unsigned int off = 1; off < parts; off <<= 1) rank += __shfl_xor(rank, off, 64);
+    if (!(threadIdx.x & (parts - 1u))) take(rank, me);
+}
 
 // The k smallest of the workgroup's entries (kPer per lane; kInfKey: none) in (key, index) order, into s.win in no order;
 // returns how many there are (k, or all of them).
@@ -570,7 +638,7 @@ __device__ __forceinline__ unsigned int short_select(ShortShared &s, const unsig
 
 // The k best of each stretch of 1,024 * kPer entries: cand[k * workgroup ...], kInfKey behind the last one.
 template <int kPer>
-__global__ __launch_bounds__(1024) void topk_local(const double *t, const uint8_t *f, size_t n, int k, Cand *cand) {
+__global__ __launch_bounds__(1024) void topk_local(const double *t, const uint8_t *f, size_t n, int k, int spread, Cand *cand) {
     __shared__ ShortShared s;
     unsigned long long rk[kPer];
     unsigned int ri[kPer];
@@ -579,6 +647,31 @@ __global__ __launch_bounds__(1024) void topk_local(const double *t, const uint8_
         const size_t i = ((size_t)blockIdx.x * kPer + q) * 1024 + threadIdx.x;
         rk[q] = i < n ? time_key(t[i], f[i]) : kInfKey;
         ri[q] = (unsigned int)i;
+    }
+    if (k <= kBoundMaxK) {
+        const unsigned int cnt = short_bound<kPer>(s, rk, ri, k);
+        if (cnt <= kShortBucket) {
+            // (where short_bound of the last launch, 2^spread entries per lane, finds the best ones of all stretches with different
+            // four lanes: its bound is close then.  In the order of their ranks it let 256 of 1,024 entries through for k = 64)
+            Cand *out = cand + (size_t)blockIdx.x * k;
+            if (cnt < (unsigned)k) {
+                for (unsigned int j = threadIdx.x; j < (unsigned)k; j += 1024) out[j] = Cand{kInfKey, 0x7fffffffffffffffll};
+                __syncthreads();
+            }
+            const unsigned int A = (unsigned)k >> 2, rot = ((blockIdx.x * (unsigned)k >> 10) * A) >> spread;
+            short_ranked(s.bucket, cnt, [&](unsigned int rank, const Cand &c) {
+                if (rank >= (unsigned)k) return;
+                unsigned int slot = rank;
+                if (rank < 4u * A) {
+                    const unsigned int b = (rank >= A ? 1u : 0u) + (rank >= 2u * A ? 1u : 0u) + (rank >= 3u * A ? 1u : 0u);
+                    unsigned int at = rank - b * A + rot;
+                    if (at >= A) at -= A;
+                    slot = 4u * at + b;
+                }
+                out[slot] = c;
+            });
+            return;
+        }
     }
     const unsigned int nwin = short_select<kPer>(s, rk, ri, k);
     for (unsigned int j = threadIdx.x; j < (unsigned)k; j += 1024)
@@ -607,24 +700,26 @@ __global__ __launch_bounds__(1024) void topk_final(const double *t, const uint8_
                 rk[q] = time_key(t[i], f[i]);
         }
     }
-    const unsigned int nwin = short_select<kPer>(s, rk, ri, k);
-    for (unsigned j = tid; j < (unsigned)k; j += 1024) {
-        if (j >= nwin) {
-            out_idx[j] = -1;
-            out_val[j] = __longlong_as_double(0x7ff0000000000000ll);
-        }
+    const Cand *list = s.bucket;
+    unsigned int cnt = k <= kBoundMaxK ? short_bound<kPer>(s, rk, ri, k) : ~0u;
+    if (cnt > kShortBucket) {
+        cnt = short_select<kPer>(s, rk, ri, k);
+        list = s.win;
     }
     // the winners in ascending (key, index) order
-    static_assert(kShortMaxK * 4 <= 1024, "four lanes per winner");
-    Cand me;
-    const unsigned int rank = short_rank<4>(s.win, nwin, me);
-    if (!(tid & 3) && rank < nwin) {
-        unsigned long long b = me.key;
+    short_ranked(list, cnt, [&](unsigned int rank, const Cand &c) {
+        if (rank >= (unsigned)k) return;
+        unsigned long long b = c.key;
         b = (b >> 63) ? (b & 0x7fffffffffffffffull) : ~b;
-        out_idx[rank] = me.idx;
+        out_idx[rank] = c.idx;
         out_val[rank] = __longlong_as_double((long long)b);
+    });
+    const unsigned int found = cnt < (unsigned)k ? cnt : (unsigned)k;
+    for (unsigned j = found + tid; j < (unsigned)k; j += 1024) {
+        out_idx[j] = -1;
+        out_val[j] = __longlong_as_double(0x7ff0000000000000ll);
     }
-    if (tid == 0 && out_count) *out_count = (int)nwin;
+    if (tid == 0 && out_count) *out_count = (int)found;
 }
 
 // Entries per workgroup of topk_local for n entries (0: topk_final alone): short stretches while the selection from what they
@@ -1476,9 +1571,10 @@ int ace_topk(ace_handle_t *h, const double *d_iter_ms, const uint8_t *d_feasible
     if (per != ~0u) {
         Cand *cand = per ? buf + p2 : nullptr;
         const unsigned int groups = per ? (unsigned int)((n + per - 1) / per) : 0u, m = per ? groups * (unsigned int)k : (unsigned int)n;
-        if (per == 4096) hipLaunchKernelGGL(topk_local<4>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, cand);
-        else if (per == 8192) hipLaunchKernelGGL(topk_local<8>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, cand);
-        else if (per) hipLaunchKernelGGL(topk_local<16>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, cand);
+        const int spread = m <= 4096 ? 2 : m <= 8192 ? 3 : 4;
+        if (per == 4096) hipLaunchKernelGGL(topk_local<4>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, spread, cand);
+        else if (per == 8192) hipLaunchKernelGGL(topk_local<8>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, spread, cand);
+        else if (per) hipLaunchKernelGGL(topk_local<16>, dim3(groups), dim3(1024), 0, s, d_iter_ms, d_feasible, n, k, spread, cand);
         const auto last = m <= 4096 ? topk_final<4> : m <= 8192 ? topk_final<8> : topk_final<16>;
         hipLaunchKernelGGL(last, dim3(1), dim3(1024), 0, s, d_iter_ms, d_feasible, cand, m, k, (long long *)d_idx, d_val, d_count);
         ACE_HIP(hipGetLastError());
