@@ -114,7 +114,7 @@ void ace_dense_kernel(const AceKernelArgs a, const AceDenseArgs d, const uint32_
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_dense_body<A, WIN>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
-template <bool COLL> __global__ __launch_bounds__(kSpreadLanes) void ace_rc_kernel(const RcArgs a, const long long first) {
+template <bool COLL> __global__ __launch_bounds__(kRcLanes, 6) void ace_rc_kernel(const RcArgs a, const long long first) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, first + (long long)blockIdx.x);
 }
@@ -767,6 +767,7 @@ struct ace_handle {
     uint32_t *d_win_rows;
     int32_t flat_rows16;       // see AceKernelArgs
     ace_u2 *d_rc_pos;          // check_recompute's tables (ace_recompute_prepare), or null
+    int32_t rc_groups, rc_waves;   // ... see RcArgs
     double *d_rc_act;
     unsigned char *host_in, *host_out;   // page-locked buffers of ace_score_host (null until the first call)
     struct StepBuffers *step;  // of ace_search_step (null until the first call)
@@ -1722,14 +1723,13 @@ int ace_recompute_prepare(ace_handle_t *h, const int32_t *type_of_pos, const dou
     if (N > kRcMaxOps || !h->d_pos_spread || h->num_types > 0xffff) return ACE_ETOOBIG;
     for (int i = 0; i < N; ++i)
         if (type_of_pos[i] < 0 || type_of_pos[i] >= h->num_types) return ACE_EINVAL;
-    RcShared s;
-    const uint32_t lds = ace_rc_layout(N, h->geom.G, nullptr, &s);
-    if (lds > kMaxLds) return ACE_ETOOBIG;
     ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_rc_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_rc_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     std::vector<ace_u2> pos;
     if (or_enomem([&] { return pos.resize((size_t)N), ACE_OK; })) return ACE_ENOMEM;
-    ace_rc_positions(type_of_pos, no_recompute, N, h->num_types, pos.data());
+    const int groups = ace_rc_positions(type_of_pos, no_recompute, N, h->num_types, pos.data()), waves = ace_rc_waves(N, h->geom.G, groups, kMaxLds);
+    RcShared s;
+    if (ace_rc_layout(N, h->geom.G, groups, waves, nullptr, &s) > kMaxLds) return ACE_ETOOBIG;
     if (h->d_rc_pos) (void)hipFree(h->d_rc_pos);
     if (h->d_rc_act) (void)hipFree(h->d_rc_act);
     h->d_rc_pos = nullptr;
@@ -1737,6 +1737,8 @@ int ace_recompute_prepare(ace_handle_t *h, const int32_t *type_of_pos, const dou
     const size_t n_act = (size_t)h->num_types * h->geom.n_mbs * h->geom.n_tp * h->geom.n_algo;
     int rc = upload((void **)&h->d_rc_pos, pos.data(), pos.size() * sizeof(ace_u2));
     if (rc == ACE_OK) rc = upload((void **)&h->d_rc_act, activations, n_act * sizeof(double));
+    h->rc_groups = groups;
+    h->rc_waves = waves;
     return rc;
 }
 
@@ -1758,10 +1760,12 @@ int ace_recompute_batch(ace_handle_t *h, const ace_batch_t *batch, double memory
     a.limit = memory_limit;
     a.peak_backward = peak_backward;
     RcShared s;
-    const uint32_t lds = ace_rc_layout(a.k.g.N, a.k.g.G, nullptr, &s);
+    a.groups = h->rc_groups;
+    a.waves = h->rc_waves;
+    const uint32_t lds = ace_rc_layout(a.k.g.N, a.k.g.G, a.groups, a.waves, nullptr, &s);
     const auto kernel = a.k.g.flags & ACE_F_COLLECTIVE_MEM ? ace_rc_kernel<true> : ace_rc_kernel<false>;
-    ace_grid_parts((uint64_t)a.k.g.P, kSpreadLanes, [&](uint64_t first, uint32_t groups) {
-        hipLaunchKernelGGL(kernel, dim3(groups), dim3(kSpreadLanes), lds, (hipStream_t)stream, a, (long long)first);
+    ace_grid_parts((uint64_t)a.k.g.P, 64u * (uint32_t)a.waves, [&](uint64_t first, uint32_t groups) {
+        hipLaunchKernelGGL(kernel, dim3(groups), dim3(64u * (uint32_t)a.waves), lds, (hipStream_t)stream, a, (long long)first);
     });
     ACE_HIP(hipGetLastError());
     return ACE_OK;

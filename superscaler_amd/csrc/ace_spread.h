@@ -308,7 +308,7 @@ template <bool BD, bool COLL> ACE_HD void spread_seg(const SpreadShared &s, int 
 // moved), and the rest of a column as a block whose places past its end read the 0.0 (which changes neither a sum nor a maximum
 // here: both start at +0.0).  Eight at a time, moved from set to set: 821 ops of one stage 25.4 us, now 18.7.
 template <bool SUM> ACE_HD double spread_next(double acc, double v) { return SUM ? acc + v : ace_max(acc, v); }
-template <bool SUM> ACE_HD double spread_column(const double *x, double acc, int lo, int hi) {
+template <bool SUM> ACE_HD double spread_column(const double *x, double acc, int lo, int hi, int zero) {
     int k = lo;
     if ((k & 1) && k < hi) acc = spread_next<SUM>(acc, x[k++]);
     if (k + 16 <= hi) {
@@ -336,7 +336,7 @@ template <bool SUM> ACE_HD double spread_column(const double *x, double acc, int
     while (k < hi) {
         double v[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = x[k + j < hi ? k + j : kSpreadLanes];
+        for (int j = 0; j < 8; ++j) v[j] = x[k + j < hi ? k + j : zero];
 #pragma unroll
         for (int j = 0; j < 8; ++j) acc = spread_next<SUM>(acc, v[j]);
         k += 8;
@@ -357,7 +357,7 @@ ACE_HD void spread_chain(const SpreadShared &s, const SpreadPlan &p, int c0, int
     lo = (lo > c0 ? lo : c0) - c0;
     hi = (hi < c0 + kSpreadLanes ? hi : c0 + kSpreadLanes) - c0;
     const double *x = s.x + col * kSpreadPitch;
-    const double acc = sums ? spread_column<true>(x, r.acc, lo, hi) : spread_column<false>(x, r.acc, lo, hi);
+    const double acc = sums ? spread_column<true>(x, r.acc, lo, hi, kSpreadLanes) : spread_column<false>(x, r.acc, lo, hi, kSpreadLanes);
     r.acc = acc;
     s.fin[col * ACE_MAX_STAGES + stage] = acc;
 }

@@ -1,0 +1,47 @@
+"""check_recompute in one launch (superscaler_amd/csrc/ace_recompute.h) where its division of the work changes: workgroups of one wavefront
+(what LDS leaves room for where every op has a type of its own), stages of more segments and of more types than a wavefront has lanes."""
+import ctypes
+import dataclasses
+
+import numpy as np
+import pytest
+
+from superscaler_amd import synth
+from superscaler_amd.recompute import update_recompute_arrays
+from tests.helpers import emu_lib
+from tests.test_recompute_kernel import cost_model, emu_recompute, limits
+from tests.test_small_batches import WORKLOADS
+
+#: 96 layers in one stage, a segment each; 134 types in one or two stages
+LONG = {"gpt3_1_3b": dict(num_layers=96, pp_choices=[1]), "wresnet_1b": dict(pp_choices=[1, 2])}
+
+
+def models(name, emu=True):
+    w = dataclasses.replace(WORKLOADS[name], **LONG.get(name, {}))
+    cm = cost_model(w, emu=emu)
+    return cm, synth.make_plans(w, cm.tables, n_plans=12, seed_offset=4)
+
+
+@pytest.mark.parametrize("lds", [0, 160 * 1024])
+@pytest.mark.parametrize("name", ["gpt3_1_3b", "wresnet_1b", "gpt_16ops", "t5_1layer"])
+def test_one_and_two_wavefronts_on_the_cpu(name, lds):
+    cm, batch = models(name)
+    room = ctypes.c_uint32.in_dll(emu_lib(), "ace_emu_rc_lds")
+    before, room.value = room.value, lds
+    try:
+        for limit in limits(cm, batch):
+            cm.settings.memory_limit = limit
+            codes, flags = emu_recompute(cm, batch)
+            assert not flags.any() and np.array_equal(codes, update_recompute_arrays(cm, batch).codes)
+    finally:
+        room.value = before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", list(LONG))
+def test_long_stages_on_the_gpu(name):
+    (cm, batch), (ref, _) = models(name, emu=False), models(name)
+    for limit in limits(ref, batch):
+        print(f"[case] {name} limit={limit}", flush=True)
+        cm.settings.memory_limit = ref.settings.memory_limit = limit
+        assert np.array_equal(cm.update_recompute_arrays(batch).codes, update_recompute_arrays(ref, batch).codes)
