@@ -809,7 +809,7 @@ __global__ __launch_bounds__(256) void gather_plans_kernel(const ace_u4 *codes_i
     gather_plans_body((first + blockIdx.x) * 256 + threadIdx.x, codes_in, hdr_in, perm, n, G, codes_out, hdr_out);
 }
 
-__global__ __launch_bounds__(kPackLanes) void pack_plans_kernel(const PackArgs a, const long long first) {
+__global__ __launch_bounds__(kPackLanes, 4) void pack_plans_kernel(const PackArgs a, const long long first) {
     __shared__ PackShared s;
     ace_pack_body(a, s, (int)threadIdx.x, first + (long long)blockIdx.x);
 }
