@@ -17,10 +17,10 @@
 // Measured, us per launch, over the table compiler's rows (27 instructions per op and role, scalars of a position by v_readlane) ->
 // over the dense tables:
 //   plans      315 ops        523 ops       821 ops (no resharding)   1,251 ops
-//    8,192     43.1 -> 31.9   67.3 -> 50.8   81.2 -> 67.9             107.3 -> 81.6
-//   16,384     43.9 -> 33.1   68.4 -> 51.4   81.7 -> 68.2             112.1 -> 86.5
-//   32,768     49.4 -> 37.3   80.1 -> 58.5   94.3 -> 74.7             149.4 -> 115.9
-//   65,536     61.4 -> 44.3   106.7 -> 76.8  125.1 -> 94.0            209.8 -> 159.0
+//    8,192     43.1 -> 31.9   67.3 -> 50.8   81.2 -> 67.1             107.3 -> 81.6
+//   16,384     43.9 -> 33.1   68.4 -> 51.4   81.7 -> 67.5             112.1 -> 86.5
+//   32,768     49.4 -> 37.3   80.1 -> 58.5   94.3 -> 73.9             149.4 -> 115.9
+//   65,536     61.4 -> 44.3   106.7 -> 76.8  125.1 -> 88.0            209.8 -> 159.0
 // Up to 16,384 plans the longest wavefront is what is waited for (the memory role of the first part: 250 cycles per op while the stages
 // of its 64 plans end, 160 afterwards, for 24 instructions), from 65,536 on the SIMDs have two and more wavefronts to issue for all
 // the time.
@@ -199,7 +199,12 @@ __device__ __forceinline__ void ace_duo_body(const AceKernelArgs &a, const AceDe
     // the part's first position is in stage `before` (it starts there), or in the one before that
     const bool opens = part == 0u || (first & 0x10u) != 0u, any = part == 0u || own != 0u;
     const uint32_t here = before + (opens ? 1u : 0u);                // one more than the index of that stage
-    if (part == 0u) __builtin_amdgcn_s_setprio(3);                  // (the longest walk of a slice)
+    // Issue priority to the longest walk of a slice, the first part's; without resharding the time role's step is half the memory's, whose
+    // walks go first then (65,536 plans of 821 ops 93.7 -> 88.0 us, 16,384 68.4 -> 67.5; with resharding 1,251 ops lose 0.7 % by it).
+    // No priorities: 523 ops, 32,768 plans 58.6 -> 64.0.
+    if (part == 0u && (role || (g.flags & ACE_F_RESHARDING))) __builtin_amdgcn_s_setprio(3);
+    else if (part == 0u) __builtin_amdgcn_s_setprio(2);
+    else if (role && !(g.flags & ACE_F_RESHARDING)) __builtin_amdgcn_s_setprio(1);
     if (grp < grp_end && __any(any)) {
         const uint32_t shift = here > 1u ? 4u * (here - 1u) : 0u, lut = d.lut_off + st.bidx * 128u, to = at * 16u + role * 2u * kPiece;
         const uint64_t glogs = shift < 64u ? st.glogs >> shift : 0ull;
