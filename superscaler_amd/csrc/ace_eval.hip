@@ -1762,7 +1762,7 @@ int ace_recompute_batch(ace_handle_t *h, const ace_batch_t *batch, double memory
     RcShared s;
     a.groups = h->rc_groups;
     a.waves = h->rc_waves;
-    const uint32_t lds = ace_rc_layout(a.k.g.N, a.k.g.G, a.groups, a.waves, nullptr, &s);
+    const uint32_t lds = ace_rc_layout(a, nullptr, &s);
     const auto kernel = a.k.g.flags & ACE_F_COLLECTIVE_MEM ? ace_rc_kernel<true> : ace_rc_kernel<false>;
     ace_grid_parts((uint64_t)a.k.g.P, 64u * (uint32_t)a.waves, [&](uint64_t first, uint32_t groups) {
         hipLaunchKernelGGL(kernel, dim3(groups), dim3(64u * (uint32_t)a.waves), lds, (hipStream_t)stream, a, (long long)first);

@@ -27,7 +27,8 @@ constexpr int kRcLanes = 128;            // the most a workgroup has
 struct RcArgs {
     AceKernelArgs k;            // batch, tables, geometry
     const ace_u2 *pos;          // [N] previous | next op of the same type << 16 (0xffff / N: none); type | no-recompute flag << 16 | group << 17
-    int32_t groups, waves;      // types in use, numbered as groups; wavefronts of a workgroup
+    int32_t groups = 0;         // types in use, numbered as groups (0: room for as many as there are ops)
+    int32_t waves = 1;          // wavefronts of a workgroup
     const double *act;          // raw activations [n_types][n_mbs][n_tp][n_algo]
     const uint8_t *status;      // [P] what scoring the batch said
     ace_u4 *codes_out;          // [G][P]
@@ -52,6 +53,7 @@ struct RcShared {
     // per stage: largest reserved sizes (forward, backward, of a collective) as their bits; input, weights, activations; its memory
     unsigned long long *reserved;
     double *in, *sums, *mem;
+    int32_t groups;             // how many `sum` and `first` have room for
 };
 // an ordinary op with a layer start behind it; an ordinary op (group numbers are below kRcMaxOps)
 enum { RC_GROUP = 0xfff, RC_LAST = 0x4000, RC_ORDINARY = 0x8000 };
@@ -63,12 +65,13 @@ __host__ __device__ __forceinline__
 #endif
 uint32_t ace_rc_layout(int N, int G, int groups, int waves, unsigned char *lds, RcShared *s) {
     uint32_t o = 0;
+    s->groups = groups ? groups : N;
     auto take = [&](uint32_t bytes) { const uint32_t at = o; o += (bytes + 15u) & ~15u; return lds + at; };
     const uint32_t n8 = (uint32_t)N * 8u + 128u;        // (chains read up to sixteen values ahead)
     s->act = reinterpret_cast<double *>(take(n8));
     s->tmp = reinterpret_cast<double *>(take(n8));
-    s->sum = reinterpret_cast<double *>(take((uint32_t)(waves * groups) * 8u));
-    s->first = reinterpret_cast<uint16_t *>(take((uint32_t)(waves * groups) * 2u));
+    s->sum = reinterpret_cast<double *>(take((uint32_t)(waves * s->groups) * 8u));
+    s->first = reinterpret_cast<uint16_t *>(take((uint32_t)(waves * s->groups) * 2u));
     s->type = reinterpret_cast<uint16_t *>(take((uint32_t)N * 2u));
     s->next = reinterpret_cast<uint16_t *>(take((uint32_t)N * 2u));
     s->codes = take((uint32_t)G * 16u + 16u);
@@ -84,6 +87,18 @@ uint32_t ace_rc_layout(int N, int G, int groups, int waves, unsigned char *lds, 
     s->mem = reinterpret_cast<double *>(take(ACE_MAX_STAGES * 8u));
     return o;
 }
+
+// ... by the arguments of a launch: the kernel and whoever sizes its LDS read the same two members, which have a value if nobody set them.
+#ifdef ACE_HOST_EMU
+inline
+#else
+__host__ __device__ __forceinline__
+#endif
+uint32_t ace_rc_layout(const RcArgs &a, unsigned char *lds, RcShared *s) {
+    return ace_rc_layout(a.k.g.N, a.k.g.G, a.groups, a.waves, lds, s);
+}
+// ... of one wavefront with room for a group per op: what arguments that say neither ask for.
+inline uint32_t ace_rc_layout(int N, int G, unsigned char *lds, RcShared *s) { return ace_rc_layout(N, G, 0, 1, lds, s); }
 
 // A wavefront's lanes: RC_EACH runs its body for every lane (`lane`, per-lane values `r`), then orders the wavefront's LDS
 // accesses; the reductions leave their result in every lane's `r`.
@@ -296,9 +311,9 @@ ACE_HD void rc_stage(const RcArgs &a, const RcShared &sh, const SpreadPlan &p, i
     const AceGeom &g = a.k.g;
     const int lo = sh.bound[s], hi = sh.bound[s + 1], len = hi - lo, nsb = n_stages - 1 - s;
     const uint32_t lut = sh.lut[(uint32_t)(p.glogs >> (4 * s)) & 15u];
-    double *act = sh.act + lo, *tmp = sh.tmp + lo, *sum = sh.sum + wave * a.groups;
+    double *act = sh.act + lo, *tmp = sh.tmp + lo, *sum = sh.sum + wave * sh.groups;
     uint8_t *codes = sh.codes + lo;
-    uint16_t *first = sh.first + wave * a.groups;
+    uint16_t *first = sh.first + wave * sh.groups;
     const uint16_t *type = sh.type + lo;
     double mem = sh.mem[s];
 #ifdef ACE_HOST_EMU
@@ -319,7 +334,7 @@ ACE_HD void rc_stage(const RcArgs &a, const RcShared &sh, const SpreadPlan &p, i
         return a.act[((ty * (uint32_t)g.n_mbs + m) * (uint32_t)g.n_tp + (tp < (uint32_t)g.n_tp ? tp : 0u)) * (uint32_t)g.n_algo + al] * (double)(nsb + 1);
     };
     RC_EACH(
-        for (int t = lane; t < a.groups; t += 64) sum[t] = 0.0;
+        for (int t = lane; t < sh.groups; t += 64) sum[t] = 0.0;
         for (int j = lane; j < len; j += 64) tmp[j] = raw(j, r.bad));
     RC_EACH(
         for (int j = lane; j < len; j += 64) {
@@ -336,10 +351,10 @@ ACE_HD void rc_stage(const RcArgs &a, const RcShared &sh, const SpreadPlan &p, i
 
     // ---- the greedy loop (:849-868): every round takes one group out of `sum` ----
     double saved = 0.0, peak = 0.0;
-    for (int left = a.groups; left >= 0; --left) {
+    for (int left = sh.groups; left >= 0; --left) {
         RC_EACH(
             r.a = 0.0; r.at = 0x7fffffff;
-            for (int t = lane; t < a.groups; t += 64) {
+            for (int t = lane; t < sh.groups; t += 64) {
                 const double v = sum[t];
                 const int at = first[t];
                 if (v > r.a || (v == r.a && v > 0.0 && at < r.at)) { r.a = v; r.at = at; }
@@ -429,7 +444,7 @@ ACE_HD void rc_fetch(const RcArgs &a, const RcShared &s, const SpreadPlan &p, lo
 template <bool COLL> ACE_HD void ace_rc_body(const RcArgs &a, unsigned char *lds_raw, int tid_, long long plan) {
     const AceGeom &g = a.k.g;
     RcShared s;
-    ace_rc_layout(g.N, g.G, a.groups, a.waves, lds_raw, &s);
+    ace_rc_layout(a, lds_raw, &s);
     SpreadShared sp;            // (the part spread_stages works on)
     sp.starts = s.starts; sp.count = s.count; sp.prefix = s.prefix; sp.bound = s.bound; sp.n_stages = s.n_stages;
 #ifdef ACE_HOST_EMU

@@ -296,6 +296,8 @@ extern "C" int ace_emu_spread(const ace_tables_t *t, const uint8_t *codes, const
 
 // LDS that check_recompute's workgroup may take: decides about its wavefronts
 extern "C" { uint32_t ace_emu_rc_lds = 160u * 1024u; }
+// ... and whether the arguments of the launch say how many groups and wavefronts there are (0: they are left as they come)
+extern "C" { int32_t ace_emu_rc_set = 1; }
 
 // ace_recompute_batch: codes and codes_out uint8 [G][P][16], flags int32 [4] zeroed by the caller.
 extern "C" int ace_emu_recompute(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, long long P, double memory_limit,
@@ -383,8 +385,11 @@ int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr,
             RcArgs r;
             r.k = a;
             ace_u2 *pos = (ace_u2 *)pool.place(nullptr, N * 8, 8);
-            r.groups = ace_rc_positions(rc->type_of_pos, rc->no_recompute, g.N, t->num_types, pos);
-            r.waves = ace_rc_waves(g.N, (int)G, r.groups, ace_emu_rc_lds);
+            const int groups = ace_rc_positions(rc->type_of_pos, rc->no_recompute, g.N, t->num_types, pos);
+            if (ace_emu_rc_set) {
+                r.groups = groups;
+                r.waves = ace_rc_waves(g.N, (int)G, groups, ace_emu_rc_lds);
+            }
             r.pos = pos;
             r.act = (const double *)pool.place(rc->activations, n_act * 8, 8);
             r.status = (const uint8_t *)pool.place(rc->status, (size_t)P, 1);
@@ -393,7 +398,7 @@ int emu_kernel(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr,
             r.limit = memory_limit;
             r.peak_backward = rc->peak_backward;
             RcShared sh;
-            const uint32_t bytes = ace_rc_layout(g.N, g.G, r.groups, r.waves, nullptr, &sh);
+            const uint32_t bytes = ace_emu_rc_set ? ace_rc_layout(r, nullptr, &sh) : ace_rc_layout(g.N, g.G, nullptr, &sh);
             unsigned char *rlds = (unsigned char *)pool.place(nullptr, bytes);
             for (long long p = 0; p < P; ++p) {
                 memset(rlds, 0xff, bytes);

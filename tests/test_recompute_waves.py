@@ -37,6 +37,21 @@ def test_one_and_two_wavefronts_on_the_cpu(name, lds):
         room.value = before
 
 
+@pytest.mark.parametrize("name", ["gpt3_1_3b", "wresnet_1b", "gpt_16ops"])
+def test_arguments_that_say_no_groups_and_no_wavefronts(name):
+    """A launch whose arguments leave both as they come, with LDS for as much as that needs: room for a group per op, one wavefront."""
+    cm, batch = models(name)
+    said = ctypes.c_int32.in_dll(emu_lib(), "ace_emu_rc_set")
+    said.value = 0
+    try:
+        for limit in limits(cm, batch):
+            cm.settings.memory_limit = limit
+            codes, flags = emu_recompute(cm, batch)
+            assert not flags.any() and np.array_equal(codes, update_recompute_arrays(cm, batch).codes)
+    finally:
+        said.value = 1
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("name", list(LONG))
 def test_long_stages_on_the_gpu(name):
