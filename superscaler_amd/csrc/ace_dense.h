@@ -19,9 +19,8 @@
 //
 // The dense tables, one block that is copied to LDS address 0 on:
 //   pairs   16 bytes {forward, backward} ms of resharding, every distinct pair once, {0, 0} first
-//   rows    per op type used: five arrays of doubles (one of the sizes kDenseArrays each): forward, backward, weights,
-//           activations, and the ranks of the two reserved sizes (16 bits each) among all that occur; indexed diag * C + code
-//           as the table compiler's rows are
+//   rows    per op type used, 40 bytes per entry: forward, backward, weights, activations, and the ranks of the two reserved sizes
+//           (16 bits each) among all that occur; entry diag * C + code as in the table compiler's rows, as many as there are
 //   slabs   per distinct (pair kind, next op's type): blocks of [code][next code] 16-bit addresses into `pairs`, one block per
 //           distinct (diag, stage size)
 //   lut     per (micro-batch size, stage size): LDS address of the diag's entries in the first row, of its block in the first slab
@@ -30,10 +29,15 @@
 // each: 115 of 760 us per 1,048,576 plans of 523 ops):
 //   reserved sizes by rank; per (op type, diag * C + code) and per (op type, output entry) a 16-bit LDS address of the distinct
 //   {input MB, intra-node ms, inter-node ms} and {output intra, inter}; types that agree in all of them share one list
-// With two algorithms and four tp sizes most codes in use are even, and diags four apart lie 256 bytes apart: from the fourth on
-// they lie 8 bytes further, so that their even codes read different banks.  Blocks of a slab are 132 bytes apart for the same reason.
+// An entry's stride of 40 bytes is ten banks of 64: like at a stride of eight bytes, the 8-byte reads of any 32 entries in a row meet no
+// bank twice.  The values' offsets within an entry are constants of the loops, whatever the tables.  (An array per value instead, of 40, 64,
+// 72 or 120 entries as a template's parameter: the same times within 1 % where a row filled its array -- 1,048,576 plans of 523 ops 547.4 and
+// 547.4 us, 65,536 of 821 93.5 and 93.1 --, and rows of 41 entries took the room of 64.)
+// With two algorithms and four tp sizes most codes in use are even, and diags four apart lie 32 entries apart: from the fourth on
+// they lie one entry further, so that their even codes read different banks.  Blocks of a slab are 132 bytes apart for the same reason.
 // Rows that do not all fit go through windows (as many ops as the rows of half the space behind the rest serve, a multiple of four),
-// consecutive windows in alternate halves, fetched by the loop itself; everything else stays resident.
+// consecutive windows in alternate halves, fetched by the loop itself; everything else stays resident.  (Sixteen rows of 80 entries, which a
+// half holds: two windows.  44 of twelve ops, with rows of 120 entries: 8,192 plans of 523 ops 90.2 -> 81.3 us, 262,144 194.8 -> 168.6.)
 // What a code byte reads that names no profiled entry (codes past the last tp size) is what it reads in the table compiler's
 // rows: the tables are filled by those addresses.
 #pragma once
@@ -51,7 +55,7 @@ constexpr int kDenseLanes = 512;
 // one of 1,024 with 20: 65,536 plans 44.9 / 41.1 us, 262,144 69.4 / 72.9, 300,000 104.6 / 99.9)
 constexpr uint32_t kDenseWinLds = 160u * 1024u;
 constexpr int kDenseWinLanes = 1024;
-constexpr uint32_t kDenseArrays[4] = {320u, 520u, 584u, 968u};   // bytes of an array of a row: up to 40, 64, 72, 120 entries (and the eight bytes further)
+constexpr uint32_t kDenseEntry = 40u, kDenseValue = 8u;          // bytes of an entry; from one of its values to the next
 
 struct AceDenseArgs {
     const ace_u4 *image;        // the tables
@@ -77,22 +81,22 @@ struct AceDenseTables {
     std::vector<int> window_start;
     uint32_t row_pitch = 0, rows_off = 0;
     AceDenseArgs args{};        // (offsets)
-    uint32_t array = 0, lds = 0;
+    uint32_t array = kDenseValue, lds = 0;
     bool ok = false;
 };
 
 // LDS behind the image: the deal's bins and permutation, and the arrival counters; windowed, the rows lie there afterwards.
 inline uint32_t ace_dense_scratch(int lanes) { return 128u + 2u * (uint32_t)lanes + 128u; }
 
-// Fills `d` (d.ok false: the tables do not fit this form).  `lds`: how much of it a workgroup of `lanes` lanes may take.
-inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed, uint32_t lds, int lanes, AceDenseTables &d) {
+// Fills `d` (d.ok false: the tables do not fit this form).  `lds`: how much of it a workgroup may take, `scratch`: what of that is for
+// the kernel's own use (windowed: before the first rows arrive); `lanes`: of a workgroup that fetches windows.
+inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed, uint32_t lds, uint32_t scratch, int lanes, AceDenseTables &d) {
     d = AceDenseTables();
     const int N = t->num_ops, C = t->n_tp * t->n_algo, ND = t->n_diag;
     if ((t->flags & ACE_F_COLLECTIVE_MEM) || N >= 32768) return;
     const bool rsh = (t->flags & ACE_F_RESHARDING) != 0;
-    const uint32_t entries = (uint32_t)(ND * C + 8), array = entries <= 40u ? kDenseArrays[0] : entries <= 64u ? kDenseArrays[1] : entries <= 72u ? kDenseArrays[2] : kDenseArrays[3];
-    if (entries > 120u) return;
-    auto diag_entry = [&](uint32_t dg) { return dg * (uint32_t)C + (C == 8 && t->n_algo == 2 && array != kDenseArrays[0] && dg >= 4u ? 1u : 0u); };
+    const uint32_t entries = (uint32_t)(ND * C + 8), further = C == 8 && t->n_algo == 2 && ND > 4 ? 1u : 0u, row_bytes = (entries + further) * kDenseEntry;
+    auto diag_entry = [&](uint32_t dg) { return dg * (uint32_t)C + (dg >= 4u ? further : 0u); };
     const size_t n_rows_all = (size_t)t->num_types * (size_t)t->row_doubles;
     auto at = [&](size_t type, size_t off) {                       // a double of a row, or of what follows it in memory
         const size_t i = type * (size_t)t->row_doubles + off;
@@ -215,37 +219,39 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
         out_of.push_back(list_of(out_lists, out));
     }
     if (in_lists.size() > 256u || out_lists.size() > 256u) return;   // (eight bits each in a record word)
-    // the constant byte K and how far apart rows and slabs lie: multiples of it, at most 255 for the last one; rows: as many as
-    // `slots` (windowed: in each half)
-    const uint32_t n_slabs = (uint32_t)slabs.size(), slab_bytes = (uint32_t)n_blocks * kBlock;
+    // How far apart rows and slabs lie, and the constant bytes whose multiples (at most 255 of each) name their places; rows: as many as
+    // `slots` (windowed: in each half, and fetched in pieces of 16 bytes, 1 KB at a time).  With resharding one constant K for both;
+    // else two of the rows alone: 248 and 8, which name any place below 63 KB, or for more rows than those reach K twice.
+    const uint32_t n_slabs = (uint32_t)slabs.size(), slab_bytes = (uint32_t)n_blocks * kBlock, row_least = windowed ? std::max(row_bytes, 1024u) : row_bytes;
     const size_t lists = (in_lists.size() * g.in_entries + out_lists.size() * g.out_entries) * 2u;
-    uint32_t K = 0, row_pitch = 0, slab_pitch = 0, slots = windowed ? 31u : (uint32_t)used.size();
+    uint32_t K = 0, K2 = 0, row_pitch = 0, slab_pitch = 0, slots = windowed ? 31u : (uint32_t)used.size();
     auto fits = [&](uint32_t n) {                                   // n rows: K and the pitches, the smallest in all
         K = 0;
         uint64_t best = ~0ull;
-        if (!rsh) {                                                 // (two constant bytes: 248 and 8)
-            row_pitch = (array * 5u + 15u) & ~15u;
-            if ((n - 1u) * row_pitch > 248u * 255u + 247u) return false;
+        const uint32_t whole = (row_least + 15u) & ~15u;
+        if (!rsh && (n - 1u) * whole <= 248u * 255u + 247u) {
+            row_pitch = whole;
             K = 248u;
+            K2 = 8u;
             best = (uint64_t)n * row_pitch * (windowed ? 2u : 1u);
         } else
             for (uint32_t k = 8; k <= 248u; k += 8u) {
-                uint32_t u = (array * 5u + k - 1u) / k;
+                uint32_t u = (row_least + k - 1u) / k;
                 const uint32_t v = (slab_bytes + k - 1u) / k;
-                u += windowed && ((u * k) & 15u) ? 1u : 0u;            // (fetched in pieces of 16 bytes)
-                if ((n - 1u) * u > 255u || (n_slabs - 1u) * v > 255u) continue;
+                u += windowed && ((u * k) & 15u) ? 1u : 0u;
+                if ((n - 1u) * u > (rsh ? 255u : 510u) || (rsh && (n_slabs - 1u) * v > 255u)) continue;
                 const uint64_t size = (uint64_t)n * u * k * (windowed ? 2u : 1u) + (uint64_t)n_slabs * v * k;
-                if (size < best) { best = size; K = k; row_pitch = u * k; slab_pitch = v * k; }
+                if (size < best) { best = size; K = K2 = k; row_pitch = u * k; slab_pitch = v * k; }
             }
         const uint64_t rest = pairs.size() * 16u + values_out.size() * 16u + values_in.size() * 24u + (size_t)t->n_mbs * (windowed ? 320u : 192u) +
                               (reserved_fwd.size() + reserved_bwd.size()) * 8u + lists + 256u;
-        return K != 0u && best + rest + (windowed ? 0u : ace_dense_scratch(lanes)) <= lds;
+        return K != 0u && best + rest + (windowed ? 0u : scratch) <= lds;
     };
     if (windowed)
         while (slots >= 4u && (!fits(slots) || slots * ((row_pitch + 1023u) / 1024u) > 4u * (uint32_t)lanes / 64u)) --slots;   // (four loads per event and wavefront)
     if (slots < 4u && windowed) return;
     if (!fits(slots)) return;
-    g.kv = rsh ? K << 24 : (248u << 24) | (8u << 16);
+    g.kv = (K << 24) | (rsh ? 0u : K2 << 16);
     // the image (what 16-bit addresses name lies in front)
     uint32_t end = 0;
     auto take = [&](size_t bytes, uint32_t align) {
@@ -266,19 +272,21 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     g.out_off = take(out_lists.size() * g.out_entries * 2u, 2u);
     const uint32_t n_rows = (uint32_t)used.size(), rows_off = take(windowed ? 0u : (size_t)n_rows * row_pitch, 16u), bytes = take(0, 16u);
     g.half = slots * row_pitch;
-    d.lds = bytes + (windowed ? std::max(2u * g.half, ace_dense_scratch(lanes)) : ace_dense_scratch(lanes));
+    d.lds = bytes + (windowed ? std::max(2u * g.half, scratch) : scratch);
     if (d.lds > lds) return;
     d.row_pitch = row_pitch;
     d.rows_off = rows_off;
     g.image16 = bytes / 16u;
-    // windows: a multiple of four ops each (or up to the last op), of at most `slots` different rows
+    // windows: a multiple of four ops each (or up to the last op), of at most `slots` different rows; two of them where one half
+    // holds every row
     std::vector<uint32_t> place(N, 0u);                             // of each position's row, from the first one (of its half) on
     if (windowed) {
+        const int longest = used.size() <= slots ? (N / 2 + 3) & ~3 : N;
         for (int i = 0; i < N;) {
             std::vector<uint32_t> seen;
             size_t good_n = 0;
             int good = -1;
-            for (int j = i; j < N;) {
+            for (int j = i; j < N && j < i + longest;) {
                 const uint32_t r = (uint32_t)row_of[types[j]];
                 if (std::find(seen.begin(), seen.end(), r) == seen.end()) {
                     if (seen.size() >= slots) break;
@@ -324,18 +332,18 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
             for (uint32_t c = 0; c < 8u; ++c) {
                 // (a code past the last one reads what follows its diag's entries)
                 const uint32_t e = dg * (uint32_t)C + c;
-                unsigned char *to = rows + r * row_pitch + (diag_entry(dg) + c) * 8u;
+                unsigned char *to = rows + r * row_pitch + (diag_entry(dg) + c) * kDenseEntry;
                 if (c >= (uint32_t)C && dg < (uint32_t)ND) continue;
                 double v[6];
                 for (uint32_t k = 0; k < 6u; ++k) v[k] = at(used[r], (size_t)t->hot_off + e * 6u + k);
-                for (uint32_t k = 0; k < 4u; ++k) memcpy(to + k * array, &v[k], 8);
+                for (uint32_t k = 0; k < 4u; ++k) memcpy(to + k * kDenseValue, &v[k], 8);
                 const uint32_t both = rank(0, v[4]) | (rank(1, v[5]) << 16);
-                memcpy(to + 4u * array, &both, 4);
+                memcpy(to + 4u * kDenseValue, &both, 4);
             }
     for (uint32_t s = 0; s < n_slabs; ++s)
         for (uint32_t b = 0; b < (uint32_t)n_blocks; ++b) put(slabs_off + s * slab_pitch + b * kBlock, slabs[s].data() + b * 64u, 128);
     for (uint32_t j = 0; j < (uint32_t)t->n_mbs * 16u; ++j) {
-        const ace_u2 z{rows_off + diag_entry(t->stage_lut[j] & 15u) * 8u, slabs_off + block_of[j] * kBlock};
+        const ace_u2 z{rows_off + diag_entry(t->stage_lut[j] & 15u) * kDenseEntry, slabs_off + block_of[j] * kBlock};
         put(g.lut_off + j * 8u, &z, 8);
         const ace_u2 other{z.x + g.half, z.y};
         if (windowed) put(g.lut_off + g.lut_half + j * 8u, &other, 8);
@@ -349,7 +357,8 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
         const uint32_t info = in ? t->pos_info[i] : 0u, at_row = in ? place[i] : 0u, slab = in ? slab_of[i] : 0u;
         const uint32_t last = in ? out_of[row_of[types[i]]] : 0u, next = in && i + 1 < (size_t)N ? in_of[row_of[types[i + 1]]] : 0u;
         ace_u4 &p = d.pos[i];
-        p.x = (odd ? 8u << 8 : 8u) | (rsh ? (at_row / K) << 24 : ((at_row / 248u) << 24) | (((at_row % 248u) / 8u) << 16));
+        const uint32_t units = std::min(at_row / K, 255u);
+        p.x = (odd ? kDenseEntry << 8 : kDenseEntry) | (units << 24) | (rsh ? 0u : ((at_row - units * K) / K2) << 16);
         p.y = rsh ? (odd ? (16u << 8) | (2u << 16) : 16u | (2u << 8)) | ((slab * (slab_pitch / K)) << 24) : 0u;
         // record word: codes of the stage's last op and of the next one in bytes 0 and 1 (odd positions with resharding: 1
         // and 2, bit 11 set), the last op's list of outputs and the next one's of inputs in the other two
@@ -358,15 +367,14 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
         d.pos_duo[i] = ace_u2{p.x, p.y};
         d.pos_duo[pos_entries + i] = ace_u2{p.x, p.z | (p.w << 12)};
     }
-    d.array = array;
     g.first_in = in_of[row_of[types[0]]];
     d.ok = true;
 }
 
 // Every row resident if they fit beside a second workgroup on the CU, else in windows.
 inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseTables &d) {
-    if (t->n_windows == 1) dense_build(t, pos_entries, false, kDenseLds, kDenseLanes, d);
-    if (!d.ok) dense_build(t, pos_entries, true, kDenseWinLds, kDenseWinLanes, d);
+    dense_build(t, pos_entries, false, kDenseLds, ace_dense_scratch(kDenseLanes), kDenseLanes, d);
+    if (!d.ok) dense_build(t, pos_entries, true, kDenseWinLds, ace_dense_scratch(kDenseWinLanes), kDenseWinLanes, d);
 }
 
 // Windowed rows: the fetch records, per event and wavefront 48 bytes = {first position of the window after the one being entered,
@@ -523,8 +531,8 @@ ACE_HD void dense_replay(const AceDenseArgs &d, const AceGeom &g, const AceLds &
 #include "ace_dense_loop_asm.inc"
 
 // The op loop: returns the number of stages of the lane's plan, and in `stored` that of the wavefront's records; `ws`: the
-// wavefront's part of the workspace.  Arrays of the rows lie A bytes apart.
-template <int A, bool WIN>
+// wavefront's part of the workspace.
+template <bool WIN>
 __device__ __forceinline__ uint32_t dense_loop(const AceKernelArgs &a, const AceDenseArgs &d, uint64_t glogs, uint32_t lut2, uint64_t zvrk, uint32_t code_off,
                                                const unsigned char *ws, uint32_t lane, uint32_t meta0, uint32_t pace, uint32_t prio, uint32_t wave, uint32_t &stored) {
     uint32_t placed;
@@ -534,8 +542,7 @@ __device__ __forceinline__ uint32_t dense_loop(const AceKernelArgs &a, const Ace
     asm volatile(TEXT : [placed] "=&v"(placed), [stored] "=&v"(stored)                                                           \
                  : [glogs] "v"(glogs), [lut2] "v"(lut2), [zvrk] "v"(zvrk), [codeoff] "v"(code_off), [place] "v"(lane * 2u),      \
                    [meta0] "v"(meta0), [codes] "s"(a.codes), [pos] "s"(d.pos), [n_ops] "s"(a.g.N), [recbase] "s"(ws),            \
-                   [gstride_lo] "s"(gs_lo), [gstride_hi] "s"(gs_hi), [kv] "s"(d.kv), [a1] "n"(A), [a2] "n"(2 * A),               \
-                   [a3] "n"(3 * A), [a4] "n"(4 * A), __VA_ARGS__                                                                  \
+                   [gstride_lo] "s"(gs_lo), [gstride_hi] "s"(gs_hi), [kv] "s"(d.kv), __VA_ARGS__ \
                  : ACE_DENSE_ASM_CLOBBERS)
 #define ACE_DENSE_RESIDENT [pace] "s"(pace), [pacemask] "s"(1u)
 #define ACE_DENSE_WINDOWED [prio] "s"(prio), [dma] "s"(d.events), [eventsize] "s"((uint32_t)(kDenseWinLanes / 64) * 48u), \
@@ -581,7 +588,7 @@ template <int LANES> __device__ __forceinline__ void dense_stage_image(const Ace
 }
 
 // One workgroup; its LDS array starts at address 0 (the kernel has no other LDS variables).
-template <int A, bool WIN> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
+template <bool WIN> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
                                                                 int tid, long long block) {
     constexpr int kLanes = WIN ? kDenseWinLanes : kDenseLanes;
     const AceGeom &g0 = a.g;
@@ -636,7 +643,7 @@ template <int A, bool WIN> __device__ __forceinline__ void ace_dense_body(const 
     uint32_t stored;
     // (windowed rows: the deeper its plans, the higher a wavefront's issue priority)
     const uint32_t prio = (uint32_t)__builtin_amdgcn_readfirstlane((int)(3u - q * 4u / (uint32_t)(kLanes / 64)));
-    const int n_st = (int)dense_loop<A, WIN>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.first_in << 24),
+    const int n_st = (int)dense_loop<WIN>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.first_in << 24),
                                              d.image16 * 16u + 128u + 2u * kLanes + (wave & 3u) * 32u, prio, wave, stored);
     dense_replay(d, g, lds, st, ws, lane, (uint32_t)__builtin_amdgcn_readfirstlane((int)stored), n_st);
     st.s = n_st;                                                    // (result() checks the count of the op loop)

@@ -48,14 +48,12 @@ inline uint32_t ace_duo_scratch(int L) { return 128u + 2u * (uint32_t)L + 2u * (
                  : [glogs] "v"(glogs), [lut2] "v"(lut2), [zvrk] "v"(zvrk), [codeoff] "v"(code_off), [recoff] "v"(rec_off),        \
                    [codes] "s"(codes), [pos] "s"(pos), [n_ops] "s"(a.g.N), [recbase] "s"(rec_base),                          \
                    [gstride_lo] "s"((uint32_t)gstride), [gstride_hi] "s"((uint32_t)(gstride >> 32)), [wsstride] "s"(ws_stride),   \
-                   [wspiece] "s"(ws_piece), [grp] "s"(grp), [cut] "s"(cut), [recnext] "v"(rec_next), [kv] "s"(d.kv),          \
-                   [a1] "n"(A), [a2] "n"(2 * A), [a3] "n"(3 * A), [a4] "n"(4 * A)                                             \
+                   [wspiece] "s"(ws_piece), [grp] "s"(grp), [cut] "s"(cut), [recnext] "v"(rec_next), [kv] "s"(d.kv)           \
                  : ACE_DUO_ASM_CLOBBERS)
 // Walks one part of the lane's plan, from 16-op group `grp` on; the stages that start in front of position `cut` are parked, the
 // first one at `rec_off`, the next at `rec_next` (kNoRecord: nowhere).  `role` is the same for the whole wavefront, and all 64
-// lanes are active.  Arrays of the rows lie A bytes apart.
+// lanes are active.
 constexpr uint32_t kNoRecord = 0x80000000u;
-template <int A>
 __device__ __forceinline__ void duo_loop(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t role, uint32_t grp, uint32_t cut, uint64_t glogs, uint32_t lut2,
                                          uint64_t zvrk, uint32_t code_off, const double *rec_base, uint32_t rec_off, uint32_t rec_next,
                                          uint32_t ws_stride, uint32_t ws_piece) {
@@ -119,7 +117,7 @@ template <> struct DuoDeal<128> { static constexpr uint32_t v[3] = {0x10101010u,
 template <> struct DuoDeal<256> { static constexpr uint32_t v[3] = {0x32103210u, 0x11110000u, 0x2222u}; };
 
 // One workgroup: L plans.  The LDS array starts at address 0 (the kernel has no other LDS variables).
-template <int A, int L>
+template <int L>
 __device__ __forceinline__ void ace_duo_body(const AceKernelArgs &a, const AceDenseArgs &d, unsigned char *lds_raw, int tid, long long block) {
     typedef DuoDeal<L> Deal;
     AceGeom g = a.g;
@@ -208,7 +206,7 @@ __device__ __forceinline__ void ace_duo_body(const AceKernelArgs &a, const AceDe
     if (grp < grp_end && __any(any)) {
         const uint32_t shift = here > 1u ? 4u * (here - 1u) : 0u, lut = d.lut_off + st.bidx * 128u, to = at * 16u + role * 2u * kPiece;
         const uint64_t glogs = shift < 64u ? st.glogs >> shift : 0ull;
-        duo_loop<A>(a, d, role, grp, part + 1u < parts ? 16u * grp_end : 0x7fffffffu, glogs >> 1, lut, lds.ld<uint64_t>(lut + ((uint32_t)glogs & 15u) * 8u),
+        duo_loop(a, d, role, grp, part + 1u < parts ? 16u * grp_end : 0x7fffffffu, glogs >> 1, lut, lds.ld<uint64_t>(lut + ((uint32_t)glogs & 15u) * 8u),
                     (uint32_t)pl * 16u, rec_base, opens ? to + before * kStride : kNoRecord, any ? to + here * kStride : kNoRecord, kStride, kPiece);
     }
     __builtin_amdgcn_s_setprio(0);

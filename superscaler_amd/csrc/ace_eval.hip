@@ -99,9 +99,9 @@ __global__ __launch_bounds__(kSpreadLanes) void ace_spread_kernel(const AceKerne
     ace_spread_body<BD, RANGED, COLL>(a, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // Mid-sized batches: several lanes per plan, see ace_duo.h.
-template <int A, int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(const AceKernelArgs a, const AceDenseArgs d) {
+template <int L> __global__ __launch_bounds__(kDuoBlock) void ace_duo_kernel(const AceKernelArgs a, const AceDenseArgs d) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_duo_body<A, L>(a, d, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_duo_body<L>(a, d, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // Large batches on the assembly loop, see ace_many.h.
 template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(const AceKernelArgs a, const uint32_t slices) {
@@ -109,10 +109,10 @@ template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(cons
     ace_many_body<WIN>(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // ... over dense tables, see ace_dense.h.
-template <int A, bool WIN> __global__ __launch_bounds__(WIN ? kDenseWinLanes : kDenseLanes, 4)
+template <bool WIN> __global__ __launch_bounds__(WIN ? kDenseWinLanes : kDenseLanes, 4)
 void ace_dense_kernel(const AceKernelArgs a, const AceDenseArgs d, const uint32_t slices) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_dense_body<A, WIN>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_dense_body<WIN>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 template <bool COLL> __global__ __launch_bounds__(kRcLanes, 6) void ace_rc_kernel(const RcArgs a, const long long first) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -758,7 +758,7 @@ struct ace_handle {
     AceGeom geom_wa;           // ... and the LDS layout of the kernel that runs it
     uint32_t lds_bytes_wa;
     AceDenseArgs dense;        // tables of ace_dense.h (device addresses; image null: they do not fit that form)
-    uint32_t dense_array, dense_lds;
+    uint32_t dense_lds;
     unsigned char *d_dense_rows;   // ... windowed: the rows
     uint8_t *d_pair_kinds;
     uint32_t *d_stage_lut;
@@ -875,10 +875,10 @@ template <bool BD, bool RANGED, bool WIN, bool DEFER> static int allow_big_lds()
     return ACE_OK;
 }
 
-template <int A> static int allow_duo_lds() {
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<A, 64>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<A, 128>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<A, 256>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+static int allow_duo_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<64>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<128>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_duo_kernel<256>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kMaxLds));
     return ACE_OK;
 }
 
@@ -887,9 +887,9 @@ template <bool WIN> static int allow_many_lds() {
     return ACE_OK;
 }
 
-template <int A> static int allow_dense_lds() {
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<A, false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<A, true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseWinLds));
+static int allow_dense_lds() {
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseWinLds));
     return ACE_OK;
 }
 
@@ -1070,7 +1070,6 @@ static int setup_dense(ace_handle *h, const ace_tables_t *t, size_t pos_entries)
     }
     if (rc != ACE_OK) return rc;
     h->dense_lds = d.lds;
-    h->dense_array = d.array;
     return ACE_OK;
 }
 
@@ -1216,10 +1215,7 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         (rc = allow_big_lds<false, false, false, false>()) || (rc = allow_big_lds<false, false, true, false>()) ||
         (rc = allow_big_lds<false, false, false, true>()) || (rc = allow_big_lds<false, false, true, true>()) ||
         (rc = allow_big_lds<true, false, false, false>()) || (rc = allow_big_lds<true, false, true, false>()) ||
-        (rc = allow_duo_lds<kDenseArrays[0]>()) || (rc = allow_duo_lds<kDenseArrays[1]>()) || (rc = allow_duo_lds<kDenseArrays[2]>()) ||
-        (rc = allow_duo_lds<kDenseArrays[3]>()) ||
-        (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) || (rc = allow_dense_lds<kDenseArrays[0]>()) || (rc = allow_dense_lds<kDenseArrays[1]>()) ||
-        (rc = allow_dense_lds<kDenseArrays[2]>()) || (rc = allow_dense_lds<kDenseArrays[3]>()) ||
+        (rc = allow_duo_lds()) || (rc = allow_many_lds<false>()) || (rc = allow_many_lds<true>()) || (rc = allow_dense_lds()) ||
         (rc = allow_big_lds<true, true, false, false>()) || (rc = allow_big_lds<true, true, true, false>())) {
         ace_destroy(h);
         return rc;
@@ -1335,11 +1331,6 @@ static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream
     else hipLaunchKernelGGL(ace_many_kernel<false>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
     return true;
 }
-template <int A>
-static void launch_dense_a(const ace_handle_t *h, const AceKernelArgs &a, size_t groups, uint32_t slices, hipStream_t s) {
-    if (h->dense.events) hipLaunchKernelGGL((ace_dense_kernel<A, true>), dim3((unsigned)groups), dim3(kDenseWinLanes), h->dense_lds, s, a, h->dense, slices);
-    else hipLaunchKernelGGL((ace_dense_kernel<A, false>), dim3((unsigned)groups), dim3(kDenseLanes), h->dense_lds, s, a, h->dense, slices);
-}
 // ... over dense tables (ace_dense.h and the table above kSpreadMaxPlain have both sides measured).
 static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     if (!h->dense.image || a.range || a.stage_out || !a.stage_ws) return false;
@@ -1347,27 +1338,17 @@ static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStrea
     const uint32_t slices = win ? ace_dense_slices(a.g.P, kDenseWinLanes / 64, 256) : ace_dense_slices(a.g.P, kDenseLanes / 64, 512), lanes = 64u * slices;
     const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
     if (a.stage_ws != h->d_stage_ws || groups * lanes > h->stage_ws_plans) return false;    // (the static scratch holds no such records)
-    if (h->dense_array == kDenseArrays[0]) launch_dense_a<kDenseArrays[0]>(h, a, groups, slices, s);
-    else if (h->dense_array == kDenseArrays[1]) launch_dense_a<kDenseArrays[1]>(h, a, groups, slices, s);
-    else if (h->dense_array == kDenseArrays[2]) launch_dense_a<kDenseArrays[2]>(h, a, groups, slices, s);
-    else launch_dense_a<kDenseArrays[3]>(h, a, groups, slices, s);
+    if (win) hipLaunchKernelGGL(ace_dense_kernel<true>, dim3((unsigned)groups), dim3(kDenseWinLanes), h->dense_lds, s, a, h->dense, slices);
+    else hipLaunchKernelGGL(ace_dense_kernel<false>, dim3((unsigned)groups), dim3(kDenseLanes), h->dense_lds, s, a, h->dense, slices);
     return true;
 }
-template <int A>
-static void launch_duo_a(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     const dim3 groups((unsigned)((a.g.P + L - 1) / L));
     const uint32_t lds = h->dense.image16 * 16u + ace_duo_scratch(L);
-    if (L == 64) hipLaunchKernelGGL((ace_duo_kernel<A, 64>), groups, dim3(kDuoBlock), lds, s, a, h->dense);
-    else if (L == 128) hipLaunchKernelGGL((ace_duo_kernel<A, 128>), groups, dim3(kDuoBlock), lds, s, a, h->dense);
-    else hipLaunchKernelGGL((ace_duo_kernel<A, 256>), groups, dim3(kDuoBlock), lds, s, a, h->dense);
+    if (L == 64) hipLaunchKernelGGL(ace_duo_kernel<64>, groups, dim3(kDuoBlock), lds, s, a, h->dense);
+    else if (L == 128) hipLaunchKernelGGL(ace_duo_kernel<128>, groups, dim3(kDuoBlock), lds, s, a, h->dense);
+    else hipLaunchKernelGGL(ace_duo_kernel<256>, groups, dim3(kDuoBlock), lds, s, a, h->dense);
 }
-static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    if (h->dense_array == kDenseArrays[0]) launch_duo_a<kDenseArrays[0]>(L, h, a, s);
-    else if (h->dense_array == kDenseArrays[1]) launch_duo_a<kDenseArrays[1]>(L, h, a, s);
-    else if (h->dense_array == kDenseArrays[2]) launch_duo_a<kDenseArrays[2]>(L, h, a, s);
-    else launch_duo_a<kDenseArrays[3]>(L, h, a, s);
-}
-
 static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     const int mid = duo_lanes(h, a);
     const int most = a.stage_out ? kSpreadMaxRecords : mid ? kSpreadMaxPlain : !a.stage_ws ? kSpreadMaxSlow : h->d_win_dma || h->dense.image ? kSpreadMaxWindowed : kSpreadMaxOther;

@@ -11,7 +11,8 @@ an op costs beside the reference's own additions:
   * costs: the pair table names the 16 bytes {forward, backward} by their LDS address; equal pairs are stored once.
   * reserved memory: the largest of a finite set of values is the one of the largest rank; forward and backward ranks are
     16 bits each, one v_pk_max_u16 for both.
-  * tables: one array of doubles per value (8-byte stride: neighbouring codes and stage sizes in different banks).
+  * tables: 40 bytes per entry, a ds_read_b64 per value (neighbouring codes and stage sizes in different banks; the values' offsets
+    are the same for all tables).
   * records: a stage that ends is parked in registers, and the parked records of all lanes are stored when one of them is
     about to park its second, some ten at a time, one behind the other in the wavefront's own part of the workspace; a
     record says whose it is.  (Stored at [stage][lane], the records were what the loop waited for: 1,048,576 plans of 16
@@ -174,7 +175,7 @@ class Dense:
     def reads(self, k1):
         x1 = k1 & 1
         for i, e in enumerate(E(x1)):
-            self.o(f"ds_read_b64 {e}, {T1}" + (f" offset:%[a{i}]" if i else ""))
+            self.o(f"ds_read_b64 {e}, {T1}" + (f" offset:{8 * i}" if i else ""))
         if self.rsh:
             self.o(f"ds_read_u16 {R(1 - x1)}, {T2}")           # where the cost of the (k1, k1 + 1) pair is
 

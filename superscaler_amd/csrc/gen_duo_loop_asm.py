@@ -124,7 +124,7 @@ class Duo:
     def reads(self, k1):
         x1 = k1 & 1
         for e, i in zip(self.E(x1), (0, 1) if self.time else (2, 3, 4)):
-            self.o(f"ds_read_b64 {e}, {T1}" + (f" offset:%[a{i}]" if i else ""))
+            self.o(f"ds_read_b64 {e}, {T1}" + (f" offset:{8 * i}" if i else ""))
         if self.rsh:
             self.o(f"ds_read_u16 {R(1 - x1)}, {T2}")
             self.o(f"ds_read_b128 {self.Z(x1)[0]}, {R(x1)}")

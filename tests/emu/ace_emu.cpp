@@ -216,6 +216,17 @@ extern "C" int ace_emu_dense(const ace_tables_t *t, const uint8_t *codes /* [P][
     return 0;
 }
 
+// What the tables of that form are like: fits, windows, bytes of LDS per workgroup, of the image, of a row (with what follows it to the
+// next one), most rows of a window.
+extern "C" void ace_emu_dense_shape(const ace_tables_t *t, int32_t *out /* [6] */) {
+    AceDenseTables d;
+    ace_dense_build(t, (size_t)((t->num_ops + 15) / 16) * 16 + 16, d);
+    size_t most = 0;
+    for (const auto &w : d.windows) most = std::max(most, w.size());
+    const int32_t v[6] = {d.ok, (int32_t)d.windows.size(), (int32_t)d.lds, (int32_t)d.image.size(), (int32_t)d.row_pitch, (int32_t)most};
+    memcpy(out, v, sizeof(v));
+}
+
 // ------------------------------------------------------------------------------------------
 // The kernel's own op loop (ace_score_loop.h) on the CPU, one lane per "workgroup", with every
 // array the kernel reads or writes placed flush against an inaccessible page: an index past an

@@ -1,0 +1,82 @@
+"""Scoring over tables of other shapes than the configured workloads': more or fewer micro-batch sizes, devices per node and op types, so
+that rows are of other lengths, fit where the configured ones do not, or go through windows.
+
+On the CPU: the tables as the library builds them, their sizes, and every plan against the C oracle.  On the GPU: the same at batch sizes
+on both sides of what decides about the kernel."""
+import ctypes
+import dataclasses
+
+import numpy as np
+import pytest
+
+from superscaler_amd import synth
+from superscaler_amd.plan import PlanBatch
+from tests.helpers import c_oracle_scores, emu_dense_score, emu_lib
+from tests.test_small_batches import tables_for, with_recompute
+
+
+def workload(name, sizes, per_node=None, gpus=None):
+    w = synth.WORKLOADS[name]
+    gpus = gpus or w.num_gpus
+    return dataclasses.replace(w, mbs_list=[1 << i for i in range(sizes)], gpus_per_node=per_node or w.gpus_per_node, num_gpus=gpus,
+                               pp_choices=[s for s in w.pp_choices if s <= gpus])
+
+
+#: (workload, micro-batch sizes, devices per node, devices): entries per row between 10 and 96
+SHAPES = {"t5, 6 sizes": ("t5_770m", 6), "t5, 8 sizes": ("t5_770m", 8), "t5, 2 of 2": ("t5_770m", 2, 2, 8), "gpt, 6 sizes": ("gpt3_13b", 6),
+          "gpt, 8 sizes": ("gpt3_1_3b", 8, 8, 32), "gpt, 7 of 4": ("gpt3_13b", 7, 4), "gpt, 8 of 2": ("gpt3_1_3b", 8, 2), "gpt, 3 of 8": ("gpt3_175b", 3, 8, 64),
+          "conv, 1 of 1": ("wresnet_1b", 1, 1, 4), "conv, 3 of 1": ("wresnet_1b", 3, 1, 4), "conv, 5 of 1": ("wresnet_1b", 5, 1, 4),
+          "conv, 1 of 2": ("wresnet_1b", 1, 2, 4), "conv, 6 sizes": ("wresnet_1b", 6)}
+
+
+def shape_of(tables):
+    """(fits, windows, LDS of a workgroup, bytes of the image, from row to row, most rows of a window)"""
+    out = np.zeros(6, dtype=np.int32)
+    ts = tables.as_struct()
+    emu_lib().ace_emu_dense_shape(ctypes.byref(ts), out.ctypes.data_as(ctypes.c_void_p))
+    return [int(x) for x in out]
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_rows_take_what_their_entries_need(shape):
+    tables = tables_for(workload(*SHAPES[shape]))
+    ok, windows, lds, _, pitch, _ = shape_of(tables)
+    entries = tables.n_diag * tables.C + 8
+    # (one entry to keep banks apart; up to 255 multiples of one constant name the places of rows: of `n` rows one is a 255th of all,
+    # rounded up to eight bytes, longer at most; a window's rows are fetched 1 KB at a time, in pieces of 16 bytes)
+    need = 40 * (entries + 1)
+    assert ok and pitch <= max(need + 8 * (need // 255 + 2), 1024 if windows else 0)
+    assert lds <= (160 if windows else 80) * 1024
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+def test_every_shape_scores_like_the_oracle(shape):
+    w = workload(*SHAPES[shape])
+    tables = tables_for(w)
+    batch = with_recompute(synth.make_plans(w, tables, n_plans=120, seed_offset=21), 0.6, 21)
+    got = emu_dense_score(tables, batch)
+    it, pk, fe, er = c_oracle_scores(tables, batch)
+    assert np.array_equal(got[0], it) and np.array_equal(got[1], pk) and np.array_equal(got[2], fe) and not got[3].any() and not er.any()
+
+
+def on_the_gpu(shape, sizes):
+    from superscaler_amd.evaluator import PlanEvaluator
+    w = workload(*SHAPES[shape])
+    tables = tables_for(w)
+    ev = PlanEvaluator(tables)
+    base = with_recompute(synth.make_plans(w, tables, n_plans=9000, seed_offset=31), 0.6, 31)
+    want = c_oracle_scores(tables, base, threads=8)
+    rng = np.random.default_rng(4)
+    for n in sizes:
+        print(f"[case] {shape} plans={n}", flush=True)
+        pick = rng.integers(0, base.n_plans, n)
+        it, pk, fe, st = ev.score_host(PlanBatch(base.codes[pick], base.hdr[pick]))
+        assert (st == 0).all() and np.array_equal(it, want[0][pick]) and np.array_equal(pk, want[1][pick]) and np.array_equal(fe, want[2][pick])
+    ev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,sizes", [("t5, 6 sizes", (70001,)), ("gpt, 6 sizes", (65537, 262145)), ("gpt, 8 sizes", (70000,)), ("t5, 2 of 2", (65537,)),
+                                         ("conv, 1 of 1", (5000, 70001)), ("conv, 1 of 2", (6200, 70001)), ("conv, 6 sizes", (65536,))])
+def test_large_batches_over_other_shapes_on_the_gpu(shape, sizes):
+    on_the_gpu(shape, sizes)
