@@ -1,9 +1,9 @@
 // Scoring of LARGE batches over dense tables: a plan per lane, like ace_many.h, but what an op costs a lane beside the
 // reference's own additions is as little as could be found: two v_dot4_u32_u8 for all addresses, one 8-byte LDS read per value,
-// one 16-byte read for both collectives' costs, and records that are stored in whole cache lines (gen_dense_loop_asm.py).  The
-// tables take less than half of a CU's LDS in the form below, so two workgroups of eight wavefronts share a CU, and one evaluates
-// its stage tails or stages its tables while the other walks.
-// Rows resident (they fit 80 KB with the rest): from 65,537 plans on.  Rows in windows: from what the kernel of small batches leaves.
+// one 16-byte read for both collectives' costs, and records that are stored in whole cache lines (gen_dense_loop_asm.py).  Where the
+// tables take less than half of a CU's LDS in the form below, two workgroups of eight wavefronts share a CU, and one evaluates
+// its stage tails or stages its tables while the other walks; else one of sixteen has it to itself.
+// Rows resident: from 65,537 plans on.  Rows in windows: from what the kernel of small batches leaves.
 // Measured, us per launch, ace_many.h -> here:
 //   plans      315 ops           523 ops           821 ops, no resharding   1,251 ops, 16 stages
 //   65,537     64.2 ->  58.9     130.1 -> 117.5    134.7 -> 113.9           285.1 -> 235.2
@@ -13,6 +13,9 @@
 //   (523 ops, 1,048,576 plans, all of one stage: 447 -> 357, all of sixteen: 1,456 -> 981)
 //   windowed rows: 134 ops, 7,681 plans 45.7 -> 32.6, 65,536 55.4 -> 41.1, 131,072 63.7 -> 48.0, 262,144 92.6 -> 72.9, 300,000 132.7 -> 99.9;
 //   230 ops, 262,144 plans 121.7 -> 88.0; 270 ops in 270 types (the C++ loop before), 100,000 plans 455.8 -> 66.0, 500,000 475.8 -> 196.6
+//   tables of more than 80 KB (all of a CU for one workgroup), in windows or as the table compiler's rows before: 523 ops with 80 entries per
+//   row 100,000 plans 123.1 -> 106.8, 262,144 195.2 -> 164.4; 1,251 ops, all sizes of the database different, 262,144 461.8 -> 388.7; 821 ops with
+//   44 entries 181.6 -> 163.3 (ace_duo.h: 8,192 plans 89.5 -> 52.6, 235.7 -> 87.8, 85.0 -> 68.5; 65,536 115.8 -> 84.1, 255.4 -> 172.3, 111.0 -> 93.6)
 // What bounds it is the issue of vector instructions: about 30 per op and wavefront of the mix of depths (35 before), and the issue
 // of everything else beside them; with fewer than four wavefronts per SIMD the latency of a step.  One workgroup of 1,024 lanes per
 // CU instead: 594 us where two of 512 took 567.
@@ -36,8 +39,7 @@
 // With two algorithms and four tp sizes most codes in use are even, and diags four apart lie 32 entries apart: from the fourth on
 // they lie one entry further, so that their even codes read different banks.  Blocks of a slab are 132 bytes apart for the same reason.
 // Rows that do not all fit go through windows (as many ops as the rows of half the space behind the rest serve, a multiple of four),
-// consecutive windows in alternate halves, fetched by the loop itself; everything else stays resident.  (Sixteen rows of 80 entries, which a
-// half holds: two windows.  44 of twelve ops, with rows of 120 entries: 8,192 plans of 523 ops 90.2 -> 81.3 us, 262,144 194.8 -> 168.6.)
+// consecutive windows in alternate halves, fetched by the loop itself; everything else stays resident.
 // What a code byte reads that names no profiled entry (codes past the last tp size) is what it reads in the table compiler's
 // rows: the tables are filled by those addresses.
 #pragma once
@@ -51,8 +53,9 @@
 
 constexpr uint32_t kDenseLds = 80u * 1024u;    // LDS of a workgroup: two per CU
 constexpr int kDenseLanes = 512;
-// ... windowed rows: one per CU, so that a window holds more ops (134 ops, two workgroups of 512 lanes per CU with windows of 8 ops against
-// one of 1,024 with 20: 65,536 plans 44.9 / 41.1 us, 262,144 69.4 / 72.9, 300,000 104.6 / 99.9)
+// ... one per CU: tables of more than that, up to all of a CU's LDS, and windowed rows, so that a window holds more ops (134 ops, two
+// workgroups of 512 lanes per CU with windows of 8 ops against one of 1,024 with 20: 65,536 plans 44.9 / 41.1 us, 262,144 69.4 / 72.9,
+// 300,000 104.6 / 99.9)
 constexpr uint32_t kDenseWinLds = 160u * 1024u;
 constexpr int kDenseWinLanes = 1024;
 constexpr uint32_t kDenseEntry = 40u, kDenseValue = 8u;          // bytes of an entry; from one of its values to the next
@@ -82,11 +85,16 @@ struct AceDenseTables {
     uint32_t row_pitch = 0, rows_off = 0;
     AceDenseArgs args{};        // (offsets)
     uint32_t array = kDenseValue, lds = 0;
+    int lanes = 0;              // of a workgroup of large batches
     bool ok = false;
 };
 
 // LDS behind the image: the deal's bins and permutation, and the arrival counters; windowed, the rows lie there afterwards.
 inline uint32_t ace_dense_scratch(int lanes) { return 128u + 2u * (uint32_t)lanes + 128u; }
+// ... that of the kernel of mid-sized batches (ace_duo.h), whose workgroup of L plans has a CU to itself: bins, permutation, the parts'
+// stage counts.
+constexpr int kDuoBlock = 1024;     // its lanes: eight wavefronts per role
+inline uint32_t ace_duo_scratch(int L) { return 128u + 2u * (uint32_t)L + 2u * (uint32_t)kDuoBlock; }
 
 // Fills `d` (d.ok false: the tables do not fit this form).  `lds`: how much of it a workgroup may take, `scratch`: what of that is for
 // the kernel's own use (windowed: before the first rows arrive); `lanes`: of a workgroup that fetches windows.
@@ -275,18 +283,17 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     d.lds = bytes + (windowed ? std::max(2u * g.half, scratch) : scratch);
     if (d.lds > lds) return;
     d.row_pitch = row_pitch;
+    d.lanes = lanes;
     d.rows_off = rows_off;
     g.image16 = bytes / 16u;
-    // windows: a multiple of four ops each (or up to the last op), of at most `slots` different rows; two of them where one half
-    // holds every row
+    // windows: a multiple of four ops each (or up to the last op), of at most `slots` different rows
     std::vector<uint32_t> place(N, 0u);                             // of each position's row, from the first one (of its half) on
     if (windowed) {
-        const int longest = used.size() <= slots ? (N / 2 + 3) & ~3 : N;
         for (int i = 0; i < N;) {
             std::vector<uint32_t> seen;
             size_t good_n = 0;
             int good = -1;
-            for (int j = i; j < N && j < i + longest;) {
+            for (int j = i; j < N;) {
                 const uint32_t r = (uint32_t)row_of[types[j]];
                 if (std::find(seen.begin(), seen.end(), r) == seen.end()) {
                     if (seen.size() >= slots) break;
@@ -371,9 +378,10 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     d.ok = true;
 }
 
-// Every row resident if they fit beside a second workgroup on the CU, else in windows.
+// Every row resident where they fit: beside a second workgroup on the CU, else in all of its LDS; windows for more than that.
 inline void ace_dense_build(const ace_tables_t *t, size_t pos_entries, AceDenseTables &d) {
     dense_build(t, pos_entries, false, kDenseLds, ace_dense_scratch(kDenseLanes), kDenseLanes, d);
+    if (!d.ok) dense_build(t, pos_entries, false, kDenseWinLds, std::max(ace_dense_scratch(kDenseWinLanes), ace_duo_scratch(256)), kDenseWinLanes, d);
     if (!d.ok) dense_build(t, pos_entries, true, kDenseWinLds, ace_dense_scratch(kDenseWinLanes), kDenseWinLanes, d);
 }
 
@@ -532,7 +540,7 @@ ACE_HD void dense_replay(const AceDenseArgs &d, const AceGeom &g, const AceLds &
 
 // The op loop: returns the number of stages of the lane's plan, and in `stored` that of the wavefront's records; `ws`: the
 // wavefront's part of the workspace.
-template <bool WIN>
+template <bool WIN, int LANES>
 __device__ __forceinline__ uint32_t dense_loop(const AceKernelArgs &a, const AceDenseArgs &d, uint64_t glogs, uint32_t lut2, uint64_t zvrk, uint32_t code_off,
                                                const unsigned char *ws, uint32_t lane, uint32_t meta0, uint32_t pace, uint32_t prio, uint32_t wave, uint32_t &stored) {
     uint32_t placed;
@@ -544,7 +552,7 @@ __device__ __forceinline__ uint32_t dense_loop(const AceKernelArgs &a, const Ace
                    [meta0] "v"(meta0), [codes] "s"(a.codes), [pos] "s"(d.pos), [n_ops] "s"(a.g.N), [recbase] "s"(ws),            \
                    [gstride_lo] "s"(gs_lo), [gstride_hi] "s"(gs_hi), [kv] "s"(d.kv), __VA_ARGS__ \
                  : ACE_DENSE_ASM_CLOBBERS)
-#define ACE_DENSE_RESIDENT [pace] "s"(pace), [pacemask] "s"(1u)
+#define ACE_DENSE_RESIDENT [pace] "s"(pace), [pacemask] "s"((uint32_t)LANES / 512u)
 #define ACE_DENSE_WINDOWED [prio] "s"(prio), [dma] "s"(d.events), [eventsize] "s"((uint32_t)(kDenseWinLanes / 64) * 48u), \
                            [waveoff] "s"(wave * 48u), [half] "s"(d.half), [luthalf] "s"(d.lut_half)
     if (WIN) {
@@ -588,9 +596,10 @@ template <int LANES> __device__ __forceinline__ void dense_stage_image(const Ace
 }
 
 // One workgroup; its LDS array starts at address 0 (the kernel has no other LDS variables).
-template <bool WIN> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
+template <bool WIN, int LANES> __device__ __forceinline__ void ace_dense_body(const AceKernelArgs &a, const AceDenseArgs &d, uint32_t slices, unsigned char *lds_raw,
                                                                 int tid, long long block) {
-    constexpr int kLanes = WIN ? kDenseWinLanes : kDenseLanes;
+    constexpr int kLanes = LANES;
+    static_assert(!WIN || LANES == kDenseWinLanes, "as many wavefronts as the fetch records say");
     const AceGeom &g0 = a.g;
     const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(tid >> 6), lane = (uint32_t)tid & 63u;
     const uint32_t lanes = 64u * slices;
@@ -643,7 +652,7 @@ template <bool WIN> __device__ __forceinline__ void ace_dense_body(const AceKern
     uint32_t stored;
     // (windowed rows: the deeper its plans, the higher a wavefront's issue priority)
     const uint32_t prio = (uint32_t)__builtin_amdgcn_readfirstlane((int)(3u - q * 4u / (uint32_t)(kLanes / 64)));
-    const int n_st = (int)dense_loop<WIN>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.first_in << 24),
+    const int n_st = (int)dense_loop<WIN, LANES>(a, d, st.glogs >> 1, lut, zvrk, (uint32_t)pl * 16u, ws, lane, ((first & 7u) << 8) | (d.first_in << 24),
                                              d.image16 * 16u + 128u + 2u * kLanes + (wave & 3u) * 32u, prio, wave, stored);
     dense_replay(d, g, lds, st, ws, lane, (uint32_t)__builtin_amdgcn_readfirstlane((int)stored), n_st);
     st.s = n_st;                                                    // (result() checks the count of the op loop)

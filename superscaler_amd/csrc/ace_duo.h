@@ -36,9 +36,6 @@ inline int ace_duo_lanes(long long plans) {
         if (plans <= 256ll * L) return L;
     return 0;
 }
-constexpr int kDuoBlock = 1024;     // lanes of a workgroup: eight wavefronts per role
-// LDS of the workgroup behind the tables: the bins of the plans' deal, its permutation and the parts' stage counts.
-inline uint32_t ace_duo_scratch(int L) { return 128u + 2u * (uint32_t)L + 2u * (uint32_t)kDuoBlock; }
 
 #ifndef ACE_HOST_EMU
 #include "ace_duo_loop_asm.inc"

@@ -109,10 +109,10 @@ template <bool WIN> __global__ __launch_bounds__(1024) void ace_many_kernel(cons
     ace_many_body<WIN>(a, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 // ... over dense tables, see ace_dense.h.
-template <bool WIN> __global__ __launch_bounds__(WIN ? kDenseWinLanes : kDenseLanes, 4)
+template <bool WIN, int LANES> __global__ __launch_bounds__(LANES, 4)
 void ace_dense_kernel(const AceKernelArgs a, const AceDenseArgs d, const uint32_t slices) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
-    ace_dense_body<WIN>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
+    ace_dense_body<WIN, LANES>(a, d, slices, lds_raw, (int)threadIdx.x, (long long)blockIdx.x);
 }
 template <bool COLL> __global__ __launch_bounds__(kRcLanes, 6) void ace_rc_kernel(const RcArgs a, const long long first) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
@@ -759,6 +759,7 @@ struct ace_handle {
     uint32_t lds_bytes_wa;
     AceDenseArgs dense;        // tables of ace_dense.h (device addresses; image null: they do not fit that form)
     uint32_t dense_lds;
+    int dense_lanes;           // of a workgroup of large batches
     unsigned char *d_dense_rows;   // ... windowed: the rows
     uint8_t *d_pair_kinds;
     uint32_t *d_stage_lut;
@@ -888,8 +889,9 @@ template <bool WIN> static int allow_many_lds() {
 }
 
 static int allow_dense_lds() {
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
-    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseWinLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<false, kDenseLanes>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<false, kDenseWinLanes>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseWinLds));
+    ACE_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&ace_dense_kernel<true, kDenseWinLanes>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDenseWinLds));
     return ACE_OK;
 }
 
@@ -1070,6 +1072,7 @@ static int setup_dense(ace_handle *h, const ace_tables_t *t, size_t pos_entries)
     }
     if (rc != ACE_OK) return rc;
     h->dense_lds = d.lds;
+    h->dense_lanes = d.lanes;
     return ACE_OK;
 }
 
@@ -1334,12 +1337,11 @@ static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream
 // ... over dense tables (ace_dense.h and the table above kSpreadMaxPlain have both sides measured).
 static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
     if (!h->dense.image || a.range || a.stage_out || !a.stage_ws) return false;
-    const bool win = h->dense.events != nullptr;
-    const uint32_t slices = win ? ace_dense_slices(a.g.P, kDenseWinLanes / 64, 256) : ace_dense_slices(a.g.P, kDenseLanes / 64, 512), lanes = 64u * slices;
+    const uint32_t slices = ace_dense_slices(a.g.P, h->dense_lanes / 64, 256 * (kDenseWinLanes / h->dense_lanes)), lanes = 64u * slices;
     const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
     if (a.stage_ws != h->d_stage_ws || groups * lanes > h->stage_ws_plans) return false;    // (the static scratch holds no such records)
-    if (win) hipLaunchKernelGGL(ace_dense_kernel<true>, dim3((unsigned)groups), dim3(kDenseWinLanes), h->dense_lds, s, a, h->dense, slices);
-    else hipLaunchKernelGGL(ace_dense_kernel<false>, dim3((unsigned)groups), dim3(kDenseLanes), h->dense_lds, s, a, h->dense, slices);
+    const auto kernel = h->dense.events ? ace_dense_kernel<true, kDenseWinLanes> : h->dense_lanes == kDenseWinLanes ? ace_dense_kernel<false, kDenseWinLanes> : ace_dense_kernel<false, kDenseLanes>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3((unsigned)h->dense_lanes), h->dense_lds, s, a, h->dense, slices);
     return true;
 }
 static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {

@@ -11,8 +11,9 @@ import pytest
 
 from superscaler_amd import synth
 from superscaler_amd.plan import PlanBatch
+from superscaler_amd.tables import compile_tables
 from tests.helpers import c_oracle_scores, emu_dense_score, emu_lib
-from tests.test_small_batches import tables_for, with_recompute
+from tests.test_small_batches import with_recompute
 
 
 def workload(name, sizes, per_node=None, gpus=None):
@@ -29,6 +30,33 @@ SHAPES = {"t5, 6 sizes": ("t5_770m", 6), "t5, 8 sizes": ("t5_770m", 8), "t5, 2 o
           "conv, 1 of 2": ("wresnet_1b", 1, 2, 4), "conv, 6 sizes": ("wresnet_1b", 6)}
 
 
+#: ... over databases in which no two sizes and no two collectives' times are equal: large images
+DISTINCT = {"t5, all sizes differ": ("t5_770m", 5), "t5, 8 differing": ("t5_770m", 8), "gpt, all sizes differ": ("gpt3_175b", 4), "gpt, 8 differing": ("gpt3_1_3b", 8),
+            "gpt, 6 differing": ("gpt3_13b", 6)}
+SHAPES.update(DISTINCT)
+
+
+def distinct_sizes(db, seed):
+    """Every input and output size, and every collective's time, a value of its own."""
+    rng = np.random.default_rng(seed)
+    for key in ("input_size", "output_size"):
+        a = db.tables[key]
+        db.tables[key] = np.round(a * rng.uniform(0.7, 1.3, a.shape) + rng.uniform(0, 1, a.shape), 3)
+    keys = sorted({"{:.0f}".format(float(x)) for x in db.tables["input_size"].ravel()}, key=float)
+    for groups in db.collectives.values():
+        for n in groups:
+            groups[n] = {k: round(float(rng.uniform(0.1, 2.0)) * (1 + float(k) * 0.01), 3) for k in keys}
+    return db
+
+
+def tables_of(shape, **settings):
+    """(workload, its compiled tables)"""
+    w = workload(*SHAPES[shape])
+    graph = synth.make_graph(w)
+    db = synth.make_db(w, graph)
+    return w, compile_tables(graph, distinct_sizes(db, 1) if shape in DISTINCT else db, dataclasses.replace(synth.make_settings(w), **settings))
+
+
 def shape_of(tables):
     """(fits, windows, LDS of a workgroup, bytes of the image, from row to row, most rows of a window)"""
     out = np.zeros(6, dtype=np.int32)
@@ -39,30 +67,34 @@ def shape_of(tables):
 
 @pytest.mark.parametrize("shape", SHAPES)
 def test_rows_take_what_their_entries_need(shape):
-    tables = tables_for(workload(*SHAPES[shape]))
+    w, tables = tables_of(shape)
     ok, windows, lds, _, pitch, _ = shape_of(tables)
     entries = tables.n_diag * tables.C + 8
     # (one entry to keep banks apart; up to 255 multiples of one constant name the places of rows: of `n` rows one is a 255th of all,
     # rounded up to eight bytes, longer at most; a window's rows are fetched 1 KB at a time, in pieces of 16 bytes)
     need = 40 * (entries + 1)
-    assert ok and pitch <= max(need + 8 * (need // 255 + 2), 1024 if windows else 0)
-    assert lds <= (160 if windows else 80) * 1024
+    assert ok and pitch <= max(need + 8 * (need // 255 + 2), 1024 if windows else 0) and lds <= 160 * 1024
+
+
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s not in ("conv, 1 of 2", "conv, 6 sizes")])
+def test_rows_that_fit_a_cu_are_resident(shape):
+    """So that mid-sized batches have their kernel, whatever the table compiler's own rows need."""
+    ok, windows, *_ = shape_of(tables_of(shape)[1])
+    assert ok and windows == 0
 
 
 @pytest.mark.parametrize("shape", SHAPES)
 def test_every_shape_scores_like_the_oracle(shape):
-    w = workload(*SHAPES[shape])
-    tables = tables_for(w)
+    w, tables = tables_of(shape)
     batch = with_recompute(synth.make_plans(w, tables, n_plans=120, seed_offset=21), 0.6, 21)
     got = emu_dense_score(tables, batch)
     it, pk, fe, er = c_oracle_scores(tables, batch)
     assert np.array_equal(got[0], it) and np.array_equal(got[1], pk) and np.array_equal(got[2], fe) and not got[3].any() and not er.any()
 
 
-def on_the_gpu(shape, sizes):
+def on_the_gpu(shape, sizes, **settings):
     from superscaler_amd.evaluator import PlanEvaluator
-    w = workload(*SHAPES[shape])
-    tables = tables_for(w)
+    w, tables = tables_of(shape, **settings)
     ev = PlanEvaluator(tables)
     base = with_recompute(synth.make_plans(w, tables, n_plans=9000, seed_offset=31), 0.6, 31)
     want = c_oracle_scores(tables, base, threads=8)
@@ -80,3 +112,12 @@ def on_the_gpu(shape, sizes):
                                          ("conv, 1 of 1", (5000, 70001)), ("conv, 1 of 2", (6200, 70001)), ("conv, 6 sizes", (65536,))])
 def test_large_batches_over_other_shapes_on_the_gpu(shape, sizes):
     on_the_gpu(shape, sizes)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,sizes", [("t5, 6 sizes", (5000, 8192, 65536)), ("t5, 8 sizes", (16385,)), ("gpt, 6 sizes", (4097, 32768, 65536)), ("conv, 5 of 1", (5000, 33000)),
+                                         ("conv, 1 of 1", (16384,)), ("t5, all sizes differ", (8192, 65536)), ("t5, 8 differing", (5000, 70001)),
+                                         ("gpt, all sizes differ", (4097, 65537)), ("gpt, 8 differing", (8192, 262145)), ("gpt, 6 differing", (20000, 131073))])
+def test_mid_sized_batches_over_other_shapes_on_the_gpu(shape, sizes):
+    on_the_gpu(shape, sizes)
+    on_the_gpu(shape, sizes[:1], resharding=False, memory_pred_type="MIN")
