@@ -122,6 +122,7 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     for (int i = 0; i < N; ++i) row_of[types[i]] = 0;
     for (int ty = 0; ty < t->num_types; ++ty)
         if (row_of[ty] == 0) { row_of[ty] = (int)used.size(); used.push_back((uint32_t)ty); }
+    if (!windowed && used.size() * row_bytes > lds) return;         // (before anything that takes time: 134 rows of 72 entries 5 ms)
     // ranks of the reserved sizes: what a running maximum from 0.0 can become (0.0: rank 0)
     std::vector<double> reserved_fwd, reserved_bwd, *const values[2] = {&reserved_fwd, &reserved_bwd};
     for (int w = 0; w < 2; ++w) {
