@@ -175,7 +175,7 @@ size_t ace_pack_host(const uint8_t *codes, const uint32_t *hdr, const uint32_t *
 /* ace_score_batch for callers that cannot allocate device memory (code under HIP graph capture, tight serving
  * loops, harnesses that forbid hipMalloc): plain scoring (no d_stage_out, no batch->d_range) of at most
  * ACE_STATIC_MAX_PLANS plans, with the deferred-stage-tail records in a static device array of the library
- * (ACE_STATIC_MAX_PLANS * 1,280 bytes = 20 MiB, held by every GPU the library runs on until the process ends)
+ * (ACE_STATIC_MAX_PLANS * 1,536 bytes = 24 MiB, held by every GPU the library runs on until the process ends)
  * instead of the handle's workspace.  It calls no hipMalloc / hipFree and no allocating library routine, and
  * leaves the handle's workspace alone.  Same results as ace_score_batch, bit for bit.  Returns ACE_ETOOBIG for a
  * larger batch.  The array is shared by every call on that GPU, whichever handle or stream: calls that overlap

@@ -11,7 +11,7 @@ HEADERS = [os.path.join(HERE, "csrc", "ace_plan_state.h"), os.path.join(HERE, "c
            os.path.join(HERE, "csrc", "ace_score_loop_asm.inc"), os.path.join(HERE, "csrc", "ace_spread.h"),
            os.path.join(HERE, "csrc", "ace_recompute.h"),
            os.path.join(HERE, "csrc", "ace_duo.h"), os.path.join(HERE, "csrc", "ace_many.h"), os.path.join(HERE, "csrc", "ace_duo_loop_asm.inc"),
-           os.path.join(HERE, "csrc", "ace_dense.h"), os.path.join(HERE, "csrc", "ace_dense_loop_asm.inc"),
+           os.path.join(HERE, "csrc", "ace_dense.h"), os.path.join(HERE, "csrc", "ace_route.h"), os.path.join(HERE, "csrc", "ace_dense_loop_asm.inc"),
            os.path.join(HERE, "csrc", "ace_edit_kernels.h"), os.path.join(HERE, "csrc", "ace_grid.h"), os.path.join(HERE, "csrc", "ace_keyset.h"),
            os.path.join(HERE, "csrc", "ace_moves_host.h"), os.path.join(HERE, "csrc", "ace_pack.h"),
            os.path.join(ROOT, "include", "ace_eval.h")]

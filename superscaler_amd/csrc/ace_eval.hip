@@ -1,6 +1,6 @@
 // MI355X (gfx950) batched plan evaluator: kernels and C ABI (see include/ace_eval.h).
 //
-// Scoring, by the size of the batch (launch_score holds the rule):
+// Scoring, by the size of the batch (ace_route.h holds the rule):
 //   ace_spread.h      small batches, and most batches of stage records and single-stage queries: a plan per workgroup, its ops
 //                     over the lanes
 //   ace_duo.h         mid-sized batches, every row resident: a plan walked by several lanes
@@ -33,13 +33,16 @@
 #include "ace_duo.h"
 #include "ace_many.h"
 #include "ace_dense.h"
+#include "ace_route.h"
 #include "ace_recompute.h"
 
-// Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans (the
-// layout ace_score_body's DEFER variant uses: [workgroup][stage][lane][ACE_WS_REC]).  Every GPU the library runs on holds
+// Scratch of ace_score_batch_static: the deferred-stage-tail records of up to ACE_STATIC_MAX_PLANS plans, in the layout of whichever kernel
+// takes them (that of the dense tables is the largest).  Every GPU the library runs on holds
 // its own copy of this array until the process ends.  In host code the array's name is only a stand-in for
 // hipGetSymbolAddress(): kernels get the per-device pointer that call returned (static_scratch_ptr), never the name.
-static __device__ __align__(256) double scratch[(size_t)ACE_STATIC_MAX_PLANS * ACE_MAX_STAGES * ACE_WS_REC];
+constexpr size_t kStaticBytes = (size_t)ACE_STATIC_MAX_PLANS * kDensePlan;
+static_assert(kDensePlan >= kWsPlan, "the larger of the two");
+static __device__ __align__(256) double scratch[kStaticBytes / sizeof(double)];
 
 namespace {
 
@@ -118,25 +121,6 @@ template <bool COLL> __global__ __launch_bounds__(kRcLanes, 6) void ace_rc_kerne
     extern __shared__ __align__(16) unsigned char lds_raw[];
     ace_rc_body<COLL>(a, lds_raw, (int)threadIdx.x, first + (long long)blockIdx.x);
 }
-
-// Batches of up to this many plans take it.  Its time grows with the number of plans once every CU has six workgroups
-// (1,536 plans); that of the others, where a lane or a few walk a plan, hardly does until the chip is full, and they cross
-// where that time is reached.  That place depends on the graph: both times grow with the ops, but not alike.  A path has one
-// limit all the same, at or below the first crossing of the graphs measured for it, so a graph that crosses later has a jump
-// there.  By what else would take the batch, in us per launch at the limit and where the graph crosses (plan per workgroup / the other):
-//   PLAIN    the mid-sized kernel                    limit  4,096: 315 ops  30 / 32, crosses at  4,300 plans; 523 ops  44 /  50,  4,650;
-//                                                                  821 ops  56 / 67,  5,000; 1,251 ops  82 /  81,  4,050
-//   WINDOWED large, windowed rows (dense tables)     limit  6,144: 118 ops  29 / 30, crosses at  6,700 plans; 134 ops 31 / 33, 6,600; 182 ops 35 / 39, 7,150;
-//                                                                  230 ops  40 / 44, 7,050; 270 ops 48 / 49, 6,150
-//   SLOW     no assembly loop (memory of collectives, more than 256 rows)
-//                                                    limit 18,432: 315 ops 161 / 161, 18,400; 523 ops 238 / 459, above 24,576 (313 / 460);
-//                                                                  134 ops  97 / 140, above 24,576 (128 / 140)
-//   RECORDS  stage records                           limit 14,336: 315 ops 134 / 136, 14,500; 523 ops 199 / 316, 23,000; 134 ops 81 / 148, above 24,576
-//            single-stage queries                           14,336: 315 ops  85 / 103, 18,000; 523 ops 80 / 179, 134 ops 53 / 124, both above 24,576
-//   OTHER    the C++ loop with deferred stage tails  limit  4,096:  62 ops  18 / 41, 11,500; 134 ops  22 / 83, 20,000
-// and at one plan 8 to 26 where a lane needs 49 to 169 (13 to 20 us is what the host needs for a launch).
-constexpr int kSpreadMaxPlain = 4096, kSpreadMaxWindowed = 6144, kSpreadMaxSlow = 18432, kSpreadMaxRecords = 14336;
-constexpr int kSpreadMaxOther = 4096;    // (tables that no assembly loop walks)
 
 // ------------------------------------------------------------------------------------------
 // top-k: radix select on the order-preserving 64-bit image of the iteration time, then a
@@ -774,6 +758,7 @@ struct ace_handle {
     struct StepBuffers *step;  // of ace_search_step (null until the first call)
     double *d_stage_ws;        // grow-only workspace for deferred stage tails
     size_t stage_ws_plans;     // capacity in plans
+    AceRouteTables route;      // what the tables allow (ace_route.h)
     int stage_ws_fixed;        // ace_reserve(..., fixed): a larger batch is an error instead of a reallocation
     std::mutex host_calls;     // held by ace_score_host and ace_search_step from their first to their last use of host_in, host_out and
                                // step: the next call, of another thread, must find the transfers of the one before ended
@@ -1076,6 +1061,26 @@ static int setup_dense(ace_handle *h, const ace_tables_t *t, size_t pos_entries)
     return ACE_OK;
 }
 
+// The assembly loop over the table compiler's rows: LDS of a workgroup, or 0 where it cannot walk them.
+static uint32_t many_lds(const ace_handle_t *h) {
+    const bool win = h->n_windows > 1;
+    if (win ? !h->d_win_dma : !(h->d_pos4 && h->geom.lut2a_lds_off && h->flat_rows16 > 0)) return 0;
+    const uint32_t tables = win ? h->lds_bytes_wa : h->lds_bytes, deal = (win ? h->geom_wa : h->geom).rk_lds_off + 128u + 2u * 1024u, lds = deal > tables ? deal : tables;
+    return lds <= kMaxLds ? lds : 0;
+}
+static AceRouteTables route_tables(const ace_handle_t *h) {
+    AceRouteTables t;
+    t.ops = h->geom.N;
+    t.spread = h->d_pos_spread != nullptr;
+    t.dense = h->dense.image != nullptr;
+    t.dense_windows = h->dense.events != nullptr;
+    t.dense_lanes = h->dense_lanes;
+    t.many = many_lds(h) != 0;
+    t.many_windows = h->n_windows > 1;
+    t.deferred = (h->n_windows == 1 || h->d_pos_types) && h->geom.N < 32768 && !(h->geom.flags & ACE_F_COLLECTIVE_MEM);
+    return t;
+}
+
 // The device address of `scratch` on the current device (looked up once per device).
 static int static_scratch_ptr(double **out) {
     int dev = -1;
@@ -1223,6 +1228,7 @@ int ace_create(const ace_tables_t *t, ace_handle_t **out) {
         ace_destroy(h);
         return rc;
     }
+    h->route = route_tables(h);
     *out = h;
     return ACE_OK;
 }
@@ -1309,71 +1315,58 @@ static void launch_spread(const AceKernelArgs &a, hipStream_t s) {
     else launch_spread_c<BD, RANGED, false>(a, s);
 }
 
-// Plain scoring on tables that the assembly loops walk with every row resident: the kernels of mid-sized and large batches.
-static bool resident_asm(const ace_handle_t *h, const AceKernelArgs &a) {
-    return !a.range && !a.stage_out && a.stage_ws && h->n_windows == 1 && a.pos4 && a.g.lut2a_lds_off && a.flat_rows16 > 0;
-}
-// Workgroup size of the kernel of mid-sized batches for this call, or 0.
-static int duo_lanes(const ace_handle_t *h, const AceKernelArgs &a) {
-    return h->dense.image && !h->dense.events && !a.range && !a.stage_out && a.stage_ws ? ace_duo_lanes(a.g.P) : 0;
-}
-// The kernel of large batches (false: it cannot take this call).
-static bool launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    const bool win = h->n_windows > 1 && h->d_win_dma && a.stage_ws && !a.range && !a.stage_out;
-    if (!win && !resident_asm(h, a)) return false;
+static void launch_many(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    const bool win = h->n_windows > 1;
     AceKernelArgs b = a;
     if (win) {                                          // (that loop lays LDS out its own way)
         b.g = h->geom_wa;
         b.g.P = a.g.P; b.g.mem_limit = a.g.mem_limit; b.g.strict = a.g.strict;
     }
-    const uint32_t slices = ace_many_slices(a.g.P), lanes = 64u * slices, tables = win ? h->lds_bytes_wa : h->lds_bytes;
-    const uint32_t deal = b.g.rk_lds_off + 128u + 2u * 1024u, lds = deal > tables ? deal : tables;
-    const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes, room = a.stage_ws == h->d_stage_ws ? h->stage_ws_plans : (size_t)ACE_STATIC_MAX_PLANS;
-    if (lds > kMaxLds || groups * lanes > room) return false;
-    if (win) hipLaunchKernelGGL(ace_many_kernel<true>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
-    else hipLaunchKernelGGL(ace_many_kernel<false>, dim3((unsigned)groups), dim3(1024), lds, s, b, slices);
-    return true;
+    const AceShares w = ace_many_shares(a.g.P);
+    hipLaunchKernelGGL(win ? ace_many_kernel<true> : ace_many_kernel<false>, dim3((unsigned)w.groups), dim3(1024), many_lds(h), s, b, w.slices);
 }
-// ... over dense tables (ace_dense.h and the table above kSpreadMaxPlain have both sides measured).
-static bool launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    if (!h->dense.image || a.range || a.stage_out || !a.stage_ws) return false;
-    const uint32_t slices = ace_dense_slices(a.g.P, h->dense_lanes / 64, 256 * (kDenseWinLanes / h->dense_lanes)), lanes = 64u * slices;
-    const size_t groups = ((size_t)a.g.P + lanes - 1) / lanes;
-    if (a.stage_ws != h->d_stage_ws || groups * lanes > h->stage_ws_plans) return false;    // (the static scratch holds no such records)
+static void launch_dense(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    const AceShares w = ace_dense_shares(h->route, a.g.P);
     const auto kernel = h->dense.events ? ace_dense_kernel<true, kDenseWinLanes> : h->dense_lanes == kDenseWinLanes ? ace_dense_kernel<false, kDenseWinLanes> : ace_dense_kernel<false, kDenseLanes>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)groups), dim3((unsigned)h->dense_lanes), h->dense_lds, s, a, h->dense, slices);
-    return true;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)w.groups), dim3((unsigned)h->dense_lanes), h->dense_lds, s, a, h->dense, w.slices);
 }
-static void launch_duo(int L, const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+static void launch_duo(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
+    const int L = ace_duo_lanes(a.g.P);
     const dim3 groups((unsigned)((a.g.P + L - 1) / L));
     const uint32_t lds = h->dense.image16 * 16u + ace_duo_scratch(L);
-    if (L == 64) hipLaunchKernelGGL(ace_duo_kernel<64>, groups, dim3(kDuoBlock), lds, s, a, h->dense);
-    else if (L == 128) hipLaunchKernelGGL(ace_duo_kernel<128>, groups, dim3(kDuoBlock), lds, s, a, h->dense);
-    else hipLaunchKernelGGL(ace_duo_kernel<256>, groups, dim3(kDuoBlock), lds, s, a, h->dense);
+    const auto kernel = L == 64 ? ace_duo_kernel<64> : L == 128 ? ace_duo_kernel<128> : ace_duo_kernel<256>;
+    hipLaunchKernelGGL(kernel, groups, dim3(kDuoBlock), lds, s, a, h->dense);
 }
-static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, hipStream_t s) {
-    const int mid = duo_lanes(h, a);
-    const int most = a.stage_out ? kSpreadMaxRecords : mid ? kSpreadMaxPlain : !a.stage_ws ? kSpreadMaxSlow : h->d_win_dma || h->dense.image ? kSpreadMaxWindowed : kSpreadMaxOther;
-    if (a.pos_spread && a.g.P <= most) {
+
+// `workspace`: bytes behind a.stage_ws.
+static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, size_t workspace, hipStream_t s) {
+    switch (ace_route(h->route, a.g.P, a.stage_out != nullptr, a.stage_ws ? workspace : 0)) {
+    case ACE_K_SPREAD:
         if (a.range) launch_spread<true, true>(a, s);
         else if (a.stage_out) launch_spread<true, false>(a, s);
         else launch_spread<false, false>(a, s);
         return;
+    case ACE_K_DUO: return launch_duo(h, a, s);
+    case ACE_K_DENSE: return launch_dense(h, a, s);
+    case ACE_K_MANY: return launch_many(h, a, s);
+    case ACE_K_DEFERRED:
+        if (h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
+        else launch_score_b<false, false, false, true>(h, a, s);
+        return;
+    case ACE_K_IN_PLACE:
+        if (a.range) launch_score_w<true, true>(h, a, s);
+        else if (a.stage_out) launch_score_w<true, false>(h, a, s);
+        else launch_score_w<false, false>(h, a, s);
     }
-    if (a.range) launch_score_w<true, true>(h, a, s);
-    else if (a.stage_out) launch_score_w<true, false>(h, a, s);
-    else if (mid) launch_duo(mid, h, a, s);
-    else if (launch_dense(h, a, s) || launch_many(h, a, s)) return;
-    else if (a.stage_ws && h->n_windows > 1) launch_score_b<false, false, true, true>(h, a, s);
-    else if (a.stage_ws) launch_score_b<false, false, false, true>(h, a, s);
-    else launch_score_w<false, false>(h, a, s);
 }
+
+static size_t ws_plan(const ace_handle_t *h) { return h->route.dense ? (size_t)kDensePlan : kWsPlan; }
 
 // Plain scoring with every row resident uses the deferred-stage-tail kernel, which needs a
 // per-plan workspace; the handle keeps one and grows it on demand.
 static int ensure_stage_ws(ace_handle_t *h, AceKernelArgs *a) {
     a->stage_ws = nullptr;
-    if (a->range || a->stage_out || (h->n_windows > 1 && !h->d_pos_types && !h->dense.image) || h->geom.N >= 32768 || (h->geom.flags & ACE_F_COLLECTIVE_MEM)) return ACE_OK;
+    if (a->range || a->stage_out || !(h->route.dense || h->route.deferred)) return ACE_OK;
     // (a block more: the kernel of large batches rounds the share of every CU up)
     const size_t need = (((size_t)a->g.P + kBlock - 1) / kBlock + 1) * kBlock;
     if (need * ACE_MAX_STAGES * (ACE_WS_REC / 2) > 0xffffffffull) return ACE_OK;   // (a workspace of 64 GiB and more: such batches take the plain kernel)
@@ -1382,7 +1375,7 @@ static int ensure_stage_ws(ace_handle_t *h, AceKernelArgs *a) {
         if (h->d_stage_ws) ACE_HIP(hipFree(h->d_stage_ws));
         h->d_stage_ws = nullptr;
         h->stage_ws_plans = 0;
-        ACE_HIP(hipMalloc((void **)&h->d_stage_ws, need * (h->dense.image ? (size_t)kDensePlan : ACE_MAX_STAGES * ACE_WS_REC * sizeof(double))));
+        ACE_HIP(hipMalloc((void **)&h->d_stage_ws, need * ws_plan(h)));
         h->stage_ws_plans = need;
     }
     a->stage_ws = h->d_stage_ws;
@@ -1415,7 +1408,7 @@ int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_lim
     if (rc) return rc;
     std::lock_guard<std::mutex> lock(h->workspace);
     if ((rc = ensure_stage_ws(h, &a))) return rc;
-    launch_score(h, a, (hipStream_t)stream);
+    launch_score(h, a, h->stage_ws_plans * ws_plan(h), (hipStream_t)stream);
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1488,12 +1481,11 @@ int ace_score_batch_static(ace_handle_t *h, const ace_batch_t *batch, double mem
     if (rc) return rc;
     int dev = -1;
     if (hipGetDevice(&dev) != hipSuccess || dev != h->device || dev < 0 || dev >= kMaxDevices) return ACE_EINVAL;
-    // (the same test as ensure_stage_ws: tables that take the kernels without deferred stage tails need no scratch)
-    const bool deferred = !((h->n_windows > 1 && !h->d_pos_types) || h->geom.N >= 32768 || (h->geom.flags & ACE_F_COLLECTIVE_MEM));
-    // looked up by ace_create on this device; the padded plan count of either workgroup size fits: ACE_STATIC_MAX_PLANS is a multiple of kBlock
+    // (tables that take the kernels without deferred stage tails need no scratch; it was looked up by ace_create on this device)
+    const bool deferred = h->route.dense || h->route.deferred;
     a.stage_ws = deferred ? g_static_ptr[dev] : nullptr;
     if (deferred && !a.stage_ws) return ACE_EINVAL;
-    launch_score(h, a, (hipStream_t)stream);
+    launch_score(h, a, kStaticBytes, (hipStream_t)stream);
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1511,7 +1503,7 @@ int ace_time_score_kernel(ace_handle_t *h, const ace_batch_t *batch, double memo
     ACE_HIP(hipEventCreate(&e0));
     ACE_HIP(hipEventCreate(&e1));
     ACE_HIP(hipEventRecord(e0, s));
-    for (int r = 0; r < reps; ++r) launch_score(h, a, s);
+    for (int r = 0; r < reps; ++r) launch_score(h, a, h->stage_ws_plans * ws_plan(h), s);
     ACE_HIP(hipEventRecord(e1, s));
     ACE_HIP(hipEventSynchronize(e1));
     float ms = 0.f;

@@ -8,6 +8,7 @@
 #include "ace_grid.h"
 #include "ace_score_loop.h"
 #include "ace_dense.h"
+#include "ace_route.h"
 #include "ace_spread.h"
 #include "ace_recompute.h"
 #include "ace_pack.h"
@@ -225,6 +226,23 @@ extern "C" void ace_emu_dense_shape(const ace_tables_t *t, int32_t *out /* [6] *
     for (const auto &w : d.windows) most = std::max(most, w.size());
     const int32_t v[6] = {d.ok, (int32_t)d.windows.size(), (int32_t)d.lds, (int32_t)d.image.size(), (int32_t)d.row_pitch, (int32_t)most};
     memcpy(out, v, sizeof(v));
+}
+
+// Which kernel a batch takes (AceKernelId).  `other`: what the table compiler's rows allow beside the dense tables (1: the assembly loop, 2: the
+// C++ loop with deferred stage tails, 3: both), which the library finds out as it lays its own tables out.
+extern "C" int ace_emu_route(const ace_tables_t *t, long long plans, int records, int other, size_t workspace) {
+    AceDenseTables d;
+    ace_dense_build(t, (size_t)((t->num_ops + 15) / 16) * 16 + 16, d);
+    AceRouteTables r{};
+    r.ops = t->num_ops;
+    r.spread = true;
+    r.dense = d.ok;
+    r.dense_windows = !d.windows.empty();
+    r.dense_lanes = d.lanes;
+    r.many = other & 1;
+    r.many_windows = t->n_windows > 1;
+    r.deferred = other & 2;
+    return ace_route(r, plans, records != 0, workspace);
 }
 
 // ------------------------------------------------------------------------------------------

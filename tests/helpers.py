@@ -55,7 +55,7 @@ def emu_lib():
     if _emu is None:
         so = os.path.join(ROOT, "tests", "emu", "libace_emu.so")
         src = os.path.join(ROOT, "tests", "emu", "ace_emu.cpp")
-        hdrs = [os.path.join(ROOT, "superscaler_amd", "csrc", h) for h in ("ace_plan_state.h", "ace_score_loop.h", "ace_spread.h", "ace_recompute.h", "ace_pack.h", "ace_grid.h", "ace_dense.h")]
+        hdrs = [os.path.join(ROOT, "superscaler_amd", "csrc", h) for h in ("ace_plan_state.h", "ace_score_loop.h", "ace_spread.h", "ace_recompute.h", "ace_pack.h", "ace_grid.h", "ace_dense.h", "ace_duo.h", "ace_many.h", "ace_route.h")]
         if (not os.path.exists(so)) or os.path.getmtime(so) < max(os.path.getmtime(f) for f in [src] + hdrs):
             subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-shared", "-fPIC",
                             "-I" + os.path.join(ROOT, "include"), "-I" + os.path.join(ROOT, "superscaler_amd", "csrc"),

@@ -1,0 +1,37 @@
+"""Which kernel scores a batch (superscaler_amd/csrc/ace_route.h): the rule as the library has it, walked on the CPU."""
+import ctypes
+
+import pytest
+
+from superscaler_amd import synth
+from tests.helpers import emu_lib
+from tests.test_small_batches import tables_for
+from tests.test_table_shapes import SHAPES, tables_of
+
+SPREAD, DUO, DENSE, MANY, DEFERRED, IN_PLACE = range(6)
+#: what the table compiler's rows allow beside the dense tables
+LOOP, DEFER = 1, 2
+STATIC = 16384 * 1536           # bytes of the library's own scratch
+
+
+def route(tables, plans, records=False, other=LOOP | DEFER, workspace=1 << 40):
+    ts = tables.as_struct()
+    return emu_lib().ace_emu_route(ctypes.byref(ts), ctypes.c_longlong(plans), int(records), other, ctypes.c_size_t(workspace))
+
+
+@pytest.mark.parametrize("name", [*synth.WORKLOADS, *SHAPES])
+def test_the_static_scratch_holds_what_any_kernel_stores(name):
+    """ace_score_batch_static takes the kernel that ace_score_batch takes."""
+    tables = tables_of(name)[1] if name in SHAPES else tables_for(synth.WORKLOADS[name])
+    for plans in (1, 4096, 4097, 6144, 6145, 7680, 9216, 9217, 16383, 16384):
+        assert route(tables, plans, workspace=STATIC) == route(tables, plans), plans
+
+
+@pytest.mark.parametrize("name,largest", [("t5, 6 sizes", DENSE), ("gpt, 6 sizes", DENSE), ("gpt, all sizes differ", DENSE), ("conv, 6 sizes", DENSE)])
+def test_every_size_has_its_kernel(name, largest):
+    tables = tables_of(name)[1]
+    mid = DENSE if name == "conv, 6 sizes" else DUO
+    assert [route(tables, n) for n in (1, 4096, 16384, 65536, 65537, 1 << 20)] == [SPREAD, SPREAD, mid, mid, largest, largest]
+    assert route(tables, 14336, records=True) == SPREAD and route(tables, 14337, records=True) == IN_PLACE
+    # without a workspace: tables whose stage tails are not deferred
+    assert route(tables, 18432, workspace=0) == SPREAD and route(tables, 18433, workspace=0) == IN_PLACE

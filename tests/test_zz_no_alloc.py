@@ -36,7 +36,9 @@ def _raw_scores(ev, torch, entry, d, limit):
     return [t.cpu().numpy() for t in outs]
 
 
-@pytest.mark.parametrize("name,sizes", [("gpt3_13b", (16384, 5000)), ("gpt3_1_3b", (3000, 64)), ("wresnet_1b", (2048, 700))])
+@pytest.mark.parametrize("name,sizes", [("gpt3_13b", (16384, 5000)), ("gpt3_1_3b", (3000, 64)), ("wresnet_1b", (2048, 700)),
+                                        # (rows in windows, above what the kernel of small batches takes)
+                                        ("wresnet_1b", (16384, 7000))])
 def test_static_entry_point_equals_score_batch(name, sizes):
     import torch
     from superscaler_amd.evaluator import PlanEvaluator
