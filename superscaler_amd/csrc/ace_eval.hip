@@ -757,7 +757,7 @@ struct ace_handle {
     unsigned char *host_in, *host_out;   // page-locked buffers of ace_score_host (null until the first call)
     struct StepBuffers *step;  // of ace_search_step (null until the first call)
     double *d_stage_ws;        // grow-only workspace for deferred stage tails
-    size_t stage_ws_plans;     // capacity in plans
+    size_t stage_ws_plans, stage_ws_bytes;     // the most plans it was asked for, its size
     AceRouteTables route;      // what the tables allow (ace_route.h)
     int stage_ws_fixed;        // ace_reserve(..., fixed): a larger batch is an error instead of a reallocation
     std::mutex host_calls;     // held by ace_score_host and ace_search_step from their first to their last use of host_in, host_out and
@@ -1360,23 +1360,21 @@ static void launch_score(const ace_handle_t *h, const AceKernelArgs &a, size_t w
     }
 }
 
-static size_t ws_plan(const ace_handle_t *h) { return h->route.dense ? (size_t)kDensePlan : kWsPlan; }
-
-// Plain scoring with every row resident uses the deferred-stage-tail kernel, which needs a
-// per-plan workspace; the handle keeps one and grows it on demand.
+// Plain scoring defers its stage tails to a per-plan workspace; the handle keeps one and grows it on demand.
 static int ensure_stage_ws(ace_handle_t *h, AceKernelArgs *a) {
     a->stage_ws = nullptr;
-    if (a->range || a->stage_out || !(h->route.dense || h->route.deferred)) return ACE_OK;
-    // (a block more: the kernel of large batches rounds the share of every CU up)
-    const size_t need = (((size_t)a->g.P + kBlock - 1) / kBlock + 1) * kBlock;
-    if (need * ACE_MAX_STAGES * (ACE_WS_REC / 2) > 0xffffffffull) return ACE_OK;   // (a workspace of 64 GiB and more: such batches take the plain kernel)
-    if (need > h->stage_ws_plans) {
+    const size_t need = a->range || a->stage_out ? 0 : ace_workspace(h->route, a->g.P), plans = ace_workspace_plans(a->g.P);
+    if (need == 0) return ACE_OK;
+    if (plans > h->stage_ws_plans) {
         if (h->stage_ws_fixed) return ACE_EFIXED;
-        if (h->d_stage_ws) ACE_HIP(hipFree(h->d_stage_ws));
-        h->d_stage_ws = nullptr;
-        h->stage_ws_plans = 0;
-        ACE_HIP(hipMalloc((void **)&h->d_stage_ws, need * ws_plan(h)));
-        h->stage_ws_plans = need;
+        if (need > h->stage_ws_bytes) {
+            if (h->d_stage_ws) ACE_HIP(hipFree(h->d_stage_ws));
+            h->d_stage_ws = nullptr;
+            h->stage_ws_plans = h->stage_ws_bytes = 0;
+            ACE_HIP(hipMalloc((void **)&h->d_stage_ws, need));
+            h->stage_ws_bytes = need;
+        }
+        h->stage_ws_plans = plans;
     }
     a->stage_ws = h->d_stage_ws;
     return ACE_OK;
@@ -1408,7 +1406,7 @@ int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_lim
     if (rc) return rc;
     std::lock_guard<std::mutex> lock(h->workspace);
     if ((rc = ensure_stage_ws(h, &a))) return rc;
-    launch_score(h, a, h->stage_ws_plans * ws_plan(h), (hipStream_t)stream);
+    launch_score(h, a, h->stage_ws_bytes, (hipStream_t)stream);
     ACE_HIP(hipGetLastError());
     return ACE_OK;
 }
@@ -1503,7 +1501,7 @@ int ace_time_score_kernel(ace_handle_t *h, const ace_batch_t *batch, double memo
     ACE_HIP(hipEventCreate(&e0));
     ACE_HIP(hipEventCreate(&e1));
     ACE_HIP(hipEventRecord(e0, s));
-    for (int r = 0; r < reps; ++r) launch_score(h, a, h->stage_ws_plans * ws_plan(h), s);
+    for (int r = 0; r < reps; ++r) launch_score(h, a, h->stage_ws_bytes, s);
     ACE_HIP(hipEventRecord(e1, s));
     ACE_HIP(hipEventSynchronize(e1));
     float ms = 0.f;

@@ -46,6 +46,18 @@ inline AceShares ace_many_shares(long long plans) {
 
 constexpr size_t kWsPlan = (size_t)ACE_MAX_STAGES * ACE_WS_REC * sizeof(double);    // workspace bytes per plan of all kernels but the dense one (kDensePlan)
 
+// Bytes of workspace that plain scoring of so many plans asks for (0: none), at most kWsMost.  The dense tables' records are the larger
+// ones: a batch that fits only without them goes over the table compiler's rows, one that does not fit either way has its stage tails
+// evaluated where they end.
+constexpr size_t kWsMost = 64ull << 30;
+// (a block more than the plans: the kernels of large batches round the share of every CU up)
+inline size_t ace_workspace_plans(long long plans) { return ((size_t)plans + 1023) / 1024 * 1024 + 1024; }
+inline size_t ace_workspace(const AceRouteTables &t, long long plans) {
+    const size_t rounded = ace_workspace_plans(plans);
+    if (t.dense && rounded * kDensePlan <= kWsMost) return rounded * kDensePlan;
+    return t.deferred && rounded * kWsPlan <= kWsMost ? rounded * kWsPlan : 0;
+}
+
 // `records`: stage records or single-stage queries; `workspace`: how many bytes of it there are.
 inline AceKernelId ace_route(const AceRouteTables &t, long long plans, bool records, size_t workspace) {
     const bool plain = !records && workspace != 0;

@@ -230,7 +230,7 @@ extern "C" void ace_emu_dense_shape(const ace_tables_t *t, int32_t *out /* [6] *
 
 // Which kernel a batch takes (AceKernelId).  `other`: what the table compiler's rows allow beside the dense tables (1: the assembly loop, 2: the
 // C++ loop with deferred stage tails, 3: both), which the library finds out as it lays its own tables out.
-extern "C" int ace_emu_route(const ace_tables_t *t, long long plans, int records, int other, size_t workspace) {
+static AceRouteTables emu_route_tables(const ace_tables_t *t, int other) {
     AceDenseTables d;
     ace_dense_build(t, (size_t)((t->num_ops + 15) / 16) * 16 + 16, d);
     AceRouteTables r{};
@@ -242,8 +242,13 @@ extern "C" int ace_emu_route(const ace_tables_t *t, long long plans, int records
     r.many = other & 1;
     r.many_windows = t->n_windows > 1;
     r.deferred = other & 2;
-    return ace_route(r, plans, records != 0, workspace);
+    return r;
 }
+extern "C" int ace_emu_route(const ace_tables_t *t, long long plans, int records, int other, size_t workspace) {
+    return ace_route(emu_route_tables(t, other), plans, records != 0, workspace);
+}
+// ... and the bytes of workspace that the library gets for it.
+extern "C" size_t ace_emu_workspace(const ace_tables_t *t, long long plans, int other) { return ace_workspace(emu_route_tables(t, other), plans); }
 
 // ------------------------------------------------------------------------------------------
 // The kernel's own op loop (ace_score_loop.h) on the CPU, one lane per "workgroup", with every

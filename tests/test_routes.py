@@ -19,6 +19,29 @@ def route(tables, plans, records=False, other=LOOP | DEFER, workspace=1 << 40):
     return emu_lib().ace_emu_route(ctypes.byref(ts), ctypes.c_longlong(plans), int(records), other, ctypes.c_size_t(workspace))
 
 
+def workspace(tables, plans, other=LOOP | DEFER):
+    ts = tables.as_struct()
+    lib = emu_lib()
+    lib.ace_emu_workspace.restype = ctypes.c_size_t
+    return lib.ace_emu_workspace(ctypes.byref(ts), ctypes.c_longlong(plans), other)
+
+
+@pytest.mark.parametrize("name,other", [("gpt3_13b", LOOP | DEFER), ("wresnet_1b", LOOP | DEFER), ("wresnet_1b", 0)])
+def test_a_workspace_is_64_gib_at_most(name, other):
+    """Counted in the bytes that the kernel stores per plan, and every kernel has room for its own."""
+    tables, most, large = tables_for(synth.WORKLOADS[name]), 64 << 30, DENSE
+    for plans in (1, 65537, 1 << 20, 44_000_000, most // 1536 - 1024, most // 1536 - 1023, 50_000_000, most // 1280 - 1024, most // 1280 - 1023, 2 ** 31 - 1):
+        have = workspace(tables, plans, other)
+        assert have <= most
+        kernel = route(tables, plans, other=other, workspace=have)
+        if plans + 1024 <= most // 1536 // 1024 * 1024:
+            assert have >= plans * 1536 and kernel in (SPREAD, DENSE)
+        elif other and plans + 1024 <= most // 1280 // 1024 * 1024:
+            assert have >= plans * 1280 and kernel == MANY
+        else:
+            assert have == 0 and kernel == IN_PLACE
+
+
 @pytest.mark.parametrize("name", [*synth.WORKLOADS, *SHAPES])
 def test_the_static_scratch_holds_what_any_kernel_stores(name):
     """ace_score_batch_static takes the kernel that ace_score_batch takes."""
