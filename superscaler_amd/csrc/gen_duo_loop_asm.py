@@ -180,34 +180,6 @@ class Duo:
         self.o(f"s_cmp_eq_u32 {S0}, %[n_ops]")
         self.o("s_cbranch_scc1 L_exit_%=")
 
-    def sums(self, k):
-        e, x = self.E(k & 1), k & 1
-        if not self.time:
-            return [(W_, e[0]), (A_, e[1])]
-        return [(FWD, e[0]), (BWD, e[1])] + ([(RSF, self.Z(x)[1]), (RSB, self.Z(x)[2])] if self.rsh else [])
-
-    def add(self, pairs):
-        for acc, v in pairs:
-            self.o(f"v_add_f64 {acc}, {acc}, {v}")
-
-    def positions(self, k):
-        if k & 7 == 0:
-            self.o(f"s_load_dwordx16 {PBUF(((k >> 3) + 1) & 1)}, {PPTR}, {64 * ((k >> 3) + 1)}")
-
-    def segments(self, k):
-        """Memory role, exec: lanes whose ops k and k + 1 are a recompute pair: running segment, saved activations, peak."""
-        act = self.E(k & 1)[1]
-        self.o(f"v_add_f64 {RUN}, {RUN}, {act}")
-        self.o(f"s_bitcmp1_b32 {P(k)[1]}, 12")
-        self.o("s_cselect_b64 exec, exec, 0")
-        self.o(f"v_add_f64 {SAVED}, {SAVED}, {act}")
-        self.o("s_not_b64 exec, exec")
-        self.o(f"v_max_f64 {PEAK}, {PEAK}, {RUN}")
-        self.o(f"v_mov_b64 {RUN}, 0")
-        self.o("s_mov_b64 exec, -1")
-        if k & 7 == 7:
-            self.o(f"s_mov_b32 {PREVFL}, {P(k)[1]}")
-
     def step(self, k):
         j, b, x, k1 = k >> 2, k & 3, k & 1, k + 1
         e = self.E(x)
