@@ -1073,10 +1073,10 @@ static AceRouteTables route_tables(const ace_handle_t *h) {
     t.ops = h->geom.N;
     t.spread = h->d_pos_spread != nullptr;
     t.dense = h->dense.image != nullptr;
-    t.dense_windows = h->dense.events != nullptr;
+    t.dense_windows = h->dense.events ? (int32_t)h->dense.n_events - 1 : 0;
     t.dense_lanes = h->dense_lanes;
     t.many = many_lds(h) != 0;
-    t.many_windows = h->n_windows > 1;
+    t.windows = h->n_windows;
     t.deferred = (h->n_windows == 1 || h->d_pos_types) && h->geom.N < 32768 && !(h->geom.flags & ACE_F_COLLECTIVE_MEM);
     return t;
 }

@@ -237,10 +237,10 @@ static AceRouteTables emu_route_tables(const ace_tables_t *t, int other) {
     r.ops = t->num_ops;
     r.spread = true;
     r.dense = d.ok;
-    r.dense_windows = !d.windows.empty();
+    r.dense_windows = (int32_t)d.windows.size();
     r.dense_lanes = d.lanes;
     r.many = other & 1;
-    r.many_windows = t->n_windows > 1;
+    r.windows = t->n_windows;
     r.deferred = other & 2;
     return r;
 }

@@ -6,7 +6,7 @@ import pytest
 from superscaler_amd import synth
 from tests.helpers import emu_lib
 from tests.test_small_batches import tables_for
-from tests.test_table_shapes import SHAPES, tables_of
+from tests.test_table_shapes import OUTSIDE, SHAPES, tables_of
 
 SPREAD, DUO, DENSE, MANY, DEFERRED, IN_PLACE = range(6)
 #: what the table compiler's rows allow beside the dense tables
@@ -42,11 +42,11 @@ def test_a_workspace_is_64_gib_at_most(name, other):
             assert have == 0 and kernel == IN_PLACE
 
 
-@pytest.mark.parametrize("name", [*synth.WORKLOADS, *SHAPES])
+@pytest.mark.parametrize("name", [*synth.WORKLOADS, *SHAPES, *OUTSIDE])
 def test_the_static_scratch_holds_what_any_kernel_stores(name):
     """ace_score_batch_static takes the kernel that ace_score_batch takes."""
-    tables = tables_of(name)[1] if name in SHAPES else tables_for(synth.WORKLOADS[name])
-    for plans in (1, 4096, 4097, 6144, 6145, 7680, 9216, 9217, 16383, 16384):
+    tables = tables_for(synth.WORKLOADS[name]) if name in synth.WORKLOADS else tables_of(name)[1]
+    for plans in (1, 4096, 4097, 4724, 4725, 6536, 6537, 7680, 8632, 8633, 8800, 8801, 9216, 9217, 16383, 16384):
         assert route(tables, plans, workspace=STATIC) == route(tables, plans), plans
 
 
@@ -58,3 +58,17 @@ def test_every_size_has_its_kernel(name, largest):
     assert route(tables, 14336, records=True) == SPREAD and route(tables, 14337, records=True) == IN_PLACE
     # without a workspace: tables whose stage tails are not deferred
     assert route(tables, 18432, workspace=0) == SPREAD and route(tables, 18433, workspace=0) == IN_PLACE
+
+
+@pytest.mark.parametrize("name,rows,most,other", [
+    # rows in windows, over dense tables: long graphs cross later, short ones sooner
+    ("conv, 38 ops", LOOP | DEFER, 4724, DENSE), ("conv, 6 sizes", LOOP | DEFER, 6536, DENSE), ("gpt, 10 sizes, 523 ops", LOOP | DEFER, 8092, DENSE),
+    ("gpt, 10 sizes", LOOP | DEFER, 11004, DENSE),
+    # ... and the table compiler's rows, resident or not
+    ("conv, 4 of 1 differing", LOOP | DEFER, 8632, MANY), ("conv, 4 of 4 differing", LOOP | DEFER, 8800, MANY), ("gpt, 8 of 8 differing", LOOP | DEFER, 8800, MANY),
+    ("conv, 38 ops, 8 differing", LOOP | DEFER, 6824, MANY),
+    # ... and the C++ loop, slower by far
+    ("conv, 8 of 1 differing", DEFER, 15900, DEFERRED), ("conv, 4 of 1 differing", DEFER, 13400, DEFERRED), ("gpt, 8 of 8 differing", DEFER, 16384, DEFERRED)])
+def test_small_batches_end_where_the_kernel_that_takes_over_is_faster(name, rows, most, other):
+    tables = tables_of(name)[1]
+    assert route(tables, most, other=rows) == SPREAD and route(tables, most + 1, other=rows) == other == route(tables, 65537, other=rows)

@@ -16,9 +16,11 @@ from tests.helpers import c_oracle_scores, emu_dense_score, emu_lib
 from tests.test_small_batches import with_recompute
 
 
-def workload(name, sizes, per_node=None, gpus=None):
+def workload(name, sizes, per_node=None, gpus=None, blocks=None):
     w = synth.WORKLOADS[name]
     gpus = gpus or w.num_gpus
+    if blocks:
+        w = dataclasses.replace(w, resnet_blocks=blocks)
     return dataclasses.replace(w, mbs_list=[1 << i for i in range(sizes)], gpus_per_node=per_node or w.gpus_per_node, num_gpus=gpus,
                                pp_choices=[s for s in w.pp_choices if s <= gpus])
 
@@ -27,13 +29,17 @@ def workload(name, sizes, per_node=None, gpus=None):
 SHAPES = {"t5, 6 sizes": ("t5_770m", 6), "t5, 8 sizes": ("t5_770m", 8), "t5, 2 of 2": ("t5_770m", 2, 2, 8), "gpt, 6 sizes": ("gpt3_13b", 6),
           "gpt, 8 sizes": ("gpt3_1_3b", 8, 8, 32), "gpt, 7 of 4": ("gpt3_13b", 7, 4), "gpt, 8 of 2": ("gpt3_1_3b", 8, 2), "gpt, 3 of 8": ("gpt3_175b", 3, 8, 64),
           "conv, 1 of 1": ("wresnet_1b", 1, 1, 4), "conv, 3 of 1": ("wresnet_1b", 3, 1, 4), "conv, 5 of 1": ("wresnet_1b", 5, 1, 4),
-          "conv, 1 of 2": ("wresnet_1b", 1, 2, 4), "conv, 6 sizes": ("wresnet_1b", 6)}
+          "conv, 1 of 2": ("wresnet_1b", 1, 2, 4), "conv, 6 sizes": ("wresnet_1b", 6), "conv, 38 ops": ("wresnet_1b", 4, 8, None, (1, 1, 1, 1)),
+          "gpt, 10 sizes": ("gpt3_175b", 10), "gpt, 10 sizes, 523 ops": ("gpt3_13b", 10)}
 
 
 #: ... over databases in which no two sizes and no two collectives' times are equal: large images
 DISTINCT = {"t5, all sizes differ": ("t5_770m", 5), "t5, 8 differing": ("t5_770m", 8), "gpt, all sizes differ": ("gpt3_175b", 4), "gpt, 8 differing": ("gpt3_1_3b", 8),
             "gpt, 6 differing": ("gpt3_13b", 6)}
 SHAPES.update(DISTINCT)
+#: ... and that the dense form has no room for: rows resident; in windows that the assembly loop fetches; in windows of rows too short for it
+OUTSIDE = {"conv, 4 of 1 differing": ("wresnet_1b", 4, 1, 4), "conv, 4 of 4 differing": ("wresnet_1b", 4, 4), "conv, 8 of 1 differing": ("wresnet_1b", 8, 1, 4),
+           "gpt, 8 of 8 differing": ("gpt3_13b", 8, 8), "conv, 38 ops, 8 differing": ("wresnet_1b", 8, 8, None, (1, 1, 1, 1))}
 
 
 def distinct_sizes(db, seed):
@@ -51,10 +57,10 @@ def distinct_sizes(db, seed):
 
 def tables_of(shape, **settings):
     """(workload, its compiled tables)"""
-    w = workload(*SHAPES[shape])
+    w = workload(*{**SHAPES, **OUTSIDE}[shape])
     graph = synth.make_graph(w)
     db = synth.make_db(w, graph)
-    return w, compile_tables(graph, distinct_sizes(db, 1) if shape in DISTINCT else db, dataclasses.replace(synth.make_settings(w), **settings))
+    return w, compile_tables(graph, distinct_sizes(db, 1) if shape in DISTINCT or shape in OUTSIDE else db, dataclasses.replace(synth.make_settings(w), **settings))
 
 
 def shape_of(tables):
@@ -76,7 +82,7 @@ def test_rows_take_what_their_entries_need(shape):
     assert ok and pitch <= max(need + 8 * (need // 255 + 2), 1024 if windows else 0) and lds <= 160 * 1024
 
 
-@pytest.mark.parametrize("shape", [s for s in SHAPES if s not in ("conv, 1 of 2", "conv, 6 sizes")])
+@pytest.mark.parametrize("shape", [s for s in SHAPES if s not in ("conv, 1 of 2", "conv, 6 sizes", "conv, 38 ops", "gpt, 10 sizes", "gpt, 10 sizes, 523 ops")])
 def test_rows_that_fit_a_cu_are_resident(shape):
     """So that mid-sized batches have their kernel, whatever the table compiler's own rows need."""
     ok, windows, *_ = shape_of(tables_of(shape)[1])
@@ -109,7 +115,7 @@ def on_the_gpu(shape, sizes, **settings):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("shape,sizes", [("t5, 6 sizes", (70001,)), ("gpt, 6 sizes", (65537, 262145)), ("gpt, 8 sizes", (70000,)), ("t5, 2 of 2", (65537,)),
-                                         ("conv, 1 of 1", (5000, 70001)), ("conv, 1 of 2", (6200, 70001)), ("conv, 6 sizes", (65536,))])
+                                         ("conv, 1 of 1", (5000, 70001)), ("conv, 1 of 2", (6537, 70001)), ("conv, 6 sizes", (65536,))])
 def test_large_batches_over_other_shapes_on_the_gpu(shape, sizes):
     on_the_gpu(shape, sizes)
 
@@ -121,3 +127,9 @@ def test_large_batches_over_other_shapes_on_the_gpu(shape, sizes):
 def test_mid_sized_batches_over_other_shapes_on_the_gpu(shape, sizes):
     on_the_gpu(shape, sizes)
     on_the_gpu(shape, sizes[:1], resharding=False, memory_pred_type="MIN")
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,sizes", [("conv, 6 sizes", (6536, 6537)), ("conv, 38 ops", (4724, 4725)), ("gpt, 10 sizes", (11004, 11005, 65537))])
+def test_windows_on_both_sides_of_their_limit_on_the_gpu(shape, sizes):
+    on_the_gpu(shape, sizes)
