@@ -199,17 +199,20 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     // what the evaluation looks up comes first (it decides how much room the rows have)
     AceDenseArgs &g = d.args;
     // what the evaluation looks up: distinct {input MB, intra, inter} and {output intra, inter}, their place per row and entry
+    // (numbered as they come.  Tables that turn out not to fit are left as soon as that is known: with every size of a database of its
+    // own, 566 types of 72 entries, a search from the front each time and a look at the end took 530 ms, this 24)
     typedef std::vector<uint64_t> Bits;
     std::vector<Bits> values_in, values_out;
-    auto place_of = [&](std::vector<Bits> &v, uint32_t ty, size_t off, size_t n) {
+    std::map<Bits, uint32_t> in_at, out_at;
+    auto place_of = [&](std::vector<Bits> &v, std::map<Bits, uint32_t> &known, uint32_t ty, size_t off, size_t n) {
         Bits b(n);
         for (size_t k = 0; k < n; ++k) {
             const double x = at(ty, off + k);
             memcpy(&b[k], &x, 8);
         }
-        const size_t i = (size_t)(std::find(v.begin(), v.end(), b) - v.begin());
-        if (i == v.size()) v.push_back(b);
-        return (uint32_t)i;
+        const auto ins = known.insert({b, (uint32_t)v.size()});
+        if (ins.second) v.push_back(b);
+        return ins.first->second;
     };
     g.in_entries = entries;
     g.out_entries = (uint32_t)(t->n_mbs * t->n_tp + 8) * (uint32_t)t->n_algo;    // (a code past the last tp size: up to index 7)
@@ -222,12 +225,13 @@ inline void dense_build(const ace_tables_t *t, size_t pos_entries, bool windowed
     };
     for (uint32_t ty : used) {
         std::vector<uint32_t> in, out;
-        for (uint32_t e = 0; e < g.in_entries; ++e) in.push_back(place_of(values_in, ty, (size_t)t->start_off + e * 3u, 3));
-        for (uint32_t e = 0; e < g.out_entries; ++e) out.push_back(place_of(values_out, ty, (size_t)t->out_off + e * 2u, 2));
+        for (uint32_t e = 0; e < g.in_entries; ++e) in.push_back(place_of(values_in, in_at, ty, (size_t)t->start_off + e * 3u, 3));
+        for (uint32_t e = 0; e < g.out_entries; ++e) out.push_back(place_of(values_out, out_at, ty, (size_t)t->out_off + e * 2u, 2));
         in_of.push_back(list_of(in_lists, in));
         out_of.push_back(list_of(out_lists, out));
+        if (in_lists.size() > 256u || out_lists.size() > 256u) return;   // (eight bits each in a record word)
+        if (pairs.size() * 16u + values_out.size() * 16u + values_in.size() * 24u > 65536u) return;   // (16-bit LDS addresses)
     }
-    if (in_lists.size() > 256u || out_lists.size() > 256u) return;   // (eight bits each in a record word)
     // How far apart rows and slabs lie, and the constant bytes whose multiples (at most 255 of each) name their places; rows: as many as
     // `slots` (windowed: in each half, and fetched in pieces of 16 bytes, 1 KB at a time).  With resharding one constant K for both;
     // else two of the rows alone: 248 and 8, which name any place below 63 KB, or for more rows than those reach K twice.
