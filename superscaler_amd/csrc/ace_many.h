@@ -1,7 +1,7 @@
 // Scoring of LARGE batches where the assembly op loop runs: the kernel of ace_score_loop.h (a plan per lane, up to sixteen
 // wavefronts per workgroup and CU) with workgroups of as many plans as make an even share.  For tables that do not fit the dense
-// form (ace_dense.h): more distinct costs or sizes than its lists hold.  Every row resident: from 65,537 plans on.  Windowed rows:
-// whatever the kernel of small batches leaves.
+// form (ace_dense.h): more distinct costs or sizes than its lists hold.  They come here from what the kernel of small batches leaves
+// (ace_route.h): the kernel of mid-sized batches (ace_duo.h) walks dense tables alone.
 //
 // The rows fill a CU's LDS, so the workgroups of a batch run in rounds of 256, and with 1,024 plans each a batch of 200,000
 // leaves a fifth of the CUs idle and the last 37,856 plans of one of 300,000 take a second round of their own.  Here a
@@ -9,7 +9,7 @@
 // that stages once and walks several rounds, with or without a barrier between them, was slower: 1,048,576 plans of 523 ops
 // 757 / 797 us instead of 729.)  Rows that are resident are staged by LDS-direct loads; windowed rows are fetched while the
 // loop walks, by all sixteen wavefronts: those without plans do nothing else.
-// Measured, us per launch, before -> now:
+// Measured, us per launch, before -> now (tables of five graphs that the dense form has taken over since):
 //   plans      315 ops          523 ops          821 ops          1,251 ops
 //   100,000   132.4 -> 69.1    263.9 -> 136.5   272.4 -> 139.8   517.1 -> 293.0     (two rounds of 256-lane workgroups before)
 //   131,072    88.9 -> 71.2    163.4 -> 141.4   161.7 -> 142.9   422.6 -> 305.1

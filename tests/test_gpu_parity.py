@@ -276,9 +276,9 @@ def test_every_settings_combination_matches_the_c_oracle(name, torch_mod):
 
 @pytest.mark.parametrize("name", ["gpt3_1_3b", "wresnet_1b"])
 def test_large_batches_of_every_loop_variant_match_the_c_oracle(name, torch_mod):
-    """The assembly op loop has one text per (resharding on / off, reserved-memory rule, rows resident / windowed), and
-    only batches of 128 workgroups or more run it over windowed rows: each of the six settings at 131,072 + 77 plans
-    against the C oracle, every plan."""
+    """The assembly op loops have one text per (resharding on / off, rows resident / windowed), and the reserved-memory rule is in
+    their tables: each of the six settings at 131,072 + 77 plans against the C oracle, every plan.  (These tables take the loop over
+    dense tables; test_table_shapes.py has some that the dense form has no room for.)"""
     import dataclasses
     from superscaler_amd.evaluator import PlanEvaluator
     w = synth.WORKLOADS[name]

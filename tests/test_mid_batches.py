@@ -69,7 +69,7 @@ def test_mid_sized_batches_on_the_gpu(name, mode, sizes):
                                              ("t5_1layer", "noreserved", (147456, 600001)), ("gpt3_1_3b", "plain", (270000,)),
                                              ("wresnet_1b", "plain", (7680, 7681, 16385, 270001)), ("resnet_1111", "min", (8000, 70000)),
                                              ("resnet_16gpus", "noreserved", (16384, 33333)),
-                                             # (no assembly loop: windowed rows of short parts, by 256 and by 1,024 lanes)
+                                             # (windowed rows of which the table compiler's are too short to be fetched)
                                              ("resnet_2tp", "plain", (4096, 4097, 131073))])
 def test_large_batches_in_even_shares_on_the_gpu(name, mode, sizes):
     from superscaler_amd.evaluator import PlanEvaluator

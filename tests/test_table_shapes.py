@@ -13,7 +13,8 @@ import pytest
 from superscaler_amd import synth
 from superscaler_amd.plan import PlanBatch
 from superscaler_amd.tables import compile_tables
-from tests.helpers import c_oracle_scores, emu_dense_score, emu_lib
+from tests.helpers import c_oracle_scores, emu_dense_score, emu_lib, emu_score
+from tests.test_mid_batches import with_rows_in_another_order
 from tests.test_small_batches import with_recompute
 
 
@@ -149,3 +150,75 @@ def test_mid_sized_batches_over_other_shapes_on_the_gpu(shape, sizes):
 @pytest.mark.parametrize("shape,sizes", [("conv, 6 sizes", (6536, 6537)), ("conv, 38 ops", (4724, 4725)), ("gpt, 10 sizes", (11004, 11005, 65537))])
 def test_windows_on_both_sides_of_their_limit_on_the_gpu(shape, sizes):
     on_the_gpu(shape, sizes)
+
+
+def outside_on_the_gpu(shape, sizes, order=False, **settings):
+    """Tables that the dense form has no room for: every plan, malformed ones among them."""
+    from superscaler_amd.evaluator import PlanEvaluator
+    w, tables = tables_of(shape, **settings)
+    base = with_recompute(synth.make_plans(w, tables, n_plans=9000, seed_offset=33), 0.6, 33)
+    assert emu_dense_score(tables, base.slice(0, 1)) is None
+    want = c_oracle_scores(tables, base, threads=8)
+    ev = PlanEvaluator(with_rows_in_another_order(tables, 5) if order else tables)
+    rng = np.random.default_rng(6)
+    for n in sizes:
+        print(f"[case] {shape} {settings} plans={n}", flush=True)
+        pick = rng.integers(0, base.n_plans, n)
+        batch = PlanBatch(base.codes[pick], base.hdr[pick])
+        bad = [0, 1, 2, 3, n - 1, *range(64, 144)]
+        batch.codes[0, 0] &= 0xEF               # no stage start in front
+        batch.codes[1, 1:] |= 16                # a stage per op
+        batch.hdr[2, 0] = 40                    # more stages than there may be
+        batch.hdr[3, 0] |= 0xff00               # no such micro-batch size
+        batch.codes[n - 1, 1:] |= 16
+        some = rng.random(batch.codes[64:144].shape) < 0.03
+        batch.codes[64:144] ^= np.where(some, rng.choice([8, 16], some.shape), 0).astype(np.uint8)     # stage and recompute bits
+        got = [x.cpu().numpy() for x in ev.score(ev.upload(batch, validate=False))[:4]]
+        good = np.ones(n, dtype=bool)
+        good[bad] = False
+        assert (got[3][good] == 0).all() and all(np.array_equal(g[good], x[pick][good]) for g, x in zip(got, want))
+        for g, x in zip(got, emu_score(tables, PlanBatch(batch.codes[bad], batch.hdr[bad]))[:4]):
+            assert np.array_equal(g[bad], x, equal_nan=True)
+    ev.close()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape,sizes", [("conv, 4 of 1 differing", (8632, 8633, 65537, 270001)), ("conv, 4 of 4 differing", (8800, 8801, 262145)),
+                                         ("conv, 8 of 1 differing", (15900, 15901, 131073)), ("gpt, 8 of 8 differing", (8801, 70001)), ("conv, 38 ops, 8 differing", (6825,))])
+def test_tables_outside_the_dense_form_on_the_gpu(shape, sizes):
+    outside_on_the_gpu(shape, sizes)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", ["conv, 4 of 1 differing", "conv, 4 of 4 differing", "conv, 8 of 1 differing"])
+def test_every_variant_of_the_older_loops_on_the_gpu(shape):
+    """One text each per resharding on or off and rule of the reserved memory, rows resident or in windows; the C++ loop likewise."""
+    for resharding in (True, False):
+        for pred, reserved in (("MAX", True), ("MIN", True), ("MAX", False)):
+            outside_on_the_gpu(shape, (131149,), resharding=resharding, memory_pred_type=pred, consider_reserved_space=reserved)
+
+
+@pytest.mark.gpu
+def test_resident_rows_in_another_order_outside_the_dense_form_on_the_gpu():
+    """... which no assembly loop walks."""
+    outside_on_the_gpu("conv, 4 of 1 differing", (13400, 13401, 131073), order=True)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("shape", ["conv, 4 of 1 differing", "conv, 4 of 4 differing", "conv, 8 of 1 differing", "conv, 1 of 2"])
+def test_static_scratch_over_other_shapes_on_the_gpu(shape):
+    import torch
+    from superscaler_amd.evaluator import PlanEvaluator
+    from tests.test_zz_no_alloc import _raw_scores
+    w, tables = tables_of(shape)
+    base = with_recompute(synth.make_plans(w, tables, n_plans=4000, seed_offset=35), 0.6, 35)
+    want = c_oracle_scores(tables, base, threads=8)
+    ev = PlanEvaluator(tables)
+    for n in (16384, 8801):
+        print(f"[case] {shape} plans={n}", flush=True)
+        pick = np.random.default_rng(n).integers(0, base.n_plans, n)
+        d = ev.upload(PlanBatch(base.codes[pick], base.hdr[pick]))
+        for entry in ("static", "plain"):
+            got = _raw_scores(ev, torch, entry, d, float(tables.settings.memory_limit))
+            assert (got[3] == 0).all() and all(np.array_equal(g, x[pick]) for g, x in zip(got, want))
+    ev.close()
