@@ -332,6 +332,8 @@ extern "C" int ace_emu_spread(const ace_tables_t *t, const uint8_t *codes, const
 extern "C" { uint32_t ace_emu_rc_lds = 160u * 1024u; }
 // ... and whether the arguments of the launch say how many groups and wavefronts there are (0: they are left as they come)
 extern "C" { int32_t ace_emu_rc_set = 1; }
+// ... and how many wavefronts it has with that much
+extern "C" int ace_emu_rc_waves(int N, int groups) { return ace_rc_waves(N, (N + 15) / 16, groups, ace_emu_rc_lds); }
 
 // ace_recompute_batch: codes and codes_out uint8 [G][P][16], flags int32 [4] zeroed by the caller.
 extern "C" int ace_emu_recompute(const ace_tables_t *t, const uint8_t *codes, const uint32_t *hdr, long long P, double memory_limit,

@@ -60,3 +60,35 @@ def test_long_stages_on_the_gpu(name):
         print(f"[case] {name} limit={limit}", flush=True)
         cm.settings.memory_limit = ref.settings.memory_limit = limit
         assert np.array_equal(cm.update_recompute_arrays(batch).codes, update_recompute_arrays(ref, batch).codes)
+
+
+def many_types(emu=True):
+    """3,974 ops, each of a type of its own: LDS has room for one wavefront's groups."""
+    w = dataclasses.replace(WORKLOADS["wresnet_1b"], resnet_blocks=(3, 4, 486, 3), mbs_list=[1], gpus_per_node=1, num_gpus=4, pp_choices=[2, 4])
+    cm = cost_model(w, emu=emu)
+    assert len(set(cm.tables.graph.type_of_pos)) == cm.tables.graph.num_ops == 3974
+    return cm, synth.make_plans(w, cm.tables, n_plans=9, seed_offset=4)
+
+
+def test_so_many_types_take_one_wavefront():
+    lib = emu_lib()
+    assert lib.ace_emu_rc_waves(3974, 3974) == 1 and lib.ace_emu_rc_waves(3974, 40) == 2 and lib.ace_emu_rc_waves(134, 134) == 2
+    cm, batch = many_types()
+    for limit in limits(cm, batch):
+        cm.settings.memory_limit = limit
+        codes, flags = emu_recompute(cm, batch)
+        assert not flags.any() and np.array_equal(codes, update_recompute_arrays(cm, batch).codes)
+
+
+@pytest.mark.gpu
+def test_one_wavefront_on_the_gpu():
+    assert emu_lib().ace_emu_rc_waves(3974, 3974) == 1
+    (cm, batch), (ref, _) = many_types(emu=False), many_types()
+    chosen = 0
+    for limit in limits(ref, batch):
+        print(f"[case] 3974 types limit={limit}", flush=True)
+        cm.settings.memory_limit = ref.settings.memory_limit = limit
+        got = cm.update_recompute_arrays(batch).codes
+        assert np.array_equal(got, update_recompute_arrays(ref, batch).codes)
+        chosen += int((got & 8).any())
+    assert chosen and cm.evaluator._rc_ready     # (the kernel took them)
