@@ -74,10 +74,10 @@ def cpu_baseline(tables, batch, threads):
 
 
 def kernel_name(tables, n_plans):
-    """The kernel that plain scoring of a batch runs (the library's choice, launch_score in ace_eval.hip), for tables that its
-    assembly loops walk, as the configured workloads' are."""
-    windowed = tables.n_windows > 1
-    if n_plans <= (6144 if windowed else 4096):
+    """The kernel that plain scoring of a batch runs (the library's rule is ace_route.h), for the configured workloads: their dense
+    tables are resident where the table compiler's rows are, which does not hold for all tables."""
+    windowed, ops = tables.n_windows > 1, tables.graph.num_ops
+    if n_plans <= (6000 + 4 * ops if windowed else 4096):
         return "ace_spread_kernel"
     if not windowed and n_plans <= 65536:
         return "ace_duo_kernel"

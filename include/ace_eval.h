@@ -152,7 +152,8 @@ void ace_destroy(ace_handle_t *h);
  *  batch of single-stage queries (batch->d_range) one record each: double[n_plans][ACE_STAGE_REC].
  *  The records of a plan whose status is not ACE_PLAN_OK hold no particular values.
  * Plain scoring (no d_stage_out, no d_range) uses a workspace owned by the handle (1,280 or, over tables in
- * the denser form, 1,536 bytes per plan, never more than 64 GiB: a batch that would need more is scored without; allocated on first use and grown when a larger batch arrives: that call allocates, unless
+ * the denser form, 1,536 bytes per plan, never more than 64 GiB: a batch that would need more is scored
+ * without; allocated on first use and grown when a larger batch arrives: that call allocates, unless
  * ace_reserve() sized or fixed it beforehand), so scoring calls on one handle must be stream-ordered with
  * respect to each other. */
 int ace_score_batch(ace_handle_t *h, const ace_batch_t *batch, double memory_limit, int strict,

@@ -24,6 +24,10 @@
 // Up to 16,384 plans the longest wavefront is what is waited for (the memory role of the first part: 250 cycles per op while the stages
 // of its 64 plans end, 160 afterwards, for 24 instructions), from 65,536 on the SIMDs have two and more wavefronts to issue for all
 // the time.
+// Tables that are resident as the table compiler lays them out and not in the dense form have no such kernel any more: with resharding
+// one constant byte names every row, so rows of more than 63 KB together go through windows (134 types of 16 entries, 134 ops: 10,000
+// plans 31.5 -> 35.5 us, 24,576 37.4 -> 39.2, 65,536 54.8 -> 45.7) or, with more distinct sizes than the lists hold, over the table
+// compiler's rows (10,000 32.5 -> 34.8, 24,576 36.6 -> 37.7, 65,536 45.8 -> 41.0); below 8,000 the kernel of small batches has them (28 against 31).
 #pragma once
 #include "ace_dense.h"
 
