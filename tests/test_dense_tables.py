@@ -92,7 +92,7 @@ def test_dense_tables_score_like_the_oracle(name, mode):
 @pytest.mark.parametrize("name,mode,sizes", [("gpt_wide_stages", "plain", (65537, 131073, 262145)), ("t5_1tp", "min", (65600, 262144)),
                                              ("gpt_3tp", "noreserved", (70001,)), ("gpt3_1_3b", "min", (65537,)), ("t5_770m", "plain", (98304,)),
                                              # (rows in windows)
-                                             ("wresnet_1b", "min", (6145, 16385, 262145)), ("resnet_1111", "plain", (65537,)),
+                                             ("wresnet_1b", "min", (6145, 6537, 16385, 262145)), ("resnet_1111", "plain", (65537,)),
                                              ("resnet_16gpus", "noreserved", (6200,)), ("gpt_6mbs_64gpus", "plain", (70001,)), ("270 types", "plain", (20001,))])
 def test_large_batches_over_dense_tables_on_the_gpu(name, mode, sizes):
     from superscaler_amd.evaluator import PlanEvaluator
